@@ -30,73 +30,104 @@ struct alignas(16) GateDev {
 };
 static_assert(sizeof(GateDev) == 80, "GateDev layout");
 
-// Gate record of the fused level path, 48 bytes.  Fan-in 1..4: the delay of
-// an output event is one lookup in the gate's delay table (u16 entries at
-// dtab + dt_off) indexed by dt_index(): the output edge class s (1..4) and,
-// per input j, whether it has an event at this time (bit 2j) and whether
-// that event fell (bit 2j+1).  Fan-in 5..6 ("wide" gates): the table at
-// dt_off holds per-input delays instead (wide_dt_index), and the truth
-// table of 4^k entries spans 4^k / 256 consecutive 256-byte blocks from
-// block `lut`.
+// Gate record of the fused level path, 48 bytes.  The walk evaluates an event
+// with two table lookups, a truth-table byte and a delay word; `walk` names
+// the form of the two tables (WalkId) and dt_off / tt_off place them.
 struct alignas(16) GateRec {
   uint32_t in_net[6];
   uint32_t out_net;
-  uint32_t dt_off;
-  uint16_t lut;   // first 256-byte truth-table block
-  uint8_t k;
-  uint8_t pad0;
+  uint32_t dt_off;  // first word of the delay table (DevProgram::d_dtab)
+  uint16_t lut;     // first 256-byte truth-table block (two-pass path)
+  uint8_t k;        // distinct inputs, 1..6 (the reference's MAX_IN_NUM, src/simulate.cu:25)
+  uint8_t walk;     // WalkId
   uint16_t dmax;
-  uint16_t job;  // instance of a batch (SAIF window)
-  uint32_t pad1[2];
+  uint16_t job;     // instance of a batch (SAIF window)
+  uint32_t tt_off;  // first word of the truth-table bytes (DevProgram::d_ttab)
+  uint32_t edge_in; // W_EO: the input whose edge the delays depend on
 };
 static_assert(sizeof(GateRec) == 48, "GateRec layout");
 
-// Largest fan-in of the lane-parallel walk; gates above it (up to 6
-// distinct inputs, the reference's MAX_IN_NUM, src/simulate.cu:25) are
-// walked by the wide-gate kernel.
+// Largest fan-in of the two-pass path, and of the walk.
 constexpr uint32_t kTileK = 4;
 constexpr uint32_t kWideK = 6;
 
-// Delay-table entries of a gate with k inputs, and the index of one entry
-// (mask: inputs with an event; fell: the subset of them that fell).
-inline constexpr uint32_t dt_size(uint32_t k) { return 4u << (2 * k); }
-
-// Wide gates: per input j, output edge class s (1..4) and whether the
-// input's own event fell: the smallest delay among its edge-independent
-// IOPATH and the one of its edge kind (tmin, 0xFFFF: none), and the delay
-// used when it is the only input with an event (tone).
-constexpr uint32_t kWideDtSize = kWideK * 4 * 2 * 2;
-__host__ __device__ inline uint32_t wide_dt_index(uint32_t j, uint32_t s, uint32_t fell,
-                                                  uint32_t one) {
-  return (((j * 4 + (s - 1)) * 2 + fell) << 1) | one;
+// How the walk evaluates an event.  f, p: the gate's value after and before
+// the event; ev: bit j = input j has an event; fell: bit j = that event fell
+// (CheckDelay == 2); sc: output edge class 1..4; idx: packed input values,
+// 2 bits per input.
+//   W_NE1..W_NE6 (fan-in 1..6, no delay depends on an input's edge)
+//     truth byte [new idx]          f << ne_shift(k)
+//     delay word [p][f][ev]         4 d - 3 + f in bits 0..17, bit 24: f != p
+//   W_EO3, W_EO4 (fan-in 3 and 4, the delays depend on the edge of one input)
+//     truth byte [old value of that input][new idx]
+//                                   (f << 1 | fell) << kEoShift
+//     delay word [p][f][fell][ev]   as W_NE
+//   W_ED1, W_ED2 (fan-in 1 and 2, edge-dependent delays; f(X..X) = X, so that p
+//   is the function of the old values from the start on)
+//     truth byte [new idx][old idx] f | (sc - 1) << 2 | fell << 4 | (f != p) << 7
+//     delay word [ev][fell][sc - 1] 4 d - 3
+//   W_GEN (any other gate)
+//     truth byte as W_NE; delay table of half-words [half][both][sc - 1][bits]:
+//     half h covers inputs 3h..3h+2, bits = per input (has an event, fell);
+//     both = 0: the delay when only this half has events (AddDelay's
+//     single-input rule when it is one event), 1: the smallest delay of its
+//     events (0xFFFF: none) when the other half has events too.
+enum WalkId : uint8_t {
+  W_NE1 = 0, W_NE2, W_NE3, W_NE4, W_NE5, W_NE6, W_EO3, W_EO4, W_ED1, W_ED2, W_GEN, W_COUNT,
+  W_DEAD = 15  // tile of a gate whose inputs were not made (a level before it failed)
+};
+inline constexpr uint32_t ne_shift(uint32_t k) { return (k < 4 ? k : 4u) + 2; }
+constexpr uint32_t kEoShift = 5;  // bits of the truth byte below f << 1 | fell
+// words of the two tables
+__host__ __device__ inline constexpr uint32_t walk_dt_words(uint32_t id, uint32_t k) {
+  return id <= W_NE6 ? 16u << k : (id <= W_EO4 ? 32u << k : (id <= W_ED2 ? 4u << (2 * k) : 512u));
 }
-__host__ __device__ inline uint32_t dt_index(uint32_t k, uint32_t s, uint32_t mask,
-                                             uint32_t fell) {
-  uint32_t bits = 0;
-  for (uint32_t j = 0; j < k; ++j)
-    bits |= (((mask >> j) & 1u) << (2 * j)) | (((fell >> j) & 1u) << (2 * j + 1));
-  return ((s - 1) << (2 * k)) | bits;
+__host__ __device__ inline constexpr uint32_t walk_tt_words(uint32_t id, uint32_t k) {
+  const uint32_t b = id == W_EO3 || id == W_EO4   ? 4u << (2 * k)
+                     : id == W_ED1 || id == W_ED2 ? 1u << (4 * k)
+                                                  : 1u << (2 * k);
+  return (b + 15) / 16 * 4;  // whole 16-byte pieces
+}
+inline constexpr uint32_t gen_dt_index(uint32_t half, uint32_t both, uint32_t s, uint32_t bits) {
+  return ((half * 2 + both) * 4 + (s - 1)) * 64 + bits;
 }
 
-// Per-gate segmentation of one level: segment c covers the leader input's
-// events [c*stride, (c+1)*stride).
+// Stack words beside one per staged word: one per lane (a step without a
+// candidate writes the slot after the lane's last one) and one for the first
+// lane's initial entry.
+constexpr uint32_t kStackSlack = 68;
+
+// LDS of one walk workgroup, in words: the tables of the tile's gate, its
+// input ranges (range_layout), and the stacks at the end.
+__host__ __device__ inline constexpr uint32_t walk_lds_need(uint32_t id, uint32_t k, uint32_t words) {
+  return walk_dt_words(id, k) + walk_tt_words(id, k) + (words + 8 * k) + (words + kStackSlack);
+}
+
+// Per-gate tiling of one level: tile i covers the leader input's words
+// [i * lt, (i + 1) * lt).
 struct GatePlan {
-  uint32_t nseg, stride, lead, pad;
+  uint32_t lt, lead;
 };
 
-// Everything one tile of the fused level kernel needs, 128 bytes, written by
-// k_tile_desc.  Input j's range covers events [B, E) of its waveform with
-// B = L - 1 (L > 0) or 0: L = first event at or after the tile's start time,
-// E = end of the range including the look-ahead halo; in_off = pool word of
-// event B.
+// Everything one tile of the walk needs, 128 bytes, written by k_tile_desc.
+// Input j's staged range starts one word before the tile (its value before
+// the tile; the state entry for the gate's first tile) and ends with the
+// look-ahead halo, n[j] words from pool word in_hi[j] << 32 | in_lo[j]; the
+// tile's own words start at index 1 of each range.
 struct alignas(16) TileDesc {
-  uint64_t in_off[4];
-  uint32_t L[4], E[4];
-  uint32_t lutw[4];                // packed truth table words (fan-in <= 3)
-  uint32_t g, ti, nseg, stride;    // gate (index in the level), tile of the gate, segments
-  uint32_t lead, k, dt_off, lut;   // leader input, fan-in, delay table, truth table id
-  uint32_t dmax, out_net, job;
-  uint32_t out_cap;  // words of the tile's output region in the level scratch
+  uint32_t in_lo[6], n[6];
+  uint32_t in_hi[2];       // byte j: bits 32..39 of input j's pool word
+  uint32_t scr_lo, scr_hi; // first word of the tile's output region in the level scratch
+  uint32_t own;            // the tile's own words (without its halo)
+  uint32_t xend;           // index in the leader's range of the tile's end (0: the gate's last tile)
+  uint32_t meta;           // WalkId | k << 4 | leader input << 8 | first tile of its gate << 12 |
+                           // edge input << 16
+  uint32_t dt_off, tt_off;
+  uint32_t dmax, job;
+  uint32_t out_cap;        // words of the tile's output region in the level scratch
+  uint32_t g, ti;          // gate (index in the level), tile of the gate
+  uint32_t out_net;
+  uint32_t pad[5];
 };
 static_assert(sizeof(TileDesc) == 128, "TileDesc layout");
 
@@ -150,61 +181,33 @@ struct TailArgs {
   uint32_t first;            // 1 in chunk 0
 };
 
+// The walk's ticket counters, each on a cache line of its own.
+constexpr uint32_t kTickets = 4, kTicketStride = 32;
+
 // Arguments of the fused level (walk) kernel.
 struct LevelArgs {
   const TileDesc* tiles;      // per tile
   const uint32_t* pool;       // input waveforms
-  const uint16_t* dtab;       // delay tables (GateRec::dt_off)
-  const uint8_t* luts;        // full truth tables (fan-in 4)
+  const uint32_t* dtab;       // delay tables (GateRec::dt_off)
+  const uint32_t* ttab;       // truth tables (GateRec::tt_off)
   const uint64_t* ntiles;     // tiles of the level (device memory)
-  const uint64_t* scr_base;   // per gate: scratch word of its first tile's region
   uint32_t* scratch;          // tile outputs
   TileOut* tout;              // per tile
   uint32_t* ovf;              // stacks of tiles that do not fit LDS
   unsigned long long ovf_cap;
   unsigned long long* ovf_used;
-  unsigned long long* ticket;   // next tile to hand out, minus the grid size (0 per level)
+  unsigned long long* ticket;   // batches handed out by each counter (0 per level)
   unsigned long long* tiles_walked;  // [0] tiles walked, [1] of them on the HBM path (per run)
   unsigned long long* ev_count;
   unsigned int* err;
   const ChunkWin* cwin;        // SAIF bounds of this chunk per instance
-  uint32_t cap;                // LDS input capacity per tile (words)
+  uint32_t lds_words;          // LDS of a workgroup
   uint32_t prefetch;           // 1: stage the next tile before storing this one
-  uint32_t* stk;               // null: stacks in LDS; else (cap + 64) words per workgroup
   uint32_t lo_rel;             // F_k in chunk time: candidates below it only pre-empt
   uint32_t hi_rel;             // F_k+1 in chunk time (0xFFFFFFFF: last chunk): candidates
                                // at or above it belong to the next chunk and are dropped
   uint32_t first;              // 1 in chunk 0: outputs start with (0, X), f before t = 0 is X
 };
-
-// Arguments of the wide-gate kernel (gates of fan-in 5..6 of one level).
-struct WideArgs {
-  const GateRec* gates;        // the level's gates
-  const uint32_t* wide;        // program gate indices of the level's wide gates
-  uint32_t nwide;
-  uint32_t g0;                 // program index of the level's first gate
-  const uint64_t* tile_base;   // per gate of the level: its (single) tile
-  const TileDesc* tiles;
-  const uint64_t* woff;
-  const uint32_t* wlen;
-  const uint32_t* pool;
-  const uint8_t* luts;
-  const uint16_t* dtab;
-  const uint64_t* scr_base;
-  uint32_t* scratch;
-  TileOut* tout;
-  unsigned long long* ev_count;
-  unsigned int* err;
-  const ChunkWin* cwin;
-  uint32_t lo_rel, hi_rel, first;
-};
-
-// LDS bytes of one fused-level workgroup for an input capacity of `cap`
-// words: inputs (cap + 128: one sentinel per input range), stacks (cap + 64,
-// when they live in LDS), truth table (256 B), delay table (2 KiB).
-inline size_t level_lds_bytes(uint32_t cap, bool stacks_in_lds) {
-  return ((uint64_t)cap + 128 + (stacks_in_lds ? cap + 64 : 0)) * 4 + 256 + 2 * dt_size(4);
-}
 
 // Per time-segment summary written by the evaluation kernel.
 struct SegSum {

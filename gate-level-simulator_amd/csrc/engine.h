@@ -47,21 +47,16 @@ struct DevProgram {
   std::vector<uint32_t> level_start;
   std::vector<GateRec> h_grec;
   std::vector<GateDev> h_gdev;
-  std::vector<uint16_t> h_dtab;
+  std::vector<uint32_t> h_dtab;  // delay tables of the walk (GateRec::dt_off)
+  std::vector<uint32_t> h_ttab;  // truth tables of the walk (GateRec::tt_off)
   std::vector<uint8_t> h_luts;   // 256-byte blocks (a fan-in 5 / 6 table spans 4 / 16)
-  std::vector<uint32_t> h_lutp;  // 16 packed words per block
-  // wide gates (fan-in 5..6): their indices in h_grec, level by level
-  // (level l: h_wide[wide_start[l] .. wide_start[l+1]))
-  std::vector<uint32_t> h_wide;
-  std::vector<uint32_t> wide_start;
   uint32_t max_k = 0;            // largest fan-in
   // device tables (valid once is_resident(); one allocation, d_block)
   GateRec* d_grec = nullptr;
   GateDev* d_gdev = nullptr;
-  uint16_t* d_dtab = nullptr;
+  uint32_t* d_dtab = nullptr;
+  uint32_t* d_ttab = nullptr;
   uint8_t* d_luts = nullptr;
-  uint32_t* d_lutp = nullptr;
-  uint32_t* d_wide = nullptr;
   std::mutex upload_mu;
   DevProgram() = default;
   DevProgram(const DevProgram&) = delete;
@@ -202,7 +197,7 @@ class Job {
   // 1: after a plain execution, capture the whole level sequence (no host
   // round trips) into a hipGraph and replay it on later executions
   uint32_t graph = 0;
-  uint32_t stack_mode = 0;  // 0: preemption stacks in LDS, 1: per-workgroup scratch in HBM
+  uint32_t stack_mode = 0;  // hbm_stacks was asked for (the walk keeps its stacks in LDS either way)
   uint32_t pool_grow = 0;   // 1: given pool and overflow-buffer sizes are starting sizes that grow
   uint32_t keep_waves = 0;  // 1: collect every gate output's waveform on the host
   // time-chunk length in time units (fused path): 0 automatic, kNoChunks one
@@ -253,6 +248,7 @@ class Job {
   void finish_stats(const uint64_t* scal, double ms);
   void run_two_pass(std::vector<hipEvent_t>& ev_eval);
   void stop_point();
+  void size_tiles();
   void* dmalloc(size_t bytes);
   bool dev_alloc(void** p, size_t bytes);  // arena or hipMalloc; false: no room
   void dev_free(void* p);                  // arena (after the stream drains) or hipFree
@@ -280,6 +276,7 @@ class Job {
   uint32_t* d_saif_job_ = nullptr;
   unsigned long long* d_win_ = nullptr;
   uint64_t* d_scal_ = nullptr;
+  unsigned long long* d_ticket_ = nullptr;
   // per-level temporaries
   uint64_t *d_nseg_ = nullptr, *d_scr_ = nullptr, *d_segbase_ = nullptr, *d_scrbase_ = nullptr;
   uint64_t *d_outlen_ = nullptr, *d_outoff_ = nullptr, *d_part_ = nullptr;
@@ -300,7 +297,8 @@ class Job {
   uint64_t ovf_words_ = 0;
   size_t cap_ovf_ = 0;
   int level_blocks_ = 0;
-  uint32_t cap_ = 0;  // LDS input capacity per tile (words)
+  uint32_t lds_words_ = 0;  // LDS of a walk workgroup
+  uint32_t wide_words_ = 0; // words per tile of a wide gate
   std::vector<void*> owned_;
   // two-pass path: initial waveform tables
   std::vector<uint64_t> h_woff_init_;
@@ -339,8 +337,6 @@ class Job {
   uint64_t allocs_ = 0;         // device allocations made since the run started
   bool static_ = false;         // run_static(): no allocation, scratch from the static array
   bool graph_scratch_in_pool_ = false;  // captured levels keep their scratch at the pool top
-  uint32_t* d_stk_ = nullptr;
-  size_t cap_stk_ = 0;
   hipGraphExec_t gexec_ = nullptr;
   std::vector<uint64_t> graph_sig_;
   bool last_replay_ = false;

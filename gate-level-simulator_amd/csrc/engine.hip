@@ -44,12 +44,13 @@ hipError_t launch_saif_nets(const uint32_t* nets, const uint32_t* job, uint32_t 
 
 // level.hip: fused path
 hipError_t launch_plan2(const GateRec* gates, uint32_t ng, const uint32_t* wlen,
-                        uint32_t seg_target, GatePlan* plan, uint64_t* ntile, uint64_t* bound,
+                        uint32_t seg_target, uint32_t wide_words, GatePlan* plan, uint64_t* ntile, uint64_t* bound,
                         unsigned int* err, const uint32_t* tail_len, hipStream_t st);
 hipError_t launch_tile_desc(const GateRec* gates, uint32_t ng, const GatePlan* plan,
-                            const uint64_t* tile_base, const uint64_t* woff, const uint32_t* wlen,
-                            const uint32_t* pool, const uint32_t* lutp, TileDesc* tiles,
-                            const uint64_t* ntiles_dev, uint64_t ntiles, hipStream_t st);
+                            const uint64_t* tile_base, const uint64_t* scr_base,
+                            const uint64_t* woff, const uint32_t* wlen, const uint32_t* pool,
+                            TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles,
+                            unsigned long long* ticket, unsigned long long* ovf_used, hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long* p, uint64_t n, unsigned long long v, hipStream_t st);
 hipError_t launch_guard(uint64_t* scal, uint64_t tiles_cap, uint64_t scratch_cap, hipStream_t st);
 hipError_t launch_pool_guard(uint64_t* scal, uint64_t pool_words, hipStream_t st);
@@ -61,14 +62,12 @@ hipError_t launch_gate_carry(const GateRec* gates, uint32_t ng, const uint64_t* 
 hipError_t launch_add_u64(unsigned long long* dst, const unsigned long long* src, uint64_t n,
                           hipStream_t st);
 hipError_t launch_compact(const TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles_cap,
-                          const TileOut* tout, const uint32_t* tile_off, const uint64_t* scr_base,
-                          const uint32_t* scratch, const uint64_t* gate_base, uint32_t* pool,
-                          uint64_t* woff, uint32_t* wlen, const unsigned int* err,
+                          const TileOut* tout, const uint32_t* tile_off, const uint32_t* scratch,
+                          const uint64_t* gate_base, uint32_t* pool, uint64_t* woff, uint32_t* wlen, const unsigned int* err,
                           unsigned long long* saif, const ChunkWin* cwin, uint32_t count_tc,
                           const TailArgs& T, hipStream_t st);
 hipError_t launch_set_scal(uint64_t* scal, uint64_t bump, hipStream_t st);
 hipError_t launch_level(const LevelArgs& a, unsigned nblocks, hipStream_t st);
-hipError_t launch_wide(const WideArgs& a, hipStream_t st);
 // chunk.hip: time chunks
 hipError_t launch_stim_count(const uint64_t* store, const uint64_t* soff, const uint32_t* slen,
                              uint32_t ns, uint64_t lb, uint64_t ub, uint64_t* cnt, uint32_t* first,
@@ -93,17 +92,28 @@ hipError_t launch_saif_stim(const uint64_t* store, const uint64_t* soff, const u
                             const uint32_t* snet, const uint32_t* sjob, uint32_t ns,
                             unsigned long long* saif, const unsigned long long* win,
                             hipStream_t st);
-int level_max_blocks(uint32_t cap, bool stacks_in_lds);
+int level_max_blocks(uint32_t lds_words);
 
-// LDS input capacity of a fused tile: 64 segments of `seg` input events
-// plus a little halo headroom.  Tiles above it (their density varies) take
-// the HBM path; a tight capacity keeps more workgroups resident per CU,
-// which pays more than the HBM path costs (200k-cell workload: 8 instead of
-// 6 workgroups per CU, 9% faster than a 1.3x headroom).
-static uint32_t tile_cap(uint32_t seg) {
-  uint64_t c = (uint64_t)seg * 64 + 64;
-  c = (c + 63) / 64 * 64;
-  return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(c, 1024), 16384);
+// LDS of a walk workgroup for tiles of 64 * seg input words on average: those
+// words twice (inputs and stacks) and 4 KiB for the gate's tables, the halo and
+// the spread of a tile's words around their mean; at least what the largest
+// tables (fan-in 6) need and at most what a CU gives one workgroup.  A tile that
+// does not fit reads HBM (0.07% of the tiles of the 200k-cell configuration; a
+// `seg` beyond every LDS size sends all of them there).  At the default of 32
+// it is 20 KiB, eight workgroups a CU: with 24 (nine) the 200k-cell
+// configuration's walk took 108 ms instead of 101, the fixed work of a tile
+// outweighing the ninth.
+static uint32_t walk_lds_words(uint32_t seg) {
+  return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(128ull * seg + 1024, 3328), 33792);
+}
+
+// Words per tile of a wide gate: 93% of what the LDS holds beside the largest
+// tables, at most 64 * seg (or those, when they ask for tiles in HBM).
+static uint32_t wide_tile_words(uint32_t seg, uint32_t lds_words) {
+  const uint64_t want = 64ull * seg;
+  if (want > 16384) return (uint32_t)std::min<uint64_t>(want, 1u << 30);
+  const uint32_t room = (lds_words - walk_lds_need(W_NE6, 6, 0)) / 2;
+  return (uint32_t)std::min<uint64_t>(want, room * 93 / 100);
 }
 
 void hip_check(hipError_t e, const char* what) {
@@ -124,86 +134,142 @@ void hip_check(hipError_t e, const char* what) {
 static constexpr uint64_t kPoolPad = 16;
 
 // scalar slots in d_scal_
-enum { S_BUMP = 0, S_TOT_A = 1, S_TOT_B = 2, S_TOT_OUT = 3, S_EVC = 4, S_TICKET = 5,
+enum { S_BUMP = 0, S_TOT_A = 1, S_TOT_B = 2, S_TOT_OUT = 3, S_EVC = 4,
        S_OVF_USED = 6, S_ERR = 7, S_TILES = 8, S_TILES_HBM = 9, S_TAILS = 10 };
 
 static uint32_t sel_delay(uint32_t r, uint32_t f, int s) {
   return s == 1 ? r : (s == 2 ? f : (s == 3 ? std::max(r, f) : std::min(r, f)));
 }
 
-// AddDelay (src/simulate.cpp:1012-1176, asserts compiled out) folded into
-// one table per gate, indexed by dt_index(k, s, mask, fell): s = output edge
-// class (1..4), mask = inputs with an event at this time, fell = the subset
-// of those whose own edge class is "fall" (CheckDelay == 2).
+// AddDelay (src/simulate.cpp:1012-1176, asserts compiled out) of one gate, by
+// input, output edge class and input edge (fall = CheckDelay == 2):
 //   * one input with an event: with a single IOPATH record for that input the
 //     record is used whatever its edge; with several, the first record whose
-//     edge matches the input's edge (fall -> negedge, else posedge), else 1;
+//     edge matches the input's edge (fall -> negedge, else posedge), else 1
+//     (`one`);
 //   * several inputs: the minimum over every edge-independent record and
-//     every record whose edge matches its input's edge, else 1.
-static void fill_delay_table(const GateDelays& D, int k, uint16_t* tab) {
-  const uint16_t NO = kNoDelay;
-  uint32_t tmin[4][4][2], tone[4][4][2];
-  for (int j = 0; j < 4; ++j)
-    for (int s = 1; s <= 4; ++s)
-      for (int fall = 0; fall < 2; ++fall) {
-        uint32_t m = 0xFFFF, one = 1;
-        if (j < k) {
-          const uint16_t* both = D.v[j][DK_BOTH];
-          const uint16_t* kind = D.v[j][fall ? DK_NEG : DK_POS];
-          if (both[0] != NO) m = std::min(m, sel_delay(both[0], both[1], s));
-          if (kind[0] != NO) m = std::min(m, sel_delay(kind[0], kind[1], s));
-          if (D.nrec[j] == 1) {
-            for (int kd = 0; kd < 3; ++kd)
-              if (D.v[j][kd][0] != NO) one = sel_delay(D.v[j][kd][0], D.v[j][kd][1], s);
-          } else if (D.nrec[j] >= 2) {
-            one = kind[0] != NO ? sel_delay(kind[0], kind[1], s) : 1;
+//     every record whose edge matches its input's edge (`any`), else 1.
+struct DelayPick {
+  uint32_t any[kWideK][4][2], one[kWideK][4][2];
+  int k;
+  DelayPick(const GateDelays& D, int k_) : k(k_) {
+    const uint16_t NO = kNoDelay;
+    for (int j = 0; j < (int)kWideK; ++j)
+      for (int s = 1; s <= 4; ++s)
+        for (int fall = 0; fall < 2; ++fall) {
+          uint32_t m = 0xFFFF, o = 1;
+          if (j < k) {
+            const uint16_t* both = D.v[j][DK_BOTH];
+            const uint16_t* kind = D.v[j][fall ? DK_NEG : DK_POS];
+            if (both[0] != NO) m = std::min(m, sel_delay(both[0], both[1], s));
+            if (kind[0] != NO) m = std::min(m, sel_delay(kind[0], kind[1], s));
+            if (D.nrec[j] == 1) {
+              for (int kd = 0; kd < 3; ++kd)
+                if (D.v[j][kd][0] != NO) o = sel_delay(D.v[j][kd][0], D.v[j][kd][1], s);
+            } else if (D.nrec[j] >= 2) {
+              o = kind[0] != NO ? sel_delay(kind[0], kind[1], s) : 1;
+            }
           }
+          any[j][s - 1][fall] = m;
+          one[j][s - 1][fall] = o;
         }
-        tmin[j][s - 1][fall] = m;
-        tone[j][s - 1][fall] = one;
-      }
-  const uint32_t full = (1u << k) - 1;
-  for (uint32_t s = 1; s <= 4; ++s)
-    for (uint32_t mask = 0; mask <= full; ++mask)
-      for (uint32_t fell = 0; fell <= full; ++fell) {
-        uint32_t d = 1;
-        if (mask != 0 && (mask & (mask - 1)) == 0) {
-          const int j = __builtin_ctz(mask);
-          d = tone[j][s - 1][(fell >> j) & 1u];
-        } else if (mask != 0) {
-          uint32_t m = 0xFFFF;
-          for (int j = 0; j < k; ++j)
-            if ((mask >> j) & 1u) m = std::min(m, tmin[j][s - 1][(fell >> j) & 1u]);
-          d = m == 0xFFFF ? 1u : m;
-        }
-        tab[dt_index((uint32_t)k, s, mask, fell)] = (uint16_t)d;
-      }
+  }
+  // inputs whose own edge matters
+  uint32_t edge_inputs() const {
+    uint32_t m = 0;
+    for (int j = 0; j < k; ++j)
+      for (int s = 0; s < 4; ++s)
+        if (any[j][s][0] != any[j][s][1] || one[j][s][0] != one[j][s][1]) m |= 1u << j;
+    return m;
+  }
+  // mask: inputs with an event; fell: the subset of them that fell
+  uint32_t delay(uint32_t s, uint32_t mask, uint32_t fell) const {
+    if (mask == 0) return 1;
+    if ((mask & (mask - 1)) == 0) {
+      const int j = __builtin_ctz(mask);
+      return one[j][s - 1][(fell >> j) & 1u];
+    }
+    uint32_t m = 0xFFFF;
+    for (int j = 0; j < k; ++j)
+      if ((mask >> j) & 1u) m = std::min(m, any[j][s - 1][(fell >> j) & 1u]);
+    return m == 0xFFFF ? 1u : m;
+  }
+};
+
+// CheckDelay (src/simulate.cpp:1178-1201) on the codes 0=0 1=X 2=Z 3=1.
+static uint32_t edge_class_of(uint32_t p, uint32_t c) {
+  static const uint8_t T[4][4] = {{0, 1, 1, 1}, {2, 0, 3, 1}, {2, 4, 0, 1}, {2, 2, 2, 0}};
+  return T[p][c];
 }
 
-// AddDelay for gates of fan-in 5..6, the same rules as fill_delay_table
-// kept per input (a full table would hold 4 << 12 entries): tmin and tone
-// of every input, output edge class and input edge, at wide_dt_index().
-static void fill_wide_delays(const GateDelays& D, int k, uint16_t* tab) {
-  const uint16_t NO = kNoDelay;
-  for (int j = 0; j < (int)kWideK; ++j)
-    for (uint32_t s = 1; s <= 4; ++s)
-      for (uint32_t fall = 0; fall < 2; ++fall) {
-        uint32_t m = 0xFFFF, one = 1;
-        if (j < k) {
-          const uint16_t* both = D.v[j][DK_BOTH];
-          const uint16_t* kind = D.v[j][fall ? DK_NEG : DK_POS];
-          if (both[0] != NO) m = std::min(m, sel_delay(both[0], both[1], (int)s));
-          if (kind[0] != NO) m = std::min(m, sel_delay(kind[0], kind[1], (int)s));
-          if (D.nrec[j] == 1) {
-            for (int kd = 0; kd < 3; ++kd)
-              if (D.v[j][kd][0] != NO) one = sel_delay(D.v[j][kd][0], D.v[j][kd][1], (int)s);
-          } else if (D.nrec[j] >= 2) {
-            one = kind[0] != NO ? sel_delay(kind[0], kind[1], (int)s) : 1;
-          }
-        }
-        tab[wide_dt_index((uint32_t)j, s, fall, 0)] = (uint16_t)m;
-        tab[wide_dt_index((uint32_t)j, s, fall, 1)] = (uint16_t)one;
+// The delay table of one gate in its WalkId's form.
+static void fill_delays(const DelayPick& P, uint32_t id, uint32_t edge_in, uint32_t* tab) {
+  const uint32_t k = (uint32_t)P.k, full = (1u << k) - 1;
+  if (id <= W_NE6) {
+    for (uint32_t p = 0; p < 4; ++p)
+      for (uint32_t f = 0; f < 4; ++f) {
+        const uint32_t s = edge_class_of(p, f);
+        for (uint32_t ev = 0; ev <= full; ++ev)
+          tab[((p << 2 | f) << k) | ev] =
+              s ? (4 * P.delay(s, ev, 0) - 3 + f) | (1u << 24) : 0u;
       }
+  } else if (id <= W_EO4) {
+    for (uint32_t p = 0; p < 4; ++p)
+      for (uint32_t f = 0; f < 4; ++f) {
+        const uint32_t s = edge_class_of(p, f);
+        for (uint32_t fell = 0; fell < 2; ++fell)
+          for (uint32_t ev = 0; ev <= full; ++ev)
+            tab[(((p << 2 | f) << 1 | fell) << k) | ev] =
+                s ? (4 * P.delay(s, ev, fell << edge_in) - 3 + f) | (1u << 24) : 0u;
+      }
+  } else if (id <= W_ED2) {
+    for (uint32_t s = 1; s <= 4; ++s)
+      for (uint32_t fell = 0; fell <= full; ++fell)
+        for (uint32_t ev = 0; ev <= full; ++ev)
+          tab[(s - 1) | (fell << 2) | (ev << (k + 2))] = 4 * P.delay(s, ev, fell) - 3;
+  } else {
+    uint16_t* t = (uint16_t*)tab;
+    for (uint32_t half = 0; half < 2; ++half)
+      for (uint32_t s = 1; s <= 4; ++s)
+        for (uint32_t bits = 0; bits < 64; ++bits) {
+          uint32_t m = 0xFFFF, n = 0, one = 1;
+          for (uint32_t q = 0; q < 3; ++q) {
+            if (!((bits >> (2 * q)) & 1u)) continue;
+            const uint32_t j = 3 * half + q, fell = (bits >> (2 * q + 1)) & 1u;
+            ++n;
+            one = P.one[j][s - 1][fell];
+            m = std::min(m, P.any[j][s - 1][fell]);
+          }
+          t[gen_dt_index(half, 0, s, bits)] = (uint16_t)(n == 1 ? one : (m == 0xFFFF ? 1u : m));
+          t[gen_dt_index(half, 1, s, bits)] = (uint16_t)m;
+        }
+  }
+}
+
+// The truth bytes of one function (4^k value codes) in a WalkId's form.
+static void fill_truth(const std::vector<uint8_t>& lut, uint32_t id, uint32_t k, uint32_t edge_in,
+                       uint8_t* tab) {
+  const uint32_t n = 1u << (2 * k);
+  if (id == W_EO3 || id == W_EO4) {
+    for (uint32_t old = 0; old < 4; ++old)
+      for (uint32_t c = 0; c < n; ++c) {
+        const uint32_t fell = edge_class_of(old, (c >> (2 * edge_in)) & 3u) == 2 ? 1u : 0u;
+        tab[old * n + c] = (uint8_t)(((lut[c] & 3u) << 1 | fell) << kEoShift);
+      }
+    return;
+  }
+  if (id != W_ED1 && id != W_ED2) {
+    for (uint32_t i = 0; i < n; ++i) tab[i] = (uint8_t)((lut[i] & 3u) << ne_shift(k));
+    return;
+  }
+  for (uint32_t c = 0; c < n; ++c)
+    for (uint32_t p = 0; p < n; ++p) {
+      const uint32_t f = lut[c] & 3u, s = edge_class_of(lut[p] & 3u, f);
+      uint32_t fell = 0;
+      for (uint32_t j = 0; j < k; ++j)
+        fell |= (edge_class_of((p >> (2 * j)) & 3u, (c >> (2 * j)) & 3u) == 2 ? 1u : 0u) << j;
+      tab[c * n + p] = (uint8_t)(f | (((s - 1) & 3u) << 2) | (fell << 4) | (s ? 0x80u : 0u));
+    }
 }
 
 // ------------------------------------------------------------- programs ---
@@ -214,12 +280,12 @@ DevProgram::~DevProgram() {
 
 size_t DevProgram::device_bytes() const {
   return h_grec.size() * sizeof(GateRec) + h_gdev.size() * sizeof(GateDev) +
-         h_dtab.size() * 2 + h_luts.size() + h_lutp.size() * 4 + h_wide.size() * 4;
+         h_dtab.size() * 4 + h_ttab.size() * 4 + h_luts.size();
 }
 
 bool DevProgram::is_resident() const { return resident.load(std::memory_order_acquire); }
 
-// The six tables share one device allocation and are published only after
+// The five tables share one device allocation and are published only after
 // it and every copy succeeded: a failed upload leaves the image
 // non-resident (all pointers null) and the next upload starts over.
 void DevProgram::upload(int dev, hipStream_t st) {
@@ -228,19 +294,18 @@ void DevProgram::upload(int dev, hipStream_t st) {
     if (dev != device) throw GlsError(GLS_E_ARG, "program image belongs to another device");
     return;
   }
-  const size_t sizes[6] = {h_grec.size() * sizeof(GateRec), h_gdev.size() * sizeof(GateDev),
-                           h_dtab.size() * 2, h_luts.size(), h_lutp.size() * 4, h_wide.size() * 4};
-  const void* srcs[6] = {h_grec.data(), h_gdev.data(), h_dtab.data(), h_luts.data(), h_lutp.data(),
-                         h_wide.data()};
-  size_t off[6], total = 0;
-  for (int i = 0; i < 6; ++i) {
+  const size_t sizes[5] = {h_grec.size() * sizeof(GateRec), h_gdev.size() * sizeof(GateDev),
+                           h_dtab.size() * 4, h_ttab.size() * 4, h_luts.size()};
+  const void* srcs[5] = {h_grec.data(), h_gdev.data(), h_dtab.data(), h_ttab.data(), h_luts.data()};
+  size_t off[5], total = 0;
+  for (int i = 0; i < 5; ++i) {
     off[i] = total;
     total += (std::max<size_t>(sizes[i], 1) + 255) / 256 * 256;
   }
   char* blk = nullptr;
   HC(hipMalloc((void**)&blk, total));
   try {
-    for (int i = 0; i < 6; ++i)
+    for (int i = 0; i < 5; ++i)
       if (sizes[i]) HC(hipMemcpyAsync(blk + off[i], srcs[i], sizes[i], hipMemcpyHostToDevice, st));
     HC(hipStreamSynchronize(st));
   } catch (...) {
@@ -252,25 +317,10 @@ void DevProgram::upload(int dev, hipStream_t st) {
   d_block = blk;
   d_grec = (GateRec*)(blk + off[0]);
   d_gdev = (GateDev*)(blk + off[1]);
-  d_dtab = (uint16_t*)(blk + off[2]);
-  d_luts = (uint8_t*)(blk + off[3]);
-  d_lutp = (uint32_t*)(blk + off[4]);
-  d_wide = (uint32_t*)(blk + off[5]);
+  d_dtab = (uint32_t*)(blk + off[2]);
+  d_ttab = (uint32_t*)(blk + off[3]);
+  d_luts = (uint8_t*)(blk + off[4]);
   resident.store(true, std::memory_order_release);
-}
-
-// Wide gates of an image, level by level.
-static void index_wide(DevProgram& P) {
-  P.h_wide.clear();
-  P.wide_start.assign(1, 0);
-  P.max_k = 0;
-  for (size_t l = 0; l + 1 < P.level_start.size(); ++l) {
-    for (uint32_t g = P.level_start[l]; g < P.level_start[l + 1]; ++g) {
-      P.max_k = std::max<uint32_t>(P.max_k, P.h_grec[g].k);
-      if (P.h_grec[g].k > kTileK) P.h_wide.push_back(g);
-    }
-    P.wide_start.push_back((uint32_t)P.h_wide.size());
-  }
 }
 
 std::shared_ptr<DevProgram> build_program_image(const Program& pg, uint32_t timescale_ps) {
@@ -290,6 +340,7 @@ std::shared_ptr<DevProgram> build_program_image(const Program& pg, uint32_t time
   if (nblk > 65535) throw GlsError(GLS_E_RANGE, "too many truth tables");
   P->h_grec.resize(P->n_gates);
   P->h_gdev.resize(P->n_gates);
+  std::map<std::pair<int, uint32_t>, uint32_t> tt_of;
   for (uint32_t i = 0; i < P->n_gates; ++i) {
     const CompiledGate& g = pg.gates[i];
     if (g.k < 1) throw GlsError(GLS_E_UNSUPPORTED, "gate without inputs");
@@ -312,24 +363,37 @@ std::shared_ptr<DevProgram> build_program_image(const Program& pg, uint32_t time
     r.lut = q.lut = (uint16_t)blk_of[g.lut];
     r.k = q.k = (uint8_t)g.k;
     r.dmax = q.dmax = D.dmax;
-    const uint32_t dts = g.k > (int)kTileK ? kWideDtSize : dt_size(g.k);
+    const DelayPick pick(D, g.k);
+    const std::vector<uint8_t>& lut = pg.luts[g.lut];
+    const uint32_t k = (uint32_t)g.k, all_x = 0x555u & ((1u << (2 * k)) - 1);
+    const uint32_t edges = pick.edge_inputs();
+    const bool one_edge = edges && !(edges & (edges - 1));
+    q.edge_in = one_edge ? (uint32_t)__builtin_ctz(edges) : 0u;
+    q.walk = (uint8_t)(!edges                                           ? W_NE1 + k - 1
+                       : one_edge && (k == 3 || k == 4)                 ? W_EO3 + k - 3
+                       : k <= 2 && (lut[all_x] & 3u) == 1u              ? W_ED1 + k - 1
+                                                                        : W_GEN);
+    const uint32_t dts = walk_dt_words(q.walk, k);
     if (P->h_dtab.size() + dts >= (1ull << 32))
       throw GlsError(GLS_E_RANGE, "delay tables exceed 2^32 entries");
     q.dt_off = (uint32_t)P->h_dtab.size();
     P->h_dtab.resize(P->h_dtab.size() + dts);
-    if (g.k > (int)kTileK) fill_wide_delays(D, g.k, P->h_dtab.data() + q.dt_off);
-    else fill_delay_table(D, g.k, P->h_dtab.data() + q.dt_off);
+    fill_delays(pick, q.walk, q.edge_in, P->h_dtab.data() + q.dt_off);
+    // truth bytes, shared by the gates of one function and form
+    const auto key = std::make_pair(g.lut, 8u * (q.walk == W_GEN ? W_NE1 + k - 1 : q.walk) + q.edge_in);
+    auto it = tt_of.find(key);
+    if (it == tt_of.end()) {
+      it = tt_of.emplace(key, (uint32_t)P->h_ttab.size()).first;
+      P->h_ttab.resize(P->h_ttab.size() + walk_tt_words(q.walk, k));
+      fill_truth(lut, q.walk, k, q.edge_in, (uint8_t*)(P->h_ttab.data() + it->second));
+    }
+    q.tt_off = it->second;
+    P->max_k = std::max(P->max_k, k);
   }
   nblk = std::max<size_t>(1, nblk);
   P->h_luts.assign(nblk * 256, 1);
-  P->h_lutp.assign(nblk * 16, 0);
-  for (size_t i = 0; i < pg.luts.size(); ++i) {
+  for (size_t i = 0; i < pg.luts.size(); ++i)
     std::memcpy(&P->h_luts[(size_t)blk_of[i] * 256], pg.luts[i].data(), pg.luts[i].size());
-    // packed 2 bits per entry for register lookups (fan-in <= 3)
-    for (size_t e = 0; e < pg.luts[i].size() && e < 256; ++e)
-      P->h_lutp[(size_t)blk_of[i] * 16 + e / 16] |= (uint32_t)(pg.luts[i][e] & 3u) << (2 * (e % 16));
-  }
-  index_wide(*P);
   return P;
 }
 
@@ -378,15 +442,20 @@ static std::shared_ptr<DevProgram> union_image(const std::vector<std::shared_ptr
                                                const std::vector<uint32_t>& net_base,
                                                const std::vector<uint32_t>& groups) {
   auto U = std::make_shared<DevProgram>();
-  std::map<const DevProgram*, std::pair<uint32_t, uint32_t>> bases;  // dtab, lut
+  struct Base {
+    uint32_t dt, tt, lut;
+  };
+  std::map<const DevProgram*, Base> bases;
   for (auto& p : parts) {
     if (bases.count(p.get())) continue;
-    bases[p.get()] = {(uint32_t)U->h_dtab.size(), (uint32_t)(U->h_luts.size() / 256)};
+    bases[p.get()] = {(uint32_t)U->h_dtab.size(), (uint32_t)U->h_ttab.size(),
+                      (uint32_t)(U->h_luts.size() / 256)};
     if (U->h_dtab.size() + p->h_dtab.size() >= (1ull << 32))
       throw GlsError(GLS_E_RANGE, "delay tables exceed 2^32 entries");
     U->h_dtab.insert(U->h_dtab.end(), p->h_dtab.begin(), p->h_dtab.end());
     U->h_luts.insert(U->h_luts.end(), p->h_luts.begin(), p->h_luts.end());
-    U->h_lutp.insert(U->h_lutp.end(), p->h_lutp.begin(), p->h_lutp.end());
+    U->h_ttab.insert(U->h_ttab.end(), p->h_ttab.begin(), p->h_ttab.end());
+    U->max_k = std::max(U->max_k, p->max_k);
   }
   if (U->h_luts.size() / 256 > 65535) throw GlsError(GLS_E_RANGE, "too many truth tables in one batch");
   size_t nlev = 0;
@@ -406,8 +475,9 @@ static std::shared_ptr<DevProgram> union_image(const std::vector<std::shared_ptr
         for (int j = 0; j < 4; ++j) r.in_net[j] = q.in_net[j];
         q.out_net += net_base[i];
         r.out_net = q.out_net;
-        q.dt_off += b.first;
-        q.lut = r.lut = (uint16_t)(q.lut + b.second);
+        q.dt_off += b.dt;
+        q.tt_off += b.tt;
+        q.lut = r.lut = (uint16_t)(q.lut + b.lut);
         q.job = (uint16_t)i;
         U->h_grec.push_back(q);
         U->h_gdev.push_back(r);
@@ -416,7 +486,6 @@ static std::shared_ptr<DevProgram> union_image(const std::vector<std::shared_ptr
     U->level_start.push_back((uint32_t)U->h_grec.size());
   }
   U->n_gates = (uint32_t)U->h_grec.size();
-  index_wide(*U);
   for (size_t i = 0; i < parts.size(); ++i) {
     U->n_nets = std::max(U->n_nets, net_base[i] + parts[i]->n_nets);
     U->n_pins += parts[i]->n_pins;
@@ -585,7 +654,7 @@ Job::~Job() {
   if (arena_) (void)hipStreamSynchronize(stream_);
   for (void* p : owned_)
     if (p) arena_ ? arena_->put(p) : (void)hipFree(p);
-  void* grown[] = {d_segmap_, d_sums_, d_carry_, d_scratch_, d_tiles_, d_tout_, d_toff_, d_stk_,
+  void* grown[] = {d_segmap_, d_sums_, d_carry_, d_scratch_, d_tiles_, d_tout_, d_toff_,
                    d_pool_,   d_ovf_,  d_tails_, d_cwin_};
   for (void* p : grown)
     if (p) arena_ ? arena_->put(p) : (void)hipFree(p);
@@ -977,6 +1046,7 @@ void Job::prepare(const std::vector<SimInstance>& inst, uint64_t pool_words) {
   d_saif_ = (unsigned long long*)dmalloc((size_t)n_nets_ * kSaifWords * sizeof(unsigned long long));
   d_win_ = (unsigned long long*)dmalloc(win_.size() * 8);
   d_scal_ = (uint64_t*)dmalloc(16 * sizeof(uint64_t));
+  d_ticket_ = (unsigned long long*)dmalloc(kTickets * kTicketStride * 8);
   uint32_t maxw = 1;
   for (size_t l = 0; l + 1 < level_start_.size(); ++l)
     maxw = std::max(maxw, level_start_[l + 1] - level_start_[l]);
@@ -1089,8 +1159,7 @@ void Job::prepare(const std::vector<SimInstance>& inst, uint64_t pool_words) {
   }
   HC(hipMemcpyAsync(d_win_, win_.data(), win_.size() * 8, hipMemcpyHostToDevice, stream_));
   HC(hipStreamSynchronize(stream_));
-  cap_ = tile_cap(seg_target ? seg_target : kDefaultSeg);
-  level_blocks_ = level_blocks_opt ? (int)level_blocks_opt : level_max_blocks(cap_, stack_mode == 0);
+  size_tiles();
   stats_ = JobStats();
   stats_.level_blocks = (uint64_t)level_blocks_;
   stats_.n_nets = n_nets_;
@@ -1100,6 +1169,14 @@ void Job::prepare(const std::vector<SimInstance>& inst, uint64_t pool_words) {
     std::fprintf(stderr, "gls: prepared %zu instance(s), pool %.1f GiB, in %.1f ms\n", inst.size(),
                  pool_words_ * 4.0 / 1073741824.0,
                  std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_prep).count());
+}
+
+// LDS and tile size of the walk for the current settings.
+void Job::size_tiles() {
+  const uint32_t seg = seg_target ? seg_target : kDefaultSeg;
+  lds_words_ = walk_lds_words(seg);
+  wide_words_ = wide_tile_words(seg, lds_words_);
+  level_blocks_ = level_blocks_opt ? (int)level_blocks_opt : level_max_blocks(lds_words_);
 }
 
 void Job::stop_point() {
@@ -1181,7 +1258,6 @@ int Job::run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_e
   uint64_t* bump = d_scal_ + S_BUMP;
   unsigned long long* evc = (unsigned long long*)(d_scal_ + S_EVC);
   unsigned int* err = (unsigned int*)(d_scal_ + S_ERR);
-  const uint32_t seg = seg_target ? seg_target : kDefaultSeg;
   const bool retry = !device_driven && !static_ && (ovf_words_opt == 0 || pool_grow);
   const uint32_t ns = G.s1 - G.s0;  // the group's stimulus signals
   const ChunkWin* cw = d_cwin_ + c.slot * net_base_.size();
@@ -1252,7 +1328,7 @@ int Job::run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_e
     uint32_t g0 = level_start_[l], ng = level_start_[l + 1] - g0;
     if (ng == 0) continue;
     const GateRec* gates = prog_->d_grec + g0;
-    HC(launch_plan2(gates, ng, d_wlen_, seg, d_plan_, d_ntile_, d_bound_, err, d_tail_len_, stream_));
+    HC(launch_plan2(gates, ng, d_wlen_, seg_target ? seg_target : kDefaultSeg, wide_words_, d_plan_, d_ntile_, d_bound_, err, d_tail_len_, stream_));
     HC(launch_scan(d_ntile_, d_tilebase_, ng, d_part_, d_scal_ + S_TOT_A, nullptr, stream_));
     HC(launch_scan(d_bound_, d_scrbase_, ng, d_part_, d_scal_ + S_TOT_B, nullptr, stream_));
     uint64_t ntiles = tiles_cap_;
@@ -1312,16 +1388,15 @@ int Job::run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_e
         scratch = d_pool_ + pool_limit;
       }
     }
-    HC(launch_tile_desc(gates, ng, d_plan_, d_tilebase_, d_woff_, d_wlen_, d_pool_, prog_->d_lutp,
-                        d_tiles_, d_scal_ + S_TOT_A, ntiles, stream_));
-    HC(launch_fill_u64((unsigned long long*)(d_scal_ + S_TICKET), 2, 0ull, stream_));  // ticket, ovf
+    HC(launch_tile_desc(gates, ng, d_plan_, d_tilebase_, d_scrbase_, d_woff_, d_wlen_, d_pool_,
+                        d_tiles_, d_scal_ + S_TOT_A, ntiles, d_ticket_,
+                        (unsigned long long*)(d_scal_ + S_OVF_USED), stream_));
     LevelArgs a;
     a.tiles = d_tiles_;
     a.pool = d_pool_;
     a.dtab = prog_->d_dtab;
-    a.luts = prog_->d_luts;
+    a.ttab = prog_->d_ttab;
     a.ntiles = d_scal_ + S_TOT_A;
-    a.scr_base = d_scrbase_;
     a.scratch = scratch;
     a.tout = d_tout_;
     a.ovf = d_ovf_;
@@ -1330,41 +1405,14 @@ int Job::run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_e
     a.ev_count = evc;
     a.err = err;
     a.cwin = cw;
-    a.cap = cap_;
+    a.lds_words = lds_words_;
     a.prefetch = prefetch;
-    a.ticket = (unsigned long long*)(d_scal_ + S_TICKET);
+    a.ticket = d_ticket_;
     a.tiles_walked = (unsigned long long*)(d_scal_ + S_TILES);
-    a.stk = nullptr;
     a.lo_rel = c.lo_rel;
     a.hi_rel = c.hi_rel;
     a.first = c.first;
     const unsigned nb = (unsigned)std::min<uint64_t>(ntiles, (uint64_t)std::max(1, level_blocks_));
-    if (stack_mode == 1) {
-      const uint64_t w = (uint64_t)std::max(1, level_blocks_) * (cap_ + 64);
-      if (!device_driven) ensure((void**)&d_stk_, cap_stk_, w * 4);
-      a.stk = d_stk_;
-    }
-    WideArgs wa;
-    wa.gates = gates;
-    wa.wide = prog_->d_wide + prog_->wide_start[l];
-    wa.nwide = prog_->wide_start[l + 1] - prog_->wide_start[l];
-    wa.g0 = g0;
-    wa.tile_base = d_tilebase_;
-    wa.tiles = d_tiles_;
-    wa.woff = d_woff_;
-    wa.wlen = d_wlen_;
-    wa.pool = d_pool_;
-    wa.luts = prog_->d_luts;
-    wa.dtab = prog_->d_dtab;
-    wa.scr_base = d_scrbase_;
-    wa.scratch = scratch;
-    wa.tout = d_tout_;
-    wa.ev_count = evc;
-    wa.err = err;
-    wa.cwin = cw;
-    wa.lo_rel = c.lo_rel;
-    wa.hi_rel = c.hi_rel;
-    wa.first = c.first;
     if (!device_driven && !static_) {
       hipEvent_t e_a, e_b;
       HC(hipEventCreate(&e_a));
@@ -1373,19 +1421,17 @@ int Job::run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_e
       ev_eval.push_back(e_b);
       HC(hipEventRecord(e_a, stream_));
       HC(launch_level(a, nb, stream_));
-      HC(launch_wide(wa, stream_));
       HC(hipEventRecord(e_b, stream_));
     } else {
       HC(launch_level(a, nb, stream_));
-      HC(launch_wide(wa, stream_));
     }
     // gate counts go to d_bound_ (free again once the scratch bases are scanned)
     HC(launch_gate_carry(gates, ng, d_tilebase_, d_ntile_, d_tout_, d_toff_, d_bound_, d_wlen_,
                          d_saif_chunk_, cw, err, T, d_evjob_chunk_, stream_));
     HC(launch_scan(d_bound_, d_outoff_, ng, d_part_, d_scal_ + S_TOT_OUT, bump, stream_));
     HC(launch_pool_guard(d_scal_, pool_limit, stream_));
-    HC(launch_compact(d_tiles_, d_scal_ + S_TOT_A, ntiles, d_tout_, d_toff_, d_scrbase_, scratch,
-                      d_outoff_, d_pool_, d_woff_, d_wlen_, err, d_saif_chunk_, cw, saif_tc, T,
+    HC(launch_compact(d_tiles_, d_scal_ + S_TOT_A, ntiles, d_tout_, d_toff_, scratch, d_outoff_, d_pool_,
+                      d_woff_, d_wlen_, err, d_saif_chunk_, cw, saif_tc, T,
                       stream_));
     HC(launch_bump(bump, d_scal_ + S_TOT_OUT, stream_));
   }
@@ -1612,10 +1658,9 @@ void Job::run_two_pass(std::vector<hipEvent_t>& ev_eval) {
 
 void Job::run() {
   HC(hipSetDevice(device_));
-  cap_ = tile_cap(seg_target ? seg_target : kDefaultSeg);
-  level_blocks_ = level_blocks_opt ? (int)level_blocks_opt : level_max_blocks(cap_, stack_mode == 0);
+  size_tiles();
   stats_.level_blocks = (uint64_t)level_blocks_;
-  const std::vector<uint64_t> sig = {cap_, (uint64_t)level_blocks_, seg_target, prefetch,
+  const std::vector<uint64_t> sig = {lds_words_, (uint64_t)level_blocks_, seg_target, prefetch,
                                      (uint64_t)mode, stack_mode, chunk_ps, keep_waves};
   last_replay_ = false;
   if (graph && gexec_ && sig == graph_sig_) {

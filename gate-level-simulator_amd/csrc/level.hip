@@ -1,29 +1,39 @@
 // Fused per-level gate evaluation (gfx950): walk, join, compact.
 //
-// Work unit: a tile = 64 consecutive time segments of one gate, one segment
-// per lane of a wavefront.  Segment c of a gate covers the events
-// [c*stride, (c+1)*stride) of the gate's longest input (the "leader"), so
-// segment boundaries are exact event times.
+// Work unit: a tile = a run of consecutive words of a gate's longest input
+// (the "leader") and the other inputs' words of the same time span, so tile
+// boundaries are exact event times.
 //
-// k_level (walk), one tile at a time per wavefront, tiles independent and
-// handed out by ticket:
+// k_level (walk), one tile at a time per wavefront, tiles independent:
 //   1. the tile's input ranges (one event before the tile for the starting
-//      values, a D_max look-ahead halo after it), its delay table and its
-//      truth table are copied into LDS with direct-to-LDS loads, each range
-//      followed by an INF sentinel (tiles too long for LDS read HBM instead
-//      and keep their stacks in the overflow buffer);
-//   2. every lane merges its segment's input events in time order (branch
-//      free), evaluates the 4-state truth table (packed in registers for
-//      fan-in <= 3), classifies the output edge, picks the SDF delay with one
-//      lookup in the gate's delay table (AddDelay folded on the host) and
-//      applies the preemption rule on a stack (LDS, or a per-workgroup HBM
-//      scratch), counting value changes as it goes; events in the halo only
-//      pre-empt;
-//   3. a wavefront scan (DPP) combines the lanes' kept lists (dedup of equal
-//      adjacent values across lanes is an associative monoid), the lanes
-//      store the tile's entries into the level scratch and lane 0 writes the
-//      tile summary (count, first/last value and time, SAIF durations).
-//   The next tile's loads are issued before the current tile is stored.
+//      values, a D_max look-ahead halo after it) and the gate's two tables
+//      are copied into LDS with direct-to-LDS loads, each range followed by an
+//      INF sentinel (tiles too long for LDS read HBM instead and keep their
+//      stacks in the overflow buffer);
+//   2. the tile's words are cut into equal shares, one per lane (lane_bounds);
+//      every lane merges its share in time order and looks every event up:
+//      a truth byte by the input values, then a delay word by the gate's old
+//      and new value and the inputs with an event (lane_walk);
+//   3. the preemption rule is applied backwards over each lane's candidates,
+//      with one suffix minimum over the wavefront for the lanes after it
+//      (keep_entries);
+//   4. the lanes' lists are joined (a list that starts with the value before
+//      it drops that entry) and stored into the level scratch, and lane 0
+//      writes the tile summary (count, first/last value and time, SAIF
+//      durations) (emit_tile).
+//   The next tile's loads are issued when the walk no longer reads its inputs.
+//
+// What bounds the walk: VALU issue, at 67% of the SIMDs' cycles with two
+// wavefronts per SIMD (LDS-limited).  1.39 VALU wave-instructions per gate
+// event on the 200k-cell configuration (gap 500 ps): about 22 (fan-in 2) to 34
+// (fan-in 4) a step and 43 steps a tile where 31 would do if the lanes' shares
+// were exact; 1,200 a tile besides.  With delays looked up by an edge class and
+// per-input event and edge bits computed each step, a halo walked by every lane,
+// the candidate lists joined by a wavefront scan of 3-word aggregates, 16 bytes a
+// store fewer and all tiles handed out by one ticket counter it was 2.04, and
+// that configuration took 154 ms over 10 Mps where it now takes 99 ms (the 2M-cell
+// configuration over 2 Mps: 615 -> 405 ms; 5- and 6-input cells, walked by one
+// thread a gate before, 6,007 cells over 150 kps: 122 -> 0.7 ms).
 // k_gate_carry: per gate, joins its tiles in order (a tile whose first entry
 //   repeats the value before it drops that entry), places them, and finishes
 //   the gate's SAIF record.
@@ -58,81 +68,57 @@ __device__ __forceinline__ uint32_t edge_cls(uint32_t pre, uint32_t cur) {
   return (uint32_t)(T >> ((pre * 4 + cur) * 4)) & 0xF;
 }
 
-// Aggregate of a run of kept candidates (for dedup + SAIF carry):
-// cnt = entries after dedup, fv/lv = first/last value, lt = last time.
-struct Agg {
-  uint32_t cnt, lt;
-  uint32_t fv, lv, has;
-};
-
-__device__ __forceinline__ Agg agg_combine(const Agg& a, const Agg& b) {
-  if (!a.has) return b;
-  if (!b.has) return a;
-  Agg r;
-  r.cnt = a.cnt + b.cnt - (a.lv == b.fv ? 1u : 0u);
-  r.fv = a.fv;
-  r.lv = b.lv;
-  r.lt = b.lt;
-  r.has = 1;
-  return r;
-}
-
 // Cross-lane moves with DPP (no LDS round trip).  Lanes without a source
-// lane (outside the row, or rows left out by ROW_MASK) receive 0, which is
-// the identity of the sums below and, for all three words, the empty Agg.
-// Control codes: row_shr:d 0x110+d, row_shl:d 0x100+d, wave_shr:1 0x138,
-// row_bcast:15 0x142, row_bcast:31 0x143.
+// lane (outside the row, or rows left out by ROW_MASK) receive OLD.
+// Control codes: row_shr:d 0x110+d, row_shl:d 0x100+d, wave_shl:1 0x130,
+// wave_shr:1 0x138, row_bcast:15 0x142, row_bcast:31 0x143.
 template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ uint32_t dpp(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROW_MASK, 0xF, false);
+__device__ __forceinline__ uint32_t dpp(uint32_t x, uint32_t old = 0) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)x, CTRL, ROW_MASK, 0xF, false);
 }
 
-__device__ __forceinline__ uint32_t agg_flags(const Agg& a) {
-  return a.fv | (a.lv << 2) | (a.has << 4);
-}
-__device__ __forceinline__ Agg agg_from(uint32_t cnt, uint32_t lt, uint32_t f) {
-  Agg r;
-  r.cnt = cnt;
-  r.lt = lt;
-  r.fv = f & 3u;
-  r.lv = (f >> 2) & 3u;
-  r.has = (f >> 4) & 1u;
-  return r;
-}
-
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ Agg agg_dpp(const Agg& a) {
-  return agg_from(dpp<CTRL, ROW_MASK>(a.cnt), dpp<CTRL, ROW_MASK>(a.lt),
-                  dpp<CTRL, ROW_MASK>(agg_flags(a)));
-}
-
-__device__ __forceinline__ Agg agg_readlane(const Agg& a, int lane) {
-  return agg_from(__builtin_amdgcn_readlane(a.cnt, lane), __builtin_amdgcn_readlane(a.lt, lane),
-                  __builtin_amdgcn_readlane(agg_flags(a), lane));
-}
-
-// Inclusive scan of the lanes' aggregates in lane order: within rows of 16
-// by row shifts, then row 0's total into row 1 and row 2's into row 3
-// (row_bcast:15), then lane 31's prefix into rows 2 and 3 (row_bcast:31).
-__device__ __forceinline__ Agg agg_wave_scan(Agg x) {
-  x = agg_combine(agg_dpp<0x111>(x), x);
-  x = agg_combine(agg_dpp<0x112>(x), x);
-  x = agg_combine(agg_dpp<0x114>(x), x);
-  x = agg_combine(agg_dpp<0x118>(x), x);
-  x = agg_combine(agg_dpp<0x142, 0xA>(x), x);
-  x = agg_combine(agg_dpp<0x143, 0xC>(x), x);
-  return x;
-}
-
-// Sum over the wavefront (uniform result).
-__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
+// Inclusive prefix sum over the wavefront: within rows of 16 by row shifts,
+// then row 0's total into row 1 and row 2's into row 3 (row_bcast:15), then
+// lane 31's prefix into rows 2 and 3 (row_bcast:31).
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
   x += dpp<0x111>(x);
   x += dpp<0x112>(x);
   x += dpp<0x114>(x);
   x += dpp<0x118>(x);
   x += dpp<0x142, 0xA>(x);
   x += dpp<0x143, 0xC>(x);
-  return __builtin_amdgcn_readlane(x, 63);
+  return x;
+}
+
+// Sum over the wavefront (uniform result).
+__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
+  return __builtin_amdgcn_readlane(wave_scan(x), 63);
+}
+
+// Inclusive prefix maximum over the wavefront.
+__device__ __forceinline__ uint32_t wave_max_scan(uint32_t x) {
+  x = max(x, dpp<0x111>(x));
+  x = max(x, dpp<0x112>(x));
+  x = max(x, dpp<0x114>(x));
+  x = max(x, dpp<0x118>(x));
+  x = max(x, dpp<0x142, 0xA>(x));
+  x = max(x, dpp<0x143, 0xC>(x));
+  return x;
+}
+
+// Minimum over the lanes after this one (all ones for lane 63): within rows
+// by row shifts, the later rows' minima from their first lanes.
+__device__ __forceinline__ uint32_t wave_min_after(uint32_t x) {
+  x = min(x, dpp<0x101>(x, 0xFFFFFFFFu));
+  x = min(x, dpp<0x102>(x, 0xFFFFFFFFu));
+  x = min(x, dpp<0x104>(x, 0xFFFFFFFFu));
+  x = min(x, dpp<0x108>(x, 0xFFFFFFFFu));
+  const uint32_t r3 = __builtin_amdgcn_readlane(x, 48);
+  const uint32_t r2 = min((uint32_t)__builtin_amdgcn_readlane(x, 32), r3);
+  const uint32_t r1 = min((uint32_t)__builtin_amdgcn_readlane(x, 16), r2);
+  const uint32_t lane = threadIdx.x;
+  const uint32_t later = lane < 16 ? r1 : (lane < 32 ? r2 : (lane < 48 ? r3 : 0xFFFFFFFFu));
+  return dpp<0x130>(min(x, later), 0xFFFFFFFFu);
 }
 
 __device__ __forceinline__ void saif_acc(unsigned long long* acc, uint32_t v, unsigned long long a,
@@ -156,54 +142,21 @@ __device__ __forceinline__ uint32_t lb_words(P a, uint32_t n, uint32_t key) {
   return lo;
 }
 
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-
-// Pointer to a tile's input ranges: LDS (staged) or HBM (too long for LDS).
-// The LDS form is a 32-bit local pointer, so its reads are ds_read.
-template <bool LDS> struct InPtr { typedef const uint32_t* T; };
-template <> struct InPtr<true> { typedef const lds_u32* T; };
-
-// Uniform (per tile) data of one gate.
-template <int K, bool LDS>
-struct TileCtx {
-  typename InPtr<LDS>::T src[K];  // input ranges, index relative to B
-  uint32_t B[K], E[K], L[K];
-  uint32_t nseg, stride, lead, dmax;
-  uint32_t span;            // the tile's own input words (out_cap - 1)
-  uint32_t lut[4];          // packed truth table, fan-in <= 3
-};
-
-template <int K, bool LDS>
-__device__ __forceinline__ uint32_t lut_eval(const TileCtx<K, LDS>& X, const uint8_t* s_lut,
-                                             uint32_t idx) {
-  // fan-in <= 2: 16 entries of 2 bits in one register; else the staged table
-  if (K <= 2) return __builtin_amdgcn_ubfe(X.lut[0], 2 * idx, 2);
-  return s_lut[idx];
+// Bit fields of TileOut::flags.
+__device__ __forceinline__ uint32_t out_flags(uint32_t fv, uint32_t lv, uint32_t has) {
+  return fv | (lv << 2) | (has << 4);
 }
-
-// Delay-table key bits of one event (dt_index): per input j, bit 2j = it has
-// an event (from `ev`, already at even positions) and bit 2j+1 = it fell
-// (CheckDelay == 2: to 0 from X/Z/1, or from 1 to X/Z) between the packed
-// input values p and c (2 bits per input).  At bit 2j+1 of c, c << 1, p and
-// p << 1 sit the input's c1, c0, p1, p0.
-__device__ __forceinline__ uint32_t event_bits(uint32_t p, uint32_t c, uint32_t ev) {
-  const uint32_t cs = c << 1, ps = p << 1;
-  const uint32_t to0 = ~c & ~cs & (p | ps);        // now 0, was not 0
-  const uint32_t from1 = (p & ps) & (c ^ cs);      // was 1, now X or Z
-  return ((to0 | from1) & 0xAAu) | ev;
-}
-
-// What one lane's walk over its segment leaves behind: its kept candidates
-// (st[0..sp), in time order), the last of them, the number of value changes
-// among them, and the number of gate events it owned.  SP: pointer to the
-// lane's region (LDS or HBM).
-template <typename SP>
-struct Lane {
-  SP st;
-  uint32_t sp, top, cnt, nown;
-};
 
 typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+
+// LDS by byte address (32-bit local pointers: the reads are ds_read with the
+// constant part of the address in the instruction).
+__device__ __forceinline__ uint32_t lds32(uint32_t a) { return *(const lds_u32*)a; }
+__device__ __forceinline__ uint32_t lds16(uint32_t a) { return *(const lds_u16*)a; }
+__device__ __forceinline__ uint32_t lds8(uint32_t a) { return *(const lds_u8*)a; }
 
 // One 4-byte direct-to-LDS load per lane: lane i's word lands at l + i.
 __device__ __forceinline__ void dma_word(const uint32_t* g, uint32_t* l) {
@@ -217,609 +170,844 @@ __device__ __forceinline__ void dma_x4(const uint32_t* g, uint32_t* l) {
 }
 
 // Wait until this wavefront has no vector-memory access in flight (direct-to-
-// LDS loads included): s_waitcnt vmcnt(0).
-__device__ __forceinline__ void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-__device__ __forceinline__ uint32_t range_start(uint32_t L) { return L > 0 ? L - 1 : 0u; }
-
-__device__ __forceinline__ uint32_t tile_words(const TileDesc& D) {
-  // loops over the fan-in run to 4 with constant indices so a descriptor
-  // held in registers is never indexed at run time
-  uint32_t total = 0;
-#pragma unroll
-  for (uint32_t j = 0; j < 4; ++j)
-    if (j < D.k) total += D.E[j] - range_start(D.L[j]);
-  return total;
+// LDS loads included): s_waitcnt vmcnt(0).  A workgroup is one wavefront, whose
+// LDS accesses stay in order: beside this wait only the compiler needs fences
+// (a barrier's would also wait for the stores in flight).
+__device__ __forceinline__ void lds_fence() { asm volatile("" ::: "memory"); }
+__device__ __forceinline__ void wait_vm() {
+  lds_fence();
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  lds_fence();
 }
 
-// LDS layout of a tile's input ranges: range j (n_j words from pool word
-// G_j) starts at P_j = R_j + G_j mod 4 with R_j a multiple of 4 words, so it
-// is copied with 16-byte loads from the aligned word G_j - G_j mod 4;
-// R_{j+1} = the multiple of 4 at or above P_j + n_j + 1 keeps the sentinel
-// word after each range.  The layout needs at most sum(n_j) + 7 K words.
-__device__ __forceinline__ void range_layout(const TileDesc& D, uint32_t P[4]) {
-  uint32_t R = 0;
+// A tile's descriptor in scalar registers.
+struct Tile {
+  uint32_t in_lo[6], n[6], in_hi[2];
+  uint64_t scr;
+  uint32_t own, xend, meta, dt_off, tt_off, dmax, job, out_cap, g;
+
+  __device__ __forceinline__ uint32_t id() const { return meta & 15u; }
+  __device__ __forceinline__ uint32_t k() const { return (meta >> 4) & 15u; }
+  __device__ __forceinline__ uint32_t lead() const { return (meta >> 8) & 15u; }
+  __device__ __forceinline__ bool starts_gate() const { return (meta >> 12) & 1u; }
+  __device__ __forceinline__ uint32_t edge_in() const { return (meta >> 16) & 15u; }
+  __device__ __forceinline__ uint64_t src(int j) const {
+    return ((uint64_t)((in_hi[j >> 2] >> (8 * (j & 3))) & 0xFFu) << 32) | in_lo[j];
+  }
+  __device__ __forceinline__ uint32_t words() const {
+    uint32_t t = 0;
 #pragma unroll
-  for (uint32_t j = 0; j < 4; ++j) {
-    const uint32_t n = D.E[j] - range_start(D.L[j]);
-    P[j] = R + ((uint32_t)D.in_off[j] & 3u);
-    if (j < D.k) R = (P[j] + n + 4) & ~3u;
+    for (uint32_t j = 0; j < kWideK; ++j) t += n[j];  // 0 beyond the fan-in
+    return t;
+  }
+};
+
+// A tile descriptor is read with one coalesced load (lane i < 32 holds
+// dword i), a tile ahead, and broadcast with readlane: its fields are scalars
+// and no load of theirs waits behind the staging loads in flight.
+__device__ __forceinline__ uint32_t desc_word(const TileDesc* p) {
+  return threadIdx.x < 32 ? ((const uint32_t*)p)[threadIdx.x] : 0u;
+}
+
+__device__ __forceinline__ Tile tile_of(uint32_t dw) {
+  uint32_t w[25];
+#pragma unroll
+  for (int i = 0; i < 25; ++i) w[i] = __builtin_amdgcn_readlane(dw, i);
+  Tile D;
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    D.in_lo[j] = w[j];
+    D.n[j] = w[6 + j];
+  }
+  D.in_hi[0] = w[12];
+  D.in_hi[1] = w[13];
+  D.scr = ((uint64_t)w[15] << 32) | w[14];
+  D.own = w[16];
+  D.xend = w[17];
+  D.meta = w[18];
+  D.dt_off = w[19];
+  D.tt_off = w[20];
+  D.dmax = w[21];
+  D.job = w[22];
+  D.out_cap = w[23];
+  D.g = w[24];
+  return D;
+}
+
+// LDS layout of a tile's input ranges (byte address of each range's index 0):
+// range j (n_j words from pool word G_j) starts at word P_j = R_j + G_j mod 4
+// with R_j a multiple of 4 words, so it is copied with 16-byte loads from the
+// aligned word G_j - G_j mod 4; R_{j+1} = the multiple of 4 at or above
+// P_j + n_j + 1 keeps the sentinel word after each range.  The layout needs at
+// most sum(n_j) + 7 K words.
+__device__ __forceinline__ void range_layout(const Tile& D, uint32_t base, uint32_t P[6]) {
+  uint32_t R = base;
+#pragma unroll
+  for (uint32_t j = 0; j < kWideK; ++j) {
+    P[j] = R + 4 * (D.in_lo[j] & 3u);
+    if (j < D.k()) R = (P[j] + 4 * D.n[j] + 16) & ~15u;
   }
 }
 
-// Issue the loads of tile D into LDS: its input ranges when they fit (laid
-// out by range_layout; the 16-byte copies may also bring up to 3 words
-// before and after a range, inside its slot), its delay table and (fan-in
-// 3 and 4) its truth table.  Completion: wait_vm().
-__device__ __forceinline__ void stage_tile(const LevelArgs& A, const TileDesc& D, bool fits,
-                                           uint32_t* s_in, uint32_t* s_lut, uint32_t* s_dt) {
+// First byte of the tile's input ranges: after its gate's tables.
+__device__ __forceinline__ uint32_t in_base(const Tile& D) {
+  return 4 * (walk_dt_words(D.id(), D.k()) + walk_tt_words(D.id(), D.k()));
+}
+__device__ __forceinline__ bool tile_fits(const LevelArgs& A, const Tile& D) {
+  return D.id() < W_COUNT && walk_lds_need(D.id(), D.k(), D.words()) <= A.lds_words;
+}
+// First byte of the tile's stacks: they end with the workgroup's LDS, so the
+// next tile's inputs can be staged at the front while they are read.
+__device__ __forceinline__ uint32_t stack_base(const LevelArgs& A, const Tile& D) {
+  return 4 * (A.lds_words - D.words() - kStackSlack);
+}
+
+// Issue the loads of a tile into LDS: its gate's tables (unless the tile
+// before was of the same gate) and its input ranges (laid out by
+// range_layout; the 16-byte copies may also bring up to 3 words before and
+// after a range, inside its slot).  Completion: wait_vm().
+__device__ __forceinline__ void stage_tile(const LevelArgs& A, const Tile& D, bool tables,
+                                           uint32_t* lds) {
   const uint32_t lane = threadIdx.x;
-  if (D.k > kTileK) return;  // wide gate: walked by k_wide
-  if (fits) {
-    uint32_t P[4];
-    range_layout(D, P);
-#pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) {
-      if (j >= D.k) break;
-      const uint32_t n = D.E[j] - range_start(D.L[j]);
-      const uint32_t a = (uint32_t)D.in_off[j] & 3u;
-      const uint32_t m = (a + n + 3) & ~3u;  // words copied, a multiple of 4
-      const uint32_t* src = A.pool + (D.in_off[j] - a);
-      uint32_t* l = s_in + (P[j] - a);
-      for (uint32_t i = 0; i < m; i += 4 * kLanes)
-        if (i + 4 * lane < m) dma_x4(src + i + 4 * lane, l + i);
-    }
+  if (tables) {
+    const uint32_t dw = walk_dt_words(D.id(), D.k()), tw = walk_tt_words(D.id(), D.k());
+    const uint32_t* dsrc = A.dtab + D.dt_off;
+    const uint32_t* tsrc = A.ttab + D.tt_off;
+#pragma unroll 1
+    for (uint32_t i = 0; i < dw; i += 4 * kLanes)
+      if (i + 4 * lane < dw) dma_x4(dsrc + i + 4 * lane, lds + i);
+#pragma unroll 1
+    for (uint32_t i = 0; i < tw; i += 4 * kLanes)
+      if (i + 4 * lane < tw) dma_x4(tsrc + i + 4 * lane, lds + dw + i);
   }
-  const uint32_t nw = dt_size(D.k) / 2;
-  const uint32_t* dsrc = (const uint32_t*)(A.dtab + D.dt_off);
-  for (uint32_t i = 0; i < nw; i += kLanes)
-    if (i + lane < nw) dma_word(dsrc + i + lane, s_dt + i);
-  if (D.k >= 3) dma_word((const uint32_t*)(A.luts + D.lut * 256u) + lane, s_lut);
+  uint32_t P[6];
+  range_layout(D, in_base(D), P);
+#pragma unroll
+  for (uint32_t j = 0; j < kWideK; ++j) {
+    if (j >= D.k()) break;
+    const uint32_t a = D.in_lo[j] & 3u;
+    const uint32_t m = (a + D.n[j] + 3) & ~3u;  // words copied, a multiple of 4
+    const uint32_t* src = A.pool + (D.src(j) - a);
+    uint32_t* l = lds + (P[j] / 4 - a);
+#pragma unroll 1
+    for (uint32_t i = 0; i < m; i += 4 * kLanes)
+      if (i + 4 * lane < m) dma_x4(src + i + 4 * lane, l + i);
+  }
 }
 
-// One lane's walk over its time segment, in two passes over the lane's
-// region of the stack buffer.
-//
-// Pass 1 merges the inputs in time order and evaluates every event without
-// branches: 4-state truth table, edge class (CheckDelay,
-// src/simulate.cpp:1178-1201), delay (one lookup in the gate's table, which
-// folds AddDelay, src/simulate.cpp:1012-1176) and candidate output time
-// o = t + d; each candidate of an owned event is appended as (o << 2 | f).
-// Events in the halo (the next segment's first D_max) only record the
-// smallest output time they make.  Look-back events, owned events and halo
-// events come in that order in time, so each has a loop of its own, tested
-// at the bottom: a step carries only its own kind's bookkeeping.
-//
-// Pass 2 applies the preemption rule of src/simulate.cpp:990-1009 in its
-// closed form: a candidate is kept iff its output time is strictly below
-// that of every later candidate (those of the lane and of the halo).  It runs
-// from the last candidate to the first, keeping the running minimum,
-// compacting kept candidates towards the end of the region (in time order)
-// and counting value changes among them.  Chunks: candidates below lo_rel
-// (made by look-back events) are never kept but still pre-empt; candidates at
-// or above hi_rel belong to the next chunk and are not kept (they pre-empt
-// only entries that are not kept either).  Only events at or after lo_rel
-// count as this chunk's gate events.
-//
-// Index 0 of every waveform is the net's state entry (its value before the
-// chunk's look-back window), so segment 0 starts at index 1 and takes its
-// starting values from index 0.
-//
-// stk_words: size of the tile's stack buffer at stk_base.  A lane's region
-// runs from its offset to the next lane's and holds its owned events + 1
-// words, enough for every candidate (and, in segment 0 of chunk 0, the
-// initial (0, X) entry).  Regions in HBM are guarded anyway: a write that
-// would leave the buffer (inputs out of order) lands on the buffer's last
-// word instead and sets bad.  LDS regions are not guarded (an LDS access
-// outside the workgroup's allocation is discarded by the hardware; all
-// inputs are time-ordered by construction).
-template <int K, bool LDS, typename SP>
-__device__ __forceinline__ Lane<SP> lane_walk(const TileCtx<K, LDS>& X, uint32_t ti,
-                                              const uint8_t* s_lut, const uint16_t* s_dt,
-                                              SP stk_base, uint32_t stk_words, uint32_t& bad,
-                                              uint32_t lo_rel, uint32_t hi_rel, bool first) {
-  const int lane = threadIdx.x;
-  const uint32_t c0 = ti * kLanes;                          // the tile's first segment
-  const uint32_t m = min((uint32_t)kLanes, X.nseg - c0);   // its segments (>= 1)
-  const uint32_t kX = 1u;
-  const uint32_t INF = 0xFFFFFFFFu;
-  uint32_t r[K], h[K], bound[K];
-  typename InPtr<LDS>::T srcL = X.src[0];
-  uint32_t BL = X.B[0], EL = X.E[0];
+// INF after every input range of a staged tile (its loads have arrived).
+__device__ __forceinline__ void put_sentinels(const Tile& D) {
+  if (threadIdx.x != 0) return;
+  uint32_t P[6];
+  range_layout(D, in_base(D), P);
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    bound[j] = X.E[j] - X.B[j];
-    if ((uint32_t)j == X.lead) {
-      srcL = X.src[j];
-      BL = X.B[j];
-      EL = X.E[j];
+  for (uint32_t j = 0; j < kWideK; ++j)
+    if (j < D.k()) *(lds_u32*)(P[j] + 4 * D.n[j]) = kWordInf;
+}
+
+// What one lane's walk leaves: candidates (or, later, kept entries) at
+// [lo, hi) in time order, and the gate events the lane owned.  SP: pointer
+// into LDS or HBM.
+template <typename SP>
+struct Lane {
+  SP lo, hi;
+  uint32_t nown;
+};
+
+// The lanes' segments.  The tile's own words, in the merged time order of
+// its inputs, are cut into equal shares: lane l starts at the event time of
+// word floor(l * own / M).  When another tile follows, M = 63 and the last
+// lane takes the halo (the dmax window after the tile): its candidates only
+// pre-empt.  A lane's candidates pre-empt those of the lanes before it through
+// one suffix minimum over the wavefront, so no lane walks another's events.
+//
+// x[j]: index of the lane's first word in input j's range (times at or after
+// the segment's start); t0 / t1: the segment's bounds as words (time << 2).
+//   fan-in 1: the index itself.
+//   fan-in 2: binary search on the merge path's diagonal (exact: 11 steps of
+//     two LDS reads for 2,000 words).
+//   fan-in 3+: a start is an event of the leader input: its index at the
+//     leader's share of the rank, the other inputs' positions by binary
+//     search, then one correction by the rank error and a second search (the
+//     merged rank of 3..6 ranges has no direct search).
+template <int K>
+__device__ __forceinline__ void lane_bounds(const uint32_t (&in)[K], const Tile& D, uint32_t k,
+                                            uint32_t (&a)[K], uint32_t& t0, uint32_t& t1) {
+  const uint32_t lane = threadIdx.x;
+  const bool more = D.xend != 0;
+  const uint32_t d = more ? lane * D.own / 63u : lane * D.own / 64u;
+  if constexpr (K == 1) {
+    a[0] = in[0] + 4 * (1 + d);
+    t0 = lds32(a[0]) & ~3u;
+  } else if constexpr (K == 2) {
+    const uint32_t nA = D.n[0] - 1, nB = D.n[1] - 1;
+    uint32_t lo = d > nB ? d - nB : 0u, hi = min(d, nA);
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      // the mid-th word of input 0 comes before the (d - 1 - mid)-th of input 1
+      if (lds32(in[0] + 4 * mid + 4) <= lds32(in[1] + 4 * (d - mid))) lo = mid + 1;
+      else hi = mid;
     }
-  }
-  constexpr bool kGuard = !std::is_same<SP, lds_u32*>::value;
-  Lane<SP> ln;
-  ln.st = stk_base;
-  ln.sp = ln.top = ln.cnt = ln.nown = 0;
-  // Lane bounds.  The tile's nominal segments (every `stride` leader events)
-  // carry uneven numbers of input events; each lane instead takes an equal
-  // share of the tile's input words.  Lane q < m first finds the word rank
-  // of nominal boundary q; lane c then places its start at the leader event
-  // interpolated between the nominal boundaries around rank c * span / 64.
-  // Lane 0 keeps the tile's start; segment 0 of the gate starts at index 1
-  // (index 0 is the state entry) at time 0.
-  const bool gate_start = c0 == 0 && lane == 0;
-  uint32_t rq = 0xFFFFFFFFu;  // rank of nominal boundary `lane` (lanes < m)
-  if ((uint32_t)lane < m) {
-    const uint32_t pq = (c0 + lane) * X.stride;
-    if (c0 + lane == 0) {
-      rq = 0;
+    a[0] = in[0] + 4 * lo + 4;
+    a[1] = in[1] + 4 * (d - lo) + 4;
+    t0 = min(lds32(a[0]), lds32(a[1])) & ~3u;
+    // a word of the same time on the other side of the cut belongs to it
+    a[0] -= lds32(a[0] - 4) >= t0 ? 4u : 0u;
+    a[1] -= lds32(a[1] - 4) >= t0 ? 4u : 0u;
+  } else {
+    uint32_t il = in[0], nl = D.n[0];
 #pragma unroll
-      for (int j = 0; j < K; ++j) rq += 1u - X.L[j];
-    } else {
-      const uint32_t tq = srcL[pq - BL] >> 2;
-      rq = 0;
-#pragma unroll
-      for (int j = 0; j < K; ++j)
-        rq += ((uint32_t)j == X.lead ? pq : X.B[j] + lb_words(X.src[j], bound[j], tq << 2)) - X.L[j];
+    for (int j = 1; j < K; ++j) {
+      il = (uint32_t)j == D.lead() ? in[j] : il;
+      nl = (uint32_t)j == D.lead() ? D.n[j] : nl;
     }
-  }
-  const uint32_t r0 = __shfl(rq, 0);
-  const uint32_t target = r0 + (uint32_t)(((uint64_t)(X.span - r0) * (uint32_t)lane) >> 6);
-  uint32_t q = 0;  // last nominal boundary at or below the target
-#pragma unroll
-  for (uint32_t step = 32; step; step >>= 1) {
-    const uint32_t cand = q + step;
-    const uint32_t rc = __shfl(rq, (int)(cand & 63u));
-    q = (cand < m && rc <= target) ? cand : q;
-  }
-  const uint32_t r_lo = __shfl(rq, (int)q);
-  const uint32_t r_nx = __shfl(rq, (int)min(q + 1, 63u));
-  const uint32_t r_hi = q + 1 < m ? r_nx : X.span;
-  const uint32_t p_lo = (c0 + q) * X.stride;
-  const uint32_t p_hi = min((c0 + q + 1) * X.stride, EL);
-  uint32_t pi = c0 * X.stride;  // lane 0: the tile's start
-  if (lane > 0) {
-    pi = p_lo;
-    if (r_hi > r_lo && p_hi > p_lo) {
-      pi = p_lo + (uint32_t)(((uint64_t)(target - r_lo) * (p_hi - p_lo)) / (r_hi - r_lo));
-      pi = min(pi, p_hi - 1);
-    }
-  }
-  pi = max(pi, 1u);
-  const uint32_t tau_c = gate_start ? 0u : srcL[pi - BL] >> 2;
-  // the segment ends where the next lane's starts; the tile's last lane ends
-  // at the next tile's first leader event (none after the gate's last tile)
-  const uint32_t tau_next = __shfl_down(tau_c, 1);
-  uint32_t tau_n = 0x3FFFFFFFu, halo_end = 0x3FFFFFFFu;
-  if (lane < kLanes - 1) {
-    tau_n = tau_next;
-  } else if (c0 + m < X.nseg) {
-    tau_n = srcL[(c0 + m) * X.stride - BL] >> 2;
-  }
-  if (tau_n != 0x3FFFFFFFu) halo_end = tau_n + X.dmax;
-  uint32_t soff = lane, idx = 0;
-#pragma unroll
-  for (int j = 0; j < K; ++j) {
-    // pj >= 1: index 0 is the state entry, and every event time is >= 1
-    uint32_t pj;
-    if (gate_start) pj = 1;
-    else if ((uint32_t)j == X.lead) pj = pi;
-    else pj = X.B[j] + lb_words(X.src[j], bound[j], tau_c << 2);
-    soff += pj - X.L[j];
-    r[j] = pj - X.B[j];
-    idx |= (X.src[j][r[j] - 1] & 3u) << (2 * j);
-    // LDS ranges end with an INF sentinel
-    h[j] = (LDS || r[j] < bound[j]) ? X.src[j][r[j]] : INF;
-  }
-  // guarded regions: the lane's words stay below the buffer end (a lane
-  // whose offset is already past it keeps the buffer's last word)
-  const uint32_t s0 = kGuard ? min(soff, stk_words - 1) : soff;
-  const uint32_t stk_lim = stk_words - s0;
-  SP st = stk_base + s0;
-  const bool init = gate_start && first;
-  // f before the first event: X at t = 0 (src/simulate.cpp:933), else the
-  // function of the starting values
-  uint32_t fprev = init ? kX : lut_eval<K>(X, s_lut, idx);
-  uint32_t nc = 0, nown = 0, hmin = INF;
-  if (init) {  // every output starts with (0, X) (src/simulate.cpp:882-887); t = 0 is rel 1
-    st[0] = (1u << 2) | kX;
-    nc = 1;
-  }
-  // pass 1: merge and evaluate.  One step takes every input event at the
-  // next event time t (w: its smallest word) and returns the gate's value
-  // after it, its output time o and whether it is a candidate (a change).
-  auto step = [&](uint32_t w, uint32_t t, uint32_t& o, bool& cand) -> uint32_t {
-    const uint32_t lim = w | 3u;
-    uint32_t ev = 0, nidx = idx;
+    const uint32_t last = more ? D.xend : nl;  // leader index of the tile's end
+    const float r = (float)(last - 1) * __builtin_amdgcn_rcpf((float)max(D.own, 1u));
+    const bool halo = more && lane == kLanes - 1;
+    const int top = max((int)last - 1, 1);
+    int x = halo ? (int)last : min(1 + (int)((float)d * r), top);
+    // lane 0 starts with the tile, also where the leader starts later
+    t0 = lane == 0 ? 4u : lds32(il + 4 * x) & ~3u;
+    // p[j]: the last word before t0.  All inputs' searches descend together
+    // (their reads overlap) in steps of powers of two; a step past the range
+    // reads its sentinel.
+    uint32_t p[K], nmax = 1;
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-      const bool take = h[j] <= lim;
-      ev |= take ? (1u << (2 * j)) : 0u;
-      nidx = take ? ((nidx & ~(3u << (2 * j))) | ((h[j] & 3u) << (2 * j))) : nidx;
-      r[j] += take ? 1u : 0u;
+      p[j] = in[j];
+      nmax = max(nmax, (uint32_t)j < k ? D.n[j] : 0u);
+    }
+    auto descend = [&](uint32_t step) {
+      for (; step; step >>= 1) {
+        uint32_t v[K], c[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+          c[j] = p[j] + 4 * step;
+          v[j] = lds32(min(c[j], in[j] + ((uint32_t)j < k ? 4 * D.n[j] : 0u)));
+        }
+#pragma unroll
+        for (int j = 0; j < K; ++j) p[j] = v[j] < t0 && (uint32_t)j < k ? c[j] : p[j];
+      }
+    };
+    const uint32_t full = 0x80000000u >> __builtin_clz(nmax);
+    descend(full);
+    uint32_t rank = 0;
+#pragma unroll
+    for (int j = 0; j < K; ++j) rank += (uint32_t)j < k ? (p[j] - in[j]) / 4 : 0u;
+    const int dx = __float2int_rn((float)((int)d - (int)rank) * r);
+    x = halo ? x : min(max(x + dx, 1), top);
+    x = (int)wave_max_scan((uint32_t)x);  // starts stay in order
+    t0 = lane == 0 ? 4u : lds32(il + 4 * x) & ~3u;
+    // the correction is small: search 32 words around the first positions,
+    // and everywhere only when a lane's lies outside
+    uint32_t p0[K];
+    bool miss = false;
+#pragma unroll
+    for (int j = 0; j < K; ++j) p[j] = p0[j] = max(p[j], in[j] + 4 * 16) - 4 * 16;
+    descend(16);
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      if ((uint32_t)j >= k) continue;
+      // the word before p0 must be before t0 (or p0 be the range's start), and
+      // the search must not have run to its end
+      miss |= p0[j] > in[j] && lds32(p0[j]) >= t0;
+      miss |= p[j] == p0[j] + 4 * 31;
+    }
+    if (__ballot(miss)) {
+#pragma unroll
+      for (int j = 0; j < K; ++j) p[j] = in[j];
+      descend(full);
     }
 #pragma unroll
-    for (int j = 0; j < K; ++j) h[j] = (LDS || r[j] < bound[j]) ? X.src[j][r[j]] : INF;
-    const uint32_t f = lut_eval<K>(X, s_lut, nidx);
-    const uint32_t sc = edge_cls(fprev, f);
-    const uint32_t key = (((sc - 1u) & 3u) << (2 * K)) | event_bits(idx, nidx, ev);
-    idx = nidx;
-    fprev = f;
-    o = t + s_dt[key];  // sc = 0 reads a valid entry that is not used
-    cand = sc != 0u;
-    return f;
-  };
-  auto next_word = [&]() -> uint32_t {
-    uint32_t w = h[0];
+    for (int j = 0; j < K; ++j) a[j] = (uint32_t)j < k ? p[j] + 4 : in[j];
+  }
+  t1 = dpp<0x130>(t0, more ? t0 + 4 * D.dmax : 0xFFFFFFFCu);
+}
+
+// One lane's walk over its segment in LDS: merges the inputs in time order
+// and evaluates every event without branches (4-state truth table, edge
+// class and AddDelay folded into the gate's tables, WalkId); each change of
+// the gate's value is appended as a candidate word o << 2 | f.
+//
+// A step takes every input event at the next event time (w: its smallest
+// word): heads h, addresses a of the next words, last words taken pw (their
+// low bits are the inputs' values), packed by alignbit into the top bits of x
+// (the old values stay below the new ones).
+//
+// Index 0 of every range is the word before the tile, so the values before a
+// segment are the low bits of the words before its first ones.
+template <int ID, int K>
+__device__ __forceinline__ Lane<lds_u32*> lane_walk(const LevelArgs& A, const Tile& D) {
+  constexpr bool NE = ID <= W_NE6, EO = ID == W_EO3 || ID == W_EO4, GEN = ID == W_GEN;
+  const uint32_t k = GEN ? D.k() : (uint32_t)K;
+  const uint32_t lane = threadIdx.x;
+  const uint32_t ttb = 4 * walk_dt_words(ID, K);  // truth bytes; the delay table is at 0
+  uint32_t P[6], in[K], a[K];
+  range_layout(D, in_base(D), P);
 #pragma unroll
-    for (int j = 1; j < K; ++j) w = min(w, h[j]);
-    return w;
-  };
-  // the lane's own events (t < tau_n): candidates go to the stack.  The
-  // halo comes after them in time, so it gets a loop of its own and the
-  // owned steps carry none of its bookkeeping.
-  // (Both loops test at the bottom: one compare a step decides both the
-  // lanes that go on and the loop's exit.)
-  auto push = [&](uint32_t o, uint32_t f, bool cand) {
-    const bool room = !kGuard || nc < stk_lim;
-    bad |= room ? 0u : 1u;
-    st[room ? nc : stk_lim - 1] = (o << 2) | f;
-    nc += (cand && room) ? 1u : 0u;
-  };
-  uint32_t w = next_word();
-  uint32_t t = w >> 2;
+  for (int j = 0; j < K; ++j) in[j] = P[j];
+  if (GEN) {
+    // unused inputs stand at input 0's sentinel
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+      if ((uint32_t)j >= k) in[j] = P[0] + 4 * D.n[0];
+  }
+  uint32_t t0, t1;
+  lane_bounds<K>(in, D, k, a, t0, t1);
+  uint32_t h[K], pw[K], x = 0, soff = lane + min(lane, 1u);
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    h[j] = lds32(a[j]);
+    pw[j] = GEN && (uint32_t)j >= k ? 0u : lds32(a[j] - 4);
+    soff += (a[j] - in[j]) / 4 - (GEN && (uint32_t)j >= k ? 0u : 1u);
+    x = __builtin_amdgcn_alignbit(pw[j], x, 2);
+  }
+  Lane<lds_u32*> ln;
+  uint32_t sp = stack_base(A, D) + 4 * soff;
+  ln.lo = (lds_u32*)sp;
+  // the gate's value before the first event: X at t = 0 (src/simulate.cpp:933),
+  // else the function of the values
+  const bool init = D.starts_gate() && A.first && lane == 0;
+  const uint32_t fsh = ne_shift(k);
+  // NE, EO: the value before, at its place in the delay table's byte offset;
+  // GEN: the value before
+  uint32_t fp = 0;
+  if (NE) {
+    fp = lds8(ttb + (x >> (32 - 2 * K)));
+    fp = init ? 1u << ne_shift(K) : fp;
+    fp <<= K > 4 ? K - 2 : 2;
+  } else if (EO) {
+    fp = lds8(ttb + (x >> (32 - 2 * K))) >> (kEoShift + 1);
+    fp = (init ? 1u : fp) << (K + 5);
+  } else if (GEN) {
+    fp = init ? 1u : lds8(ttb + (x >> 20)) >> fsh;
+  }
+  if (init) {  // every output starts with (0, X) (src/simulate.cpp:882-887); t = 0 is rel 1
+    *(lds_u32*)sp = (1u << 2) | 1u;
+    sp += 4;
+  }
+  uint32_t w = h[0];
+#pragma unroll
+  for (int j = 1; j < K; ++j) w = min(w, h[j]);
   // look-back events (t < lo_rel, chunks after the first) come first: they
   // make candidates but are not this chunk's gate events
-  const uint32_t t_own = min(lo_rel, tau_n);
-  while (t < t_own) {
-    uint32_t o;
-    bool cand;
-    const uint32_t f = step(w, t, o, cand);
-    push(o, f, cand);
-    w = next_word();
-    t = w >> 2;
+  const uint32_t lo_w = A.lo_rel << 2;
+  uint32_t bound = t1;
+  bool look = __ballot(w < lo_w && w < t1) != 0;
+  if (look) bound = min(lo_w, t1);
+  uint32_t nown = 0;
+  // The two lookups of a step and its push are spread over the steps after it,
+  // so that a step waits only for its heads: fa, ea, la are the truth byte
+  // (being read), events and time of the step before; vb, lb, tb the delay
+  // word (being read), time and truth byte of the one before that.  The first
+  // values stand for a step without a change.
+  uint32_t fa = 0, ea = 0, la = 0, vb = 0, lb = 0, tb = 0;
+  if (NE) fa = fp >> (K > 4 ? K - 2 : 2);
+  if (EO) fa = fp >> (K + 5 - kEoShift - 1);
+  const uint32_t xs = 32 - 4 * K + 2 * D.edge_in();  // EO: the edge input's old value in x
+  auto push = [&] {
+    if constexpr (NE || EO) {
+      uint32_t o;
+      asm("v_mad_u32_u24 %0, %1, 1, %2" : "=v"(o) : "v"(vb), "v"(lb));
+      *(lds_u32*)sp = o;
+      sp += __builtin_amdgcn_ubfe(vb, 22, 3);
+    } else {
+      *(lds_u32*)sp = lb + vb + (tb & 3u);
+      sp += (tb >> 7) << 2;
+    }
+  };
+  auto look_up = [&] {
+    if constexpr (NE) {
+      vb = lds32(ea | (fa << (K > 4 ? K - 4 : 0)) | fp);
+      fp = fa << (K > 4 ? K - 2 : 2);
+    } else if constexpr (EO) {
+      vb = lds32(ea | (fa << (K + 2 - kEoShift)) | fp);
+      fp = (fa >> (kEoShift + 1)) << (K + 5);
+    } else {
+      vb = lds32((ea << (K + 2)) | (fa & (((4u << K) - 1u) << 2)));
+      tb = fa;
+    }
+    lb = la;
+  };
+  for (;;) {
+    while (w < bound) {
+      const uint32_t lim = w | 3u;
+      uint32_t e = 0;
+      const uint32_t xo = x;
+#pragma unroll
+      for (int j = 0; j < K; ++j) {
+        const bool take = K == 1 || h[j] <= lim;
+        const uint32_t s4 = take ? 4u : 0u;
+        pw[j] = take ? h[j] : pw[j];
+        a[j] += s4;
+        e |= s4 << j;
+        x = __builtin_amdgcn_alignbit(pw[j], x, 2);
+      }
+#pragma unroll
+      for (int j = 0; j < K; ++j) h[j] = lds32(a[j]);
+      if constexpr (!GEN) {
+        push();
+        look_up();
+        if constexpr (EO)
+          fa = lds8(ttb + ((__builtin_amdgcn_ubfe(x, xs, 2) << (2 * K)) | (x >> (32 - 2 * K))));
+        else
+          fa = lds8(ttb + (x >> (NE ? 32 - 2 * K : 32 - 4 * K)));
+        ea = e;
+        la = lim;
+      } else {
+        const uint32_t f = lds8(ttb + (x >> 20)) >> fsh;
+        const uint32_t sc = edge_cls(fp, f);
+        // per input: bit 2j an event, bit 2j+1 it fell (CheckDelay == 2: to 0
+        // from X/Z/1, or from 1 to X/Z)
+        const uint32_t c = x >> 20, p = xo >> 20;
+        const uint32_t cs = c << 1, ps = p << 1;
+        const uint32_t fell = (~c & ~cs & (p | ps)) | ((p & ps) & (c ^ cs));
+        uint32_t ev = 0;
+#pragma unroll
+        for (int j = 0; j < K; ++j) ev |= ((e >> (2 + j)) & 1u) << (2 * j);
+        const uint32_t bits = (fell & 0xAAAu) | ev;
+        const uint32_t b0 = bits & 63u, b1 = bits >> 6;
+        const uint32_t s0 = ((sc - 1u) & 3u) << 6;
+        const bool both = (b0 & 0x15u) && (b1 & 0x15u);
+        const uint32_t bo = both ? 256u : 0u;
+        const uint32_t d0 = lds16(2 * (bo + s0 + b0)), d1 = lds16(2 * (512u + bo + s0 + b1));
+        uint32_t dd = both ? min(d0, d1) : ((b0 & 0x15u) ? d0 : d1);
+        dd = both && dd == 0xFFFFu ? 1u : dd;
+        *(lds_u32*)sp = lim + 4 * dd - 3 + f;
+        sp += sc != 0u ? 4u : 0u;
+        fp = f;
+      }
+      ++nown;
+      w = h[0];
+#pragma unroll
+      for (int j = 1; j < K; ++j) w = min(w, h[j]);
+    }
+    if (!look) break;
+    look = false;
+    nown = 0;
+    bound = t1;
   }
-  while (t < tau_n) {  // the end of every input (INF) is never below tau_n
-    uint32_t o;
-    bool cand;
-    const uint32_t f = step(w, t, o, cand);
-    ++nown;
-    push(o, f, cand);
-    w = next_word();
-    t = w >> 2;
+  if constexpr (!GEN) {
+    push();
+    look_up();
+    push();
   }
-  // the halo (tau_n <= t < halo_end): only the smallest output time of its
-  // candidates is kept
-  while (t < halo_end) {
-    uint32_t o;
-    bool cand;
-    step(w, t, o, cand);
-    hmin = cand ? min(hmin, o) : hmin;
-    w = next_word();
-    t = w >> 2;
-  }
-  // pass 2: keep the candidates strictly earlier than every later one,
-  // compacted (in time order) to the end of the region
-  uint32_t runmin = min(hmin, hi_rel), j = nc, cnt = 0, lastv = 4u;
-  for (uint32_t i = nc; i-- > 0;) {
-    const uint32_t e = st[i];
-    const uint32_t o = e >> 2;
-    const bool keep = o >= lo_rel && o < runmin;
-    runmin = min(runmin, o);
-    st[keep ? j - 1 : i] = e;
-    j -= keep ? 1u : 0u;
-    const uint32_t v = e & 3u;
-    cnt += (keep && v != lastv) ? 1u : 0u;
-    lastv = keep ? v : lastv;
-  }
-  ln.st = st + j;
-  ln.sp = nc - j;
-  // the last kept candidate: the first one kept going backwards, now at the
-  // region's last slot
-  ln.top = j < nc ? st[nc - 1] : 0u;
-  ln.cnt = cnt;
+  ln.hi = (lds_u32*)sp;
   ln.nown = nown;
   return ln;
 }
 
-// Tile context and walk for fan-in K, then `finish` with the lanes' stacks.
-// Tiles that fit LDS read their inputs there (LDS pointers) and keep their
-// stacks in LDS or in this workgroup's slice of the stack scratch; tiles that
-// do not fit read their inputs from HBM and keep their stacks in the
-// overflow buffer.
-template <int K, typename F>
-__device__ __forceinline__ void walk_k(const LevelArgs& A, const TileDesc& D, bool fits,
-                                       uint32_t* s_in, uint32_t* s_st, const uint8_t* s_lut,
-                                       const uint16_t* s_dt, F&& finish) {
-  const int lane = threadIdx.x;
-  uint32_t B[K], E[K], L[K], pos[4], total = 0;
-  range_layout(D, pos);
+// The same walk for a tile too long for LDS: inputs read from HBM, the
+// gate's tables too, stacks in the overflow buffer, lanes at equal shares of
+// the leader's words.  Rare (a tile's words are kept to its LDS share), so it
+// is one form for every gate.  Writes that would leave the lane's buffer
+// (inputs out of order) land on its last word and set bad.
+__device__ __forceinline__ void hbm_walk(const LevelArgs& A, const Tile& D, uint32_t* stk,
+                                      uint32_t stk_words, Lane<uint32_t*>& ln, uint32_t& bad) {
+  const uint32_t lane = threadIdx.x;
+  const uint32_t k = D.k(), id = D.id();
+  const bool more = D.xend != 0;
+  const uint32_t* in[6];
+  uint32_t r[6], h[6], pw[6];
+  const uint32_t* lead = nullptr;
+  uint32_t nl = 0;
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    L[j] = D.L[j];
-    E[j] = D.E[j];
-    B[j] = range_start(L[j]);
-    total += E[j] - B[j];
+  for (uint32_t j = 0; j < kWideK; ++j) {
+    in[j] = A.pool + D.src(j);
+    if (j == D.lead()) {
+      lead = in[j];
+      nl = D.n[j];
+    }
   }
-  auto fill = [&](auto& X) {
-    X.nseg = D.nseg;
-    X.stride = D.stride;
-    X.lead = D.lead;
-    X.dmax = D.dmax;
-    X.span = D.out_cap - 1;
+  const uint32_t last = more ? D.xend : nl;  // leader index of the tile's end
+  const uint32_t M = more ? 63u : 64u;
+  const uint32_t xl = 1u + (uint32_t)((uint64_t)(last - 1) * min(lane, M) / M);
+  uint32_t t0 = xl < nl ? lead[xl] & ~3u : 0xFFFFFFFCu;
+  t0 = lane == 0 ? 4u : t0;
+  const uint32_t t1 = dpp<0x130>(t0, more ? t0 + 4 * D.dmax : 0xFFFFFFFCu);
+  uint32_t soff = lane, idx = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) X.lut[q] = D.lutw[q];
+  for (uint32_t j = 0; j < kWideK; ++j) {
+    r[j] = 0;
+    h[j] = kWordInf;
+    pw[j] = 0;
+    if (j >= k) continue;
+    r[j] = 1 + lb_words(in[j] + 1, D.n[j] - 1, t0);
+    pw[j] = in[j][r[j] - 1];
+    h[j] = r[j] < D.n[j] ? in[j][r[j]] : kWordInf;
+    soff += r[j] - 1;
+    idx |= (pw[j] & 3u) << (2 * j);
+  }
+  const uint32_t s0 = min(soff, stk_words - 1), lim_n = stk_words - s0;
+  uint32_t* st = stk + s0;
+  const uint8_t* tt = (const uint8_t*)(A.ttab + D.tt_off);
+  const uint32_t* dt = A.dtab + D.dt_off;
+  const bool ed = id == W_ED1 || id == W_ED2, eo = id == W_EO3 || id == W_EO4;
+  const uint32_t fsh = ne_shift(k);
+  const bool init = D.starts_gate() && A.first && lane == 0;
+  uint32_t fp = 1u, nc = 0, nown = 0;
+  if (init) st[nc++] = (1u << 2) | 1u;
+  else fp = ed ? tt[(idx << (2 * k)) | idx] & 3u : (uint32_t)tt[idx] >> (eo ? kEoShift + 1 : fsh);
+  for (;;) {
+    uint32_t w = h[0];
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-      X.L[j] = L[j];
-      X.E[j] = E[j];
-      X.B[j] = B[j];
+    for (uint32_t j = 1; j < kWideK; ++j) w = min(w, h[j]);
+    if (w >= t1) break;
+    const uint32_t lim = w | 3u;
+    uint32_t ev = 0, nidx = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kWideK; ++j) {
+      if (h[j] <= lim) {
+        ev |= 1u << j;
+        pw[j] = h[j];
+        ++r[j];
+        h[j] = r[j] < D.n[j] ? in[j][r[j]] : kWordInf;
+      }
+      nidx |= (pw[j] & 3u) << (2 * j);
+    }
+    uint32_t o;
+    bool cand;
+    if (ed) {
+      const uint32_t t = tt[(nidx << (2 * k)) | idx];
+      o = lim + dt[(ev << (k + 2)) | ((t >> 2) & ((4u << k) - 1u))] + (t & 3u);
+      cand = (t >> 7) != 0;
+    } else if (eo) {
+      const uint32_t old = (idx >> (2 * D.edge_in())) & 3u;
+      const uint32_t t = (uint32_t)tt[(old << (2 * k)) | nidx] >> kEoShift;
+      o = lim + (dt[(((fp << 3) | t) << k) | ev] & 0x3FFFFu);
+      cand = (t >> 1) != fp;
+      fp = t >> 1;
+    } else {
+      const uint32_t f = (uint32_t)tt[nidx] >> fsh;
+      cand = f != fp;
+      if (id != W_GEN) {
+        o = lim + (dt[(((fp << 2) | f) << k) | ev] & 0x3FFFFu);
+      } else {
+        const uint32_t sc = edge_cls(fp, f);
+        uint32_t bits = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kWideK; ++j) {
+          const uint32_t p = (idx >> (2 * j)) & 3u, c = (nidx >> (2 * j)) & 3u;
+          bits |= ((ev >> j) & 1u) << (2 * j);
+          bits |= (edge_cls(p, c) == 2u ? 2u : 0u) << (2 * j);
+        }
+        const uint32_t b0 = bits & 63u, b1 = bits >> 6, s = ((sc - 1u) & 3u) << 6;
+        const bool both = (b0 & 0x15u) && (b1 & 0x15u);
+        const uint16_t* q = (const uint16_t*)dt;
+        const uint32_t d0 = q[(both ? 256u : 0u) + s + b0], d1 = q[(both ? 768u : 512u) + s + b1];
+        uint32_t dd = both ? min(d0, d1) : ((b0 & 0x15u) ? d0 : d1);
+        dd = both && dd == 0xFFFFu ? 1u : dd;
+        o = lim + 4 * dd - 3 + f;
+      }
+      fp = f;
+    }
+    if (cand) {
+      const bool room = nc < lim_n;
+      bad |= room ? 0u : 1u;
+      st[room ? nc : lim_n - 1] = o;
+      nc += room ? 1u : 0u;
+    }
+    nown += (w >> 2) >= A.lo_rel ? 1u : 0u;
+    idx = nidx;
+  }
+  ln.lo = st;
+  ln.hi = st + nc;
+  ln.nown = nown;
+}
+
+// The preemption rule of src/simulate.cpp:990-1009 in its closed form: a
+// candidate is kept iff its output time is strictly below that of every
+// later candidate.  Backwards over the lane's candidates with a running
+// minimum, kept ones compacted (in time order) to the end of the region and
+// an entry that repeats its predecessor's value dropped; then the later
+// lanes' minimum (one suffix minimum over the wavefront) and the chunk's end
+// (candidates at or above hi_rel belong to the next chunk) cut the list from
+// the end.  Look-back candidates below lo_rel only pre-empt.
+template <typename SP>
+__device__ __forceinline__ void keep_entries(const LevelArgs& A, Lane<SP>& ln, bool halo_lane) {
+  SP q = ln.hi, jp = ln.hi;
+  uint32_t rm = 0xFFFFFFFFu, lastv = 4u, left = (uint32_t)(ln.hi - ln.lo);
+  const uint32_t lo_w = A.lo_rel << 2;
+  auto take = [&](uint32_t e) {
+    if (e < rm) {
+      rm = e & ~3u;
+      if (e >= lo_w) {
+        const uint32_t v = e & 3u;
+        jp -= v != lastv ? 1 : 0;
+        *jp = e;
+        lastv = v;
+      }
     }
   };
-  if (fits) {
-    TileCtx<K, true> X;
-    fill(X);
-    const lds_u32* in = (const lds_u32*)s_in;
+  while (left >= 4) {
+    uint32_t e4[4];  // four reads in flight
 #pragma unroll
-    for (int j = 0; j < K; ++j) X.src[j] = in + pos[j];
-    uint32_t bad = 0;
-    if (A.stk) {
-      finish(lane_walk<K, true>(X, D.ti, s_lut, s_dt, A.stk + (uint64_t)blockIdx.x * (A.cap + kLanes),
-                                A.cap + kLanes, bad, A.lo_rel, A.hi_rel, A.first != 0));
-    } else {
-      finish(lane_walk<K, true>(X, D.ti, s_lut, s_dt, (lds_u32*)s_st, A.cap + kLanes, bad, A.lo_rel,
-                                A.hi_rel, A.first != 0));
-    }
-    if (bad) atomicOr(A.err, ERR_ORDER);
-    return;
-  }
-  TileCtx<K, false> X;
-  fill(X);
+    for (int i = 0; i < 4; ++i) e4[i] = q[-1 - i];
 #pragma unroll
-  for (int j = 0; j < K; ++j) X.src[j] = A.pool + D.in_off[j];
-  unsigned long long base = 0;
-  const unsigned long long need = (unsigned long long)total + kLanes;
-  if (lane == 0) base = atomicAdd(A.ovf_used, need);
-  base = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
-         (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base);  // lane 0's value
-  if (base + need > A.ovf_cap) {
-    // no room: the tile's output is left empty (so the level's waveforms stay
-    // in time order) and the run reports the error
-    if (lane == 0) atomicOr(A.err, ERR_OVERFLOW);
-    Lane<uint32_t*> ln;
-    ln.st = A.ovf;
-    ln.sp = ln.top = ln.cnt = ln.nown = 0;
-    finish(ln);
-    return;
+    for (int i = 0; i < 4; ++i) take(e4[i]);
+    q -= 4;
+    left -= 4;
   }
-  uint32_t bad = 0;
-  finish(lane_walk<K, false>(X, D.ti, s_lut, s_dt, A.ovf + base, (uint32_t)need, bad, A.lo_rel,
-                             A.hi_rel, A.first != 0));
-  if (bad) atomicOr(A.err, ERR_ORDER);
+  if (left) {
+    uint32_t e4[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) e4[i] = (uint32_t)i < left ? q[-1 - i] : kWordInf;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) take(e4[i]);
+  }
+  const uint32_t hi_w = A.hi_rel == 0xFFFFFFFFu ? 0xFFFFFFFFu : A.hi_rel << 2;
+  const uint32_t cut = min(wave_min_after(rm), hi_w);
+  SP te = ln.hi;
+  while (te > jp && te[-1] >= cut) --te;
+  if (halo_lane) te = jp;
+  ln.lo = jp;
+  ln.hi = te;
 }
 
-// The tile's output inside the tile: wavefront scan of the lane aggregates
-// (dedup across lane boundaries is an associative monoid).
-struct TileSum {
-  Agg carry;         // everything before this lane's first entry, inside the tile
-  Agg tile;          // the whole tile
-  uint32_t e_first;  // the lane's first stack entry
-  uint32_t ft;       // time of the tile's first entry
-};
-
-template <typename SP>
-__device__ __forceinline__ TileSum combine_tile(const Lane<SP>& ln) {
-  const uint32_t sp = ln.sp;
-  const uint32_t e_first = sp ? ln.st[0] : 0u;
-  Agg mine;
-  mine.cnt = ln.cnt;
-  mine.has = sp > 0 ? 1u : 0u;
-  mine.fv = e_first & 3u;
-  mine.lv = ln.top & 3u;
-  mine.lt = ln.top >> 2;
-  const Agg inc = agg_wave_scan(mine);
-  TileSum r;
-  r.carry = agg_dpp<0x138>(inc);  // lane - 1 (empty for lane 0)
-  r.tile = agg_readlane(inc, 63);
-  r.e_first = e_first;
-  const uint64_t has = __ballot(sp > 0);
-  r.ft = has ? (uint32_t)__builtin_amdgcn_readlane(e_first, __ffsll((long long)has) - 1) >> 2 : 0u;
-  return r;
-}
-
-// Store the tile's entries (deduplicated inside the tile) at dst, sum the
-// SAIF durations between them (32 bits per lane: times < 2^30; the lanes'
-// intervals are disjoint pieces of the tile's span, so the sums fit too) and
-// write the tile summary.  out_cap: words of the tile's output region (never
-// reached for time-ordered inputs; stores beyond it are dropped and the
-// count is clamped, with ERR_ORDER).
-template <typename SP>
+// Join the lanes' lists (a list that starts with the value before it drops
+// that entry), store the tile's entries at dst, sum the SAIF durations
+// between them (32 bits per lane: times < 2^30; the lanes' intervals are
+// disjoint pieces of the tile's span, so the sums fit too) and write the tile
+// summary.  out_cap: words of the tile's output region (never reached for
+// time-ordered inputs; entries beyond it are dropped, with ERR_ORDER).
+// `before_stores` runs just before the first store.
+template <typename SP, typename F>
 __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const Lane<SP>& ln,
-                                          const TileSum& T, uint32_t* dst, uint32_t out_cap,
-                                          unsigned long long w_start, unsigned long long w_end,
-                                          unsigned long long& wave_ev) {
+                                          uint32_t* dst, uint32_t out_cap, unsigned long long w_start,
+                                          unsigned long long w_end, unsigned long long& wave_ev,
+                                          F&& before_stores) {
   const int lane = threadIdx.x;
-  const uint32_t sp = ln.sp;
-  const SP st = ln.st;
-  const Agg& carry = T.carry;
+  const uint32_t n = (uint32_t)(ln.hi - ln.lo);
+  const uint32_t e_first = n ? ln.lo[0] : 0u, e_last = n ? ln.hi[-1] : 0u;
+  const uint64_t mask = __ballot(n > 0);
+  const uint64_t below = mask & ((1ull << lane) - 1ull);
+  const uint32_t prev = __shfl(e_last, below ? 63 - __clzll((long long)below) : 0);
+  const uint32_t dup = (n && below && ((prev ^ e_first) & 3u) == 0u) ? 1u : 0u;
+  const uint32_t mine = n - dup;
+  const uint32_t incl = wave_scan(mine);
+  const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+  uint32_t ft = 0, lt = 0;  // the tile's first and last entries
+  if (mask) {
+    ft = __builtin_amdgcn_readlane(e_first, __ffsll((long long)mask) - 1);
+    lt = __builtin_amdgcn_readlane(e_last, 63 - __clzll((long long)mask));
+  }
   const uint32_t s32 = (uint32_t)min(w_start, 0x7FFFFFFFull);
   const uint32_t e32 = (uint32_t)min(w_end, 0x7FFFFFFFull);
-  uint32_t pvv = carry.has ? carry.lv : 4u;
-  uint32_t pct = max(min(carry.has ? carry.lt : (T.e_first >> 2), e32), s32);
-  const uint32_t ct0 = pct;
-  uint32_t a0 = 0, a1 = 0;
-  uint32_t w = carry.has ? carry.cnt : 0u;  // lane's first slot in the tile output
-  // four stack reads in flight per step; indices past the last entry read
-  // the last entry again, which adds nothing (same value: no store; same
-  // time: no duration), so every step takes all four
-  for (uint32_t i = 0; i < sp; i += 4) {
-    uint32_t e4[4];
+  const uint32_t w = min(incl - mine, out_cap);
+  uint32_t a0 = 0, a3 = 0;
+  uint32_t pv = below ? prev & 3u : 4u;
+  uint32_t pt = max(min((below ? prev : e_first) >> 2, e32), s32);
+  auto add = [&](uint32_t e) {
+    const uint32_t t = max(min(e >> 2, e32), s32), len = t - pt;
+    a0 += pv == 0u ? len : 0u;
+    a3 += pv == 3u ? len : 0u;
+    pv = e & 3u;
+    pt = t;
+  };
+  before_stores();
+  if (n) {
+    // the interval before the lane's first entry, which is not stored again
+    // when it repeats the value before it
+    add(e_first);
+    uint32_t* dp = dst + w;
+    uint32_t left = min(mine, out_cap - w);  // entries that the region takes
+    SP p = ln.lo + dup;
+    // whole groups of four: four reads in flight, one store
+    while (left >= 4) {
+      uint32_t e4[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) e4[q] = st[min(i + q, sp - 1)];
+      for (int q = 0; q < 4; ++q) e4[q] = p[q];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t e = e4[q];
-      const uint32_t v = e & 3u;
-      const uint32_t ct = max(min(e >> 2, e32), s32);
-      const uint32_t len = ct - pct;
-      a0 += pvv == 0u ? len : 0u;
-      a1 += pvv == 3u ? len : 0u;
-      if (v != pvv) {
-        // past out_cap (inputs out of time order: the run fails with
-        // ERR_ORDER) stores land on the region's last word
-        dst[min(w, out_cap - 1u)] = e;
-        ++w;
+      for (int q = 0; q < 4; ++q) add(e4[q]);
+      __builtin_memcpy(dp, e4, 16);
+      dp += 4;
+      p += 4;
+      left -= 4;
+    }
+    // the rest; repeating the last entry adds nothing
+    if (left) {
+      uint32_t e4[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) e4[q] = (uint32_t)q < left ? p[q] : e_last;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        add(e4[q]);
+        if ((uint32_t)q < left) dp[q] = e4[q];
       }
-      pvv = v;
-      pct = ct;
     }
   }
-  const uint32_t t0 = wave_sum(a0), t1 = wave_sum(a1), tx = wave_sum(pct - ct0 - a0 - a1);
+  const uint32_t t0 = wave_sum(a0), t1 = wave_sum(a3);
   const uint32_t ev = wave_sum(ln.nown);
   if (lane == 0) {
     TileOut o;
-    o.cnt = min(T.tile.cnt, out_cap);
-    if (T.tile.cnt > out_cap) atomicOr(A.err, ERR_ORDER);
-    o.ft = T.ft;
-    o.lt = T.tile.lt;
-    o.flags = agg_flags(T.tile);
+    o.cnt = min(total, out_cap);
+    if (total > out_cap) atomicOr(A.err, ERR_ORDER);
+    o.ft = ft >> 2;
+    o.lt = lt >> 2;
+    o.flags = out_flags(ft & 3u, lt & 3u, mask ? 1u : 0u);
     o.t0 = t0;
     o.t1 = t1;
-    o.tx = tx;
+    // the intervals between the tile's entries add up to its span
+    o.tx = max(min(lt >> 2, e32), s32) - max(min(ft >> 2, e32), s32) - t0 - t1;
     o.ev = ev;
     A.tout[tk] = o;
     wave_ev += ev;
   }
 }
 
-// A tile descriptor is read with one coalesced load (lane i < 32 holds
-// dword i) and broadcast to every lane with readlane.  The fields then live
-// in registers: no per-field loads (whose waits, s_waitcnt vmcnt, would also
-// wait for the staging DMA in flight) on the walk's path.
-__device__ __forceinline__ uint32_t desc_word(const TileDesc* p) {
-  const uint32_t lane = threadIdx.x;
-  return lane < 32 ? ((const uint32_t*)p)[lane] : 0u;
-}
-
-__device__ __forceinline__ TileDesc desc_of(uint32_t w) {
-  uint32_t f[32];
-#pragma unroll
-  for (int i = 0; i < 32; ++i) f[i] = __builtin_amdgcn_readlane(w, i);
-  TileDesc D;
-  __builtin_memcpy(&D, f, sizeof D);
-  return D;
-}
-
-// Scratch word of a tile's output region: its gate's region, then the
-// tile's first own event in the gate's merged input order plus one slack
-// word per earlier tile (a tile keeps at most its own events + 1 entries).
-__device__ __forceinline__ uint64_t tile_scratch(const uint64_t* scr_base, const TileDesc& D) {
-  uint64_t p = scr_base[D.g] + D.ti;
-#pragma unroll
-  for (uint32_t j = 0; j < 4; ++j)
-    if (j < D.k) p += D.L[j];
-  return p;
-}
-
 // Persistent, software-pipelined walk kernel.  Tiles are independent (no
 // tile waits for another): workgroup b starts with tile b and then draws
-// tickets for the next one; the next tile's inputs are staged into LDS while
-// the current tile is stored.  A static round-robin schedule left the
-// workgroups that drew many tiles too long for LDS as a long tail (14%
-// slower on the 200k-cell workload).
+// tickets for the next one.  The next tile's descriptor and ticket are on the
+// way during the walk; its inputs are staged into LDS from the end of the
+// walk on, behind the current tile's stacks, and waited for before the current
+// tile's first store (a later wait would include the stores).  A static
+// round-robin schedule left the workgroups that drew many tiles too long for
+// LDS as a long tail (14% slower on the 200k-cell workload).
 __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
-  // dynamic LDS: inputs (cap + 128 words), stacks (cap + 64, unless they are
-  // in HBM), truth table (64 words), delay table (512 words)
+  // dynamic LDS, A.lds_words: tables, inputs, ..., stacks (walk_lds_need)
   extern __shared__ uint32_t s_dyn[];
-  uint32_t* s_in = s_dyn;
-  uint32_t* s_st = A.stk ? nullptr : s_dyn + A.cap + 2 * kLanes;
-  uint32_t* s_lut = A.stk ? s_dyn + A.cap + 2 * kLanes : s_st + A.cap + kLanes;
-  uint32_t* s_dt = s_lut + 64;
-  const uint8_t* lut8 = (const uint8_t*)s_lut;
-  const uint16_t* dt16 = (const uint16_t*)s_dt;
   const int lane = threadIdx.x;
   unsigned long long wave_ev = 0;  // gate events of this wavefront (lane 0)
   unsigned long long wave_tiles = 0, wave_hbm = 0;
   const uint64_t ntiles = *A.ntiles;  // uniform: one scalar load
-  // Tiles are handed out in batches of B consecutive tiles (the first batch
-  // of workgroup b is b's, later ones come from a ticket counter): one atomic
-  // per batch instead of per tile (a single counter serves only so many
-  // atomics per second), and consecutive tiles of one gate share its tables
-  // in L2.  Small levels use B = 1 so every workgroup gets a tile.
-  const uint64_t B = max(1ull, min(8ull, (unsigned long long)(ntiles / (16ull * gridDim.x))));
-  uint64_t tk = (uint64_t)blockIdx.x * B;
-  uint64_t bend = min(tk + B, ntiles);  // end of the current batch
-  bool fits = false;
-  uint32_t dw = 0;  // descriptor of tile tk, one dword per lane
-  if (tk < ntiles) {
-    dw = desc_word(A.tiles + tk);
-    const TileDesc D0 = desc_of(dw);
-    fits = tile_words(D0) <= A.cap;
-    stage_tile(A, D0, fits, s_in, s_lut, s_dt);
-  }
-  while (tk < ntiles) {
-    const TileDesc D = desc_of(dw);
-    const bool wide = D.k > kTileK;  // uniform: the tile is k_wide's
+  // Tiles are handed out in two parts.  The first half is split into
+  // one run of consecutive tiles per workgroup (consecutive tiles of one gate
+  // keep its tables in LDS).  The rest is drawn by ticket in batches of B, so
+  // that workgroups with slow tiles take fewer and the level's tail stays
+  // short.  One counter serves about 70 M tickets a second, which held levels of
+  // short waveforms (one or two tiles a gate) to 70 M tiles a second: four
+  // counters hand out every fourth batch each, and a workgroup whose counter
+  // has run out goes on to the next.
+  const uint64_t n_run = max(1ull, (unsigned long long)(ntiles / 2 / gridDim.x));
+  const uint64_t t_drawn = n_run * gridDim.x;  // first tile handed out by ticket
+  const uint32_t B = (uint32_t)max(
+      1ull, min(8ull, (unsigned long long)((ntiles - min(t_drawn, ntiles)) / (16ull * gridDim.x))));
+  uint64_t tk = (uint64_t)blockIdx.x * n_run;
+  if (tk >= ntiles) return;
+  uint64_t bend = min(tk + n_run, ntiles);  // end of the current run or batch
+  uint32_t counter = (blockIdx.x >> 3) & (kTickets - 1), used_up = 0;
+  unsigned long long drawn = 0;  // lane 0: the drawn ticket
+  auto draw = [&] {
+    if (lane == 0 && t_drawn < ntiles) drawn = atomicAdd(A.ticket + counter * kTicketStride, 1ull);
+  };
+  auto drawn_batch = [&]() -> uint64_t {  // first tile of the drawn batch (ntiles: none left)
+    while (t_drawn < ntiles && used_up < kTickets) {
+      const uint64_t i = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(drawn >> 32)) << 32) |
+                         (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)drawn);
+      const uint64_t t = t_drawn + (counter + kTickets * i) * B;
+      if (t < ntiles) return t;
+      if (++used_up == kTickets) break;
+      counter = (counter + 1) & (kTickets - 1);
+      draw();
+    }
+    return ntiles;
+  };
+  if (tk + 1 >= bend) draw();
+  Tile D = tile_of(desc_word(A.tiles + tk));
+  bool fits = tile_fits(A, D);
+  uint32_t tab_g = 0xFFFFFFFFu;  // gate whose tables are in LDS
+  if (fits) {
+    stage_tile(A, D, true, s_dyn);
+    tab_g = D.g;
     wait_vm();
-    if (fits && !wide && lane == 0) {  // INF sentinel after every input range
-      // one lane, constant indices: the descriptor stays in registers (an
-      // index chosen by lane would put it in per-lane scratch memory)
-      uint32_t P[4];
-      range_layout(D, P);
-#pragma unroll
-      for (uint32_t j = 0; j < 4; ++j)
-        if (j < D.k) s_in[P[j] + D.E[j] - range_start(D.L[j])] = 0xFFFFFFFFu;
-    }
-    __syncthreads();
-    // the emit's scalars, loaded now so the walk covers their latency
-    uint32_t* dst = A.scratch + tile_scratch(A.scr_base, D);
-    const unsigned long long w_start = A.cwin[D.job].lo, w_end = A.cwin[D.job].hi;
-    // the next tile: the next of this batch, or the first of a batch drawn
-    // from the ticket counter (dynamic schedule: workgroups that drew slow
-    // tiles, e.g. ones too long for LDS, take fewer, so the level's tail stays
-    // short); its descriptor load completes during the walk
-    uint64_t tn = tk + 1, bend_n = bend;
+    put_sentinels(D);
+  }
+  for (;;) {
+    // the tile after this one: the next of its run, or the first of the batch
+    // drawn a tile ago
+    uint64_t tn = tk + 1;
     if (tn >= bend) {
-      uint64_t t0 = 0;
-      if (lane == 0) t0 = (uint64_t)gridDim.x * B + atomicAdd(A.ticket, (unsigned long long)B);
-      tn = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(t0 >> 32)) << 32) |
-           (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)t0);
-      bend_n = min(tn + B, ntiles);
+      tn = drawn_batch();
+      bend = min(tn + B, ntiles);
     }
-    const uint32_t dw_n = tn < ntiles ? desc_word(A.tiles + tn) : 0u;
-    bool fits_n = false;
-    auto finish = [&](const auto& ln) {
-      __syncthreads();  // inputs, truth and delay tables no longer read
-      const TileSum T = combine_tile(ln);
-      if (A.prefetch && tn < ntiles) {  // stage the next tile while this one is stored
-        const TileDesc Dn = desc_of(dw_n);
-        fits_n = tile_words(Dn) <= A.cap;
-        stage_tile(A, Dn, fits_n, s_in, s_lut, s_dt);
-      }
-      emit_tile(A, tk, ln, T, dst, D.out_cap, w_start, w_end, wave_ev);
+    const bool more_tiles = tn < ntiles;
+    const uint32_t dwn = more_tiles ? desc_word(A.tiles + tn) : 0u;
+    if (more_tiles && tn + 1 >= bend) draw();
+    const ChunkWin* W = A.cwin + D.job;
+    const unsigned long long w_start = W->lo, w_end = W->hi;
+    lds_fence();
+    Tile Dn = D;
+    bool fits_n = false, staged = false;
+    auto stage_next = [&] {
+      if (!fits_n || staged) return;
+      stage_tile(A, Dn, Dn.g != tab_g, s_dyn);
+      tab_g = Dn.g;
+      staged = true;
     };
-    switch (wide ? 0u : D.k) {
-      case 0: break;
-      case 1: walk_k<1>(A, D, fits, s_in, s_st, lut8, dt16, finish); break;
-      case 2: walk_k<2>(A, D, fits, s_in, s_st, lut8, dt16, finish); break;
-      case 3: walk_k<3>(A, D, fits, s_in, s_st, lut8, dt16, finish); break;
-      default: walk_k<4>(A, D, fits, s_in, s_st, lut8, dt16, finish); break;
+    auto finish = [&](auto& ln) {
+      // inputs and tables are no longer read
+      lds_fence();
+      if (more_tiles) {
+        Dn = tile_of(dwn);
+        fits_n = tile_fits(A, Dn);
+        if (A.prefetch &&
+            !(fits && in_base(Dn) + 4 * (Dn.words() + 8 * Dn.k()) > stack_base(A, D)))
+          stage_next();
+      }
+      const bool halo = D.xend != 0 && lane == kLanes - 1;
+      keep_entries(A, ln, halo);
+      if (halo) ln.nown = 0;
+      emit_tile(A, tk, ln, A.scratch + D.scr, D.out_cap, w_start, w_end, wave_ev, [&] {
+        if (staged) {
+          wait_vm();
+          put_sentinels(Dn);
+        }
+      });
+    };
+    if (fits) {
+      Lane<lds_u32*> ln;
+      switch (D.id()) {
+        case W_NE1: ln = lane_walk<W_NE1, 1>(A, D); break;
+        case W_NE2: ln = lane_walk<W_NE2, 2>(A, D); break;
+        case W_NE3: ln = lane_walk<W_NE3, 3>(A, D); break;
+        case W_NE4: ln = lane_walk<W_NE4, 4>(A, D); break;
+        case W_NE5: ln = lane_walk<W_NE5, 5>(A, D); break;
+        case W_NE6: ln = lane_walk<W_NE6, 6>(A, D); break;
+        case W_EO3: ln = lane_walk<W_EO3, 3>(A, D); break;
+        case W_EO4: ln = lane_walk<W_EO4, 4>(A, D); break;
+        case W_ED1: ln = lane_walk<W_ED1, 1>(A, D); break;
+        case W_ED2: ln = lane_walk<W_ED2, 2>(A, D); break;
+        default: ln = lane_walk<W_GEN, 6>(A, D); break;
+      }
+      finish(ln);
+    } else {
+      Lane<uint32_t*> ln;
+      ln.lo = ln.hi = A.ovf;
+      ln.nown = 0;
+      if (D.id() < W_COUNT) {
+        const unsigned long long need = (unsigned long long)D.words() + kStackSlack;
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(A.ovf_used, need);
+        base = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
+               (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base);  // lane 0's value
+        uint32_t bad = 0;
+        if (base + need > A.ovf_cap) {
+          // no room: the tile's output is left empty (so the level's waveforms
+          // stay in time order) and the run reports the error
+          if (lane == 0) atomicOr(A.err, ERR_OVERFLOW);
+        } else {
+          hbm_walk(A, D, A.ovf + base, (uint32_t)need, ln, bad);
+        }
+        if (bad) atomicOr(A.err, ERR_ORDER);
+      }
+      finish(ln);
     }
-    if ((wide || !A.prefetch) && tn < ntiles) {
-      __syncthreads();
-      const TileDesc Dn = desc_of(dw_n);
-      fits_n = tile_words(Dn) <= A.cap;
-      stage_tile(A, Dn, fits_n, s_in, s_lut, s_dt);
+    if (more_tiles && fits_n && !staged) {
+      lds_fence();
+      stage_next();
+      wait_vm();
+      put_sentinels(Dn);
     }
-    __syncthreads();
+    lds_fence();
     ++wave_tiles;
     wave_hbm += fits ? 0u : 1u;
+    if (!more_tiles) break;
     tk = tn;
-    bend = bend_n;
     fits = fits_n;
-    dw = dw_n;
+    D = Dn;
   }
-  if (lane == 0 && wave_ev) atomicAdd(A.ev_count, wave_ev);
-  if (lane == 0 && wave_tiles) {
+  if (lane == 0) {
+    if (wave_ev) atomicAdd(A.ev_count, wave_ev);
     atomicAdd(A.tiles_walked, wave_tiles);
     if (wave_hbm) atomicAdd(A.tiles_walked + 1, wave_hbm);
   }
@@ -874,7 +1062,7 @@ __global__ void k_gate_carry(const GateRec* __restrict__ gates, uint32_t ng,
     lv = T.tails[T.tail_off[G.out_net] + tl - 1] & 3u;
     has = 1;
   }
-  unsigned long long acc[3] = {0, 0, 0}, tc = 0, gev = 0;
+  unsigned long long acc[3] = {0, 0, 0}, tc = 0, gev = 0, any = 0;
   for (uint64_t c = 0; c < n; c += 64) {
     const bool in = c + (uint64_t)lane < n;
     const uint64_t t = t0 + c + (uint64_t)lane;
@@ -899,8 +1087,11 @@ __global__ void k_gate_carry(const GateRec* __restrict__ gates, uint32_t ng,
       acc[2] += S.tx;
       // the tile's first entry against the previous tile's last value
       tc += (p_has && is_toggle(p_lv, my_fv) && S.ft > W.tc_lo && S.ft <= W.tc_hi) ? 1u : 0u;
-      gev += S.ev;
     }
+    // an instance counts the events of its tiles with entries; the tiles of a
+    // wide gate count as one
+    gev += ne || G.k > kTileK ? S.ev : 0u;
+    any |= mask;
     // inclusive scan of the joined counts over the step
     uint32_t incl = mine;
 #pragma unroll
@@ -930,7 +1121,7 @@ __global__ void k_gate_carry(const GateRec* __restrict__ gates, uint32_t ng,
     sa[2] = s2;
     sa[3] = s3;
     // a level whose tiles ran out of overflow stacks runs again: count it then
-    if (ev_job && s4 && !(*err & ERR_OVERFLOW)) atomicAdd(ev_job + G.job, s4);
+    if (ev_job && s4 && any && !(*err & ERR_OVERFLOW)) atomicAdd(ev_job + G.job, s4);
   }
 }
 
@@ -942,7 +1133,7 @@ __global__ void k_gate_carry(const GateRec* __restrict__ gates, uint32_t ng,
 // waveforms are left empty.
 __global__ void k_compact(const TileDesc* __restrict__ tiles, const uint64_t* __restrict__ ntiles,
                           const TileOut* __restrict__ tout, const uint32_t* __restrict__ tile_off,
-                          const uint64_t* __restrict__ scr_base, const uint32_t* __restrict__ scratch,
+                          const uint32_t* __restrict__ scratch,
                           const uint64_t* __restrict__ gate_base, uint32_t* __restrict__ pool,
                           uint64_t* __restrict__ woff, uint32_t* __restrict__ wlen,
                           const unsigned int* __restrict__ err, unsigned long long* __restrict__ saif,
@@ -974,7 +1165,7 @@ __global__ void k_compact(const TileDesc* __restrict__ tiles, const uint64_t* __
     if (!((S.flags >> 4) & 1u)) continue;
     const uint32_t off = tile_off[t] & 0x7FFFFFFFu, skip = tile_off[t] >> 31;
     const uint32_t n = S.cnt - skip;
-    const uint32_t* src = scratch + tile_scratch(scr_base, D) + skip;
+    const uint32_t* src = scratch + (((uint64_t)D.scr_hi << 32) | D.scr_lo) + skip;
     uint32_t* dst = pool + gate_base[D.g] + off;
     // four loads in flight per lane before their stores: the copy of a tile
     // waits for memory about n / 256 times instead of n / 64
@@ -1004,158 +1195,19 @@ __global__ void k_compact(const TileDesc* __restrict__ tiles, const uint64_t* __
   }
 }
 
-// Wide gates (5 or 6 distinct inputs): one thread walks a gate's whole
-// chunk, with the walk's rules in sequence (the same merge, truth table,
-// edge class, AddDelay per input, preemption in closed form, chunk
-// bounds), and leaves its tile output and summary exactly as a one-tile
-// lane walk would (k_gate_carry and k_compact then treat it like any other
-// tile).  The candidates are built in the tile's output region itself
-// (it holds every input word + 1) and compacted in place.
-__global__ void k_wide(WideArgs A) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= A.nwide) return;
-  // a level over the captured capacities was skipped (no descriptors)
-  if (*A.err & ERR_CAPACITY) return;
-  const uint32_t g = A.wide[i] - A.g0;
-  const GateRec& G = A.gates[g];
-  const uint64_t tk = A.tile_base[g];
-  const uint32_t cap = A.tiles[tk].out_cap;
-  uint32_t* st = A.scratch + A.scr_base[g];
-  const uint8_t* lut = A.luts + (uint32_t)G.lut * 256u;
-  const uint16_t* tab = A.dtab + G.dt_off;
-  const uint32_t k = G.k;
-  const uint32_t kX = 1u, INF = 0xFFFFFFFFu;
-  const uint32_t* in[kWideK];
-  uint32_t n[kWideK], r[kWideK], h[kWideK];
-  uint32_t idx = 0;
-#pragma unroll
-  for (uint32_t j = 0; j < kWideK; ++j) {
-    if (j < k) {
-      in[j] = A.pool + A.woff[G.in_net[j]];
-      n[j] = A.wlen[G.in_net[j]];
-      idx |= (in[j][0] & 3u) << (2 * j);  // the state entry
-      r[j] = 1;
-      h[j] = n[j] > 1 ? in[j][1] : INF;
-    } else {
-      in[j] = nullptr;
-      n[j] = r[j] = 0;
-      h[j] = INF;
-    }
-  }
-  const bool init = A.first != 0;
-  uint32_t fprev = init ? kX : lut[idx];
-  uint32_t nc = 0, nown = 0, bad = 0;
-  if (init) st[nc++] = (1u << 2) | kX;  // (0, X) at rel 1; cap >= 1
-  for (;;) {
-    uint32_t w = h[0];
-#pragma unroll
-    for (uint32_t j = 1; j < kWideK; ++j) w = min(w, h[j]);
-    const uint32_t t = w >> 2;
-    if (t >= 0x3FFFFFFFu) break;  // every input at its end
-    const uint32_t lim = w | 3u;
-    uint32_t mask = 0, nidx = idx;
-#pragma unroll
-    for (uint32_t j = 0; j < kWideK; ++j) {
-      if (h[j] <= lim) {
-        mask |= 1u << j;
-        nidx = (nidx & ~(3u << (2 * j))) | ((h[j] & 3u) << (2 * j));
-        ++r[j];
-        h[j] = r[j] < n[j] ? in[j][r[j]] : INF;
-      }
-    }
-    const uint32_t f = lut[nidx];
-    const uint32_t sc = edge_cls(fprev, f);
-    if (sc != 0u) {
-      uint32_t d;
-      if ((mask & (mask - 1u)) == 0u) {
-        const uint32_t j = __builtin_ctz(mask);
-        const uint32_t p = (idx >> (2 * j)) & 3u, c = (nidx >> (2 * j)) & 3u;
-        const uint32_t fell = ((c == 0u && p != 0u) || (p == 3u && (c == 1u || c == 2u))) ? 1u : 0u;
-        d = tab[wide_dt_index(j, sc, fell, 1)];
-      } else {
-        uint32_t m = 0xFFFFu;
-#pragma unroll
-        for (uint32_t j = 0; j < kWideK; ++j) {
-          if (!((mask >> j) & 1u)) continue;
-          const uint32_t p = (idx >> (2 * j)) & 3u, c = (nidx >> (2 * j)) & 3u;
-          const uint32_t fell = ((c == 0u && p != 0u) || (p == 3u && (c == 1u || c == 2u))) ? 1u : 0u;
-          m = min(m, (uint32_t)tab[wide_dt_index(j, sc, fell, 0)]);
-        }
-        d = m == 0xFFFFu ? 1u : m;
-      }
-      if (nc < cap) st[nc++] = ((t + d) << 2) | f;
-      else bad = 1;
-    }
-    nown += t >= A.lo_rel ? 1u : 0u;
-    idx = nidx;
-    fprev = f;
-  }
-  // keep the candidates strictly earlier than every later one (and inside
-  // [lo_rel, hi_rel)), compacted in time order to the end of the list
-  uint32_t runmin = A.hi_rel, jj = nc, cnt = 0, top = 0, lastv = 4u, has = 0;
-  for (uint32_t q = nc; q-- > 0;) {
-    const uint32_t e = st[q];
-    const uint32_t o = e >> 2;
-    const bool keep = o >= A.lo_rel && o < runmin;
-    runmin = min(runmin, o);
-    if (keep) {
-      st[--jj] = e;
-      cnt += (e & 3u) != lastv ? 1u : 0u;
-      lastv = e & 3u;
-      if (!has) top = e;
-      has = 1;
-    }
-  }
-  // entries (deduplicated) to the front of the region, SAIF durations
-  // between them, summary
-  const ChunkWin W = A.cwin[G.job];
-  const uint32_t s32 = (uint32_t)min(W.lo, 0x7FFFFFFFull);
-  const uint32_t e32 = (uint32_t)min(W.hi, 0x7FFFFFFFull);
-  const uint32_t sp = nc - jj;
-  const uint32_t e_first = sp ? st[jj] : 0u;
-  uint32_t pvv = 4u, pct = max(min(e_first >> 2, e32), s32);
-  const uint32_t ct0 = pct;
-  uint32_t a0 = 0, a1 = 0, wpos = 0;
-  for (uint32_t q = 0; q < sp; ++q) {
-    const uint32_t e = st[jj + q];
-    const uint32_t v = e & 3u;
-    const uint32_t ct = max(min(e >> 2, e32), s32);
-    const uint32_t len = ct - pct;
-    a0 += pvv == 0u ? len : 0u;
-    a1 += pvv == 3u ? len : 0u;
-    if (v != pvv) st[wpos++] = e;  // wpos <= q <= jj + q: read before written
-    pvv = v;
-    pct = ct;
-  }
-  TileOut o;
-  o.cnt = min(cnt, cap);
-  o.ft = sp ? e_first >> 2 : 0u;
-  o.lt = has ? top >> 2 : 0u;
-  o.flags = has ? ((e_first & 3u) | ((top & 3u) << 2) | (1u << 4)) : 0u;
-  o.t0 = a0;
-  o.t1 = a1;
-  o.tx = pct - ct0 - a0 - a1;
-  o.ev = nown;
-  A.tout[tk] = o;
-  if (cnt > cap || bad) atomicOr(A.err, ERR_ORDER);
-  if (nown) atomicAdd(A.ev_count, (unsigned long long)nown);
-}
-
-hipError_t launch_wide(const WideArgs& a, hipStream_t st) {
-  if (a.nwide == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_wide, dim3((a.nwide + 63) / 64), dim3(64), 0, st, a);
-  return hipGetLastError();
-}
-
 // Start-of-run scalars: bump pointer past the stimulus words, all else 0.
 __global__ void k_set_scal(uint64_t* scal, uint64_t bump) {
   if (blockIdx.x == 0 && threadIdx.x < 16) scal[threadIdx.x] = threadIdx.x == 0 ? bump : 0;
 }
 
-// per gate: leader, stride, segments, tiles, output bound
+// Per gate: leader (the input with the most words), words of the leader per
+// tile, tiles, output bound.  A tile of a gate of fan-in 1..4 holds 64 times
+// the leader's words of a lane share of about seg_target input words, spread
+// evenly over the gate's tiles; a wide gate's tiles hold wide_words input words
+// (its tables leave less LDS).
 __global__ void k_plan2(const GateRec* __restrict__ gates, uint32_t ng,
                         const uint32_t* __restrict__ wlen, uint32_t seg_target,
-                        GatePlan* __restrict__ plan, uint64_t* __restrict__ ntile,
+                        uint32_t wide_words, GatePlan* __restrict__ plan, uint64_t* __restrict__ ntile,
                         uint64_t* __restrict__ bound, unsigned int* __restrict__ err,
                         const uint32_t* __restrict__ tail_len) {
   uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1173,35 +1225,22 @@ __global__ void k_plan2(const GateRec* __restrict__ gates, uint32_t ng,
   }
   // a tile's offset inside its gate's waveform travels in 31 bits
   if (N + 1 >= (1ull << 30)) atomicOr(err, ERR_RANGE);
-  if (G.k > kTileK) {  // wide gate: one tile, walked by k_wide
-    GatePlan P;
-    P.nseg = 1;
-    P.stride = nl > 0 ? nl : 1u;
-    P.lead = lead;
-    P.pad = 0;
-    plan[g] = P;
-    ntile[g] = 1;
-    bound[g] = N + 2 + tail_len[G.out_net];
-    return;
-  }
-  // leader events per segment so that a segment holds ~seg_target input
-  // events; then the gate's tiles are filled evenly (the stride that spreads
-  // the leader's events over all 64 segments of each of those tiles, never
-  // larger), so a small gate's single tile uses every lane
-  uint64_t s = N > 0 ? (uint64_t)seg_target * nl / N : 1;
-  if (s < 1) s = 1;
-  if (nl > 0) {
-    const uint64_t nt0 = ((nl + s - 1) / s + kLanes - 1) / kLanes;
-    s = (nl + nt0 * kLanes - 1) / (nt0 * kLanes);
-  }
-  uint32_t ns = nl > 0 ? (uint32_t)((nl + s - 1) / s) : 1u;
   GatePlan P;
-  P.nseg = ns;
-  P.stride = (uint32_t)s;
+  if (G.k > kTileK) {
+    const uint32_t nt0 = (uint32_t)max<uint64_t>(1, (N + wide_words - 1) / wide_words);
+    P.lt = max(1u, (nl + nt0 - 1) / nt0);
+  } else {
+    uint64_t s = N > 0 ? (uint64_t)seg_target * nl / N : 1;
+    if (s < 1) s = 1;
+    if (nl > 0) {
+      const uint64_t nt0 = ((nl + s - 1) / s + kLanes - 1) / kLanes;
+      s = (nl + nt0 * kLanes - 1) / (nt0 * kLanes);
+    }
+    P.lt = (uint32_t)min<uint64_t>(s * kLanes, 0xFFFFFFFFu);
+  }
   P.lead = lead;
-  P.pad = 0;
   plan[g] = P;
-  const uint32_t nt = (ns + kLanes - 1) / kLanes;
+  const uint32_t nt = max(1u, (uint32_t)(((uint64_t)nl + P.lt - 1) / P.lt));
   ntile[g] = nt;
   // scratch words of the gate's tile outputs: every tile keeps at most its
   // own input events + 1 entries; the gate's tail is added so that the
@@ -1209,26 +1248,31 @@ __global__ void k_plan2(const GateRec* __restrict__ gates, uint32_t ng,
   bound[g] = N + nt + 1 + tail_len[G.out_net];
 }
 
-// per (tile, input): the tile's descriptor (gate, tile index within the
-// gate, segmentation, tables) and input j's range
+// Per tile: its descriptor; thread j of the tile's four takes inputs j and
+// j + 4.
 __global__ void k_tile_desc(const GateRec* __restrict__ gates, uint32_t ng,
                             const GatePlan* __restrict__ plan,
                             const uint64_t* __restrict__ tile_base,
+                            const uint64_t* __restrict__ scr_base,
                             const uint64_t* __restrict__ woff, const uint32_t* __restrict__ wlen,
-                            const uint32_t* __restrict__ pool, const uint32_t* __restrict__ lutp,
-                            TileDesc* __restrict__ tiles, const uint64_t* __restrict__ ntiles) {
+                            const uint32_t* __restrict__ pool, TileDesc* __restrict__ tiles,
+                            const uint64_t* __restrict__ ntiles, unsigned long long* __restrict__ ticket,
+                            unsigned long long* __restrict__ ovf_used) {
+  // the walk's tickets and overflow stacks start over
+  if (blockIdx.x == 0 && threadIdx.x < kTickets) ticket[threadIdx.x * kTicketStride] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *ovf_used = 0;
   // a tile's first own word of each input is the previous tile's end: the
   // block's tiles pass them on through LDS (each boundary searched once)
-  __shared__ uint32_t s_first[256];
+  __shared__ uint32_t s_first[2][256];
   const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t t = x >> 2;
-  const int j = (int)(x & 3);
+  const int j0 = (int)(x & 3);
   const uint64_t nt = *ntiles;
   const bool valid = t < nt;
   // gate of tile t: binary search over tile_base by the tile's first
   // thread, passed to the other three
   uint32_t g = 0;
-  if (valid && j == 0) {
+  if (valid && j0 == 0) {
     uint32_t lo = 0, hi = ng;
     while (hi - lo > 1) {
       uint32_t mid = (lo + hi) >> 1;
@@ -1240,70 +1284,55 @@ __global__ void k_tile_desc(const GateRec* __restrict__ gates, uint32_t ng,
   g = __shfl(g, (int)((threadIdx.x & 63u) & ~3u));
   GateRec G;
   GatePlan P;
-  uint32_t ti = 0, L = 0, c0 = 0, clast = 0, n = 0;
+  uint32_t ti = 0, nl = 0, L[2] = {0, 0};
   const uint32_t* lw = nullptr;
-  const uint32_t* iw = nullptr;
-  bool narrow_in = false;  // input j of a gate of fan-in <= 4
   if (valid) {
     G = gates[g];
     P = plan[g];
     ti = (uint32_t)(t - tile_base[g]);
-    narrow_in = G.k <= kTileK && (uint32_t)j < G.k;
-    if (narrow_in) {
-      lw = pool + woff[G.in_net[P.lead]];
-      iw = pool + woff[G.in_net[j]];
-      n = wlen[G.in_net[j]];
-      c0 = ti * kLanes;
-      clast = min(c0 + kLanes - 1, P.nseg - 1);
-      if (c0 > 0) {
-        const uint32_t tau_lo = lw[c0 * P.stride] >> 2;
-        L = (uint32_t)j == P.lead ? c0 * P.stride : lb_words(iw, n, tau_lo << 2);
+    lw = pool + woff[G.in_net[P.lead]];
+    nl = wlen[G.in_net[P.lead]];
+    if (ti > 0) {
+      const uint32_t tau_lo = lw[ti * P.lt] >> 2;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint32_t j = j0 + 4 * q;
+        if (j < G.k)
+          L[q] = j == P.lead ? ti * P.lt
+                             : lb_words(pool + woff[G.in_net[j]], wlen[G.in_net[j]], tau_lo << 2);
       }
     }
   }
-  s_first[threadIdx.x] = L;
+  s_first[0][threadIdx.x] = L[0];
+  s_first[1][threadIdx.x] = L[1];
   __syncthreads();
   if (!valid) return;
   TileDesc& D = tiles[t];
-  D.lutw[j] = lutp[(uint32_t)G.lut * 16u + j];
-  if (j == 0) {
-    D.g = g;
-    D.ti = ti;
-    D.nseg = P.nseg;
-    D.stride = P.stride;
-    D.lead = P.lead;
-    D.k = G.k;
-    D.dt_off = G.dt_off;
-    D.lut = G.lut;
-    D.dmax = G.dmax;
-    D.out_net = G.out_net;
-    D.job = G.job;
-  }
   // own input words of the tile (up to the next tile's first words), summed
-  // over the tile's four threads: its output region in the level scratch
-  // holds that many entries plus one
-  uint32_t span = 0;
-  if (G.k > kTileK) {
-    // wide gate (one tile): no staged ranges; the output region holds all
-    // input words + 1 (threads 0 and 1 also count inputs 4 and 5)
-    D.L[j] = 0;
-    D.E[j] = 0;
-    D.in_off[j] = 0;
-    span = wlen[G.in_net[j]];
-    if ((uint32_t)j + 4 < G.k) span += wlen[G.in_net[j + 4]];
-  } else if (!narrow_in) {
-    D.L[j] = 0;
-    D.E[j] = 0;
-    D.in_off[j] = 0;
-  } else {
+  // over the tile's threads: its output region in the level scratch holds
+  // that many entries plus one
+  uint32_t span = 0, own = 0, xend = 0, dead = 0, lsum = 0, hi8[2] = {0, 0};
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const uint32_t j = j0 + 4 * q;
+    if (j >= G.k) {
+      if (j < kWideK) {
+        D.in_lo[j] = 0;
+        D.n[j] = 0;
+      }
+      continue;
+    }
+    const uint64_t off = woff[G.in_net[j]];
+    const uint32_t n = wlen[G.in_net[j]];
+    const uint32_t* iw = pool + off;
     uint32_t E = n, Ln = n;
-    if (clast + 1 < P.nseg) {
+    if ((ti + 1) * (uint64_t)P.lt < nl) {
       // the next tile is this gate's: its first words end this one
-      const uint32_t tau_nx = lw[(clast + 1) * P.stride] >> 2;
+      const uint32_t tau_nx = lw[(ti + 1) * P.lt] >> 2;
       if (threadIdx.x + 4 < blockDim.x && t + 1 < nt)
-        Ln = s_first[threadIdx.x + 4];
+        Ln = s_first[q][threadIdx.x + 4];
       else
-        Ln = (uint32_t)j == P.lead ? (clast + 1) * P.stride : lb_words(iw, n, tau_nx << 2);
+        Ln = j == P.lead ? (ti + 1) * P.lt : lb_words(iw, n, tau_nx << 2);
       // halo end: the first word at or after tau_nx + dmax lies at or after
       // Ln, usually at it; step forward with doubling strides, then search
       // only inside the last stride (every word before a is below the key)
@@ -1319,15 +1348,49 @@ __global__ void k_tile_desc(const GateRec* __restrict__ gates, uint32_t ng,
         if (b > n) b = n;
         E = a + 1 + lb_words(iw + a + 1, b - a - 1, key);
       }
+      if (j == P.lead) xend = (ti + 1) * P.lt - (L[q] > 0 ? L[q] - 1 : 0u);
     }
-    D.L[j] = L;
-    D.E[j] = E;
-    D.in_off[j] = woff[G.in_net[j]] + (L > 0 ? L - 1 : 0u);
-    span = Ln - L;
+    const uint32_t B = L[q] > 0 ? L[q] - 1 : 0u;
+    D.in_lo[j] = (uint32_t)(off + B);
+    D.n[j] = E - B;
+    hi8[q] = (uint32_t)((off + B) >> 32) << (8 * j0);
+    span += Ln - L[q];
+    own += Ln - max(L[q], 1u);
+    lsum += L[q];
+    dead |= n == 0 ? 1u : 0u;
   }
-  span += __shfl_xor(span, 1);
-  span += __shfl_xor(span, 2);
-  if (j == 0) D.out_cap = span + 1;
+#pragma unroll
+  for (int d = 1; d < 4; d <<= 1) {
+    span += __shfl_xor(span, d);
+    own += __shfl_xor(own, d);
+    xend |= __shfl_xor(xend, d);
+    dead |= __shfl_xor(dead, d);
+    lsum += __shfl_xor(lsum, d);
+    hi8[0] |= __shfl_xor(hi8[0], d);
+    hi8[1] |= __shfl_xor(hi8[1], d);
+  }
+  if (j0 == 0) {
+    D.in_hi[0] = hi8[0];
+    D.in_hi[1] = hi8[1];
+    // a gate's region, then the tile's first own event in the gate's merged
+    // input order plus one slack word per earlier tile (a tile keeps at most
+    // its own events + 1 entries)
+    const uint64_t scr = scr_base[g] + ti + lsum;
+    D.scr_lo = (uint32_t)scr;
+    D.scr_hi = (uint32_t)(scr >> 32);
+    D.own = dead ? 0u : own;
+    D.xend = xend;
+    D.meta = (dead ? (uint32_t)W_DEAD : (uint32_t)G.walk) | ((uint32_t)G.k << 4) | (P.lead << 8) |
+             ((ti == 0 ? 1u : 0u) << 12) | (G.edge_in << 16);
+    D.dt_off = G.dt_off;
+    D.tt_off = G.tt_off;
+    D.dmax = G.dmax;
+    D.job = G.job;
+    D.out_cap = span + 1;
+    D.g = g;
+    D.ti = ti;
+    D.out_net = G.out_net;
+  }
 }
 
 __global__ void k_fill_u64(unsigned long long* p, uint64_t n, unsigned long long v) {
@@ -1336,21 +1399,22 @@ __global__ void k_fill_u64(unsigned long long* p, uint64_t n, unsigned long long
 }
 
 hipError_t launch_plan2(const GateRec* gates, uint32_t ng, const uint32_t* wlen,
-                        uint32_t seg_target, GatePlan* plan, uint64_t* ntile, uint64_t* bound,
+                        uint32_t seg_target, uint32_t wide_words, GatePlan* plan, uint64_t* ntile, uint64_t* bound,
                         unsigned int* err, const uint32_t* tail_len, hipStream_t st) {
-  k_plan2<<<(ng + 255) / 256, 256, 0, st>>>(gates, ng, wlen, seg_target, plan, ntile, bound, err,
-                                            tail_len);
+  k_plan2<<<(ng + 255) / 256, 256, 0, st>>>(gates, ng, wlen, seg_target, wide_words, plan, ntile, bound,
+                                            err, tail_len);
   return hipGetLastError();
 }
 
 hipError_t launch_tile_desc(const GateRec* gates, uint32_t ng, const GatePlan* plan,
-                            const uint64_t* tile_base, const uint64_t* woff, const uint32_t* wlen,
-                            const uint32_t* pool, const uint32_t* lutp, TileDesc* tiles,
-                            const uint64_t* ntiles_dev, uint64_t ntiles, hipStream_t st) {
+                            const uint64_t* tile_base, const uint64_t* scr_base,
+                            const uint64_t* woff, const uint32_t* wlen, const uint32_t* pool,
+                            TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles,
+                            unsigned long long* ticket, unsigned long long* ovf_used, hipStream_t st) {
   if (ntiles == 0) return hipSuccess;
   const uint64_t threads = ntiles * 4;
-  k_tile_desc<<<(unsigned)((threads + 255) / 256), 256, 0, st>>>(gates, ng, plan, tile_base, woff,
-                                                                  wlen, pool, lutp, tiles, ntiles_dev);
+  k_tile_desc<<<(unsigned)((threads + 255) / 256), 256, 0, st>>>(
+      gates, ng, plan, tile_base, scr_base, woff, wlen, pool, tiles, ntiles_dev, ticket, ovf_used);
   return hipGetLastError();
 }
 
@@ -1402,16 +1466,15 @@ hipError_t launch_gate_carry(const GateRec* gates, uint32_t ng, const uint64_t* 
 }
 
 hipError_t launch_compact(const TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles_cap,
-                          const TileOut* tout, const uint32_t* tile_off, const uint64_t* scr_base,
+                          const TileOut* tout, const uint32_t* tile_off,
                           const uint32_t* scratch, const uint64_t* gate_base, uint32_t* pool,
                           uint64_t* woff, uint32_t* wlen, const unsigned int* err,
                           unsigned long long* saif, const ChunkWin* cwin, uint32_t count_tc,
                           const TailArgs& T, hipStream_t st) {
   if (ntiles_cap == 0) return hipSuccess;
   const uint64_t blocks = std::min<uint64_t>((ntiles_cap + 3) / 4, 8192);  // 4 wavefronts each
-  k_compact<<<(unsigned)blocks, 256, 0, st>>>(tiles, ntiles_dev, tout, tile_off, scr_base, scratch,
-                                              gate_base, pool, woff, wlen, err, saif, cwin, count_tc,
-                                              T);
+  k_compact<<<(unsigned)blocks, 256, 0, st>>>(tiles, ntiles_dev, tout, tile_off, scratch, gate_base,
+                                              pool, woff, wlen, err, saif, cwin, count_tc, T);
   return hipGetLastError();
 }
 
@@ -1428,20 +1491,21 @@ hipError_t launch_set_scal(uint64_t* scal, uint64_t bump, hipStream_t st) {
 
 hipError_t launch_level(const LevelArgs& a, unsigned nblocks, hipStream_t st) {
   if (nblocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_level, dim3(nblocks), dim3(kLanes), level_lds_bytes(a.cap, a.stk == nullptr),
-                     st, a);
+  hipLaunchKernelGGL(k_level, dim3(nblocks), dim3(kLanes), a.lds_words * 4, st, a);
   return hipGetLastError();
 }
 
-int level_max_blocks(uint32_t cap, bool stacks_in_lds) {
+int level_max_blocks(uint32_t lds_words) {
   int per_cu = 0, dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 2048;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_level, kLanes,
-                                                   level_lds_bytes(cap, stacks_in_lds)) != hipSuccess)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_level, kLanes, lds_words * 4) != hipSuccess)
     per_cu = 4;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 256;
-  return per_cu * cus;
+  // LDS is handed out in pieces of 1,280 bytes, 160 KiB per CU
+  const uint32_t piece = (lds_words * 4 + 1279) / 1280;
+  per_cu = std::min<int>(per_cu, (int)(128 / std::max(1u, piece)));
+  return std::max(per_cu, 1) * cus;
 }
 
 }  // namespace gls

@@ -122,8 +122,8 @@ typedef struct {
   uint32_t graph;        /* 1: fused path only; after the first execution the whole level
                             sequence is captured into a hipGraph with no host round trip
                             between levels, and later executions replay it */
-  uint32_t hbm_stacks;   /* 1: the fused kernel keeps its preemption stacks in a per-workgroup
-                            HBM scratch instead of LDS (half the LDS, more resident workgroups) */
+  uint32_t hbm_stacks;   /* accepted for callers that set it; the fused kernel's preemption
+                            stacks are in LDS either way (HBM for tiles too long for LDS) */
   uint32_t pool_grow;    /* 1: pool_bytes and ovf_words are only starting sizes; both grow as
                             with 0 */
   uint32_t ovf_words;    /* fused path: words of the stack buffer for tiles too long for LDS, per
