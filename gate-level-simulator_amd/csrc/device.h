@@ -181,8 +181,90 @@ struct TailArgs {
   uint32_t first;            // 1 in chunk 0
 };
 
+// Run scalars in device memory (64-bit slots).  The levels of a chunk run with
+// no host round trip: each level's kernels read its counts here, and the plan
+// kernel trips the chunk (S_TRIP) when a level needs more room than it has (or
+// the caller asked to stop); every later kernel then returns at once and the
+// host reads why, makes room and goes on from that level.
+enum ScalSlot {
+  S_BUMP = 0,     // pool words used
+  S_TOT_A = 1,    // tiles of the level
+  S_TOT_B = 2,    // scratch words of the level
+  S_TOT_OUT = 3,  // output words of the level (two-pass path)
+  S_EVC = 4,      // gate events of the run
+  S_EVL = 5,      // gate events of the level
+  S_OVF_USED = 6, // overflow stack words the level asked for
+  S_ERR = 7,      // error flags
+  S_TILES = 8, S_TILES_HBM = 9,  // tiles walked, of them on the HBM path
+  S_TAILS = 10,   // words of the chunk's gate-output tails
+  S_TRIP = 11,    // 0, or the tripped level + 1
+  S_WHY = 12,     // TripWhy
+  S_SCRATCH = 13, // address of the level scratch
+  S_LIMIT = 14,   // pool word that the level's outputs must not reach
+  S_OUTBASE = 15, // pool word of the level's first output
+  S_STIM = 16,    // pool words of the chunk's stimulus
+  S_DONE = 17,    // blocks of the running scan that are done
+  S_CLOCK = 18,   // start of the level's walk
+  S_EVAL = 19,    // ticks spent in walks
+  S_LEVELS = 20,  // walks run
+  S_IN_W = 21, S_OUT_W = 22,     // waveform words read by gates, written by gates
+  S_COUNT = 24
+};
+enum TripWhy : unsigned { TRIP_STOP = 1, TRIP_PROJECTED, TRIP_ROOM, TRIP_OVERFLOW, TRIP_STIM, TRIP_POOL };
+
 // The walk's ticket counters, each on a cache line of its own.
 constexpr uint32_t kTickets = 4, kTicketStride = 32;
+
+// Gates per block of the plan's and the join's scans (a gate's prefix = its
+// block's, in `part`, plus its own inside the block), and signals per block of
+// the stimulus cut.
+constexpr uint32_t kPlanGates = 1024, kJoinGates = 32, kStimSignals = 256;
+
+// Plan of one level.
+struct PlanArgs {
+  const GateRec* gates;
+  uint32_t ng;
+  const uint32_t* wlen;
+  const uint32_t* tail_len;
+  uint32_t seg_target, wide_words;
+  GatePlan* plan;
+  uint32_t* ntile;      // tiles per gate
+  uint32_t* tile_loc;   // tiles before the gate in its block
+  uint64_t* scr_loc;    // scratch words before the gate in its block
+  uint64_t* part;       // per block: tiles, scratch words before it
+  uint64_t* scal;
+  unsigned long long* ticket;
+  // room: tile arrays, pool, a scratch apart from the pool (when allowed)
+  uint64_t tiles_cap, pool_words, apart_cap;
+  uint32_t* pool;
+  uint32_t* apart;
+  uint32_t allow_apart;
+  uint32_t level;       // level + 1, for S_TRIP
+  // automatic chunks: trip when the chunk's outputs so far, over `done_gates`
+  // of `all_gates`, project to more than proj_cap words (0: not asked)
+  double proj_cap, all_gates, done_gates;
+  const uint32_t* stop; // host flag: nonzero trips the chunk (null: none)
+};
+
+// Join of one level's tiles.
+struct JoinArgs {
+  const GateRec* gates;
+  uint32_t ng;
+  const uint32_t* ntile;
+  const uint32_t* tile_loc;
+  const uint64_t* plan_part;
+  const TileOut* tout;
+  uint32_t* tile_off;
+  uint64_t* out_loc;    // output words before the gate in its block
+  uint64_t* part;       // per block: output words before it
+  uint32_t* wlen;
+  unsigned long long* saif;
+  const ChunkWin* cwin;
+  uint64_t* scal;
+  unsigned long long* ev_job;  // batches: gate events per instance (null: none)
+  uint32_t level;       // level + 1, for S_TRIP
+  uint32_t ovf_trip;    // 1: a level that ran out of overflow stacks is run again
+};
 
 // Arguments of the fused level (walk) kernel.
 struct LevelArgs {
@@ -190,16 +272,11 @@ struct LevelArgs {
   const uint32_t* pool;       // input waveforms
   const uint32_t* dtab;       // delay tables (GateRec::dt_off)
   const uint32_t* ttab;       // truth tables (GateRec::tt_off)
-  const uint64_t* ntiles;     // tiles of the level (device memory)
-  uint32_t* scratch;          // tile outputs
+  uint64_t* scal;
   TileOut* tout;              // per tile
   uint32_t* ovf;              // stacks of tiles that do not fit LDS
   unsigned long long ovf_cap;
-  unsigned long long* ovf_used;
   unsigned long long* ticket;   // batches handed out by each counter (0 per level)
-  unsigned long long* tiles_walked;  // [0] tiles walked, [1] of them on the HBM path (per run)
-  unsigned long long* ev_count;
-  unsigned int* err;
   const ChunkWin* cwin;        // SAIF bounds of this chunk per instance
   uint32_t lds_words;          // LDS of a workgroup
   uint32_t prefetch;           // 1: stage the next tile before storing this one

@@ -125,6 +125,10 @@ class DevArena {
   bool get_large(size_t want, size_t min_bytes, void** p, size_t* got);
   void put(void* p);
   void trim();  // frees every cached block
+  // pinned host pages of kPage bytes
+  static constexpr size_t kPage = 4096;
+  void* get_page();
+  void put_page(void* p);
   // frees every cached block when the device has less than 4 GiB (or 1.5%
   // of its memory) free: the HIP runtime needs room of its own
   void keep_headroom();
@@ -139,6 +143,7 @@ class DevArena {
   std::mutex mu_;
   std::multimap<size_t, void*> free_;          // cached blocks by size
   std::map<void*, size_t> live_;               // blocks handed out, with their sizes
+  std::vector<void*> pages_;                   // cached pinned pages
   uint64_t cached_ = 0, max_cached_;
   uint64_t hits_ = 0, misses_ = 0;
 };
@@ -239,11 +244,17 @@ class Job {
   bool try_ensure(void** p, size_t& cap, size_t need);
   Chunk make_chunk(size_t k, uint64_t F, uint64_t Fn, uint64_t prev_lb) const;
   void put_chunk_windows(const Chunk& c, bool capture);
-  int run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_eval,
-                bool device_driven, double* grow_hint);
-  void end_chunk(const Chunk& c, const Group& G, bool device_driven);
-  void run_chunks(std::vector<hipEvent_t>& ev_eval);
-  void run_group_chunks(const Group& G, std::vector<hipEvent_t>& ev_eval);
+  int run_chunk(const Chunk& c, const Group& G, bool device_driven, double* grow_hint,
+                const std::function<void()>& after);
+  void launch_level_of(size_t l, const Chunk& c, const Group& G, bool device_driven, double proj_cap);
+  void close_chunk(const Chunk& c, const Group& G);
+  void keep_tails(const Group& G);
+  void run_chunks();
+  void run_group_chunks(const Group& G);
+  void read_scal();
+  void write_scal();
+  void make_events();
+  void drop_graph();
   void build_graph();
   void finish_stats(const uint64_t* scal, double ms);
   void run_two_pass(std::vector<hipEvent_t>& ev_eval);
@@ -287,7 +298,8 @@ class Job {
   SegCarry* d_carry_ = nullptr;
   uint32_t* d_scratch_ = nullptr;
   // fused path
-  uint64_t *d_ntile_ = nullptr, *d_bound_ = nullptr, *d_tilebase_ = nullptr;
+  uint32_t *d_ntile_ = nullptr, *d_tileloc_ = nullptr;
+  uint64_t *d_scrloc_ = nullptr, *d_outloc_ = nullptr, *d_planpart_ = nullptr, *d_outpart_ = nullptr;
   size_t cap_tiles_ = 0, cap_tout_ = 0, cap_toff_ = 0;
   GatePlan* d_plan_ = nullptr;
   TileDesc* d_tiles_ = nullptr;
@@ -331,12 +343,20 @@ class Job {
   std::vector<Group> groups_;
   std::vector<std::vector<uint64_t>> gsched_;  // per group: its F_1 .. F_K
   size_t gsched_count_ = 0;                     // chunks of the group being run
-  uint64_t max_tiles_ = 0, tiles_cap_ = 0, max_scratch_ = 0, scratch_cap_ = 0;
+  // pinned page: run scalars, the device's view of should_stop, chunk windows
+  static constexpr size_t kStopAt = 1024, kPinnedWinAt = 2048;
+  static constexpr size_t kPinnedWin = (DevArena::kPage - kPinnedWinAt) / sizeof(ChunkWin);
+  unsigned char* pinned_ = nullptr;
+  uint32_t* stop_flag() const { return (uint32_t*)(pinned_ + kStopAt); }
+  uint64_t h_scal_[S_COUNT] = {};  // the device's run scalars when last read
+  hipEvent_t e0_ = nullptr, e1_ = nullptr;
+  double clock_khz_ = 100000;      // of the device's wall clock (S_EVAL)
   uint64_t max_tails_ = 0, max_bump_ = 0;
   uint64_t pool_reallocs_ = 0;  // pool allocations made while running
   uint64_t allocs_ = 0;         // device allocations made since the run started
   bool static_ = false;         // run_static(): no allocation, scratch from the static array
-  bool graph_scratch_in_pool_ = false;  // captured levels keep their scratch at the pool top
+  bool scratch_apart_ = false;  // the chunk's level scratch does not fit the pool's free top
+  bool capturing_ = false;
   hipGraphExec_t gexec_ = nullptr;
   std::vector<uint64_t> graph_sig_;
   bool last_replay_ = false;

@@ -18,7 +18,7 @@ namespace gls {
 hipError_t launch_scan(const uint64_t* in, uint64_t* out, uint64_t n, uint64_t* part,
                        uint64_t* total, const uint64_t* base, hipStream_t st);
 uint64_t scan_part_size(uint64_t n);
-hipError_t launch_plan(const GateDev* gates, uint32_t ng, const uint32_t* wlen, uint32_t seg_target,
+hipError_t launch_plan2p(const GateDev* gates, uint32_t ng, const uint32_t* wlen, uint32_t seg_target,
                        uint64_t* nseg, uint64_t* scr, uint32_t* gnseg, hipStream_t st);
 hipError_t launch_segmap(uint32_t ng, const uint64_t* seg_base, const uint32_t* gnseg,
                          uint32_t* segmap, hipStream_t st);
@@ -43,55 +43,53 @@ hipError_t launch_saif_nets(const uint32_t* nets, const uint32_t* job, uint32_t 
                             hipStream_t st);
 
 // level.hip: fused path
-hipError_t launch_plan2(const GateRec* gates, uint32_t ng, const uint32_t* wlen,
-                        uint32_t seg_target, uint32_t wide_words, GatePlan* plan, uint64_t* ntile, uint64_t* bound,
-                        unsigned int* err, const uint32_t* tail_len, hipStream_t st);
+hipError_t launch_plan(const PlanArgs& a, hipStream_t st);
 hipError_t launch_tile_desc(const GateRec* gates, uint32_t ng, const GatePlan* plan,
-                            const uint64_t* tile_base, const uint64_t* scr_base,
+                            const uint32_t* tile_loc, const uint64_t* scr_loc, const uint64_t* part,
                             const uint64_t* woff, const uint32_t* wlen, const uint32_t* pool,
-                            TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles,
-                            unsigned long long* ticket, unsigned long long* ovf_used, hipStream_t st);
+                            TileDesc* tiles, const uint64_t* scal, uint64_t guess, hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long* p, uint64_t n, unsigned long long v, hipStream_t st);
-hipError_t launch_guard(uint64_t* scal, uint64_t tiles_cap, uint64_t scratch_cap, hipStream_t st);
-hipError_t launch_pool_guard(uint64_t* scal, uint64_t pool_words, hipStream_t st);
-hipError_t launch_gate_carry(const GateRec* gates, uint32_t ng, const uint64_t* tile_base,
-                             const uint64_t* ntile, const TileOut* tout, uint32_t* tile_off,
-                             uint64_t* gate_cnt, uint32_t* wlen, unsigned long long* saif,
-                             const ChunkWin* cwin, const unsigned int* err, const TailArgs& T,
-                             unsigned long long* ev_job, hipStream_t st);
-hipError_t launch_add_u64(unsigned long long* dst, const unsigned long long* src, uint64_t n,
-                          hipStream_t st);
-hipError_t launch_compact(const TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles_cap,
-                          const TileOut* tout, const uint32_t* tile_off, const uint32_t* scratch,
-                          const uint64_t* gate_base, uint32_t* pool, uint64_t* woff, uint32_t* wlen, const unsigned int* err,
-                          unsigned long long* saif, const ChunkWin* cwin, uint32_t count_tc,
-                          const TailArgs& T, hipStream_t st);
-hipError_t launch_set_scal(uint64_t* scal, uint64_t bump, hipStream_t st);
 hipError_t launch_level(const LevelArgs& a, unsigned nblocks, hipStream_t st);
-// chunk.hip: time chunks
-hipError_t launch_stim_count(const uint64_t* store, const uint64_t* soff, const uint32_t* slen,
-                             uint32_t ns, uint64_t lb, uint64_t ub, uint64_t* cnt, uint32_t* first,
-                             hipStream_t st);
+hipError_t launch_join(const JoinArgs& a, const TailArgs& T, hipStream_t st);
+hipError_t launch_compact(const TileDesc* tiles, const TileOut* tout, const uint32_t* tile_off,
+                          const uint64_t* out_loc, const uint64_t* part, uint32_t* pool,
+                          uint64_t* woff, const uint64_t* scal, unsigned long long* saif,
+                          const ChunkWin* cwin, uint32_t count_tc, const TailArgs& T, uint64_t guess,
+                          hipStream_t st);
+hipError_t launch_run_begin(uint64_t* scal, unsigned long long* saif, uint64_t n_saif,
+                            unsigned long long* wtot, uint64_t n_nets, unsigned long long* evjob,
+                            uint64_t n_jobs, hipStream_t st);
+hipError_t launch_word_counts(const GateRec* gates, uint32_t ng, const unsigned long long* wtot,
+                              uint64_t* scal, hipStream_t st);
+hipError_t launch_stim_plan(const uint64_t* store, const uint64_t* soff, const uint32_t* slen,
+                            uint32_t ns, uint64_t lb, uint64_t ub, uint64_t* cnt, uint32_t* first,
+                            uint64_t* loc, uint64_t* part, uint64_t pool_words, uint64_t* scal,
+                            hipStream_t st);
 hipError_t launch_stim_copy(const uint64_t* store, const uint64_t* soff, const uint32_t* snet,
                             uint32_t ns, uint64_t lb, const uint64_t* cnt, const uint32_t* first,
-                            const uint64_t* base, uint32_t* pool, uint64_t pool_words,
-                            uint64_t* woff, uint32_t* wlen, unsigned int* err, hipStream_t st);
+                            const uint64_t* loc, const uint64_t* part, uint32_t* pool, uint64_t* woff,
+                            uint32_t* wlen, const uint64_t* scal, hipStream_t st);
+hipError_t launch_tail_len(const GateRec* gates, uint32_t ng, const uint64_t* woff,
+                           const uint32_t* wlen, const uint32_t* pool, uint32_t key, uint64_t* len,
+                           uint64_t* src, uint64_t* loc, uint64_t* part, uint64_t* scal,
+                           hipStream_t st);
+hipError_t launch_tail_copy(const GateRec* gates, uint32_t ng, const uint64_t* len,
+                            const uint64_t* src, const uint64_t* loc, const uint64_t* part,
+                            const uint32_t* pool, uint32_t* tails, uint64_t cap, uint32_t* tail_len,
+                            uint64_t* tail_off, uint64_t* scal, hipStream_t st);
+// chunk.hip: time chunks
 hipError_t launch_tails_init(const GateRec* gates, uint32_t ng, uint32_t* tail_len,
                              uint64_t* tail_off, uint32_t* tails, hipStream_t st);
 hipError_t launch_saif_accum(const GateRec* gates, uint32_t ng, const unsigned long long* chunk,
                              unsigned long long* saif, const uint32_t* wlen,
-                             const uint32_t* tail_len, unsigned long long* wtot, hipStream_t st);
-hipError_t launch_tail_len(const GateRec* gates, uint32_t ng, const uint64_t* woff,
-                           const uint32_t* wlen, const uint32_t* pool, uint32_t key, uint64_t* len,
-                           uint64_t* src, hipStream_t st);
-hipError_t launch_tail_copy(const GateRec* gates, uint32_t ng, const uint64_t* len,
-                            const uint64_t* src, const uint64_t* off, const uint32_t* pool,
-                            uint32_t* tails, uint64_t cap, uint32_t* tail_len, uint64_t* tail_off,
-                            unsigned int* err, hipStream_t st);
+                             const uint32_t* tail_len, unsigned long long* wtot, const uint64_t* scal,
+                             hipStream_t st);
+hipError_t launch_add_u64(unsigned long long* dst, const unsigned long long* src, uint64_t n,
+                          const uint64_t* scal, hipStream_t st);
 hipError_t launch_saif_stim(const uint64_t* store, const uint64_t* soff, const uint32_t* slen,
                             const uint32_t* snet, const uint32_t* sjob, uint32_t ns,
                             unsigned long long* saif, const unsigned long long* win,
-                            hipStream_t st);
+                            unsigned long long* wtot, hipStream_t st);
 int level_max_blocks(uint32_t lds_words);
 
 // LDS of a walk workgroup for tiles of 64 * seg input words on average: those
@@ -132,10 +130,6 @@ void hip_check(hipError_t e, const char* what) {
 // input ranges with 16-byte copies that may read up to 3 words beyond a
 // range's last word.
 static constexpr uint64_t kPoolPad = 16;
-
-// scalar slots in d_scal_
-enum { S_BUMP = 0, S_TOT_A = 1, S_TOT_B = 2, S_TOT_OUT = 3, S_EVC = 4,
-       S_OVF_USED = 6, S_ERR = 7, S_TILES = 8, S_TILES_HBM = 9, S_TAILS = 10 };
 
 static uint32_t sel_delay(uint32_t r, uint32_t f, int s) {
   return s == 1 ? r : (s == 2 ? f : (s == 3 ? std::max(r, f) : std::min(r, f)));
@@ -508,6 +502,7 @@ static bool trace_on() {
 DevArena::~DevArena() {
   std::lock_guard<std::mutex> lk(mu_);
   trim_locked();
+  for (void* p : pages_) (void)hipHostFree(p);
 }
 
 size_t DevArena::size_class(size_t bytes) {
@@ -608,6 +603,27 @@ void DevArena::keep_headroom() {
   keep_headroom_locked();
 }
 
+// Pinned pages for run scalars and stop flags: as many as jobs ran at once.
+void* DevArena::get_page() {
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (!pages_.empty()) {
+      void* p = pages_.back();
+      pages_.pop_back();
+      return p;
+    }
+  }
+  void* p = nullptr;
+  hip_check(hipHostMalloc(&p, kPage, hipHostMallocDefault), "hipHostMalloc");
+  return p;
+}
+
+void DevArena::put_page(void* p) {
+  std::lock_guard<std::mutex> lk(mu_);
+  if (pages_.size() < 64) pages_.push_back(p);
+  else (void)hipHostFree(p);
+}
+
 uint64_t DevArena::cached_bytes() {
   std::lock_guard<std::mutex> lk(mu_);
   return cached_;
@@ -650,6 +666,8 @@ Job::Job(int device, hipStream_t stream, DevArena* arena)
 Job::~Job() {
   const auto t0 = std::chrono::steady_clock::now();
   if (gexec_) (void)hipGraphExecDestroy(gexec_);
+  if (e0_) (void)hipEventDestroy(e0_);
+  if (e1_) (void)hipEventDestroy(e1_);
   // blocks go back to the arena only once this job's work has drained
   if (arena_) (void)hipStreamSynchronize(stream_);
   for (void* p : owned_)
@@ -658,6 +676,7 @@ Job::~Job() {
                    d_pool_,   d_ovf_,  d_tails_, d_cwin_};
   for (void* p : grown)
     if (p) arena_ ? arena_->put(p) : (void)hipFree(p);
+  if (pinned_) arena_ ? arena_->put_page(pinned_) : (void)hipHostFree(pinned_);
   if (trace_on())
     std::fprintf(stderr, "gls: job buffers released in %.1f ms\n",
                  std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count());
@@ -763,11 +782,7 @@ bool Job::grow_pool(uint64_t need, uint64_t used) {
   d_pool_ = p;
   dev_bytes_ += (n - pool_words_) * sizeof(uint32_t);
   pool_words_ = n;
-  if (gexec_) {
-    HC(hipGraphExecDestroy(gexec_));
-    gexec_ = nullptr;
-    graph_sig_.clear();
-  }
+  drop_graph();
   return true;
 }
 
@@ -808,11 +823,7 @@ bool Job::refresh_pool(uint64_t words) {
   dev_bytes_ += (n + kPoolPad) * sizeof(uint32_t);
   const bool grew = n > pool_words_;
   pool_words_ = n;
-  if (gexec_) {
-    HC(hipGraphExecDestroy(gexec_));
-    gexec_ = nullptr;
-    graph_sig_.clear();
-  }
+  drop_graph();
   return grew;
 }
 
@@ -1045,22 +1056,28 @@ void Job::prepare(const std::vector<SimInstance>& inst, uint64_t pool_words) {
   d_wlen_ = (uint32_t*)dmalloc(n_nets_ * sizeof(uint32_t));
   d_saif_ = (unsigned long long*)dmalloc((size_t)n_nets_ * kSaifWords * sizeof(unsigned long long));
   d_win_ = (unsigned long long*)dmalloc(win_.size() * 8);
-  d_scal_ = (uint64_t*)dmalloc(16 * sizeof(uint64_t));
+  d_scal_ = (uint64_t*)dmalloc(S_COUNT * sizeof(uint64_t));
   d_ticket_ = (unsigned long long*)dmalloc(kTickets * kTicketStride * 8);
+  if (!pinned_) {
+    if (arena_) pinned_ = (unsigned char*)arena_->get_page();
+    else HC(hipHostMalloc((void**)&pinned_, DevArena::kPage, hipHostMallocDefault));
+  }
+  int khz = 0;
+  HC(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_));
+  clock_khz_ = khz > 0 ? khz : 100000;
+  // the scans' block counter starts at zero (every scan leaves it so)
+  HC(launch_fill_u64((unsigned long long*)d_scal_, S_COUNT, 0ull, stream_));
   uint32_t maxw = 1;
   for (size_t l = 0; l + 1 < level_start_.size(); ++l)
     maxw = std::max(maxw, level_start_[l + 1] - level_start_[l]);
-  for (uint64_t** p : {&d_outoff_, &d_ntile_, &d_bound_, &d_tilebase_, &d_scrbase_})
-    *p = (uint64_t*)dmalloc(maxw * 8ull);
   if (mode == 1) {
-    for (uint64_t** p : {&d_nseg_, &d_scr_, &d_segbase_, &d_outlen_})
+    for (uint64_t** p : {&d_outoff_, &d_scrbase_, &d_nseg_, &d_scr_, &d_segbase_, &d_outlen_})
       *p = (uint64_t*)dmalloc(maxw * 8ull);
+    d_part_ = (uint64_t*)dmalloc(scan_part_size(maxw) * 8ull);
+    d_gnseg_ = (uint32_t*)dmalloc(maxw * 4ull);
     d_saif_nets_ = (uint32_t*)dmalloc(saif_net_list_.size() * 4);
     d_saif_job_ = (uint32_t*)dmalloc(saif_net_job_.size() * 4);
   }
-  d_part_ = (uint64_t*)dmalloc(scan_part_size(maxw) * 8ull);
-  d_gnseg_ = (uint32_t*)dmalloc(maxw * 4ull);
-  d_plan_ = (GatePlan*)dmalloc(maxw * sizeof(GatePlan));
   // stacks of tiles that do not fit LDS; an automatic size grows when a
   // level runs out of it (the level is run again)
   ovf_words_ = ovf_words_opt ? ovf_words_opt : (1ull << 24);
@@ -1074,11 +1091,18 @@ void Job::prepare(const std::vector<SimInstance>& inst, uint64_t pool_words) {
     d_scnt_ = (uint64_t*)dmalloc(n_sig_ * 8ull);
     d_sbase_ = (uint64_t*)dmalloc(n_sig_ * 8ull);
     d_sfirst_ = (uint32_t*)dmalloc(n_sig_ * 4ull);
-    d_spart_ = (uint64_t*)dmalloc(scan_part_size(n_sig_) * 8ull);
+    d_spart_ = (uint64_t*)dmalloc((n_sig_ / kStimSignals + 1) * 8ull);
+    d_plan_ = (GatePlan*)dmalloc(maxw * sizeof(GatePlan));
+    d_ntile_ = (uint32_t*)dmalloc(maxw * 4ull);
+    d_tileloc_ = (uint32_t*)dmalloc(maxw * 4ull);
+    d_scrloc_ = (uint64_t*)dmalloc(maxw * 8ull);
+    d_outloc_ = (uint64_t*)dmalloc(maxw * 8ull);
+    d_planpart_ = (uint64_t*)dmalloc((maxw / kPlanGates + 1) * 16ull);
+    d_outpart_ = (uint64_t*)dmalloc((maxw / kJoinGates + 1) * 8ull);
     d_tail_len_ = (uint32_t*)dmalloc(n_nets_ * 4ull);
     d_tail_off_ = (uint64_t*)dmalloc(n_nets_ * 8ull);
     for (uint64_t** p : {&d_tlen_g_, &d_tsrc_g_, &d_toff_g_}) *p = (uint64_t*)dmalloc(n_gates_ * 8ull);
-    d_gpart_ = (uint64_t*)dmalloc(scan_part_size(n_gates_) * 8ull);
+    d_gpart_ = (uint64_t*)dmalloc((n_gates_ / kPlanGates + 1) * 8ull);
     d_saif_chunk_ = (unsigned long long*)dmalloc((size_t)n_nets_ * kSaifWords * 8);
     d_wtot_ = (unsigned long long*)dmalloc(n_nets_ * 8ull);
     d_evjob_ = d_evjob_chunk_ = nullptr;
@@ -1229,37 +1253,54 @@ void Job::put_chunk_windows(const Chunk& c, bool capture) {
     if (need > cap_cwin_) throw GlsError(GLS_E_STATE, "chunk windows not sized for the capture");
   } else {
     ensure((void**)&d_cwin_, cap_cwin_, need);
+    if (n <= kPinnedWin) {
+      // through the pinned page: its last copy was done before the last
+      // chunk's results came back
+      ChunkWin* p = (ChunkWin*)(pinned_ + kPinnedWinAt);
+      std::copy(w.begin(), w.end(), p);
+      HC(hipMemcpyAsync(d_cwin_ + c.slot * n, p, n * sizeof(ChunkWin), hipMemcpyHostToDevice, stream_));
+      return;
+    }
   }
   HC(hipMemcpyAsync(d_cwin_ + c.slot * n, w.data(), n * sizeof(ChunkWin), hipMemcpyHostToDevice,
                     stream_));
   HC(hipStreamSynchronize(stream_));
 }
 
-// One chunk: its stimulus cut into the pool, then every level.  Per level:
-// plan the tiles (k_plan2, two scans), describe them (k_tile_desc), walk
-// every tile independently into the level scratch (k_level), join the tiles
-// of each gate and finish its SAIF share (k_gate_carry), place the gates in
-// the pool behind their tails (scan) and copy the outputs there
-// (k_compact).  Plain: one host round trip per level sizes the tile arrays
-// and the scratch.  Device-driven (graph capture): no host round trip; the
-// arrays keep the capacities learned by an earlier plain run, kernels read
-// the level's counts from device memory, and k_guard skips a level that
-// would not fit (reported as an error after the run).
-//
-// Plain runs with an automatically sized overflow stack buffer check, at
-// the next host round trip, whether the previous level ran out of it; if so
-// the buffer doubles and that level runs again from its starting state
-// (bump pointer and event count; its outputs and SAIF shares are
-// rewritten).  A plain chunk that cannot fit the pool (or, with automatic
-// chunks, is projected not to) returns CHUNK_SHORTER before its results
-// are used; *grow_hint then suggests a length factor (0: none).
-int Job::run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_eval,
-                   bool device_driven, double* grow_hint) {
-  uint64_t* bump = d_scal_ + S_BUMP;
-  unsigned long long* evc = (unsigned long long*)(d_scal_ + S_EVC);
-  unsigned int* err = (unsigned int*)(d_scal_ + S_ERR);
-  const bool retry = !device_driven && !static_ && (ovf_words_opt == 0 || pool_grow);
-  const uint32_t ns = G.s1 - G.s0;  // the group's stimulus signals
+// Run scalars to the host (h_scal_), once the stream has drained.  While a
+// caller that may stop the run (a job's cancel or deadline) waits, its flag
+// goes to the device as soon as it is raised: the next level's plan trips.
+void Job::read_scal() {
+  HC(hipMemcpyAsync(pinned_, d_scal_, S_COUNT * 8, hipMemcpyDeviceToHost, stream_));
+  if (should_stop) {
+    for (;;) {
+      const hipError_t e = hipStreamQuery(stream_);
+      if (e == hipSuccess) break;
+      if (e != hipErrorNotReady) HC(e);
+      (void)hipGetLastError();
+      if (should_stop()) __atomic_store_n(stop_flag(), 1u, __ATOMIC_RELAXED);
+      std::this_thread::yield();
+    }
+  }
+  HC(hipStreamSynchronize(stream_));
+  std::memcpy(h_scal_, pinned_, sizeof h_scal_);
+}
+
+void Job::write_scal() {
+  std::memcpy(pinned_, h_scal_, sizeof h_scal_);
+  HC(hipMemcpyAsync(d_scal_, pinned_, sizeof h_scal_, hipMemcpyHostToDevice, stream_));
+  HC(hipStreamSynchronize(stream_));
+}
+
+// Launches of level l of chunk c: plan the tiles (k_plan), describe them
+// (k_tile_desc), walk every tile independently into the level scratch
+// (k_level), join the tiles of each gate, finish its SAIF share and place it in
+// the pool behind its tail (k_join), and copy the outputs there (k_compact).
+// No host round trip: the kernels read the level's counts from device memory.
+void Job::launch_level_of(size_t l, const Chunk& c, const Group& G, bool device_driven, double proj_cap) {
+  const uint32_t g0 = level_start_[l], ng = level_start_[l + 1] - g0;
+  if (ng == 0) return;
+  const GateRec* gates = prog_->d_grec + g0;
   const ChunkWin* cw = d_cwin_ + c.slot * net_base_.size();
   TailArgs T;
   T.tail_len = d_tail_len_;
@@ -1267,175 +1308,177 @@ int Job::run_chunk(const Chunk& c, const Group& G, std::vector<hipEvent_t>& ev_e
   T.tails = d_tails_;
   T.shift = c.shift;
   T.first = c.first;
-  *grow_hint = 0;
+  // expected tiles, for launch widths: one a gate and one per 1,024 words of
+  // the estimated input words of the level's share of the chunk
+  const double share = c.Fn == kChunkEnd ? 1.0 : std::min(1.0, (double)(c.Fn - c.F) / (double)G.horizon);
+  const uint64_t guess = ng + (uint64_t)(G.est_words * share * ng / std::max(1u, G.g1 - G.g0) / 512.0);
+  PlanArgs p;
+  p.gates = gates;
+  p.ng = ng;
+  p.wlen = d_wlen_;
+  p.tail_len = d_tail_len_;
+  p.seg_target = seg_target ? seg_target : kDefaultSeg;
+  p.wide_words = wide_words_;
+  p.plan = d_plan_;
+  p.ntile = d_ntile_;
+  p.tile_loc = d_tileloc_;
+  p.scr_loc = d_scrloc_;
+  p.part = d_planpart_;
+  p.scal = d_scal_;
+  p.ticket = d_ticket_;
+  p.tiles_cap = std::min({cap_tiles_ / sizeof(TileDesc), cap_tout_ / sizeof(TileOut), cap_toff_ / 4});
+  p.pool_words = pool_words_;
+  p.apart_cap = d_scratch_ ? cap_scratch_ / 4 : 0;
+  p.pool = d_pool_;
+  p.apart = d_scratch_;
+  p.allow_apart = !(pool_auto_ && !static_) || scratch_apart_ || device_driven ? 1u : 0u;
+  p.level = (uint32_t)l + 1;
+  // automatic chunks: a chunk projected (by its gates so far) not to fit the
+  // largest pool is cut short before it runs further
+  const uint64_t group_gates = G.g1 - G.g0, done_g = g0 - G.g0;
+  p.proj_cap = done_g >= std::max<uint64_t>(64, group_gates / 32) ? proj_cap : 0.0;
+  p.all_gates = (double)group_gates;
+  p.done_gates = (double)done_g;
+  p.stop = should_stop && !device_driven ? stop_flag() : nullptr;
+  HC(launch_plan(p, stream_));
+  HC(launch_tile_desc(gates, ng, d_plan_, d_tileloc_, d_scrloc_, d_planpart_, d_woff_, d_wlen_, d_pool_,
+                      d_tiles_, d_scal_, guess, stream_));
+  LevelArgs a;
+  a.tiles = d_tiles_;
+  a.pool = d_pool_;
+  a.dtab = prog_->d_dtab;
+  a.ttab = prog_->d_ttab;
+  a.scal = d_scal_;
+  a.tout = d_tout_;
+  a.ovf = d_ovf_;
+  a.ovf_cap = ovf_words_;
+  a.ticket = d_ticket_;
+  a.cwin = cw;
+  a.lds_words = lds_words_;
+  a.prefetch = prefetch;
+  a.lo_rel = c.lo_rel;
+  a.hi_rel = c.hi_rel;
+  a.first = c.first;
+  HC(launch_level(a, (unsigned)std::min<uint64_t>(guess, (uint64_t)std::max(1, level_blocks_)), stream_));
+  JoinArgs j;
+  j.gates = gates;
+  j.ng = ng;
+  j.ntile = d_ntile_;
+  j.tile_loc = d_tileloc_;
+  j.plan_part = d_planpart_;
+  j.tout = d_tout_;
+  j.tile_off = d_toff_;
+  j.out_loc = d_outloc_;
+  j.part = d_outpart_;
+  j.wlen = d_wlen_;
+  j.saif = d_saif_chunk_;
+  j.cwin = cw;
+  j.scal = d_scal_;
+  j.ev_job = d_evjob_chunk_;
+  j.level = (uint32_t)l + 1;
+  j.ovf_trip = !device_driven && !static_ && (ovf_words_opt == 0 || pool_grow) ? 1u : 0u;
+  HC(launch_join(j, T, stream_));
+  HC(launch_compact(d_tiles_, d_tout_, d_toff_, d_outloc_, d_outpart_, d_pool_, d_woff_, d_scal_,
+                    d_saif_chunk_, cw, saif_tc, T, guess, stream_));
+}
 
+// One chunk: its stimulus cut into the pool, then every level, with no host
+// round trip between levels; `after` launches what follows the last level (it
+// does nothing when the chunk tripped).  Plain runs then read the run scalars:
+// a level that tripped is given the room it asked for (tile arrays, pool, a
+// scratch apart, a larger overflow stack buffer; its own kernels changed
+// nothing that a second run of it does not rewrite) and the chunk goes on from
+// there.  A chunk that cannot fit the pool (or, with automatic chunks, is
+// projected not to) returns CHUNK_SHORTER before its results are used;
+// *grow_hint then suggests a length factor (0: none).  Device-driven (graph
+// capture): the arrays keep their capacities, a trip is an error after the run.
+//
+// One host round trip per chunk: with one per level (the counts read back to
+// size arrays and launches) the 300-cell netlist's run took 1.4 ms for 12
+// levels.
+int Job::run_chunk(const Chunk& c, const Group& G, bool device_driven, double* grow_hint,
+                   const std::function<void()>& after) {
+  const uint32_t ns = G.s1 - G.s0;  // the group's stimulus signals
+  *grow_hint = 0;
+  scratch_apart_ = false;
   if (d_evjob_chunk_) HC(launch_fill_u64(d_evjob_chunk_, net_base_.size(), 0ull, stream_));
-  // the chunk's stimulus at the start of the pool
-  HC(launch_stim_count(d_store_, d_soff_ + G.s0, d_slen_ + G.s0, ns, c.lb,
-                       c.Fn == kChunkEnd ? ~0ull : c.Fn, d_scnt_, d_sfirst_, stream_));
-  if (ns) HC(launch_scan(d_scnt_, d_sbase_, ns, d_spart_, bump, nullptr, stream_));
-  else HC(launch_fill_u64((unsigned long long*)bump, 1, 0ull, stream_));
-  uint64_t stim_chunk = 0;
-  if (!device_driven) {
-    HC(hipMemcpyAsync(&stim_chunk, bump, 8, hipMemcpyDeviceToHost, stream_));
-    HC(hipStreamSynchronize(stream_));
-    if (stim_chunk + 1024 > pool_words_) {
+  const uint64_t group_gates = G.g1 - G.g0;
+  const bool projected = !device_driven && chunk_ps == 0;
+  double proj_cap = 0;
+  if (projected) proj_cap = (double)(pool_auto_ && !static_ ? pool_max_words() : pool_words_);
+  bool stim = true;
+  size_t next = G.L0;  // level to run next
+  for (;;) {
+    if (stim) {  // the chunk's stimulus at the start of the pool
+      HC(launch_stim_plan(d_store_, d_soff_ + G.s0, d_slen_ + G.s0, ns, c.lb,
+                          c.Fn == kChunkEnd ? ~0ull : c.Fn, d_scnt_, d_sfirst_, d_sbase_, d_spart_,
+                          pool_words_, d_scal_, stream_));
+      HC(launch_stim_copy(d_store_, d_soff_ + G.s0, d_snet_ + G.s0, ns, c.lb, d_scnt_, d_sfirst_,
+                          d_sbase_, d_spart_, d_pool_, d_woff_, d_wlen_, d_scal_, stream_));
+      stim = false;
+    }
+    for (size_t l = next; l < G.L1; ++l) {
+      if (!device_driven) stop_point();
+      launch_level_of(l, c, G, device_driven, proj_cap);
+    }
+    after();
+    if (device_driven) return CHUNK_OK;
+    read_scal();
+    if (!h_scal_[S_TRIP]) return CHUNK_OK;
+    const uint64_t why = h_scal_[S_WHY], used = h_scal_[S_BUMP], stim_chunk = h_scal_[S_STIM];
+    next = (size_t)(h_scal_[S_TRIP] - 1);
+    h_scal_[S_TRIP] = h_scal_[S_WHY] = 0;
+    if (why == TRIP_STOP) {
+      stop_point();
+      throw GlsError(GLS_E_CANCELLED, "job cancelled or past its deadline");
+    }
+    if (why == TRIP_STIM) {
       // nothing in the pool to keep yet
       if (pool_auto_) refresh_pool(std::max<uint64_t>(2 * stim_chunk, 2 * pool_words_));
       if (stim_chunk + 1024 > pool_words_) return CHUNK_SHORTER;
-    }
-  }
-  HC(launch_stim_copy(d_store_, d_soff_ + G.s0, d_snet_ + G.s0, ns, c.lb, d_scnt_, d_sfirst_,
-                      d_sbase_, d_pool_, pool_words_, d_woff_, d_wlen_, err, stream_));
-
-  size_t prev = SIZE_MAX;  // last level run
-  uint64_t prev_bump = 0, prev_evc = 0, prev_err = 0;
-  // true when the previous level overflowed and was rolled back
-  auto rolled_back = [&](const uint64_t* h) {
-    if (!retry || prev == SIZE_MAX || !(h[S_ERR] & 2u)) return false;
-    uint64_t s[8];
-    std::memcpy(s, h, sizeof s);
-    s[S_BUMP] = prev_bump;
-    s[S_EVC] = prev_evc;
-    s[S_ERR] = prev_err;
-    HC(hipMemcpyAsync(d_scal_, s, sizeof s, hipMemcpyHostToDevice, stream_));
-    HC(hipStreamSynchronize(stream_));
-    ovf_words_ *= 2;
-    ensure((void**)&d_ovf_, cap_ovf_, ovf_words_ * 4);
-    if (gexec_) {  // a captured graph holds the old buffer
-      HC(hipGraphExecDestroy(gexec_));
-      gexec_ = nullptr;
-      graph_sig_.clear();
-    }
-    return true;
-  };
-  const bool projected = !device_driven && chunk_ps == 0;
-  const uint64_t group_gates = G.g1 - G.g0;
-  size_t next = G.L0;  // level to run next
-  while (next <= G.L1) {
-    const size_t l = next++;
-    if (!device_driven) stop_point();
-    if (l == G.L1) {  // after the last level: did it overflow?
-      if (!retry || prev == SIZE_MAX) break;
-      uint64_t h[8];
-      HC(hipMemcpyAsync(h, d_scal_, sizeof h, hipMemcpyDeviceToHost, stream_));
-      HC(hipStreamSynchronize(stream_));
-      if (!rolled_back(h)) break;
-      next = prev;  // run it again
-      prev = SIZE_MAX;
-      continue;
-    }
-    uint32_t g0 = level_start_[l], ng = level_start_[l + 1] - g0;
-    if (ng == 0) continue;
-    const GateRec* gates = prog_->d_grec + g0;
-    HC(launch_plan2(gates, ng, d_wlen_, seg_target ? seg_target : kDefaultSeg, wide_words_, d_plan_, d_ntile_, d_bound_, err, d_tail_len_, stream_));
-    HC(launch_scan(d_ntile_, d_tilebase_, ng, d_part_, d_scal_ + S_TOT_A, nullptr, stream_));
-    HC(launch_scan(d_bound_, d_scrbase_, ng, d_part_, d_scal_ + S_TOT_B, nullptr, stream_));
-    uint64_t ntiles = tiles_cap_;
-    // The level scratch lives in the unused top of the event pool when twice
-    // its size is free above the bump (the level's outputs, at most the
-    // scratch size, then land below it); otherwise in an allocation of its
-    // own.  The pool guard keeps the outputs clear of a scratch in the pool.
-    uint32_t* scratch = d_scratch_;
-    uint64_t pool_limit = pool_words_;
-    if (!device_driven) {
-      uint64_t h[8];
-      HC(hipMemcpyAsync(h, d_scal_, sizeof h, hipMemcpyDeviceToHost, stream_));
-      HC(hipStreamSynchronize(stream_));
-      if (rolled_back(h)) {
-        next = prev;  // run the previous level again
-        prev = SIZE_MAX;
-        continue;
-      }
-      prev = l;
-      prev_bump = h[S_BUMP];
-      prev_evc = h[S_EVC];
-      prev_err = h[S_ERR];
-      ntiles = h[S_TOT_A];
-      const uint64_t scr = h[S_TOT_B], used = h[S_BUMP];
-      if (ntiles >= 0xFFFFFFF0ull) throw GlsError(GLS_E_RANGE, "too many tiles in one level");
-      // automatic chunks: a chunk projected (by its gates so far) not to fit
-      // the largest pool is cut short before it runs further
-      const uint64_t done_g = g0 - G.g0;
-      if (projected && done_g >= std::max<uint64_t>(64, group_gates / 32) && used > stim_chunk) {
-        const double proj = (double)(used - stim_chunk) * group_gates / done_g;
-        const double cap = (double)(pool_auto_ && !static_ ? pool_max_words() : pool_words_);
-        if (((double)stim_chunk + proj) * 1.35 > cap) {
-          *grow_hint = std::max(0.05, 0.85 * (cap / 1.35 - stim_chunk) / proj);
-          return CHUNK_SHORTER;
-        }
-      }
-      if (!try_ensure((void**)&d_tiles_, cap_tiles_, ntiles * sizeof(TileDesc)) ||
-          !try_ensure((void**)&d_tout_, cap_tout_, ntiles * sizeof(TileOut)) ||
-          !try_ensure((void**)&d_toff_, cap_toff_, ntiles * 4))
+      stim = true;
+      next = G.L0;
+    } else if (why == TRIP_PROJECTED) {
+      const uint64_t done_g = level_start_[next] - G.g0;
+      const double proj = (double)(used - stim_chunk) * (double)group_gates / (double)done_g;
+      *grow_hint = std::max(0.05, 0.85 * (proj_cap / 1.35 - (double)stim_chunk) / proj);
+      return CHUNK_SHORTER;
+    } else if (why == TRIP_OVERFLOW) {
+      ovf_words_ *= 2;
+      ensure((void**)&d_ovf_, cap_ovf_, ovf_words_ * 4);
+      drop_graph();  // a captured graph holds the old buffer
+      h_scal_[S_ERR] &= ~2ull;
+    } else if (why == TRIP_ROOM) {
+      const uint64_t tiles = h_scal_[S_TOT_A], scr = h_scal_[S_TOT_B];
+      if (tiles >= 0xFFFFFFF0ull) throw GlsError(GLS_E_RANGE, "too many tiles in one level");
+      if (!try_ensure((void**)&d_tiles_, cap_tiles_, tiles * sizeof(TileDesc)) ||
+          !try_ensure((void**)&d_tout_, cap_tout_, tiles * sizeof(TileOut)) ||
+          !try_ensure((void**)&d_toff_, cap_toff_, tiles * 4))
         return CHUNK_SHORTER;
       grow_pool(used + 2 * scr, used);
-      if (used <= pool_words_ && 2 * scr <= pool_words_ - used) {
-        pool_limit = pool_words_ - scr;
-        scratch = d_pool_ + pool_limit;
-      } else {
+      if (!(used <= pool_words_ && 2 * scr <= pool_words_ - used)) {
         // outputs in the pool, scratch apart
         if (used + scr > pool_words_ && !grow_pool(used + scr, used)) return CHUNK_SHORTER;
         if (!try_ensure((void**)&d_scratch_, cap_scratch_, scr * 4)) return CHUNK_SHORTER;
-        scratch = d_scratch_;
+        scratch_apart_ = true;
       }
-      max_tiles_ = std::max(max_tiles_, ntiles);
-      max_scratch_ = std::max(max_scratch_, scr);
-    } else {
-      HC(launch_guard(d_scal_, tiles_cap_, scratch_cap_, stream_));
-      if (graph_scratch_in_pool_) {
-        pool_limit = pool_words_ - scratch_cap_;
-        scratch = d_pool_ + pool_limit;
-      }
+    } else {  // TRIP_POOL: reported from the error flags
+      return CHUNK_OK;
     }
-    HC(launch_tile_desc(gates, ng, d_plan_, d_tilebase_, d_scrbase_, d_woff_, d_wlen_, d_pool_,
-                        d_tiles_, d_scal_ + S_TOT_A, ntiles, d_ticket_,
-                        (unsigned long long*)(d_scal_ + S_OVF_USED), stream_));
-    LevelArgs a;
-    a.tiles = d_tiles_;
-    a.pool = d_pool_;
-    a.dtab = prog_->d_dtab;
-    a.ttab = prog_->d_ttab;
-    a.ntiles = d_scal_ + S_TOT_A;
-    a.scratch = scratch;
-    a.tout = d_tout_;
-    a.ovf = d_ovf_;
-    a.ovf_cap = ovf_words_;
-    a.ovf_used = (unsigned long long*)(d_scal_ + S_OVF_USED);
-    a.ev_count = evc;
-    a.err = err;
-    a.cwin = cw;
-    a.lds_words = lds_words_;
-    a.prefetch = prefetch;
-    a.ticket = d_ticket_;
-    a.tiles_walked = (unsigned long long*)(d_scal_ + S_TILES);
-    a.lo_rel = c.lo_rel;
-    a.hi_rel = c.hi_rel;
-    a.first = c.first;
-    const unsigned nb = (unsigned)std::min<uint64_t>(ntiles, (uint64_t)std::max(1, level_blocks_));
-    if (!device_driven && !static_) {
-      hipEvent_t e_a, e_b;
-      HC(hipEventCreate(&e_a));
-      HC(hipEventCreate(&e_b));
-      ev_eval.push_back(e_a);
-      ev_eval.push_back(e_b);
-      HC(hipEventRecord(e_a, stream_));
-      HC(launch_level(a, nb, stream_));
-      HC(hipEventRecord(e_b, stream_));
-    } else {
-      HC(launch_level(a, nb, stream_));
-    }
-    // gate counts go to d_bound_ (free again once the scratch bases are scanned)
-    HC(launch_gate_carry(gates, ng, d_tilebase_, d_ntile_, d_tout_, d_toff_, d_bound_, d_wlen_,
-                         d_saif_chunk_, cw, err, T, d_evjob_chunk_, stream_));
-    HC(launch_scan(d_bound_, d_outoff_, ng, d_part_, d_scal_ + S_TOT_OUT, bump, stream_));
-    HC(launch_pool_guard(d_scal_, pool_limit, stream_));
-    HC(launch_compact(d_tiles_, d_scal_ + S_TOT_A, ntiles, d_tout_, d_toff_, scratch, d_outoff_, d_pool_,
-                      d_woff_, d_wlen_, err, d_saif_chunk_, cw, saif_tc, T,
-                      stream_));
-    HC(launch_bump(bump, d_scal_ + S_TOT_OUT, stream_));
+    write_scal();
   }
-  return CHUNK_OK;
+}
+
+void Job::make_events() {
+  if (!e0_) HC(hipEventCreate(&e0_));
+  if (!e1_) HC(hipEventCreate(&e1_));
+}
+
+void Job::drop_graph() {
+  if (!gexec_) return;
+  HC(hipGraphExecDestroy(gexec_));
+  gexec_ = nullptr;
+  graph_sig_.clear();
 }
 
 // Gate-output waveforms of a finished chunk to the host: each gate net's
@@ -1464,28 +1507,32 @@ void Job::fetch_chunk_waves(const Chunk& c, const Group& G) {
   }
 }
 
-// After a chunk: its SAIF shares join the totals, its waveforms go to the
-// host (keep_waves, plain runs), and the gate outputs' tails for the next
-// chunk are cut from their waveforms.
-void Job::end_chunk(const Chunk& c, const Group& G, bool device_driven) {
+// Launched behind a chunk's last level: its SAIF shares join the totals and,
+// when another chunk follows, the gate outputs' tails for it are cut from their
+// waveforms (their words end up in S_TAILS); after the run's last chunk the
+// words read and written are counted.
+void Job::close_chunk(const Chunk& c, const Group& G) {
   const GateRec* gates = prog_->d_grec + G.g0;
   const uint32_t ng = G.g1 - G.g0;
-  HC(launch_saif_accum(gates, ng, d_saif_chunk_, d_saif_, d_wlen_, d_tail_len_, d_wtot_, stream_));
-  if (d_evjob_) HC(launch_add_u64(d_evjob_, d_evjob_chunk_, net_base_.size(), stream_));
-  if (!device_driven && keep_waves) fetch_chunk_waves(c, G);
-  if (c.Fn == kChunkEnd || ng == 0) return;
-  const uint32_t key = (uint32_t)((c.Fn - wmax_) - c.lb + 1);  // lb of the next chunk
-  HC(launch_tail_len(gates, ng, d_woff_, d_wlen_, d_pool_, key, d_tlen_g_, d_tsrc_g_, stream_));
-  HC(launch_scan(d_tlen_g_, d_toff_g_, ng, d_gpart_, d_scal_ + S_TAILS, nullptr, stream_));
-  if (!device_driven) {
-    uint64_t total = 0;
-    HC(hipMemcpyAsync(&total, d_scal_ + S_TAILS, 8, hipMemcpyDeviceToHost, stream_));
-    HC(hipStreamSynchronize(stream_));
-    ensure((void**)&d_tails_, cap_tails_, std::max<uint64_t>(total, 1) * 4);
-    max_tails_ = std::max(max_tails_, total);
+  HC(launch_saif_accum(gates, ng, d_saif_chunk_, d_saif_, d_wlen_, d_tail_len_, d_wtot_, d_scal_,
+                       stream_));
+  if (d_evjob_) HC(launch_add_u64(d_evjob_, d_evjob_chunk_, net_base_.size(), d_scal_, stream_));
+  if (c.Fn == kChunkEnd) {
+    if (&G == &groups_.back())
+      HC(launch_word_counts(prog_->d_grec, n_gates_, d_wtot_, d_scal_, stream_));
+    if (&G == &groups_.back() && !capturing_ && !static_) HC(hipEventRecord(e1_, stream_));
+    return;
   }
-  HC(launch_tail_copy(gates, ng, d_tlen_g_, d_tsrc_g_, d_toff_g_, d_pool_, d_tails_, cap_tails_ / 4,
-                      d_tail_len_, d_tail_off_, (unsigned int*)(d_scal_ + S_ERR), stream_));
+  const uint32_t key = (uint32_t)((c.Fn - wmax_) - c.lb + 1);  // lb of the next chunk
+  HC(launch_tail_len(gates, ng, d_woff_, d_wlen_, d_pool_, key, d_tlen_g_, d_tsrc_g_, d_toff_g_, d_gpart_,
+                     d_scal_, stream_));
+}
+
+// The tails cut by close_chunk to the tail store.
+void Job::keep_tails(const Group& G) {
+  const uint32_t ng = G.g1 - G.g0;
+  HC(launch_tail_copy(prog_->d_grec + G.g0, ng, d_tlen_g_, d_tsrc_g_, d_toff_g_, d_gpart_, d_pool_,
+                      d_tails_, cap_tails_ / 4, d_tail_len_, d_tail_off_, d_scal_, stream_));
 }
 
 // A plain run of every chunk.  Automatic chunks: the first chunk is the
@@ -1494,12 +1541,13 @@ void Job::end_chunk(const Chunk& c, const Group& G, bool device_driven) {
 // fit) is run again shorter, the pool taking the largest size free HBM
 // allows, and each next chunk aims at 60% of that pool by the output rate of
 // the one before.
-void Job::run_chunks(std::vector<hipEvent_t>& ev_eval) {
-  HC(launch_set_scal(d_scal_, 0, stream_));
-  HC(launch_fill_u64(d_saif_, (uint64_t)n_nets_ * kSaifWords, 0ull, stream_));
-  HC(launch_fill_u64(d_wtot_, n_nets_, 0ull, stream_));
-  if (d_evjob_) HC(launch_fill_u64(d_evjob_, net_base_.size(), 0ull, stream_));
-  HC(launch_saif_stim(d_store_, d_soff_, d_slen_, d_snet_, d_sjob_, n_sig_, d_saif_, d_win_, stream_));
+void Job::run_chunks() {
+  HC(launch_run_begin(d_scal_, d_saif_, (uint64_t)n_nets_ * kSaifWords, d_wtot_, n_nets_, d_evjob_,
+                      net_base_.size(), stream_));
+  std::memset(h_scal_, 0, sizeof h_scal_);
+  if (should_stop) __atomic_store_n(stop_flag(), 0u, __ATOMIC_RELAXED);
+  HC(launch_saif_stim(d_store_, d_soff_, d_slen_, d_snet_, d_sjob_, n_sig_, d_saif_, d_win_, d_wtot_,
+                      stream_));
   waves_.clear();
   if (keep_waves) waves_.assign(n_nets_, {});
   sched_.clear();
@@ -1507,8 +1555,24 @@ void Job::run_chunks(std::vector<hipEvent_t>& ev_eval) {
   stats_.chunk_retries = 0;
   max_bump_ = 0;
   max_tails_ = 0;
+  if (!static_) {
+    // tile arrays from the waveform estimate (one tile a gate and one per 1,024
+    // input words of the widest level, two inputs a gate), at most 1/32 of the
+    // pool; a level that has more trips once and they grow
+    uint32_t maxw = 1;
+    for (size_t l = 0; l + 1 < level_start_.size(); ++l)
+      maxw = std::max(maxw, level_start_[l + 1] - level_start_[l]);
+    double words = 0;
+    for (const Group& G : groups_)
+      words = std::max(words, std::min(G.est_words, (double)pool_words_) / std::max(1u, G.g1 - G.g0));
+    const uint64_t n = 2 * (uint64_t)maxw + 64 +
+                       (uint64_t)std::min(words * maxw / 512.0, (double)pool_words_ * 4 / 32 / 164);
+    ensure((void**)&d_tiles_, cap_tiles_, n * sizeof(TileDesc));
+    ensure((void**)&d_tout_, cap_tout_, n * sizeof(TileOut));
+    ensure((void**)&d_toff_, cap_toff_, n * 4);
+  }
   for (size_t q = 0; q < groups_.size(); ++q) {
-    run_group_chunks(groups_[q], ev_eval);
+    run_group_chunks(groups_[q]);
     gsched_[q].assign(sched_.end() - (std::ptrdiff_t)gsched_count_, sched_.end());
   }
   stats_.chunks = sched_.size();
@@ -1516,7 +1580,7 @@ void Job::run_chunks(std::vector<hipEvent_t>& ev_eval) {
 
 // The time chunks of one instance group, from its own time 0: the group's
 // gate outputs start from X tails.
-void Job::run_group_chunks(const Group& G, std::vector<hipEvent_t>& ev_eval) {
+void Job::run_group_chunks(const Group& G) {
   const uint32_t ng = G.g1 - G.g0;
   ensure((void**)&d_tails_, cap_tails_, std::max<size_t>(ng, 1) * 4);
   HC(launch_tails_init(prog_->d_grec + G.g0, ng, d_tail_len_, d_tail_off_, d_tails_, stream_));
@@ -1558,29 +1622,26 @@ void Job::run_group_chunks(const Group& G, std::vector<hipEvent_t>& ev_eval) {
   for (;;) {
     const uint64_t Fn = (F + L >= horizon) ? kChunkEnd : F + L;
     const Chunk c = make_chunk(k, F, Fn, prev_lb);
-    uint64_t snap[16];
-    HC(hipMemcpyAsync(snap, d_scal_, sizeof snap, hipMemcpyDeviceToHost, stream_));
-    HC(hipStreamSynchronize(stream_));
+    uint64_t snap[S_COUNT];
+    std::memcpy(snap, h_scal_, sizeof snap);
     put_chunk_windows(c, false);
     double hint = 0;
     const auto tc0 = std::chrono::steady_clock::now();
     const uint64_t re0 = pool_reallocs_;
-    const int res = run_chunk(c, G, ev_eval, false, &hint);
-    if (trace_on()) {
-      uint64_t b = 0;
-      HC(hipMemcpyAsync(&b, d_scal_ + S_BUMP, 8, hipMemcpyDeviceToHost, stream_));
-      HC(hipStreamSynchronize(stream_));
+    const int res = run_chunk(c, G, false, &hint, [&] { close_chunk(c, G); });
+    if (trace_on())
       std::fprintf(stderr, "gls: chunk %zu [%llu, %llu) L=%llu %s bump=%llu pool=%llu reallocs=%llu %.1f ms\n",
                    k, (unsigned long long)F, (unsigned long long)(Fn == kChunkEnd ? 0 : Fn),
-                   (unsigned long long)L, res == CHUNK_OK ? "ok" : "shorter", (unsigned long long)b,
-                   (unsigned long long)pool_words_, (unsigned long long)(pool_reallocs_ - re0),
+                   (unsigned long long)L, res == CHUNK_OK ? "ok" : "shorter",
+                   (unsigned long long)h_scal_[S_BUMP], (unsigned long long)pool_words_,
+                   (unsigned long long)(pool_reallocs_ - re0),
                    std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - tc0).count());
-    }
     if (res != CHUNK_OK) {
       if (chunk_ps != 0)
         throw GlsError(GLS_E_OOM, "event pool exhausted (raise the pool size or allow time chunks)");
-      HC(hipStreamSynchronize(stream_));
-      HC(hipMemcpyAsync(d_scal_, snap, sizeof snap, hipMemcpyHostToDevice, stream_));
+      for (int i : {S_EVAL, S_LEVELS}) snap[i] = h_scal_[i];  // the walks' time stays counted
+      std::memcpy(h_scal_, snap, sizeof snap);
+      write_scal();
       uint64_t nl = hint > 0 ? (uint64_t)((double)L * std::min(0.5, hint)) : L / 2;
       if (L <= lmin) throw GlsError(GLS_E_OOM, "event pool exhausted by the shortest time chunk");
       L = std::max<uint64_t>(nl, lmin);
@@ -1589,11 +1650,15 @@ void Job::run_group_chunks(const Group& G, std::vector<hipEvent_t>& ev_eval) {
       refresh_pool(pool_max_words());  // the chunk starts over: nothing to keep
       continue;
     }
-    uint64_t used = 0;
-    HC(hipMemcpyAsync(&used, d_scal_ + S_BUMP, 8, hipMemcpyDeviceToHost, stream_));
-    HC(hipStreamSynchronize(stream_));
+    const uint64_t used = h_scal_[S_BUMP];
     max_bump_ = std::max(max_bump_, used);
-    end_chunk(c, G, false);
+    if (keep_waves) fetch_chunk_waves(c, G);
+    if (Fn != kChunkEnd && G.g1 > G.g0) {
+      const uint64_t total = h_scal_[S_TAILS];
+      ensure((void**)&d_tails_, cap_tails_, std::max<uint64_t>(total, 1) * 4);
+      max_tails_ = std::max(max_tails_, total);
+      keep_tails(G);
+    }
     sched_.push_back(Fn);
     ++gsched_count_;
     if (Fn == kChunkEnd) break;
@@ -1622,7 +1687,7 @@ void Job::run_two_pass(std::vector<hipEvent_t>& ev_eval) {
     uint32_t g0 = level_start_[l], ng = level_start_[l + 1] - g0;
     if (ng == 0) continue;
     const GateDev* gates = prog_->d_gdev + g0;
-    HC(launch_plan(gates, ng, d_wlen_, seg, d_nseg_, d_scr_, d_gnseg_, stream_));
+    HC(launch_plan2p(gates, ng, d_wlen_, seg, d_nseg_, d_scr_, d_gnseg_, stream_));
     HC(launch_scan(d_nseg_, d_segbase_, ng, d_part_, d_scal_ + S_TOT_A, nullptr, stream_));
     HC(launch_scan(d_scr_, d_scrbase_, ng, d_part_, d_scal_ + S_TOT_B, nullptr, stream_));
     uint64_t h[3];
@@ -1666,21 +1731,15 @@ void Job::run() {
   if (graph && gexec_ && sig == graph_sig_) {
     // replay the captured chunk and level sequence: no host round trip
     auto w0 = std::chrono::steady_clock::now();
-    hipEvent_t e0, e1;
-    HC(hipEventCreate(&e0));
-    HC(hipEventCreate(&e1));
-    HC(hipEventRecord(e0, stream_));
+    make_events();
+    HC(hipEventRecord(e0_, stream_));
     HC(hipGraphLaunch(gexec_, stream_));
-    HC(hipEventRecord(e1, stream_));
-    HC(hipEventSynchronize(e1));
+    HC(hipEventRecord(e1_, stream_));
+    read_scal();
     float ms = 0;
-    HC(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    uint64_t h[16];
-    HC(hipMemcpyAsync(h, d_scal_, sizeof h, hipMemcpyDeviceToHost, stream_));
-    HC(hipStreamSynchronize(stream_));
-    if (h[S_ERR] & 8u)
+    HC(hipEventElapsedTime(&ms, e0_, e1_));
+    const uint64_t* h = h_scal_;
+    if ((h[S_ERR] & 8u) || h[S_TRIP])
       throw GlsError(GLS_E_STATE, "device-driven run outgrew the capacities of its first run");
     stats_.eval_ms = ms;
     stats_.eval_launches = 1;
@@ -1695,13 +1754,9 @@ void Job::run() {
   }
   auto w0 = std::chrono::steady_clock::now();
   allocs_ = 0;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  if (!static_) {
-    HC(hipEventCreate(&e0));
-    HC(hipEventCreate(&e1));
-  }
+  if (!static_) make_events();
   if (mode == 1) {
-    uint64_t scal[16] = {0};
+    uint64_t scal[S_COUNT] = {0};
     scal[S_BUMP] = stim_words_;
     HC(hipMemcpyAsync(d_woff_, h_woff_init_.data(), n_nets_ * 8ull, hipMemcpyHostToDevice, stream_));
     HC(hipMemcpyAsync(d_wlen_, h_wlen_init_.data(), n_nets_ * 4ull, hipMemcpyHostToDevice, stream_));
@@ -1709,34 +1764,29 @@ void Job::run() {
     HC(launch_fill_u64(d_saif_, (uint64_t)n_nets_ * kSaifWords, 0ull, stream_));
     HC(hipStreamSynchronize(stream_));
   }
-  if (e0) HC(hipEventRecord(e0, stream_));
+  if (!static_) HC(hipEventRecord(e0_, stream_));
   std::vector<hipEvent_t> ev_eval;
   try {
     if (mode == 1) {
       HC(launch_saif_nets(d_saif_nets_, d_saif_job_, (uint32_t)saif_net_list_.size(), d_woff_,
                           d_wlen_, d_pool_, d_saif_, d_win_, stream_));
       run_two_pass(ev_eval);
+      if (!static_) HC(hipEventRecord(e1_, stream_));
+      read_scal();
     } else {
-      run_chunks(ev_eval);
+      run_chunks();  // records e1_ behind the last chunk and reads the scalars
     }
   } catch (...) {
     (void)hipStreamSynchronize(stream_);
     for (hipEvent_t e : ev_eval) (void)hipEventDestroy(e);
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
     throw;
   }
+  const uint64_t* h = h_scal_;
   float ms = 0;
-  if (e0) {
-    HC(hipEventRecord(e1, stream_));
-    HC(hipEventSynchronize(e1));
-    HC(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-  } else {
-    HC(hipStreamSynchronize(stream_));
+  if (!static_)
+    HC(hipEventElapsedTime(&ms, e0_, e1_));
+  else
     ms = (float)std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
-  }
   double eval_ms = 0;
   for (size_t i = 0; i + 1 < ev_eval.size(); i += 2) {
     float x = 0;
@@ -1744,11 +1794,8 @@ void Job::run() {
     eval_ms += x;
   }
   for (hipEvent_t e : ev_eval) (void)hipEventDestroy(e);
-  stats_.eval_ms = eval_ms;
-  stats_.eval_launches = ev_eval.size() / 2;
-  uint64_t h[16];
-  HC(hipMemcpyAsync(h, d_scal_, sizeof h, hipMemcpyDeviceToHost, stream_));
-  HC(hipStreamSynchronize(stream_));
+  stats_.eval_ms = mode == 1 ? eval_ms : static_ ? 0.0 : (double)h[S_EVAL] / clock_khz_;
+  stats_.eval_launches = mode == 1 ? ev_eval.size() / 2 : static_ ? 0 : h[S_LEVELS];
   finish_stats(h, ms);
   if (mode == 1 && keep_waves) {
     // two-pass: every waveform sits in the pool in absolute time
@@ -1880,16 +1927,7 @@ void Job::build_graph() {
   }
   if (keep_waves && sched_.size() > 1)
     throw GlsError(GLS_E_UNSUPPORTED, "graph replay keeps waveforms of one-chunk runs only");
-  tiles_cap_ = std::max<uint64_t>(1, max_tiles_);
-  scratch_cap_ = std::max<uint64_t>(1, max_scratch_);
-  ensure((void**)&d_tiles_, cap_tiles_, tiles_cap_ * sizeof(TileDesc));
-  ensure((void**)&d_tout_, cap_tout_, tiles_cap_ * sizeof(TileOut));
-  ensure((void**)&d_toff_, cap_toff_, tiles_cap_ * 4);
   ensure((void**)&d_tails_, cap_tails_, std::max<uint64_t>(max_tails_, 1) * 4);
-  // the replay's bump sequence is the plain run's: a scratch at the pool top
-  // stays clear of every level's outputs when it fits above the largest bump
-  graph_scratch_in_pool_ = max_bump_ <= pool_words_ && scratch_cap_ <= pool_words_ - max_bump_;
-  if (!graph_scratch_in_pool_) ensure((void**)&d_scratch_, cap_scratch_, scratch_cap_ * 4);
   // every chunk's windows in a slot of its own (the groups' chunks in turn)
   const size_t K = sched_.size();
   ensure((void**)&d_cwin_, cap_cwin_, std::max<size_t>(K, 1) * net_base_.size() * sizeof(ChunkWin));
@@ -1908,29 +1946,29 @@ void Job::build_graph() {
   }
   hipGraph_t g = nullptr;
   HC(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed));
+  capturing_ = true;
   try {
-    HC(launch_set_scal(d_scal_, 0, stream_));
-    HC(launch_fill_u64(d_saif_, (uint64_t)n_nets_ * kSaifWords, 0ull, stream_));
-    HC(launch_fill_u64(d_wtot_, n_nets_, 0ull, stream_));
-    if (d_evjob_) HC(launch_fill_u64(d_evjob_, net_base_.size(), 0ull, stream_));
-    HC(launch_saif_stim(d_store_, d_soff_, d_slen_, d_snet_, d_sjob_, n_sig_, d_saif_, d_win_,
+    HC(launch_run_begin(d_scal_, d_saif_, (uint64_t)n_nets_ * kSaifWords, d_wtot_, n_nets_, d_evjob_,
+                        net_base_.size(), stream_));
+    HC(launch_saif_stim(d_store_, d_soff_, d_slen_, d_snet_, d_sjob_, n_sig_, d_saif_, d_win_, d_wtot_,
                         stream_));
-    std::vector<hipEvent_t> none;
     for (size_t q = 0; q < groups_.size(); ++q) {
       const Group& G = groups_[q];
       HC(launch_tails_init(prog_->d_grec + G.g0, G.g1 - G.g0, d_tail_len_, d_tail_off_, d_tails_,
                            stream_));
       for (const Chunk& c : chunks[q]) {
         double hint = 0;
-        run_chunk(c, G, none, true, &hint);
-        end_chunk(c, G, true);
+        run_chunk(c, G, true, &hint, [&] { close_chunk(c, G); });
+        if (c.Fn != kChunkEnd) keep_tails(G);
       }
     }
   } catch (...) {
+    capturing_ = false;
     (void)hipStreamEndCapture(stream_, &g);
     if (g) (void)hipGraphDestroy(g);
     throw;
   }
+  capturing_ = false;
   HC(hipStreamEndCapture(stream_, &g));
   hipError_t e = hipGraphInstantiate(&gexec_, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
@@ -1963,23 +2001,16 @@ void Job::finish_stats(const uint64_t* h, double ms) {
   // algorithmic bytes: every input waveform read once per reading gate, every
   // output written once (whole-run waveform lengths), 3 u64 SAIF counters per
   // net, CSR metadata
-  std::vector<uint64_t> W(n_nets_, 0);
+  uint64_t in_w = h[S_IN_W], out_w = h[S_OUT_W];
   if (mode == 1) {
     std::vector<uint32_t> wlen(n_nets_);
     HC(hipMemcpyAsync(wlen.data(), d_wlen_, n_nets_ * 4ull, hipMemcpyDeviceToHost, stream_));
     HC(hipStreamSynchronize(stream_));
-    for (uint32_t n = 0; n < n_nets_; ++n) W[n] = wlen[n];
-  } else {
-    HC(hipMemcpyAsync(W.data(), d_wtot_, n_nets_ * 8ull, hipMemcpyDeviceToHost, stream_));
-    HC(hipStreamSynchronize(stream_));
-    for (uint32_t s = 0; s < n_sig_; ++s) W[h_snet_[s]] = h_slen_[s];
+    for (const GateRec& g : prog_->h_grec) {
+      for (int j = 0; j < g.k; ++j) in_w += wlen[g.in_net[j]];
+      out_w += wlen[g.out_net];
+    }
   }
-  uint64_t in_w = 0, out_w = 0;
-  for (const GateRec& g : prog_->h_grec) {
-    for (int j = 0; j < g.k; ++j) in_w += W[g.in_net[j]];
-    out_w += W[g.out_net];
-  }
-  if (prog_->h_grec.size() != n_gates_) in_w = out_w = 0;
   stats_.in_words = in_w;
   stats_.out_words = out_w;
   stats_.alg_bytes = 4 * (in_w + out_w) + 24ull * n_nets_ + 16ull * n_gates_ + 4ull * stats_.n_pins;

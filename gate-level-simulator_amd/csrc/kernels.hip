@@ -1,7 +1,7 @@
 // Level kernels of the plain per-level simulator (gfx950).
 //
 // For each topological level:
-//   k_plan         per gate: input event count N, leader input, segment count
+//   k_plan_2p      per gate: input event count N, leader input, segment count
 //   scan (x2)      segment bases and scratch bases over the level's gates
 //   k_segmap       segment -> gate map
 //   k_eval         one lane per time segment of one gate: k-way merge of the
@@ -89,7 +89,7 @@ GLS_DEV uint32_t pick_delay(const GateDev& G, uint32_t mask, const uint32_t* pre
 }
 
 // ------------------------------------------------------------------ plan ----
-__global__ void k_plan(const GateDev* __restrict__ gates, uint32_t ng,
+__global__ void k_plan_2p(const GateDev* __restrict__ gates, uint32_t ng,
                        const uint32_t* __restrict__ wlen, uint32_t seg_target,
                        uint64_t* __restrict__ nseg_out, uint64_t* __restrict__ scr_out,
                        uint32_t* __restrict__ gnseg) {
@@ -482,9 +482,9 @@ hipError_t launch_scan(const uint64_t* in, uint64_t* out, uint64_t n, uint64_t* 
 
 uint64_t scan_part_size(uint64_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
 
-hipError_t launch_plan(const GateDev* gates, uint32_t ng, const uint32_t* wlen, uint32_t seg_target,
+hipError_t launch_plan2p(const GateDev* gates, uint32_t ng, const uint32_t* wlen, uint32_t seg_target,
                        uint64_t* nseg, uint64_t* scr, uint32_t* gnseg, hipStream_t st) {
-  k_plan<<<blocks_for(ng, 256), 256, 0, st>>>(gates, ng, wlen, seg_target, nseg, scr, gnseg);
+  k_plan_2p<<<blocks_for(ng, 256), 256, 0, st>>>(gates, ng, wlen, seg_target, nseg, scr, gnseg);
   GLS_CHECK_LAUNCH();
   return hipSuccess;
 }

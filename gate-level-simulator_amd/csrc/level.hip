@@ -841,7 +841,7 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
   if (lane == 0) {
     TileOut o;
     o.cnt = min(total, out_cap);
-    if (total > out_cap) atomicOr(A.err, ERR_ORDER);
+    if (total > out_cap) atomicOr((unsigned int*)(A.scal + S_ERR), ERR_ORDER);
     o.ft = ft >> 2;
     o.lt = lt >> 2;
     o.flags = out_flags(ft & 3u, lt & 3u, mask ? 1u : 0u);
@@ -869,7 +869,11 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   const int lane = threadIdx.x;
   unsigned long long wave_ev = 0;  // gate events of this wavefront (lane 0)
   unsigned long long wave_tiles = 0, wave_hbm = 0;
-  const uint64_t ntiles = *A.ntiles;  // uniform: one scalar load
+  if (A.scal[S_TRIP]) return;
+  if (blockIdx.x == 0 && lane == 0) A.scal[S_CLOCK] = (uint64_t)wall_clock64();
+  const uint64_t ntiles = A.scal[S_TOT_A];  // uniform: one scalar load
+  uint32_t* const scratch = (uint32_t*)A.scal[S_SCRATCH];
+  unsigned int* const err = (unsigned int*)(A.scal + S_ERR);
   // Tiles are handed out in two parts.  The first half is split into
   // one run of consecutive tiles per workgroup (consecutive tiles of one gate
   // keep its tables in LDS).  The rest is drawn by ticket in batches of B, so
@@ -947,7 +951,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       const bool halo = D.xend != 0 && lane == kLanes - 1;
       keep_entries(A, ln, halo);
       if (halo) ln.nown = 0;
-      emit_tile(A, tk, ln, A.scratch + D.scr, D.out_cap, w_start, w_end, wave_ev, [&] {
+      emit_tile(A, tk, ln, scratch + D.scr, D.out_cap, w_start, w_end, wave_ev, [&] {
         if (staged) {
           wait_vm();
           put_sentinels(Dn);
@@ -977,18 +981,18 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       if (D.id() < W_COUNT) {
         const unsigned long long need = (unsigned long long)D.words() + kStackSlack;
         unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(A.ovf_used, need);
+        if (lane == 0) base = atomicAdd((unsigned long long*)(A.scal + S_OVF_USED), need);
         base = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base);  // lane 0's value
         uint32_t bad = 0;
         if (base + need > A.ovf_cap) {
           // no room: the tile's output is left empty (so the level's waveforms
           // stay in time order) and the run reports the error
-          if (lane == 0) atomicOr(A.err, ERR_OVERFLOW);
+          if (lane == 0) atomicOr(err, ERR_OVERFLOW);
         } else {
           hbm_walk(A, D, A.ovf + base, (uint32_t)need, ln, bad);
         }
-        if (bad) atomicOr(A.err, ERR_ORDER);
+        if (bad) atomicOr(err, ERR_ORDER);
       }
       finish(ln);
     }
@@ -1007,9 +1011,347 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
     D = Dn;
   }
   if (lane == 0) {
-    if (wave_ev) atomicAdd(A.ev_count, wave_ev);
-    atomicAdd(A.tiles_walked, wave_tiles);
-    if (wave_hbm) atomicAdd(A.tiles_walked + 1, wave_hbm);
+    unsigned long long* n = (unsigned long long*)A.scal;
+    if (wave_ev) atomicAdd(n + S_EVL, wave_ev);
+    atomicAdd(n + S_TILES, wave_tiles);
+    if (wave_hbm) atomicAdd(n + S_TILES_HBM, wave_hbm);
+  }
+}
+
+// Exclusive scan of one value per thread over a block of T threads.
+template <int T>
+__device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* sh, uint64_t& total) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  uint64_t x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  __syncthreads();
+  if (lane == 63) sh[wid] = x;
+  __syncthreads();
+  uint64_t before = 0, tot = 0;
+#pragma unroll
+  for (int i = 0; i < T / 64; ++i) {
+    if (i < wid) before += sh[i];
+    tot += sh[i];
+  }
+  total = tot;
+  return before + x - v;
+}
+
+// Scans over blocks in one launch: every block leaves its totals in `part`
+// (agent-scope stores: the blocks run on XCDs with L2s of their own) and
+// counts itself done; the last one turns the totals into prefixes.  No block
+// waits for another.
+__device__ __forceinline__ void put_part(uint64_t* p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool last_block(uint64_t* done) {
+  __shared__ uint32_t s_last;
+  if (threadIdx.x == 0) {  // the thread that stored the block's totals
+    const unsigned long long n = __hip_atomic_fetch_add((unsigned long long*)done, 1ull,
+                                                        __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = n + 1 == gridDim.x ? 1u : 0u;
+    if (s_last) *done = 0;  // for the next scan
+  }
+  __syncthreads();
+  return s_last != 0;
+}
+// part[stride * b] for every block b: totals to exclusive prefixes; returns
+// the sum.
+template <int T>
+__device__ __forceinline__ uint64_t scan_parts(uint64_t* part, uint32_t stride, uint64_t* sh) {
+  uint64_t carry = 0;
+  for (uint32_t b0 = 0; b0 < gridDim.x; b0 += T * 4) {
+    uint64_t v[4], sum = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      const uint32_t b = b0 + threadIdx.x * 4 + i;
+      v[i] = b < gridDim.x ? __hip_atomic_load(part + (uint64_t)stride * b, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT)
+                           : 0;
+      sum += v[i];
+    }
+    uint64_t tot, x = carry + block_scan<T>(sum, sh, tot);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      const uint32_t b = b0 + threadIdx.x * 4 + i;
+      if (b < gridDim.x) part[(uint64_t)stride * b] = x;
+      x += v[i];
+    }
+    carry += tot;
+  }
+  return carry;
+}
+
+// Plan of a level, four consecutive gates per thread: per gate its leader
+// (the input with the most words), words of the leader per tile, tiles and
+// output bound, and their prefixes over the level; then, in the block that
+// finishes last, whether the level has room, where its scratch lies, and the
+// walk's counters.  A tile of a gate of fan-in 1..4 holds 64 times the leader's
+// words of a lane share of about seg_target input words, spread evenly over the
+// gate's tiles; a wide gate's tiles hold wide_words input words (its tables
+// leave less LDS).
+//
+// One launch: with the plan, two three-kernel scans, the capacity check and
+// the clears as launches of their own, a level of the 300-cell netlist spent
+// 9 of its 18 launches (25 of 48 us) before its first descriptor.
+__global__ __launch_bounds__(256) void k_plan(PlanArgs A) {
+  __shared__ uint64_t sh[4];
+  if (A.scal[S_TRIP]) return;
+  const uint32_t g0 = blockIdx.x * kPlanGates + threadIdx.x * 4;
+  uint32_t nt4[4];
+  uint64_t bd4[4], nt_sum = 0, bd_sum = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t g = g0 + i;
+    nt4[i] = 0;
+    bd4[i] = 0;
+    if (g >= A.ng) continue;
+    const GateRec& G = A.gates[g];
+    uint64_t N = 0;
+    uint32_t nl = 0, lead = 0;
+    for (int j = 0; j < G.k; ++j) {
+      const uint32_t n = A.wlen[G.in_net[j]];
+      N += n;
+      if (j == 0 || n > nl) {
+        nl = n;
+        lead = j;
+      }
+    }
+    // a tile's offset inside its gate's waveform travels in 31 bits
+    if (N + 1 >= (1ull << 30)) atomicOr((unsigned int*)(A.scal + S_ERR), ERR_RANGE);
+    GatePlan P;
+    if (G.k > kTileK) {
+      const uint32_t nt0 = (uint32_t)max<uint64_t>(1, (N + A.wide_words - 1) / A.wide_words);
+      P.lt = max(1u, (nl + nt0 - 1) / nt0);
+    } else {
+      uint64_t s = N > 0 ? (uint64_t)A.seg_target * nl / N : 1;
+      if (s < 1) s = 1;
+      if (nl > 0) {
+        const uint64_t nt0 = ((nl + s - 1) / s + kLanes - 1) / kLanes;
+        s = (nl + nt0 * kLanes - 1) / (nt0 * kLanes);
+      }
+      P.lt = (uint32_t)min<uint64_t>(s * kLanes, 0xFFFFFFFFu);
+    }
+    P.lead = lead;
+    A.plan[g] = P;
+    nt4[i] = max(1u, (uint32_t)(((uint64_t)nl + P.lt - 1) / P.lt));
+    A.ntile[g] = nt4[i];
+    // scratch words of the gate's tile outputs: every tile keeps at most its
+    // own input events + 1 entries; the gate's tail is added so that the
+    // level's waveforms (tails + joined entries) never exceed the scratch
+    bd4[i] = N + nt4[i] + 1 + A.tail_len[G.out_net];
+    nt_sum += nt4[i];
+    bd_sum += bd4[i];
+  }
+  uint64_t nt_tot, bd_tot;
+  uint64_t t = block_scan<256>(nt_sum, sh, nt_tot);
+  uint64_t b = block_scan<256>(bd_sum, sh, bd_tot);
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    if (g0 + i < A.ng) {
+      A.tile_loc[g0 + i] = (uint32_t)t;
+      A.scr_loc[g0 + i] = b;
+    }
+    t += nt4[i];
+    b += bd4[i];
+  }
+  if (threadIdx.x == 0) {
+    put_part(A.part + 2 * blockIdx.x, nt_tot);
+    put_part(A.part + 2 * blockIdx.x + 1, bd_tot);
+  }
+  if (!last_block(A.scal + S_DONE)) return;
+  const uint64_t tiles = scan_parts<256>(A.part, 2, sh);
+  const uint64_t scr = scan_parts<256>(A.part + 1, 2, sh);
+  if (threadIdx.x < kTickets) A.ticket[threadIdx.x * kTicketStride] = 0;
+  if (threadIdx.x != 0) return;
+  const uint64_t used = A.scal[S_BUMP], stim = A.scal[S_STIM];
+  unsigned why = 0;
+  if (A.stop && __hip_atomic_load(A.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) why = TRIP_STOP;
+  if (!why && A.proj_cap > 0 && used > stim) {
+    const double proj = (double)(used - stim) * A.all_gates / A.done_gates;
+    if (((double)stim + proj) * 1.35 > A.proj_cap) why = TRIP_PROJECTED;
+  }
+  // The level scratch lives in the unused top of the event pool when twice its
+  // size is free above the bump (the level's outputs, at most the scratch size,
+  // then land below it); otherwise in an allocation of its own.
+  if (!why) {
+    if (tiles > A.tiles_cap) {
+      why = TRIP_ROOM;
+    } else if (used <= A.pool_words && 2 * scr <= A.pool_words - used) {
+      A.scal[S_LIMIT] = A.pool_words - scr;
+      A.scal[S_SCRATCH] = (uint64_t)(A.pool + (A.pool_words - scr));
+    } else if (A.allow_apart && used + scr <= A.pool_words && scr <= A.apart_cap) {
+      A.scal[S_LIMIT] = A.pool_words;
+      A.scal[S_SCRATCH] = (uint64_t)A.apart;
+    } else {
+      why = TRIP_ROOM;
+    }
+  }
+  A.scal[S_TOT_A] = tiles;
+  A.scal[S_TOT_B] = scr;
+  A.scal[S_EVL] = 0;
+  A.scal[S_OVF_USED] = 0;
+  if (why) {
+    A.scal[S_TRIP] = A.level;
+    A.scal[S_WHY] = why;
+  }
+}
+
+// Per tile: its descriptor; thread j of the tile's four takes inputs j and
+// j + 4.
+__global__ __launch_bounds__(256) void k_tile_desc(
+    const GateRec* __restrict__ gates, uint32_t ng, const GatePlan* __restrict__ plan,
+    const uint32_t* __restrict__ tile_loc, const uint64_t* __restrict__ scr_loc,
+    const uint64_t* __restrict__ part, const uint64_t* __restrict__ woff,
+    const uint32_t* __restrict__ wlen, const uint32_t* __restrict__ pool,
+    TileDesc* __restrict__ tiles, const uint64_t* __restrict__ scal) {
+  // a tile's first own word of each input is the previous tile's end: the
+  // block's tiles pass them on through LDS (each boundary searched once)
+  __shared__ uint32_t s_first[2][256];
+  if (scal[S_TRIP]) return;
+  const uint64_t nt = scal[S_TOT_A];
+  const uint32_t nb = (ng + kPlanGates - 1) / kPlanGates;
+  for (uint64_t t0 = (uint64_t)blockIdx.x * 64; t0 < nt; t0 += (uint64_t)gridDim.x * 64) {
+    const uint64_t t = t0 + (threadIdx.x >> 2);
+    const int j0 = (int)(threadIdx.x & 3);
+    const bool valid = t < nt;
+    // gate of tile t: binary search over the plan's blocks, then in the block,
+    // by the tile's first thread, passed to the other three
+    uint32_t g = 0, ti = 0;
+    if (valid && j0 == 0) {
+      uint32_t lo = 0, hi = nb;
+      while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (part[2 * mid] <= t) lo = mid;
+        else hi = mid;
+      }
+      const uint32_t r = (uint32_t)(t - part[2 * lo]);
+      lo *= kPlanGates;
+      hi = min(lo + kPlanGates, ng);
+      while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (tile_loc[mid] <= r) lo = mid;
+        else hi = mid;
+      }
+      g = lo;
+      ti = r - tile_loc[lo];
+    }
+    const int q0 = (int)((threadIdx.x & 63u) & ~3u);
+    g = __shfl(g, q0);
+    ti = __shfl(ti, q0);
+    GateRec G;
+    GatePlan P;
+    uint32_t nl = 0, L[2] = {0, 0};
+    const uint32_t* lw = nullptr;
+    if (valid) {
+      G = gates[g];
+      P = plan[g];
+      lw = pool + woff[G.in_net[P.lead]];
+      nl = wlen[G.in_net[P.lead]];
+      if (ti > 0) {
+        const uint32_t tau_lo = lw[ti * P.lt] >> 2;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t j = j0 + 4 * q;
+          if (j < G.k)
+            L[q] = j == P.lead ? ti * P.lt
+                               : lb_words(pool + woff[G.in_net[j]], wlen[G.in_net[j]], tau_lo << 2);
+        }
+      }
+    }
+    __syncthreads();  // the block's tiles before these are done with s_first
+    s_first[0][threadIdx.x] = L[0];
+    s_first[1][threadIdx.x] = L[1];
+    __syncthreads();
+    if (!valid) continue;
+    TileDesc& D = tiles[t];
+    // own input words of the tile (up to the next tile's first words), summed
+    // over the tile's threads: its output region in the level scratch holds
+    // that many entries plus one
+    uint32_t span = 0, own = 0, xend = 0, dead = 0, lsum = 0, hi8[2] = {0, 0};
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const uint32_t j = j0 + 4 * q;
+      if (j >= G.k) {
+        if (j < kWideK) {
+          D.in_lo[j] = 0;
+          D.n[j] = 0;
+        }
+        continue;
+      }
+      const uint64_t off = woff[G.in_net[j]];
+      const uint32_t n = wlen[G.in_net[j]];
+      const uint32_t* iw = pool + off;
+      uint32_t E = n, Ln = n;
+      if ((ti + 1) * (uint64_t)P.lt < nl) {
+        // the next tile is this gate's: its first words end this one
+        const uint32_t tau_nx = lw[(ti + 1) * P.lt] >> 2;
+        if (threadIdx.x + 4 < blockDim.x && t + 1 < nt)
+          Ln = s_first[q][threadIdx.x + 4];
+        else
+          Ln = j == P.lead ? (ti + 1) * P.lt : lb_words(iw, n, tau_nx << 2);
+        // halo end: the first word at or after tau_nx + dmax lies at or after
+        // Ln, usually at it; step forward with doubling strides, then search
+        // only inside the last stride (every word before a is below the key)
+        const uint32_t key = (tau_nx + G.dmax) << 2;
+        E = Ln;
+        if (E < n && iw[E] < key) {
+          uint32_t a = E, d = 1, b = a + 1;
+          while (b < n && iw[b] < key) {
+            a = b;
+            d <<= 1;
+            b = a + d;
+          }
+          if (b > n) b = n;
+          E = a + 1 + lb_words(iw + a + 1, b - a - 1, key);
+        }
+        if (j == P.lead) xend = (ti + 1) * P.lt - (L[q] > 0 ? L[q] - 1 : 0u);
+      }
+      const uint32_t B = L[q] > 0 ? L[q] - 1 : 0u;
+      D.in_lo[j] = (uint32_t)(off + B);
+      D.n[j] = E - B;
+      hi8[q] = (uint32_t)((off + B) >> 32) << (8 * j0);
+      span += Ln - L[q];
+      own += Ln - max(L[q], 1u);
+      lsum += L[q];
+      dead |= n == 0 ? 1u : 0u;
+    }
+#pragma unroll
+    for (int d = 1; d < 4; d <<= 1) {
+      span += __shfl_xor(span, d);
+      own += __shfl_xor(own, d);
+      xend |= __shfl_xor(xend, d);
+      dead |= __shfl_xor(dead, d);
+      lsum += __shfl_xor(lsum, d);
+      hi8[0] |= __shfl_xor(hi8[0], d);
+      hi8[1] |= __shfl_xor(hi8[1], d);
+    }
+    if (j0 == 0) {
+      D.in_hi[0] = hi8[0];
+      D.in_hi[1] = hi8[1];
+      // a gate's region, then the tile's first own event in the gate's merged
+      // input order plus one slack word per earlier tile (a tile keeps at most
+      // its own events + 1 entries)
+      const uint64_t scr = part[2 * (g / kPlanGates) + 1] + scr_loc[g] + ti + lsum;
+      D.scr_lo = (uint32_t)scr;
+      D.scr_hi = (uint32_t)(scr >> 32);
+      D.own = dead ? 0u : own;
+      D.xend = xend;
+      D.meta = (dead ? (uint32_t)W_DEAD : (uint32_t)G.walk) | ((uint32_t)G.k << 4) | (P.lead << 8) |
+               ((ti == 0 ? 1u : 0u) << 12) | (G.edge_in << 16);
+      D.dt_off = G.dt_off;
+      D.tt_off = G.tt_off;
+      D.dmax = G.dmax;
+      D.job = G.job;
+      D.out_cap = span + 1;
+      D.g = g;
+      D.ti = ti;
+      D.out_net = G.out_net;
+    }
   }
 }
 
@@ -1017,145 +1359,192 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
 // entry repeats the last value before it drops that entry), place each
 // tile's output (offset inside the gate, bit 31: first entry dropped), and
 // add up the SAIF durations: inside tiles, between tiles, and from the last
-// entry to the window end.  One wavefront per gate, 64 tiles per step: each
+// entry to the window end.  Eight lanes per gate, 8 tiles per step: each
 // lane takes the last value and time of the nearest non-empty tile before
 // it (a ballot of the non-empty lanes, then a shuffle; the step's first
 // non-empty tile takes them from the previous step), the offsets are an
 // exclusive scan of the joined counts, and the sums are reduced at the end.
-// In a batch (ev_job set) the gate's events are added to its instance's
-// count for the chunk.
-__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) x += __shfl_xor(x, d);
-  return x;
-}
-
-__global__ void k_gate_carry(const GateRec* __restrict__ gates, uint32_t ng,
-                             const uint64_t* __restrict__ tile_base,
-                             const uint64_t* __restrict__ ntile, const TileOut* __restrict__ tout,
-                             uint32_t* __restrict__ tile_off, uint64_t* __restrict__ gate_cnt,
-                             uint32_t* __restrict__ wlen, unsigned long long* __restrict__ saif,
-                             const ChunkWin* __restrict__ cwin, const unsigned int* __restrict__ err,
-                             TailArgs T, unsigned long long* __restrict__ ev_job) {
-  const int lane = threadIdx.x & 63;
-  const uint32_t g = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-  if (g >= ng) return;  // uniform over the wavefront
-  const GateRec& G = gates[g];
-  if (*err & ERR_CAPACITY) {  // the level was skipped: its tiles were never walked
-    if (lane == 0) {
-      gate_cnt[g] = 0;
-      wlen[G.out_net] = 0;
-    }
-    return;
+// (A wavefront per gate left most lanes idle: gates have 2 to 40 tiles.)  In a
+// batch (ev_job set) the gates' events are added to their instance's count
+// for the chunk, one atomic per block of one instance (one per gate held the
+// batching mix's joins to 88 us a level).
+//
+// The block that finishes last places the gates in the pool and closes the
+// level: bump pointer, gate events, or a trip when the level ran out of
+// overflow stacks.
+__global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
+  __shared__ uint64_t sh[4];
+  __shared__ uint32_t s_cnt[kJoinGates], s_job[kJoinGates];
+  __shared__ unsigned long long s_ev[kJoinGates];
+  if (A.scal[S_TRIP]) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    A.scal[S_EVAL] += (uint64_t)wall_clock64() - A.scal[S_CLOCK];
+    A.scal[S_LEVELS] += 1;
   }
-  const ChunkWin W = cwin[G.job];
-  const unsigned long long start = W.lo, end = W.hi;
-  const uint64_t t0 = tile_base[g], n = ntile[g];
-  // carried from the previous step: count so far, last value and time.  The
-  // gate's waveform starts with its tail (state entry and look-back
-  // entries); after chunk 0 the first new entry is compared with the tail's
-  // last value, which holds from before the chunk (time 0 is clipped to
-  // the chunk's SAIF start).
-  const uint32_t tl = T.tail_len[G.out_net];
-  uint32_t cnt = tl, lv = 0, lt = 0, has = 0;
-  if (!T.first && tl) {
-    lv = T.tails[T.tail_off[G.out_net] + tl - 1] & 3u;
-    has = 1;
+  const uint32_t grp = threadIdx.x >> 3, l8 = threadIdx.x & 7u;
+  const int sh8 = (int)(threadIdx.x & 56u);  // the group's first lane in its wavefront
+  const uint32_t g = blockIdx.x * kJoinGates + grp;
+  if (l8 == 0) {
+    s_cnt[grp] = 0;
+    s_ev[grp] = 0;
+    s_job[grp] = 0xFFFFFFFFu;
   }
-  unsigned long long acc[3] = {0, 0, 0}, tc = 0, gev = 0, any = 0;
-  for (uint64_t c = 0; c < n; c += 64) {
-    const bool in = c + (uint64_t)lane < n;
-    const uint64_t t = t0 + c + (uint64_t)lane;
-    TileOut S = {};
-    if (in) S = tout[t];
-    const bool ne = in && ((S.flags >> 4) & 1u);
-    const uint64_t mask = __ballot(ne);
-    const uint32_t my_lv = (S.flags >> 2) & 3u, my_lt = S.lt, my_fv = S.flags & 3u;
-    // nearest non-empty tile below this lane in the step, if any
-    const uint64_t below = mask & ((1ull << lane) - 1ull);
-    const int pl = below ? 63 - __clzll((long long)below) : 0;
-    const uint32_t s_lv = __shfl(my_lv, pl), s_lt = __shfl(my_lt, pl);
-    const uint32_t p_has = below ? 1u : has;
-    const uint32_t p_lv = below ? s_lv : lv, p_lt = below ? s_lt : lt;
-    uint32_t mine = 0, skip = 0;
-    if (ne) {
-      skip = (p_has && p_lv == my_fv) ? 1u : 0u;
-      mine = S.cnt - skip;
-      if (p_has) saif_acc(acc, p_lv, p_lt, S.ft, start, end);
-      acc[0] += S.t0;
-      acc[1] += S.t1;
-      acc[2] += S.tx;
-      // the tile's first entry against the previous tile's last value
-      tc += (p_has && is_toggle(p_lv, my_fv) && S.ft > W.tc_lo && S.ft <= W.tc_hi) ? 1u : 0u;
-    }
-    // an instance counts the events of its tiles with entries; the tiles of a
-    // wide gate count as one
-    gev += ne || G.k > kTileK ? S.ev : 0u;
-    any |= mask;
-    // inclusive scan of the joined counts over the step
-    uint32_t incl = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t v = __shfl_up(incl, d);
-      if (lane >= d) incl += v;
-    }
-    if (in) tile_off[t] = (cnt + incl - mine) | (skip << 31);
-    cnt += __shfl(incl, 63);
-    if (mask) {  // the step's last non-empty tile carries on
-      const int ll = 63 - __clzll((long long)mask);
-      lv = __shfl(my_lv, ll);
-      lt = __shfl(my_lt, ll);
+  if (g < A.ng) {
+    const GateRec& G = A.gates[g];
+    const ChunkWin W = A.cwin[G.job];
+    const unsigned long long start = W.lo, end = W.hi;
+    const uint64_t t0 = A.plan_part[2 * (g / kPlanGates)] + A.tile_loc[g];
+    const uint32_t n = A.ntile[g];
+    // carried from the previous step: count so far, last value and time.  The
+    // gate's waveform starts with its tail (state entry and look-back
+    // entries); after chunk 0 the first new entry is compared with the tail's
+    // last value, which holds from before the chunk (time 0 is clipped to
+    // the chunk's SAIF start).
+    const uint32_t tl = T.tail_len[G.out_net];
+    uint32_t cnt = tl, lv = 0, lt = 0, has = 0, any = 0;
+    if (!T.first && tl) {
+      lv = T.tails[T.tail_off[G.out_net] + tl - 1] & 3u;
       has = 1;
     }
+    unsigned long long acc[3] = {0, 0, 0}, tc = 0, gev = 0;
+    for (uint32_t c = 0; c < n; c += 8) {
+      const bool in = c + l8 < n;
+      const uint64_t t = t0 + c + l8;
+      TileOut S = {};
+      if (in) S = A.tout[t];
+      const bool ne = in && ((S.flags >> 4) & 1u);
+      const uint32_t mask = (uint32_t)(__ballot(ne) >> sh8) & 0xFFu;
+      const uint32_t my_lv = (S.flags >> 2) & 3u, my_lt = S.lt, my_fv = S.flags & 3u;
+      // nearest non-empty tile below this lane in the step, if any
+      const uint32_t below = mask & ((1u << l8) - 1u);
+      const int pl = below ? 31 - __clz((int)below) : 0;
+      const uint32_t s_lv = __shfl(my_lv, pl, 8), s_lt = __shfl(my_lt, pl, 8);
+      const uint32_t p_has = below ? 1u : has;
+      const uint32_t p_lv = below ? s_lv : lv, p_lt = below ? s_lt : lt;
+      uint32_t mine = 0, skip = 0;
+      if (ne) {
+        skip = (p_has && p_lv == my_fv) ? 1u : 0u;
+        mine = S.cnt - skip;
+        if (p_has) saif_acc(acc, p_lv, p_lt, S.ft, start, end);
+        acc[0] += S.t0;
+        acc[1] += S.t1;
+        acc[2] += S.tx;
+        // the tile's first entry against the previous tile's last value
+        tc += (p_has && is_toggle(p_lv, my_fv) && S.ft > W.tc_lo && S.ft <= W.tc_hi) ? 1u : 0u;
+      }
+      // an instance counts the events of its tiles with entries; the tiles of a
+      // wide gate count as one
+      gev += ne || G.k > kTileK ? S.ev : 0u;
+      any |= mask;
+      // inclusive scan of the joined counts over the step
+      uint32_t incl = mine;
+#pragma unroll
+      for (int d = 1; d < 8; d <<= 1) {
+        const uint32_t v = __shfl_up(incl, d, 8);
+        if ((int)l8 >= d) incl += v;
+      }
+      if (in) A.tile_off[t] = (cnt + incl - mine) | (skip << 31);
+      cnt += __shfl(incl, 7, 8);
+      if (mask) {  // the step's last non-empty tile carries on
+        const int ll = 31 - __clz((int)mask);
+        lv = __shfl(my_lv, ll, 8);
+        lt = __shfl(my_lt, ll, 8);
+        has = 1;
+      }
+    }
+    if (has && l8 == 0) saif_acc(acc, lv, lt, end > lt ? end : (unsigned long long)lt, start, end);
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) {
+      acc[0] += __shfl_xor(acc[0], d, 8);
+      acc[1] += __shfl_xor(acc[1], d, 8);
+      acc[2] += __shfl_xor(acc[2], d, 8);
+      tc += __shfl_xor(tc, d, 8);
+      gev += __shfl_xor(gev, d, 8);
+    }
+    if (l8 == 0) {
+      s_cnt[grp] = cnt;
+      s_job[grp] = G.job;
+      s_ev[grp] = any ? gev : 0ull;
+      A.wlen[G.out_net] = cnt;
+      unsigned long long* sa = A.saif + (uint64_t)kSaifWords * G.out_net;
+      sa[0] = acc[0];
+      sa[1] = acc[1];
+      sa[2] = acc[2];
+      sa[3] = tc;
+    }
   }
-  if (has && lane == 0) saif_acc(acc, lv, lt, end > lt ? end : (unsigned long long)lt, start, end);
-  const unsigned long long s0 = wave_sum_u64(acc[0]), s1 = wave_sum_u64(acc[1]);
-  const unsigned long long s2 = wave_sum_u64(acc[2]), s3 = wave_sum_u64(tc);
-  const unsigned long long s4 = ev_job ? wave_sum_u64(gev) : 0ull;
-  if (lane == 0) {
-    gate_cnt[g] = cnt;
-    wlen[G.out_net] = cnt;
-    unsigned long long* sa = saif + (uint64_t)kSaifWords * G.out_net;
-    sa[0] = s0;
-    sa[1] = s1;
-    sa[2] = s2;
-    sa[3] = s3;
-    // a level whose tiles ran out of overflow stacks runs again: count it then
-    if (ev_job && s4 && any && !(*err & ERR_OVERFLOW)) atomicAdd(ev_job + G.job, s4);
+  __syncthreads();
+  const unsigned int err = *(const unsigned int*)(A.scal + S_ERR);
+  if (threadIdx.x < 64) {  // the first wavefront: prefixes over the block's gates
+    const uint32_t i = threadIdx.x;
+    const uint64_t mine = i < kJoinGates ? s_cnt[i] : 0u;
+    uint64_t x = mine;
+#pragma unroll
+    for (int d = 1; d < (int)kJoinGates; d <<= 1) {
+      const uint64_t y = __shfl_up(x, d, 64);
+      if ((int)i >= d) x += y;
+    }
+    const uint32_t gi = blockIdx.x * kJoinGates + i;
+    if (i < kJoinGates && gi < A.ng) A.out_loc[gi] = x - mine;
+    const uint64_t tot = __shfl(x, kJoinGates - 1, 64);
+    if (i == 0) put_part(A.part + blockIdx.x, tot);
+    // a level whose tiles ran out of overflow stacks runs again: counted then
+    if (A.ev_job && !(err & ERR_OVERFLOW)) {
+      const uint32_t job = i < kJoinGates ? s_job[i] : 0xFFFFFFFFu;
+      unsigned long long ev = i < kJoinGates ? s_ev[i] : 0ull;
+      const uint32_t job0 = __shfl(job, 0, 64);
+      if (__ballot(job != job0 && job != 0xFFFFFFFFu)) {
+        if (job != 0xFFFFFFFFu && ev) atomicAdd(A.ev_job + job, ev);
+      } else {
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) ev += __shfl_xor(ev, d);
+        if (i == 0 && ev) atomicAdd(A.ev_job + job0, ev);
+      }
+    }
   }
+  if (!last_block(A.scal + S_DONE)) return;
+  const uint64_t total = scan_parts<256>(A.part, 1, sh);
+  if (threadIdx.x != 0) return;
+  if (A.ovf_trip && (err & ERR_OVERFLOW)) {
+    A.scal[S_TRIP] = A.level;
+    A.scal[S_WHY] = TRIP_OVERFLOW;
+    return;
+  }
+  const uint64_t base = A.scal[S_BUMP];
+  if (base + total > A.scal[S_LIMIT]) {  // (outputs never exceed the scratch's size)
+    atomicOr((unsigned int*)(A.scal + S_ERR), ERR_CAPACITY | ERR_POOL);
+    A.scal[S_TRIP] = A.level;
+    A.scal[S_WHY] = TRIP_POOL;
+    return;
+  }
+  A.scal[S_OUTBASE] = base;
+  A.scal[S_BUMP] = base + total;
+  A.scal[S_EVC] += A.scal[S_EVL];
 }
 
 // Copy every tile's joined output from the scratch into the gate's dense
 // waveform in the pool (one wavefront per tile, coalesced); the gate's first
 // tile also copies the gate's tail (state and look-back entries, moved to
-// this chunk's time base) to the front.  When the level does not fit the
-// pool (error flag set by k_pool_guard) nothing is copied and the level's
-// waveforms are left empty.
-__global__ void k_compact(const TileDesc* __restrict__ tiles, const uint64_t* __restrict__ ntiles,
-                          const TileOut* __restrict__ tout, const uint32_t* __restrict__ tile_off,
-                          const uint32_t* __restrict__ scratch,
-                          const uint64_t* __restrict__ gate_base, uint32_t* __restrict__ pool,
-                          uint64_t* __restrict__ woff, uint32_t* __restrict__ wlen,
-                          const unsigned int* __restrict__ err, unsigned long long* __restrict__ saif,
-                          const ChunkWin* __restrict__ cwin, uint32_t count_tc, TailArgs T) {
+// this chunk's time base) to the front.
+__global__ __launch_bounds__(256) void k_compact(
+    const TileDesc* __restrict__ tiles, const TileOut* __restrict__ tout,
+    const uint32_t* __restrict__ tile_off, const uint64_t* __restrict__ out_loc,
+    const uint64_t* __restrict__ part, uint32_t* __restrict__ pool, uint64_t* __restrict__ woff,
+    const uint64_t* __restrict__ scal, unsigned long long* __restrict__ saif,
+    const ChunkWin* __restrict__ cwin, uint32_t count_tc, TailArgs T) {
+  if (scal[S_TRIP]) return;
   const int lane = threadIdx.x & 63;
   const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / 64);
-  const bool failed = (*err & ERR_CAPACITY) != 0;
-  const uint64_t nt = *ntiles;
+  const uint64_t nt = scal[S_TOT_A], base = scal[S_OUTBASE];
+  const uint32_t* scratch = (const uint32_t*)scal[S_SCRATCH];
   for (uint64_t t = (uint64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; t < nt; t += waves) {
     const TileDesc& D = tiles[t];
-    if (failed) {
-      if (D.ti == 0 && lane == 0) {
-        woff[D.out_net] = 0;
-        wlen[D.out_net] = 0;
-      }
-      continue;
-    }
+    const uint64_t gate = base + part[D.g / kJoinGates] + out_loc[D.g];
     if (D.ti == 0) {
-      if (lane == 0) woff[D.out_net] = gate_base[D.g];
+      if (lane == 0) woff[D.out_net] = gate;
       const uint32_t tl = T.tail_len[D.out_net];
       const uint32_t* ts = T.tails + T.tail_off[D.out_net];
-      uint32_t* td = pool + gate_base[D.g];
+      uint32_t* td = pool + gate;
       for (uint32_t q = lane; q < tl; q += 64) {
         const uint32_t w = ts[q], tt = w >> 2;
         td[q] = ((tt > T.shift ? tt - T.shift : 0u) << 2) | (w & 3u);
@@ -1166,7 +1555,7 @@ __global__ void k_compact(const TileDesc* __restrict__ tiles, const uint64_t* __
     const uint32_t off = tile_off[t] & 0x7FFFFFFFu, skip = tile_off[t] >> 31;
     const uint32_t n = S.cnt - skip;
     const uint32_t* src = scratch + (((uint64_t)D.scr_hi << 32) | D.scr_lo) + skip;
-    uint32_t* dst = pool + gate_base[D.g] + off;
+    uint32_t* dst = pool + gate + off;
     // four loads in flight per lane before their stores: the copy of a tile
     // waits for memory about n / 256 times instead of n / 64
     uint32_t q = lane;
@@ -1180,7 +1569,7 @@ __global__ void k_compact(const TileDesc* __restrict__ tiles, const uint64_t* __
     for (; q < n; q += 64) dst[q] = src[q];
     if (count_tc) {
       // SAIF TC inside the tile: 0<->1 changes between its consecutive
-      // entries (the first entry against the previous tile is k_gate_carry's)
+      // entries (the first entry against the previous tile is k_join's)
       const uint32_t* e = src - skip;
       const ChunkWin W = cwin[D.job];
       uint32_t c = 0;
@@ -1195,201 +1584,202 @@ __global__ void k_compact(const TileDesc* __restrict__ tiles, const uint64_t* __
   }
 }
 
-// Start-of-run scalars: bump pointer past the stimulus words, all else 0.
-__global__ void k_set_scal(uint64_t* scal, uint64_t bump) {
-  if (blockIdx.x == 0 && threadIdx.x < 16) scal[threadIdx.x] = threadIdx.x == 0 ? bump : 0;
+// ------------------------------------------------------- stimulus and tails ---
+
+// first index of a sorted 64-bit word range whose time (word >> 2) is at or
+// after `t`
+__device__ __forceinline__ uint32_t lb_time64(const uint64_t* a, uint32_t n, uint64_t t) {
+  uint32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if ((a[mid] >> 2) < t) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
 }
 
-// Per gate: leader (the input with the most words), words of the leader per
-// tile, tiles, output bound.  A tile of a gate of fan-in 1..4 holds 64 times
-// the leader's words of a lane share of about seg_target input words, spread
-// evenly over the gate's tiles; a wide gate's tiles hold wide_words input words
-// (its tables leave less LDS).
-__global__ void k_plan2(const GateRec* __restrict__ gates, uint32_t ng,
-                        const uint32_t* __restrict__ wlen, uint32_t seg_target,
-                        uint32_t wide_words, GatePlan* __restrict__ plan, uint64_t* __restrict__ ntile,
-                        uint64_t* __restrict__ bound, unsigned int* __restrict__ err,
-                        const uint32_t* __restrict__ tail_len) {
-  uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= ng) return;
-  const GateRec& G = gates[g];
-  uint64_t N = 0;
-  uint32_t nl = 0, lead = 0;
-  for (int j = 0; j < G.k; ++j) {
-    uint32_t n = wlen[G.in_net[j]];
-    N += n;
-    if (j == 0 || n > nl) {
-      nl = n;
-      lead = j;
-    }
+// Per stimulus signal: the range [lb, ub) of its resident waveform, the chunk
+// words it needs (one state entry + the range) and their prefixes; the chunk
+// trips when its stimulus does not leave the pool 1,024 words.
+__global__ __launch_bounds__(256) void k_stim_plan(const uint64_t* __restrict__ store,
+                                                   const uint64_t* __restrict__ soff,
+                                                   const uint32_t* __restrict__ slen, uint32_t ns,
+                                                   uint64_t lb, uint64_t ub, uint64_t* __restrict__ cnt,
+                                                   uint32_t* __restrict__ first,
+                                                   uint64_t* __restrict__ loc, uint64_t* __restrict__ part,
+                                                   uint64_t pool_words, uint64_t* __restrict__ scal) {
+  __shared__ uint64_t sh[4];
+  if (scal[S_TRIP]) return;
+  const uint32_t s = blockIdx.x * kStimSignals + threadIdx.x;
+  uint64_t n = 0;
+  if (s < ns) {
+    const uint64_t* w = store + soff[s];
+    const uint32_t len = slen[s];
+    const uint32_t i = lb ? lb_time64(w, len, lb) : 0u;
+    const uint32_t j = lb_time64(w, len, ub);
+    first[s] = i;
+    n = 1ull + (j - i);
+    cnt[s] = n;
   }
-  // a tile's offset inside its gate's waveform travels in 31 bits
-  if (N + 1 >= (1ull << 30)) atomicOr(err, ERR_RANGE);
-  GatePlan P;
-  if (G.k > kTileK) {
-    const uint32_t nt0 = (uint32_t)max<uint64_t>(1, (N + wide_words - 1) / wide_words);
-    P.lt = max(1u, (nl + nt0 - 1) / nt0);
-  } else {
-    uint64_t s = N > 0 ? (uint64_t)seg_target * nl / N : 1;
-    if (s < 1) s = 1;
-    if (nl > 0) {
-      const uint64_t nt0 = ((nl + s - 1) / s + kLanes - 1) / kLanes;
-      s = (nl + nt0 * kLanes - 1) / (nt0 * kLanes);
-    }
-    P.lt = (uint32_t)min<uint64_t>(s * kLanes, 0xFFFFFFFFu);
+  uint64_t tot;
+  const uint64_t x = block_scan<256>(n, sh, tot);
+  if (s < ns) loc[s] = x;
+  if (threadIdx.x == 0) put_part(part + blockIdx.x, tot);
+  if (!last_block(scal + S_DONE)) return;
+  const uint64_t total = scan_parts<256>(part, 1, sh);
+  if (threadIdx.x != 0) return;
+  scal[S_BUMP] = scal[S_STIM] = total;
+  if (total + 1024 > pool_words) {
+    scal[S_TRIP] = ~0ull;
+    scal[S_WHY] = TRIP_STIM;
   }
-  P.lead = lead;
-  plan[g] = P;
-  const uint32_t nt = max(1u, (uint32_t)(((uint64_t)nl + P.lt - 1) / P.lt));
-  ntile[g] = nt;
-  // scratch words of the gate's tile outputs: every tile keeps at most its
-  // own input events + 1 entries; the gate's tail is added so that the
-  // level's waveforms (tails + joined entries) never exceed the scratch
-  bound[g] = N + nt + 1 + tail_len[G.out_net];
 }
 
-// Per tile: its descriptor; thread j of the tile's four takes inputs j and
-// j + 4.
-__global__ void k_tile_desc(const GateRec* __restrict__ gates, uint32_t ng,
-                            const GatePlan* __restrict__ plan,
-                            const uint64_t* __restrict__ tile_base,
-                            const uint64_t* __restrict__ scr_base,
-                            const uint64_t* __restrict__ woff, const uint32_t* __restrict__ wlen,
-                            const uint32_t* __restrict__ pool, TileDesc* __restrict__ tiles,
-                            const uint64_t* __restrict__ ntiles, unsigned long long* __restrict__ ticket,
-                            unsigned long long* __restrict__ ovf_used) {
-  // the walk's tickets and overflow stacks start over
-  if (blockIdx.x == 0 && threadIdx.x < kTickets) ticket[threadIdx.x * kTicketStride] = 0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *ovf_used = 0;
-  // a tile's first own word of each input is the previous tile's end: the
-  // block's tiles pass them on through LDS (each boundary searched once)
-  __shared__ uint32_t s_first[2][256];
-  const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t t = x >> 2;
-  const int j0 = (int)(x & 3);
-  const uint64_t nt = *ntiles;
-  const bool valid = t < nt;
-  // gate of tile t: binary search over tile_base by the tile's first
-  // thread, passed to the other three
-  uint32_t g = 0;
-  if (valid && j0 == 0) {
-    uint32_t lo = 0, hi = ng;
-    while (hi - lo > 1) {
-      uint32_t mid = (lo + hi) >> 1;
-      if (tile_base[mid] <= t) lo = mid;
+// One wavefront per stimulus signal: state entry at relative time 0, then
+// the range in relative time (abs - lb + 1 >= 1); sets the net's waveform.
+__global__ __launch_bounds__(256) void k_stim_copy(
+    const uint64_t* __restrict__ store, const uint64_t* __restrict__ soff,
+    const uint32_t* __restrict__ snet, uint32_t ns, uint64_t lb, const uint64_t* __restrict__ cnt,
+    const uint32_t* __restrict__ first, const uint64_t* __restrict__ loc,
+    const uint64_t* __restrict__ part, uint32_t* __restrict__ pool, uint64_t* __restrict__ woff,
+    uint32_t* __restrict__ wlen, const uint64_t* __restrict__ scal) {
+  if (scal[S_TRIP]) return;
+  const uint32_t s = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
+  const int lane = threadIdx.x & 63;
+  if (s >= ns) return;
+  const uint64_t base = part[s / kStimSignals] + loc[s];
+  const uint64_t* w = store + soff[s] + first[s];
+  const uint32_t n = (uint32_t)(cnt[s] - 1);
+  uint32_t* d = pool + base;
+  if (lane == 0) {
+    d[0] = first[s] > 0 ? (uint32_t)(w[-1] & 3u) : 1u;  // X before the first entry
+    woff[snet[s]] = base;
+    wlen[snet[s]] = n + 1;
+  }
+  for (uint32_t q = lane; q < n; q += 64) {
+    const uint64_t e = w[q];
+    d[1 + q] = (uint32_t)((((e >> 2) - lb + 1) << 2) | (e & 3u));
+  }
+}
+
+// End of chunk k, per gate output: where its tail for chunk k+1 starts in
+// its chunk waveform (relative time of chunk k): the last entry before
+// `key` (lb_k+1 in chunk k's time; index 0, the state entry, is below it)
+// and everything after it.  Tails are short, so the search gallops back
+// from the end.  Their prefixes place them in the tail store.
+__global__ __launch_bounds__(256) void k_tail_len(const GateRec* __restrict__ gates, uint32_t ng,
+                                                  const uint64_t* __restrict__ woff,
+                                                  const uint32_t* __restrict__ wlen,
+                                                  const uint32_t* __restrict__ pool, uint32_t key,
+                                                  uint64_t* __restrict__ len, uint64_t* __restrict__ src,
+                                                  uint64_t* __restrict__ loc, uint64_t* __restrict__ part,
+                                                  uint64_t* __restrict__ scal) {
+  __shared__ uint64_t sh[4];
+  if (scal[S_TRIP]) return;
+  const uint32_t kw = key << 2;
+  uint64_t n4[4], sum = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t g = blockIdx.x * kPlanGates + threadIdx.x * 4 + i;
+    n4[i] = 0;
+    if (g >= ng) continue;
+    const uint32_t net = gates[g].out_net;
+    const uint32_t* w = pool + woff[net];
+    const uint32_t n = wlen[net];
+    // w[lo] < kw; every index at or after hi is >= kw (hi = n: none checked)
+    uint32_t lo = 0, hi = n, d = 1;
+    while (hi > lo + 1) {
+      const uint32_t p = hi - min(d, hi - lo - 1);
+      if (w[p] < kw) {
+        lo = p;
+        break;
+      }
+      hi = p;
+      d <<= 1;
+    }
+    while (hi > lo + 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (w[mid] < kw) lo = mid;
       else hi = mid;
     }
-    g = lo;
+    n4[i] = n - lo;
+    len[g] = n - lo;
+    src[g] = woff[net] + lo;
+    sum += n - lo;
   }
-  g = __shfl(g, (int)((threadIdx.x & 63u) & ~3u));
-  GateRec G;
-  GatePlan P;
-  uint32_t ti = 0, nl = 0, L[2] = {0, 0};
-  const uint32_t* lw = nullptr;
-  if (valid) {
-    G = gates[g];
-    P = plan[g];
-    ti = (uint32_t)(t - tile_base[g]);
-    lw = pool + woff[G.in_net[P.lead]];
-    nl = wlen[G.in_net[P.lead]];
-    if (ti > 0) {
-      const uint32_t tau_lo = lw[ti * P.lt] >> 2;
+  uint64_t tot, x = block_scan<256>(sum, sh, tot);
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const uint32_t j = j0 + 4 * q;
-        if (j < G.k)
-          L[q] = j == P.lead ? ti * P.lt
-                             : lb_words(pool + woff[G.in_net[j]], wlen[G.in_net[j]], tau_lo << 2);
-      }
-    }
+  for (uint32_t i = 0; i < 4; ++i) {
+    const uint32_t g = blockIdx.x * kPlanGates + threadIdx.x * 4 + i;
+    if (g < ng) loc[g] = x;
+    x += n4[i];
   }
-  s_first[0][threadIdx.x] = L[0];
-  s_first[1][threadIdx.x] = L[1];
-  __syncthreads();
-  if (!valid) return;
-  TileDesc& D = tiles[t];
-  // own input words of the tile (up to the next tile's first words), summed
-  // over the tile's threads: its output region in the level scratch holds
-  // that many entries plus one
-  uint32_t span = 0, own = 0, xend = 0, dead = 0, lsum = 0, hi8[2] = {0, 0};
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const uint32_t j = j0 + 4 * q;
-    if (j >= G.k) {
-      if (j < kWideK) {
-        D.in_lo[j] = 0;
-        D.n[j] = 0;
-      }
-      continue;
-    }
-    const uint64_t off = woff[G.in_net[j]];
-    const uint32_t n = wlen[G.in_net[j]];
-    const uint32_t* iw = pool + off;
-    uint32_t E = n, Ln = n;
-    if ((ti + 1) * (uint64_t)P.lt < nl) {
-      // the next tile is this gate's: its first words end this one
-      const uint32_t tau_nx = lw[(ti + 1) * P.lt] >> 2;
-      if (threadIdx.x + 4 < blockDim.x && t + 1 < nt)
-        Ln = s_first[q][threadIdx.x + 4];
-      else
-        Ln = j == P.lead ? (ti + 1) * P.lt : lb_words(iw, n, tau_nx << 2);
-      // halo end: the first word at or after tau_nx + dmax lies at or after
-      // Ln, usually at it; step forward with doubling strides, then search
-      // only inside the last stride (every word before a is below the key)
-      const uint32_t key = (tau_nx + G.dmax) << 2;
-      E = Ln;
-      if (E < n && iw[E] < key) {
-        uint32_t a = E, d = 1, b = a + 1;
-        while (b < n && iw[b] < key) {
-          a = b;
-          d <<= 1;
-          b = a + d;
-        }
-        if (b > n) b = n;
-        E = a + 1 + lb_words(iw + a + 1, b - a - 1, key);
-      }
-      if (j == P.lead) xend = (ti + 1) * P.lt - (L[q] > 0 ? L[q] - 1 : 0u);
-    }
-    const uint32_t B = L[q] > 0 ? L[q] - 1 : 0u;
-    D.in_lo[j] = (uint32_t)(off + B);
-    D.n[j] = E - B;
-    hi8[q] = (uint32_t)((off + B) >> 32) << (8 * j0);
-    span += Ln - L[q];
-    own += Ln - max(L[q], 1u);
-    lsum += L[q];
-    dead |= n == 0 ? 1u : 0u;
+  if (threadIdx.x == 0) put_part(part + blockIdx.x, tot);
+  if (!last_block(scal + S_DONE)) return;
+  const uint64_t total = scan_parts<256>(part, 1, sh);
+  if (threadIdx.x == 0) scal[S_TAILS] = total;
+}
+
+// Copies each gate output's tail into the tail store (kept in chunk k's
+// relative time; k_compact moves it to chunk k+1's).  A store too small for
+// the chunk (a replayed sequence that outgrew its first run) flags
+// ERR_CAPACITY and copies nothing past its end.
+__global__ void k_tail_copy(const GateRec* __restrict__ gates, uint32_t ng,
+                            const uint64_t* __restrict__ len, const uint64_t* __restrict__ src,
+                            const uint64_t* __restrict__ loc, const uint64_t* __restrict__ part,
+                            const uint32_t* __restrict__ pool, uint32_t* __restrict__ tails,
+                            uint64_t cap, uint32_t* __restrict__ tail_len,
+                            uint64_t* __restrict__ tail_off, uint64_t* __restrict__ scal) {
+  if (scal[S_TRIP]) return;
+  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= ng) return;
+  const uint32_t net = gates[g].out_net;
+  const uint64_t n = len[g], o = part[g / kPlanGates] + loc[g];
+  if (o + n > cap) {
+    atomicOr((unsigned int*)(scal + S_ERR), ERR_CAPACITY);
+    tail_len[net] = 0;
+    tail_off[net] = 0;
+    return;
   }
-#pragma unroll
-  for (int d = 1; d < 4; d <<= 1) {
-    span += __shfl_xor(span, d);
-    own += __shfl_xor(own, d);
-    xend |= __shfl_xor(xend, d);
-    dead |= __shfl_xor(dead, d);
-    lsum += __shfl_xor(lsum, d);
-    hi8[0] |= __shfl_xor(hi8[0], d);
-    hi8[1] |= __shfl_xor(hi8[1], d);
+  const uint32_t* s = pool + src[g];
+  for (uint64_t q = 0; q < n; ++q) tails[o + q] = s[q];
+  tail_len[net] = (uint32_t)n;
+  tail_off[net] = o;
+}
+
+// Start of a run: scalars, SAIF counters, waveform lengths and instance event
+// counts to zero.
+__global__ void k_run_begin(uint64_t* scal, unsigned long long* saif, uint64_t n_saif,
+                            unsigned long long* wtot, uint64_t n_nets, unsigned long long* evjob,
+                            uint64_t n_jobs) {
+  const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+  if (i0 < S_COUNT) scal[i0] = 0;
+  for (uint64_t i = i0; i < n_saif; i += step) saif[i] = 0;
+  for (uint64_t i = i0; i < n_nets; i += step) wtot[i] = 0;
+  if (evjob)
+    for (uint64_t i = i0; i < n_jobs; i += step) evjob[i] = 0;
+}
+
+// End of a run: waveform words read by the gates and written by them (wtot:
+// whole-run waveform lengths of every net).
+__global__ __launch_bounds__(256) void k_word_counts(const GateRec* __restrict__ gates, uint32_t ng,
+                                                     const unsigned long long* __restrict__ wtot,
+                                                     uint64_t* __restrict__ scal) {
+  __shared__ uint64_t sh[4];
+  if (scal[S_TRIP]) return;
+  uint64_t in = 0, out = 0;
+  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += gridDim.x * blockDim.x) {
+    const GateRec& G = gates[g];
+    for (int j = 0; j < G.k; ++j) in += wtot[G.in_net[j]];
+    out += wtot[G.out_net];
   }
-  if (j0 == 0) {
-    D.in_hi[0] = hi8[0];
-    D.in_hi[1] = hi8[1];
-    // a gate's region, then the tile's first own event in the gate's merged
-    // input order plus one slack word per earlier tile (a tile keeps at most
-    // its own events + 1 entries)
-    const uint64_t scr = scr_base[g] + ti + lsum;
-    D.scr_lo = (uint32_t)scr;
-    D.scr_hi = (uint32_t)(scr >> 32);
-    D.own = dead ? 0u : own;
-    D.xend = xend;
-    D.meta = (dead ? (uint32_t)W_DEAD : (uint32_t)G.walk) | ((uint32_t)G.k << 4) | (P.lead << 8) |
-             ((ti == 0 ? 1u : 0u) << 12) | (G.edge_in << 16);
-    D.dt_off = G.dt_off;
-    D.tt_off = G.tt_off;
-    D.dmax = G.dmax;
-    D.job = G.job;
-    D.out_cap = span + 1;
-    D.g = g;
-    D.ti = ti;
-    D.out_net = G.out_net;
+  uint64_t ti, to;
+  block_scan<256>(in, sh, ti);
+  block_scan<256>(out, sh, to);
+  if (threadIdx.x == 0) {
+    atomicAdd((unsigned long long*)(scal + S_IN_W), (unsigned long long)ti);
+    atomicAdd((unsigned long long*)(scal + S_OUT_W), (unsigned long long)to);
   }
 }
 
@@ -1398,94 +1788,102 @@ __global__ void k_fill_u64(unsigned long long* p, uint64_t n, unsigned long long
   if (i < n) p[i] = v;
 }
 
-hipError_t launch_plan2(const GateRec* gates, uint32_t ng, const uint32_t* wlen,
-                        uint32_t seg_target, uint32_t wide_words, GatePlan* plan, uint64_t* ntile, uint64_t* bound,
-                        unsigned int* err, const uint32_t* tail_len, hipStream_t st) {
-  k_plan2<<<(ng + 255) / 256, 256, 0, st>>>(gates, ng, wlen, seg_target, wide_words, plan, ntile, bound,
-                                            err, tail_len);
+// ------------------------------------------------------- launch helpers ----
+
+static inline unsigned nblk(uint64_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
+
+hipError_t launch_plan(const PlanArgs& a, hipStream_t st) {
+  if (a.ng == 0) return hipSuccess;
+  k_plan<<<nblk(a.ng, kPlanGates), 256, 0, st>>>(a);
   return hipGetLastError();
 }
 
+// `guess`: expected tiles, for the launch width alone
 hipError_t launch_tile_desc(const GateRec* gates, uint32_t ng, const GatePlan* plan,
-                            const uint64_t* tile_base, const uint64_t* scr_base,
+                            const uint32_t* tile_loc, const uint64_t* scr_loc, const uint64_t* part,
                             const uint64_t* woff, const uint32_t* wlen, const uint32_t* pool,
-                            TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles,
-                            unsigned long long* ticket, unsigned long long* ovf_used, hipStream_t st) {
-  if (ntiles == 0) return hipSuccess;
-  const uint64_t threads = ntiles * 4;
-  k_tile_desc<<<(unsigned)((threads + 255) / 256), 256, 0, st>>>(
-      gates, ng, plan, tile_base, scr_base, woff, wlen, pool, tiles, ntiles_dev, ticket, ovf_used);
+                            TileDesc* tiles, const uint64_t* scal, uint64_t guess, hipStream_t st) {
+  const unsigned nb = (unsigned)std::min<uint64_t>(guess / 64 + 1, 8192);
+  k_tile_desc<<<nb, 256, 0, st>>>(gates, ng, plan, tile_loc, scr_loc, part, woff, wlen, pool, tiles,
+                                  scal);
   return hipGetLastError();
 }
 
 hipError_t launch_fill_u64(unsigned long long* p, uint64_t n, unsigned long long v,
                            hipStream_t st) {
   if (n == 0) return hipSuccess;
-  k_fill_u64<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(p, n, v);
+  k_fill_u64<<<nblk(n, 256), 256, 0, st>>>(p, n, v);
   return hipGetLastError();
 }
 
-// Device-driven levels: when the tile count or the level's scratch does not
-// fit the arrays sized by the first run, the level is skipped (tile count 0)
-// and the error flag says why.
-__global__ void k_guard(uint64_t* scal, uint64_t tiles_cap, uint64_t scratch_cap) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  // scal: 1 tiles of the level, 2 scratch words of the level, 7 error flags
-  if (scal[1] > tiles_cap || scal[2] > scratch_cap) {
-    scal[1] = 0;
-    scal[2] = 0;
-    atomicOr((unsigned int*)(scal + 7), ERR_CAPACITY);
-  }
-}
-
-// After the level's output size is known: when it does not fit the pool,
-// flag the error (the compaction then leaves the level empty) and reserve
-// nothing.  scal: 0 bump, 3 output words of the level.
-__global__ void k_pool_guard(uint64_t* scal, uint64_t pool_words) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (scal[0] + scal[3] > pool_words) {
-    scal[3] = 0;
-    atomicOr((unsigned int*)(scal + 7), ERR_CAPACITY | ERR_POOL);
-  }
-}
-
-hipError_t launch_pool_guard(uint64_t* scal, uint64_t pool_words, hipStream_t st) {
-  k_pool_guard<<<1, 64, 0, st>>>(scal, pool_words);
+hipError_t launch_join(const JoinArgs& a, const TailArgs& T, hipStream_t st) {
+  if (a.ng == 0) return hipSuccess;
+  k_join<<<nblk(a.ng, kJoinGates), 256, 0, st>>>(a, T);
   return hipGetLastError();
 }
 
-hipError_t launch_gate_carry(const GateRec* gates, uint32_t ng, const uint64_t* tile_base,
-                             const uint64_t* ntile, const TileOut* tout, uint32_t* tile_off,
-                             uint64_t* gate_cnt, uint32_t* wlen, unsigned long long* saif,
-                             const ChunkWin* cwin, const unsigned int* err, const TailArgs& T,
-                             unsigned long long* ev_job, hipStream_t st) {
+hipError_t launch_compact(const TileDesc* tiles, const TileOut* tout, const uint32_t* tile_off,
+                          const uint64_t* out_loc, const uint64_t* part, uint32_t* pool,
+                          uint64_t* woff, const uint64_t* scal, unsigned long long* saif,
+                          const ChunkWin* cwin, uint32_t count_tc, const TailArgs& T, uint64_t guess,
+                          hipStream_t st) {
+  const unsigned nb = (unsigned)std::min<uint64_t>(guess / 4 + 1, 8192);  // 4 wavefronts each
+  k_compact<<<nb, 256, 0, st>>>(tiles, tout, tile_off, out_loc, part, pool, woff, scal, saif, cwin,
+                                count_tc, T);
+  return hipGetLastError();
+}
+
+hipError_t launch_run_begin(uint64_t* scal, unsigned long long* saif, uint64_t n_saif,
+                            unsigned long long* wtot, uint64_t n_nets, unsigned long long* evjob,
+                            uint64_t n_jobs, hipStream_t st) {
+  const unsigned nb = (unsigned)std::min<uint64_t>(nblk(std::max<uint64_t>(n_saif, S_COUNT), 256), 2048);
+  k_run_begin<<<nb, 256, 0, st>>>(scal, saif, n_saif, wtot, n_nets, evjob, n_jobs);
+  return hipGetLastError();
+}
+
+hipError_t launch_word_counts(const GateRec* gates, uint32_t ng, const unsigned long long* wtot,
+                              uint64_t* scal, hipStream_t st) {
   if (ng == 0) return hipSuccess;
-  k_gate_carry<<<(ng + 3) / 4, 256, 0, st>>>(gates, ng, tile_base, ntile, tout, tile_off, gate_cnt,
-                                             wlen, saif, cwin, err, T, ev_job);  // one wavefront per gate
+  k_word_counts<<<std::min(nblk(ng, 256), 1024u), 256, 0, st>>>(gates, ng, wtot, scal);
   return hipGetLastError();
 }
 
-hipError_t launch_compact(const TileDesc* tiles, const uint64_t* ntiles_dev, uint64_t ntiles_cap,
-                          const TileOut* tout, const uint32_t* tile_off,
-                          const uint32_t* scratch, const uint64_t* gate_base, uint32_t* pool,
-                          uint64_t* woff, uint32_t* wlen, const unsigned int* err,
-                          unsigned long long* saif, const ChunkWin* cwin, uint32_t count_tc,
-                          const TailArgs& T, hipStream_t st) {
-  if (ntiles_cap == 0) return hipSuccess;
-  const uint64_t blocks = std::min<uint64_t>((ntiles_cap + 3) / 4, 8192);  // 4 wavefronts each
-  k_compact<<<(unsigned)blocks, 256, 0, st>>>(tiles, ntiles_dev, tout, tile_off, scratch, gate_base,
-                                              pool, woff, wlen, err, saif, cwin, count_tc, T);
+hipError_t launch_stim_plan(const uint64_t* store, const uint64_t* soff, const uint32_t* slen,
+                            uint32_t ns, uint64_t lb, uint64_t ub, uint64_t* cnt, uint32_t* first,
+                            uint64_t* loc, uint64_t* part, uint64_t pool_words, uint64_t* scal,
+                            hipStream_t st) {
+  k_stim_plan<<<std::max(1u, nblk(ns, kStimSignals)), 256, 0, st>>>(store, soff, slen, ns, lb, ub, cnt,
+                                                                    first, loc, part, pool_words, scal);
   return hipGetLastError();
 }
 
-hipError_t launch_guard(uint64_t* scal, uint64_t tiles_cap, uint64_t scratch_cap, hipStream_t st) {
-  k_guard<<<1, 64, 0, st>>>(scal, tiles_cap, scratch_cap);
+hipError_t launch_stim_copy(const uint64_t* store, const uint64_t* soff, const uint32_t* snet,
+                            uint32_t ns, uint64_t lb, const uint64_t* cnt, const uint32_t* first,
+                            const uint64_t* loc, const uint64_t* part, uint32_t* pool, uint64_t* woff,
+                            uint32_t* wlen, const uint64_t* scal, hipStream_t st) {
+  if (ns == 0) return hipSuccess;
+  k_stim_copy<<<nblk(ns, 4), 256, 0, st>>>(store, soff, snet, ns, lb, cnt, first, loc, part, pool, woff,
+                                           wlen, scal);
   return hipGetLastError();
 }
 
+hipError_t launch_tail_len(const GateRec* gates, uint32_t ng, const uint64_t* woff,
+                           const uint32_t* wlen, const uint32_t* pool, uint32_t key, uint64_t* len,
+                           uint64_t* src, uint64_t* loc, uint64_t* part, uint64_t* scal,
+                           hipStream_t st) {
+  if (ng == 0) return hipSuccess;
+  k_tail_len<<<nblk(ng, kPlanGates), 256, 0, st>>>(gates, ng, woff, wlen, pool, key, len, src, loc, part,
+                                                   scal);
+  return hipGetLastError();
+}
 
-hipError_t launch_set_scal(uint64_t* scal, uint64_t bump, hipStream_t st) {
-  k_set_scal<<<1, 64, 0, st>>>(scal, bump);
+hipError_t launch_tail_copy(const GateRec* gates, uint32_t ng, const uint64_t* len,
+                            const uint64_t* src, const uint64_t* loc, const uint64_t* part,
+                            const uint32_t* pool, uint32_t* tails, uint64_t cap, uint32_t* tail_len,
+                            uint64_t* tail_off, uint64_t* scal, hipStream_t st) {
+  if (ng == 0) return hipSuccess;
+  k_tail_copy<<<nblk(ng, 256), 256, 0, st>>>(gates, ng, len, src, loc, part, pool, tails, cap, tail_len,
+                                             tail_off, scal);
   return hipGetLastError();
 }
 
@@ -1502,7 +1900,8 @@ int level_max_blocks(uint32_t lds_words) {
     per_cu = 4;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 256;
-  // LDS is handed out in pieces of 1,280 bytes, 160 KiB per CU
+  // LDS is handed out in pieces of 1,280 bytes, 160 KiB per CU (workgroups
+  // that do not fit at once would start their fixed runs late)
   const uint32_t piece = (lds_words * 4 + 1279) / 1280;
   per_cu = std::min<int>(per_cu, (int)(128 / std::max(1u, piece)));
   return std::max(per_cu, 1) * cus;
