@@ -31,7 +31,11 @@ struct gls_design {
   // VCD decides which nets are driven from outside; its other signals and
   // their order do not change the program)
   std::mutex mu;
-  std::map<std::vector<std::string>, std::shared_ptr<const Program>> progs;
+  struct Compiled {
+    std::shared_ptr<const Program> pg;
+    std::shared_ptr<const NetTable> nets;  // built for the first run
+  };
+  std::map<std::vector<std::string>, Compiled> progs;
 };
 struct gls_stim {
   Stimulus st;
@@ -75,39 +79,63 @@ static std::vector<std::string> program_key(const Netlist& nl, const std::vector
   return k;
 }
 
-std::shared_ptr<const Program> design_program(gls_design* d, const std::vector<std::string>& names) {
+// The compiled program for the set of driven nets, with its net table when
+// `nets` is asked for.
+static std::shared_ptr<const Program> design_program(gls_design* d, const std::vector<std::string>& names,
+                                                     std::shared_ptr<const NetTable>* nets = nullptr) {
   auto key = program_key(d->nl, names);
   std::lock_guard<std::mutex> lk(d->mu);
   auto it = d->progs.find(key);
-  if (it != d->progs.end()) return it->second;
-  auto pg = std::make_shared<const Program>(compile_program(d->nl, d->lib, names));
-  d->progs.emplace(std::move(key), pg);
-  return pg;
+  if (it == d->progs.end()) {
+    auto pg = std::make_shared<const Program>(compile_program(d->nl, d->lib, names));
+    it = d->progs.emplace(std::move(key), gls_design::Compiled{pg, nullptr}).first;
+  }
+  if (nets) {
+    if (!it->second.nets) {
+      const Program& pg = *it->second.pg;
+      auto t = std::make_shared<NetTable>();
+      t->names = pg.net_names;
+      t->in_saif = pg.in_saif;
+      t->is_gate.assign(t->names.size(), 0);
+      for (auto& g : pg.gates) t->is_gate[g.out_net] = 1;
+      t->by_name.reserve(t->names.size());
+      for (size_t i = 0; i < t->names.size(); ++i) t->by_name.emplace(t->names[i], (int)i);
+      it->second.nets = std::move(t);
+    }
+    *nets = it->second.nets;
+  }
+  return it->second.pg;
 }
 
 RunInst make_inst(gls_design* d, const gls_stim* s, uint64_t dumpon, uint64_t dumpoff) {
   RunInst r;
-  r.pg = design_program(d, s->st.names);
-  r.names = r.pg->net_names;
-  r.in_saif = r.pg->in_saif;
-  r.is_gate.assign(r.names.size(), 0);
-  for (auto& g : r.pg->gates) r.is_gate[g.out_net] = 1;
-  for (size_t i = 0; i < r.names.size(); ++i) r.by_name.emplace(r.names[i], (int)i);
+  r.pg = design_program(d, s->st.names, &r.nets);
+  std::shared_ptr<NetTable> own;  // the shared table and the stimulus's own signals
   for (auto& nm : s->st.names) {
     int id = d->nl.net(nm);
     if (id < 0) {  // a VCD signal the netlist does not use: SAIF record only
-      auto it = r.by_name.find(nm);
-      if (it != r.by_name.end()) id = it->second;
-      else {
-        id = (int)r.names.size();
-        r.names.push_back(nm);
-        r.in_saif.push_back(1);
-        r.is_gate.push_back(0);
-        r.by_name.emplace(nm, id);
+      const NetTable& t = own ? *own : *r.nets;
+      auto it = t.by_name.find(nm);
+      if (it != t.by_name.end()) {
+        id = it->second;
+      } else {
+        if (!own) {
+          own = std::make_shared<NetTable>();
+          own->names = r.nets->names;
+          own->in_saif = r.nets->in_saif;
+          own->is_gate = r.nets->is_gate;
+          own->by_name = r.nets->by_name;
+        }
+        id = (int)own->names.size();
+        own->names.push_back(nm);
+        own->in_saif.push_back(1);
+        own->is_gate.push_back(0);
+        own->by_name.emplace(nm, id);
       }
     }
     r.stim_nets.push_back(id);
   }
+  if (own) r.nets = std::move(own);
   r.st = &s->st;
   r.start = dumpon;
   r.end = dumpoff;
@@ -115,21 +143,11 @@ RunInst make_inst(gls_design* d, const gls_stim* s, uint64_t dumpon, uint64_t du
   return r;
 }
 
-std::string inst_saif(const RunInst& in, const std::vector<uint64_t>& saif, uint32_t base,
-                      bool with_tc) {
-  std::vector<SaifRecord> recs;
-  for (size_t n = 0; n < in.names.size(); ++n) {
-    if (!in.in_saif[n]) continue;
-    SaifRecord s;
-    const uint64_t* c = &saif[(size_t)kSaifWords * (base + n)];
-    s.name = in.names[n];
-    s.t0 = c[0];
-    s.t1 = c[1];
-    s.tx = c[2];
-    s.tc = c[3];
-    recs.push_back(std::move(s));
-  }
-  return saif_text(std::move(recs), in.start, in.end, in.timescale_ps, with_tc);
+size_t inst_saif(const RunInst& in, const std::vector<uint64_t>& saif, uint32_t base, bool with_tc,
+                 char* buf, size_t cap) {
+  static_assert(kSaifWords == 4, "SaifLayout reads four counters a net");
+  return in.nets->saif().text(saif.data() + (size_t)kSaifWords * base, in.start, in.end,
+                              in.timescale_ps, with_tc, buf, cap);
 }
 }  // namespace gls
 
@@ -280,7 +298,7 @@ int gls_design_load(const char* path, gls_design** out) {
   d->gv_text = std::move(t.gv);
   d->sdf_text = std::move(t.sdf);
   d->progs.emplace(program_key(d->nl, declared_inputs(d->nl)),
-                   std::make_shared<const Program>(std::move(pg)));
+                   gls_design::Compiled{std::make_shared<const Program>(std::move(pg)), nullptr});
   *out = d.release();
   API_END
 }
@@ -528,9 +546,9 @@ static const RunInst& inst_of(const gls_run* r, size_t i) {
   return r->inst[i];
 }
 
-static std::string make_saif(const gls_run* r, size_t i) {
+static size_t make_saif(const gls_run* r, size_t i, char* buf, size_t cap) {
   if (!r->executed) throw GlsError(GLS_E_STATE, "run not executed");
-  return inst_saif(inst_of(r, i), r->saif, r->job->net_base(i), r->saif_tc);
+  return inst_saif(inst_of(r, i), r->saif, r->job->net_base(i), r->saif_tc, buf, cap);
 }
 
 int gls_run_instances(const gls_run* r, size_t* n) {
@@ -543,16 +561,10 @@ int gls_run_instances(const gls_run* r, size_t* n) {
 int gls_run_write_saif(const gls_run* r, const char* path) {
   API_BEGIN
   if (!r || !path) throw GlsError(GLS_E_ARG, "null argument");
-  write_file(path, make_saif(r, 0));
+  std::string text(make_saif(r, 0, nullptr, 0), '\0');
+  make_saif(r, 0, &text[0], text.size());
+  write_file(path, text);
   API_END
-}
-
-static void copy_text(const std::string& s, char* buf, size_t cap, size_t* len) {
-  *len = s.size();
-  if (buf) {
-    if (cap < s.size()) throw GlsError(GLS_E_ARG, "buffer too small");
-    std::memcpy(buf, s.data(), s.size());
-  }
 }
 
 int gls_run_saif_text(const gls_run* r, char* buf, size_t cap, size_t* len) {
@@ -562,7 +574,8 @@ int gls_run_saif_text(const gls_run* r, char* buf, size_t cap, size_t* len) {
 int gls_run_instance_saif_text(const gls_run* r, size_t i, char* buf, size_t cap, size_t* len) {
   API_BEGIN
   if (!r || !len) throw GlsError(GLS_E_ARG, "null argument");
-  copy_text(make_saif(r, i), buf, cap, len);
+  *len = make_saif(r, i, buf, cap);
+  if (buf && cap < *len) throw GlsError(GLS_E_ARG, "buffer too small");
   API_END
 }
 
@@ -571,8 +584,8 @@ int gls_run_net_saif(const gls_run* r, const char* net, uint64_t v[3]) {
   if (!r || !net || !v) throw GlsError(GLS_E_ARG, "null argument");
   if (!r->executed) throw GlsError(GLS_E_STATE, "run not executed");
   const RunInst& in = inst_of(r, 0);
-  auto it = in.by_name.find(net);
-  if (it == in.by_name.end()) throw GlsError(GLS_E_ARG, std::string("unknown net ") + net);
+  auto it = in.nets->by_name.find(net);
+  if (it == in.nets->by_name.end()) throw GlsError(GLS_E_ARG, std::string("unknown net ") + net);
   for (int i = 0; i < 3; ++i) v[i] = r->saif[(size_t)kSaifWords * it->second + i];
   API_END
 }
@@ -583,8 +596,8 @@ int gls_run_net_toggles(const gls_run* r, const char* net, uint64_t* tc) {
   if (!r->executed) throw GlsError(GLS_E_STATE, "run not executed");
   if (!r->saif_tc) throw GlsError(GLS_E_STATE, "toggle counts need the saif_tc option");
   const RunInst& in = inst_of(r, 0);
-  auto it = in.by_name.find(net);
-  if (it == in.by_name.end()) throw GlsError(GLS_E_ARG, std::string("unknown net ") + net);
+  auto it = in.nets->by_name.find(net);
+  if (it == in.nets->by_name.end()) throw GlsError(GLS_E_ARG, std::string("unknown net ") + net);
   *tc = r->saif[(size_t)kSaifWords * it->second + 3];
   API_END
 }
@@ -595,7 +608,7 @@ int gls_run_net_toggles(const gls_run* r, const char* net, uint64_t* tc) {
 static void net_words(const gls_run* r, size_t i, int id, std::vector<uint64_t>& out) {
   const RunInst& in = inst_of(r, i);
   out.clear();
-  if (in.is_gate[id]) {
+  if (in.nets->is_gate[id]) {
     const auto& W = r->job->waves();
     const size_t n = r->job->net_base(i) + (size_t)id;
     if (n < W.size()) out = W[n];
@@ -614,8 +627,8 @@ static void net_words(const gls_run* r, size_t i, int id, std::vector<uint64_t>&
 static int net_id(const gls_run* r, const char* net) {
   if (!r->executed || !r->keep_waves) throw GlsError(GLS_E_STATE, "waveforms not kept");
   const RunInst& in = inst_of(r, 0);
-  auto it = in.by_name.find(net);
-  if (it == in.by_name.end()) throw GlsError(GLS_E_ARG, std::string("unknown net ") + net);
+  auto it = in.nets->by_name.find(net);
+  if (it == in.nets->by_name.end()) throw GlsError(GLS_E_ARG, std::string("unknown net ") + net);
   return it->second;
 }
 
@@ -670,10 +683,10 @@ int gls_run_instance_waves_hash(const gls_run* r, size_t i, uint64_t* hash) {
   const uint32_t base = r->job->net_base(i);
   uint64_t total = 0;
   static const std::vector<uint64_t> empty;
-  for (size_t n = 0; n < in.names.size(); ++n) {
-    if (!in.is_gate[n]) continue;
+  for (size_t n = 0; n < in.nets->names.size(); ++n) {
+    if (!in.nets->is_gate[n]) continue;
     uint64_t h = 1469598103934665603ull;
-    for (unsigned char ch : in.names[n]) h = (h ^ ch) * 1099511628211ull;
+    for (unsigned char ch : in.nets->names[n]) h = (h ^ ch) * 1099511628211ull;
     const std::vector<uint64_t>& w = base + n < W.size() ? W[base + n] : empty;
     for (uint64_t e : w) {
       const uint32_t x = (uint32_t)e;
@@ -833,7 +846,8 @@ int gls_server_job_info(gls_server* s, uint64_t job, gls_job_info* info) {
 int gls_server_job_saif_text(gls_server* s, uint64_t job, char* buf, size_t cap, size_t* len) {
   API_BEGIN
   if (!s || !len) throw GlsError(GLS_E_ARG, "null argument");
-  copy_text(s->srv->saif(job), buf, cap, len);
+  *len = s->srv->saif(job, buf, cap);
+  if (buf && cap < *len) throw GlsError(GLS_E_ARG, "buffer too small");
   API_END
 }
 

@@ -1223,57 +1223,120 @@ std::string vcd_text(const Stimulus& st) {
 // ---------------------------------------------------------------- SAIF ----
 // Record layout of src/simulate.cpp:85-88,162-163,303-304,373-378 with the
 // header of src/simulate.cu:457-481; nets in lexicographic order.
-std::string saif_text(std::vector<SaifRecord> recs, uint64_t start, uint64_t end, int timescale_ps,
-                      bool with_tc) {
-  std::sort(recs.begin(), recs.end(),
-            [](const SaifRecord& a, const SaifRecord& b) { return a.name < b.name; });
-  std::string o;
-  o.reserve(recs.size() * 64 + 128);
+SaifLayout::SaifLayout(const std::vector<std::string>& names, const std::vector<uint8_t>& in_saif) {
+  std::vector<uint32_t> hier;
+  for (uint32_t n = 0; n < names.size(); ++n)
+    if (in_saif[n]) net_.push_back(n);
+  std::sort(net_.begin(), net_.end(), [&](uint32_t a, uint32_t b) { return names[a] < names[b]; });
+  auto nested = [&](uint32_t n) {
+    const std::string& s = names[n];
+    const size_t lb = s.find('[');
+    return lb != std::string::npos && lb + 1 < s.size() && !(s[lb + 1] >= '0' && s[lb + 1] <= '9');
+  };
+  std::stable_partition(net_.begin(), net_.end(), [&](uint32_t n) { return !nested(n); });
+  while (flat_ < net_.size() && !nested(net_[flat_])) ++flat_;
+  head_at_.reserve(net_.size() + 1);
+  head_at_.push_back(0);
+  for (size_t r = 0; r < net_.size(); ++r) {
+    const std::string& s = names[net_[r]];
+    if (r < flat_) {
+      head_ += "      (" + s + "\n         (T0 ";
+    } else {
+      const size_t lb = s.find('['), rb = s.find(']');
+      head_ += "   (INSTANCE " + s.substr(0, lb) + "\n      (NET\n         (" +
+               s.substr(lb + 1, rb - lb - 1) + "\n            (T0 ";
+    }
+    head_at_.push_back(head_.size());
+  }
+}
+
+static size_t u64_digits(uint64_t v) {
+  size_t n = 1;
+  for (; v >= 10000; v /= 10000) n += 4;
+  return n + (v >= 10) + (v >= 100) + (v >= 1000);
+}
+
+static char* put_u64(char* p, uint64_t v) {
+  char* const end = p + u64_digits(v);
+  char* q = end;
+  do {
+    *--q = (char)('0' + v % 10);
+    v /= 10;
+  } while (v);
+  return end;
+}
+
+template <size_t N>
+static char* put_lit(char* p, const char (&s)[N]) {
+  std::memcpy(p, s, N - 1);
+  return p + N - 1;
+}
+
+size_t SaifLayout::text(const uint64_t* counts, uint64_t start, uint64_t end, int timescale_ps,
+                        bool with_tc, char* buf, size_t cap) const {
   const char* unit = "ps";
   long long res = timescale_ps;
   if (timescale_ps % 1000000 == 0) { unit = "us"; res = timescale_ps / 1000000; }
   else if (timescale_ps % 1000 == 0) { unit = "ns"; res = timescale_ps / 1000; }
-  char buf[256];
-  std::snprintf(buf, sizeof buf, "(TIMESCALE %lld %s)\n(DURATION %llu)\n(INSTANCE root\n   (NET\n",
-                res, unit, (unsigned long long)(end - start));
-  o += buf;
-  std::vector<const SaifRecord*> hier;
-  for (auto& r : recs) {
-    size_t lb = r.name.find('[');
-    if (lb != std::string::npos && lb + 1 < r.name.size() &&
-        !(r.name[lb + 1] >= '0' && r.name[lb + 1] <= '9')) {
-      hier.push_back(&r);
-      continue;
+  char top[256];
+  const size_t n_top =
+      (size_t)std::snprintf(top, sizeof top, "(TIMESCALE %lld %s)\n(DURATION %llu)\n(INSTANCE root\n   (NET\n",
+                            res, unit, (unsigned long long)(end - start));
+  static const char kMid[] = "   )\n\n", kEnd[] = ")\n";
+  static const char kFlat[] = ")\n      )\n", kNested[] = ")\n         )\n      )\n   )\n";
+  const size_t n = net_.size();
+  auto size_of = [&](size_t r) {
+    const uint64_t* c = counts + 4 * (size_t)net_[r];
+    size_t z = head_at_[r + 1] - head_at_[r] + u64_digits(c[0]) + u64_digits(c[1]) + u64_digits(c[2]) +
+               2 * 6 + (r < flat_ ? sizeof kFlat - 1 : sizeof kNested - 1);
+    if (with_tc) z += 6 + u64_digits(c[3]);
+    return z;
+  };
+  auto put = [&](char* p, size_t r) {
+    const uint64_t* c = counts + 4 * (size_t)net_[r];
+    const size_t h = head_at_[r + 1] - head_at_[r];
+    std::memcpy(p, head_.data() + head_at_[r], h);
+    p = put_u64(p + h, c[0]);
+    p = put_u64(put_lit(p, ") (T1 "), c[1]);
+    p = put_u64(put_lit(p, ") (TX "), c[2]);
+    if (with_tc) p = put_u64(put_lit(p, ") (TC "), c[3]);
+    return r < flat_ ? put_lit(p, kFlat) : put_lit(p, kNested);
+  };
+  // a stretch of records per thread: all measured, then all written
+  const size_t T = std::max<size_t>(1, std::min<size_t>((size_t)host_threads(0), n / 4096));
+  std::vector<size_t> at(T + 1, 0);  // stretch i's bytes, then its first byte
+  auto in_stretches = [&](auto&& work) {
+    std::vector<std::thread> th;
+    size_t started = 1;
+    try {
+      th.reserve(T);
+      for (; started < T; ++started) th.emplace_back(work, started);
+    } catch (...) {  // no more threads: this one takes the rest
     }
-    o += "      (" + r.name + "\n";
-    if (with_tc)
-      std::snprintf(buf, sizeof buf, "         (T0 %llu) (T1 %llu) (TX %llu) (TC %llu)\n      )\n",
-                    (unsigned long long)r.t0, (unsigned long long)r.t1, (unsigned long long)r.tx,
-                    (unsigned long long)r.tc);
-    else
-      std::snprintf(buf, sizeof buf, "         (T0 %llu) (T1 %llu) (TX %llu)\n      )\n",
-                    (unsigned long long)r.t0, (unsigned long long)r.t1, (unsigned long long)r.tx);
-    o += buf;
-  }
-  o += "   )\n\n";
-  for (auto* r : hier) {
-    size_t lb = r->name.find('['), rb = r->name.find(']');
-    std::string inst = r->name.substr(0, lb);
-    std::string net = r->name.substr(lb + 1, rb - lb - 1);
-    o += "   (INSTANCE " + inst + "\n      (NET\n         (" + net + "\n";
-    if (with_tc)
-      std::snprintf(buf, sizeof buf,
-                    "            (T0 %llu) (T1 %llu) (TX %llu) (TC %llu)\n         )\n      )\n   )\n",
-                    (unsigned long long)r->t0, (unsigned long long)r->t1, (unsigned long long)r->tx,
-                    (unsigned long long)r->tc);
-    else
-      std::snprintf(buf, sizeof buf,
-                    "            (T0 %llu) (T1 %llu) (TX %llu)\n         )\n      )\n   )\n",
-                    (unsigned long long)r->t0, (unsigned long long)r->t1, (unsigned long long)r->tx);
-    o += buf;
-  }
-  o += ")\n";
-  return o;
+    work((size_t)0);
+    for (size_t i = started; i < T; ++i) work(i);
+    for (auto& t : th) t.join();
+  };
+  in_stretches([&](size_t i) {
+    size_t z = 0;
+    for (size_t r = n * i / T; r < n * (i + 1) / T; ++r) z += size_of(r);
+    at[i + 1] = z;
+  });
+  for (size_t i = 0; i < T; ++i) at[i + 1] += at[i];
+  const size_t all = n_top + at[T] + sizeof kMid - 1 + sizeof kEnd - 1;
+  if (!buf || cap < all) return all;
+  std::memcpy(buf, top, n_top);
+  in_stretches([&](size_t i) {
+    const size_t a = n * i / T, b = n * (i + 1) / T;
+    char* p = buf + n_top + at[i] + (a > flat_ ? sizeof kMid - 1 : 0);
+    for (size_t r = a; r < b; ++r) {
+      if (r == flat_) p = put_lit(p, kMid);
+      p = put(p, r);
+    }
+  });
+  if (flat_ == n) std::memcpy(buf + n_top + at[T], kMid, sizeof kMid - 1);
+  std::memcpy(buf + all - (sizeof kEnd - 1), kEnd, sizeof kEnd - 1);
+  return all;
 }
 
 }  // namespace gls

@@ -35,18 +35,28 @@ std::string gv_text(const Netlist& nl, const Library& lib);
 std::string sdf_text(const Netlist& nl, const Library& lib);
 std::string vcd_text(const Stimulus& st);
 
-// SAIF report.  One record per net; `hier` records are nets named
-// "inst[pin]" (outputs an instance leaves unconnected), written as nested
-// INSTANCE blocks like the reference's CPU writer (src/simulate.cpp:305-377).
-struct SaifRecord {
-  std::string name;
-  uint64_t t0 = 0, t1 = 0, tx = 0;
-  uint64_t tc = 0;  // 0<->1 transitions in (start, end]
+// SAIF report of a set of nets: one record per net with in_saif set, in name
+// order; nets named "inst[pin]" (outputs an instance leaves unconnected) follow
+// as nested INSTANCE blocks like the reference's CPU writer
+// (src/simulate.cpp:305-377).  The order and the records' fixed text depend on
+// the names alone and are laid out once; a report then only adds the counters.
+class SaifLayout {
+ public:
+  SaifLayout(const std::vector<std::string>& names, const std::vector<uint8_t>& in_saif);
+  // The report's size; written to `buf` when it is not null and holds it
+  // (cap).  counts: T0, T1, TX, TC of net n at counts[4 n].  with_tc: each
+  // record also carries (TC n) after (TX ...); off is the reference's
+  // three-field record (src/simulate.cu:133-135).  Large reports are measured
+  // and written by several threads, each its own stretch of records.
+  size_t text(const uint64_t* counts, uint64_t start, uint64_t end, int timescale_ps, bool with_tc,
+              char* buf, size_t cap) const;
+
+ private:
+  std::string head_;              // every record's text up to its first counter
+  std::vector<uint64_t> head_at_; // record r: [head_at_[r], head_at_[r + 1])
+  std::vector<uint32_t> net_;     // record -> net, records in report order
+  size_t flat_ = 0;               // records before the nested ones
 };
-// with_tc: each record also carries (TC n) after (TX ...); off by default,
-// which is the reference's three-field record (src/simulate.cu:133-135).
-std::string saif_text(std::vector<SaifRecord> recs, uint64_t start, uint64_t end,
-                      int timescale_ps = 1, bool with_tc = false);
 
 std::string read_file(const std::string& path);
 void write_file(const std::string& path, const std::string& data);

@@ -76,7 +76,7 @@ uint64_t Server::pool_cap_words() const {
 // image when it is not resident yet.
 uint64_t Server::estimate(const Rec& r, bool* resident) const {
   const RunInst& in = r.inst;
-  const uint64_t gates = in.pg->gates.size(), nets = in.names.size();
+  const uint64_t gates = in.pg->gates.size(), nets = in.nets->names.size();
   uint64_t stim = 0;
   for (auto& w : in.st->waves) stim += w.size();
   const uint64_t pool = job_pool_words(in, opt_.pool_factor, pool_cap_words());
@@ -310,7 +310,7 @@ bool Server::run_group(const std::vector<Rec*>& group, hipStream_t stream) {
   const Clock::time_point now = Clock::now();
   for (size_t i = 0; i < group.size(); ++i) {
     Rec* r = group[i];
-    const size_t n = r->inst.names.size();
+    const size_t n = r->inst.nets->names.size();
     std::vector<uint64_t> mine(saif.begin() + (size_t)kSaifWords * base[i],
                                saif.begin() + (size_t)kSaifWords * (base[i] + n));
     // a job cancelled (or past its deadline) while its batch ran keeps no result
@@ -383,13 +383,13 @@ ServerJobInfo Server::info(uint64_t id) {
   return it->second->info;
 }
 
-std::string Server::saif(uint64_t id) {
+size_t Server::saif(uint64_t id, char* buf, size_t cap) {
   std::lock_guard<std::mutex> lk(mu_);
   auto it = jobs_.find(id);
   if (it == jobs_.end()) throw GlsError(GLS_E_ARG, "unknown job");
   Rec* r = it->second.get();
   if (r->info.status != 0) throw GlsError(GLS_E_STATE, "job not finished successfully");
-  return inst_saif(r->inst, r->saif, 0, false);
+  return inst_saif(r->inst, r->saif, 0, false, buf, cap);
 }
 
 void Server::drain() {

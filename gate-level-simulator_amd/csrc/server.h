@@ -19,26 +19,42 @@
 #include <vector>
 
 #include "engine.h"
+#include "formats.h"
 
 namespace gls {
 
-// One simulation as the C-ABI sees it: program, names for the SAIF writer,
-// stimulus, window.
-struct RunInst {
-  std::shared_ptr<const Program> pg;
-  std::vector<int> stim_nets;
-  std::vector<std::string> names;  // all net names incl. stimulus-only signals
+// The nets of a run: the program's, and the stimulus signals that the netlist
+// does not use.  Built once per compiled program and shared by its runs (a
+// stimulus with signals of its own has a copy).
+struct NetTable {
+  std::vector<std::string> names;
   std::vector<uint8_t> in_saif;
   std::vector<uint8_t> is_gate;
   std::unordered_map<std::string, int> by_name;
+  const SaifLayout& saif() const {  // laid out on first use
+    std::call_once(once_, [this] { saif_ = std::make_unique<SaifLayout>(names, in_saif); });
+    return *saif_;
+  }
+
+ private:
+  mutable std::once_flag once_;
+  mutable std::unique_ptr<SaifLayout> saif_;
+};
+
+// One simulation as the C-ABI sees it: program, nets, stimulus, window.
+struct RunInst {
+  std::shared_ptr<const Program> pg;
+  std::shared_ptr<const NetTable> nets;
+  std::vector<int> stim_nets;
   const Stimulus* st = nullptr;
   uint64_t start = 0, end = 0;
   int timescale_ps = 1;
 };
 
-// SAIF text of one instance; with_tc adds each net's (TC n) toggle count.
-std::string inst_saif(const RunInst& in, const std::vector<uint64_t>& saif, uint32_t base,
-                      bool with_tc);
+// SAIF text of one instance: its size, written to buf when that holds it
+// (cap); with_tc adds each net's (TC n) toggle count.
+size_t inst_saif(const RunInst& in, const std::vector<uint64_t>& saif, uint32_t base, bool with_tc,
+                 char* buf, size_t cap);
 
 struct ServerOptions {
   uint64_t device_budget = 0;  // bytes of HBM the server may use (0: 90% of free)
@@ -84,7 +100,8 @@ class Server {
   // still queued/running at the timeout).
   int wait(uint64_t id, double timeout_s);
   ServerJobInfo info(uint64_t id);
-  std::string saif(uint64_t id);
+  // size of a done job's SAIF text, written to buf when that holds it
+  size_t saif(uint64_t id, char* buf, size_t cap);
   ServerStats stats();
   void drain();
 
