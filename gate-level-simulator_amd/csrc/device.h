@@ -188,8 +188,8 @@ struct TailArgs {
 // host reads why, makes room and goes on from that level.
 enum ScalSlot {
   S_BUMP = 0,     // pool words used
-  S_TOT_A = 1,    // tiles of the level
-  S_TOT_B = 2,    // scratch words of the level
+  S_TOT_A = 1,    // tiles and scratch words that the last planned level asked for
+  S_TOT_B = 2,
   S_TOT_OUT = 3,  // output words of the level (two-pass path)
   S_EVC = 4,      // gate events of the run
   S_EVL = 5,      // gate events of the level
@@ -199,7 +199,6 @@ enum ScalSlot {
   S_TAILS = 10,   // words of the chunk's gate-output tails
   S_TRIP = 11,    // 0, or the tripped level + 1
   S_WHY = 12,     // TripWhy
-  S_SCRATCH = 13, // address of the level scratch
   S_LIMIT = 14,   // pool word that the level's outputs must not reach
   S_OUTBASE = 15, // pool word of the level's first output
   S_STIM = 16,    // pool words of the chunk's stimulus
@@ -208,7 +207,10 @@ enum ScalSlot {
   S_EVAL = 19,    // ticks spent in walks
   S_LEVELS = 20,  // walks run
   S_IN_W = 21, S_OUT_W = 22,     // waveform words read by gates, written by gates
-  S_COUNT = 24
+  // of the level in hand and the one planned while its outputs are copied
+  // (LevelArgs::slot): tiles, address of the level scratch
+  S_NTILES = 23, S_SCRATCH = 25,
+  S_COUNT = 32
 };
 enum TripWhy : unsigned { TRIP_STOP = 1, TRIP_PROJECTED, TRIP_ROOM, TRIP_OVERFLOW, TRIP_STIM, TRIP_POOL };
 
@@ -218,7 +220,7 @@ constexpr uint32_t kTickets = 4, kTicketStride = 32;
 // Gates per block of the plan's and the join's scans (a gate's prefix = its
 // block's, in `part`, plus its own inside the block), and signals per block of
 // the stimulus cut.
-constexpr uint32_t kPlanGates = 1024, kJoinGates = 32, kStimSignals = 256;
+constexpr uint32_t kPlanGates = 256, kJoinGates = 32, kStimSignals = 256;
 
 // Plan of one level.
 struct PlanArgs {
@@ -240,10 +242,28 @@ struct PlanArgs {
   uint32_t* apart;
   uint32_t allow_apart;
   uint32_t level;       // level + 1, for S_TRIP
+  uint32_t slot;        // 0 or 1
   // automatic chunks: trip when the chunk's outputs so far, over `done_gates`
   // of `all_gates`, project to more than proj_cap words (0: not asked)
   double proj_cap, all_gates, done_gates;
   const uint32_t* stop; // host flag: nonzero trips the chunk (null: none)
+};
+
+// Compaction of one level's outputs.
+struct CompactArgs {
+  const TileDesc* tiles;
+  const TileOut* tout;
+  const uint32_t* tile_off;
+  const uint64_t* out_loc;
+  const uint64_t* part;
+  uint32_t* pool;
+  uint64_t* woff;
+  const uint64_t* scal;
+  unsigned long long* saif;
+  const ChunkWin* cwin;
+  uint32_t count_tc;
+  uint32_t level;       // level + 1
+  uint32_t slot;
 };
 
 // Join of one level's tiles.
@@ -280,6 +300,7 @@ struct LevelArgs {
   const ChunkWin* cwin;        // SAIF bounds of this chunk per instance
   uint32_t lds_words;          // LDS of a workgroup
   uint32_t prefetch;           // 1: stage the next tile before storing this one
+  uint32_t slot;
   uint32_t lo_rel;             // F_k in chunk time: candidates below it only pre-empt
   uint32_t hi_rel;             // F_k+1 in chunk time (0xFFFFFFFF: last chunk): candidates
                                // at or above it belong to the next chunk and are dropped

@@ -246,7 +246,8 @@ class Job {
   void put_chunk_windows(const Chunk& c, bool capture);
   int run_chunk(const Chunk& c, const Group& G, bool device_driven, double* grow_hint,
                 const std::function<void()>& after);
-  void launch_level_of(size_t l, const Chunk& c, const Group& G, bool device_driven, double proj_cap);
+  PlanArgs plan_args(size_t l, const Group& G, uint32_t slot, bool device_driven, double proj_cap);
+  void launch_levels(size_t next, const Chunk& c, const Group& G, bool device_driven, double proj_cap);
   void close_chunk(const Chunk& c, const Group& G);
   void keep_tails(const Group& G);
   void run_chunks();

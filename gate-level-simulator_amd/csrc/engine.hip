@@ -47,14 +47,12 @@ hipError_t launch_plan(const PlanArgs& a, hipStream_t st);
 hipError_t launch_tile_desc(const GateRec* gates, uint32_t ng, const GatePlan* plan,
                             const uint32_t* tile_loc, const uint64_t* scr_loc, const uint64_t* part,
                             const uint64_t* woff, const uint32_t* wlen, const uint32_t* pool,
-                            TileDesc* tiles, const uint64_t* scal, uint64_t guess, hipStream_t st);
+                            TileDesc* tiles, const uint64_t* scal, uint32_t slot, uint64_t guess,
+                            hipStream_t st);
 hipError_t launch_fill_u64(unsigned long long* p, uint64_t n, unsigned long long v, hipStream_t st);
 hipError_t launch_level(const LevelArgs& a, unsigned nblocks, hipStream_t st);
 hipError_t launch_join(const JoinArgs& a, const TailArgs& T, hipStream_t st);
-hipError_t launch_compact(const TileDesc* tiles, const TileOut* tout, const uint32_t* tile_off,
-                          const uint64_t* out_loc, const uint64_t* part, uint32_t* pool,
-                          uint64_t* woff, const uint64_t* scal, unsigned long long* saif,
-                          const ChunkWin* cwin, uint32_t count_tc, const TailArgs& T, uint64_t guess,
+hipError_t launch_compact(const CompactArgs& a, const TailArgs& T, const PlanArgs* next, uint64_t guess,
                           hipStream_t st);
 hipError_t launch_run_begin(uint64_t* scal, unsigned long long* saif, uint64_t n_saif,
                             unsigned long long* wtot, uint64_t n_nets, unsigned long long* evjob,
@@ -1292,29 +1290,11 @@ void Job::write_scal() {
   HC(hipStreamSynchronize(stream_));
 }
 
-// Launches of level l of chunk c: plan the tiles (k_plan), describe them
-// (k_tile_desc), walk every tile independently into the level scratch
-// (k_level), join the tiles of each gate, finish its SAIF share and place it in
-// the pool behind its tail (k_join), and copy the outputs there (k_compact).
-// No host round trip: the kernels read the level's counts from device memory.
-void Job::launch_level_of(size_t l, const Chunk& c, const Group& G, bool device_driven, double proj_cap) {
-  const uint32_t g0 = level_start_[l], ng = level_start_[l + 1] - g0;
-  if (ng == 0) return;
-  const GateRec* gates = prog_->d_grec + g0;
-  const ChunkWin* cw = d_cwin_ + c.slot * net_base_.size();
-  TailArgs T;
-  T.tail_len = d_tail_len_;
-  T.tail_off = d_tail_off_;
-  T.tails = d_tails_;
-  T.shift = c.shift;
-  T.first = c.first;
-  // expected tiles, for launch widths: one a gate and one per 1,024 words of
-  // the estimated input words of the level's share of the chunk
-  const double share = c.Fn == kChunkEnd ? 1.0 : std::min(1.0, (double)(c.Fn - c.F) / (double)G.horizon);
-  const uint64_t guess = ng + (uint64_t)(G.est_words * share * ng / std::max(1u, G.g1 - G.g0) / 512.0);
+PlanArgs Job::plan_args(size_t l, const Group& G, uint32_t slot, bool device_driven, double proj_cap) {
+  const uint32_t g0 = level_start_[l];
   PlanArgs p;
-  p.gates = gates;
-  p.ng = ng;
+  p.gates = prog_->d_grec + g0;
+  p.ng = level_start_[l + 1] - g0;
   p.wlen = d_wlen_;
   p.tail_len = d_tail_len_;
   p.seg_target = seg_target ? seg_target : kDefaultSeg;
@@ -1333,6 +1313,7 @@ void Job::launch_level_of(size_t l, const Chunk& c, const Group& G, bool device_
   p.apart = d_scratch_;
   p.allow_apart = !(pool_auto_ && !static_) || scratch_apart_ || device_driven ? 1u : 0u;
   p.level = (uint32_t)l + 1;
+  p.slot = slot;
   // automatic chunks: a chunk projected (by its gates so far) not to fit the
   // largest pool is cut short before it runs further
   const uint64_t group_gates = G.g1 - G.g0, done_g = g0 - G.g0;
@@ -1340,46 +1321,95 @@ void Job::launch_level_of(size_t l, const Chunk& c, const Group& G, bool device_
   p.all_gates = (double)group_gates;
   p.done_gates = (double)done_g;
   p.stop = should_stop && !device_driven ? stop_flag() : nullptr;
-  HC(launch_plan(p, stream_));
-  HC(launch_tile_desc(gates, ng, d_plan_, d_tileloc_, d_scrloc_, d_planpart_, d_woff_, d_wlen_, d_pool_,
-                      d_tiles_, d_scal_, guess, stream_));
-  LevelArgs a;
-  a.tiles = d_tiles_;
-  a.pool = d_pool_;
-  a.dtab = prog_->d_dtab;
-  a.ttab = prog_->d_ttab;
-  a.scal = d_scal_;
-  a.tout = d_tout_;
-  a.ovf = d_ovf_;
-  a.ovf_cap = ovf_words_;
-  a.ticket = d_ticket_;
-  a.cwin = cw;
-  a.lds_words = lds_words_;
-  a.prefetch = prefetch;
-  a.lo_rel = c.lo_rel;
-  a.hi_rel = c.hi_rel;
-  a.first = c.first;
-  HC(launch_level(a, (unsigned)std::min<uint64_t>(guess, (uint64_t)std::max(1, level_blocks_)), stream_));
-  JoinArgs j;
-  j.gates = gates;
-  j.ng = ng;
-  j.ntile = d_ntile_;
-  j.tile_loc = d_tileloc_;
-  j.plan_part = d_planpart_;
-  j.tout = d_tout_;
-  j.tile_off = d_toff_;
-  j.out_loc = d_outloc_;
-  j.part = d_outpart_;
-  j.wlen = d_wlen_;
-  j.saif = d_saif_chunk_;
-  j.cwin = cw;
-  j.scal = d_scal_;
-  j.ev_job = d_evjob_chunk_;
-  j.level = (uint32_t)l + 1;
-  j.ovf_trip = !device_driven && !static_ && (ovf_words_opt == 0 || pool_grow) ? 1u : 0u;
-  HC(launch_join(j, T, stream_));
-  HC(launch_compact(d_tiles_, d_tout_, d_toff_, d_outloc_, d_outpart_, d_pool_, d_woff_, d_scal_,
-                    d_saif_chunk_, cw, saif_tc, T, guess, stream_));
+  return p;
+}
+
+// Launches of levels [next, G.L1) of chunk c.  Per level: describe the planned
+// tiles (k_tile_desc), walk every tile independently into the level scratch
+// (k_level), join the tiles of each gate, finish its SAIF share and place it in
+// the pool behind its tail (k_join), and copy the outputs there while the next
+// level is planned (k_compact).  No host round trip: the kernels read the
+// levels' counts from device memory.
+void Job::launch_levels(size_t next, const Chunk& c, const Group& G, bool device_driven, double proj_cap) {
+  std::vector<size_t> levels;
+  for (size_t l = next; l < G.L1; ++l)
+    if (level_start_[l + 1] > level_start_[l]) levels.push_back(l);
+  if (levels.empty()) return;
+  const ChunkWin* cw = d_cwin_ + c.slot * net_base_.size();
+  TailArgs T;
+  T.tail_len = d_tail_len_;
+  T.tail_off = d_tail_off_;
+  T.tails = d_tails_;
+  T.shift = c.shift;
+  T.first = c.first;
+  const double share = c.Fn == kChunkEnd ? 1.0 : std::min(1.0, (double)(c.Fn - c.F) / (double)G.horizon);
+  HC(launch_plan(plan_args(levels[0], G, 0, device_driven, proj_cap), stream_));
+  for (size_t i = 0; i < levels.size(); ++i) {
+    if (!device_driven) stop_point();
+    const size_t l = levels[i];
+    const uint32_t slot = (uint32_t)(i & 1);
+    const uint32_t g0 = level_start_[l], ng = level_start_[l + 1] - g0;
+    const GateRec* gates = prog_->d_grec + g0;
+    // expected tiles, for launch widths: one a gate and one per 512 words of
+    // the waveform estimate of the level's share of the chunk
+    const uint64_t guess = ng + (uint64_t)(G.est_words * share * ng / std::max(1u, G.g1 - G.g0) / 512.0);
+    HC(launch_tile_desc(gates, ng, d_plan_, d_tileloc_, d_scrloc_, d_planpart_, d_woff_, d_wlen_, d_pool_,
+                        d_tiles_, d_scal_, slot, guess, stream_));
+    LevelArgs a;
+    a.tiles = d_tiles_;
+    a.pool = d_pool_;
+    a.dtab = prog_->d_dtab;
+    a.ttab = prog_->d_ttab;
+    a.scal = d_scal_;
+    a.tout = d_tout_;
+    a.ovf = d_ovf_;
+    a.ovf_cap = ovf_words_;
+    a.ticket = d_ticket_;
+    a.cwin = cw;
+    a.lds_words = lds_words_;
+    a.prefetch = prefetch;
+    a.slot = slot;
+    a.lo_rel = c.lo_rel;
+    a.hi_rel = c.hi_rel;
+    a.first = c.first;
+    HC(launch_level(a, (unsigned)std::min<uint64_t>(guess, (uint64_t)std::max(1, level_blocks_)), stream_));
+    JoinArgs j;
+    j.gates = gates;
+    j.ng = ng;
+    j.ntile = d_ntile_;
+    j.tile_loc = d_tileloc_;
+    j.plan_part = d_planpart_;
+    j.tout = d_tout_;
+    j.tile_off = d_toff_;
+    j.out_loc = d_outloc_;
+    j.part = d_outpart_;
+    j.wlen = d_wlen_;
+    j.saif = d_saif_chunk_;
+    j.cwin = cw;
+    j.scal = d_scal_;
+    j.ev_job = d_evjob_chunk_;
+    j.level = (uint32_t)l + 1;
+    j.ovf_trip = !device_driven && !static_ && (ovf_words_opt == 0 || pool_grow) ? 1u : 0u;
+    HC(launch_join(j, T, stream_));
+    CompactArgs k;
+    k.tiles = d_tiles_;
+    k.tout = d_tout_;
+    k.tile_off = d_toff_;
+    k.out_loc = d_outloc_;
+    k.part = d_outpart_;
+    k.pool = d_pool_;
+    k.woff = d_woff_;
+    k.scal = d_scal_;
+    k.saif = d_saif_chunk_;
+    k.cwin = cw;
+    k.count_tc = saif_tc;
+    k.level = (uint32_t)l + 1;
+    k.slot = slot;
+    PlanArgs np;
+    const bool more = i + 1 < levels.size();
+    if (more) np = plan_args(levels[i + 1], G, slot ^ 1u, device_driven, proj_cap);
+    HC(launch_compact(k, T, more ? &np : nullptr, guess, stream_));
+  }
 }
 
 // One chunk: its stimulus cut into the pool, then every level, with no host
@@ -1417,10 +1447,7 @@ int Job::run_chunk(const Chunk& c, const Group& G, bool device_driven, double* g
                           d_sbase_, d_spart_, d_pool_, d_woff_, d_wlen_, d_scal_, stream_));
       stim = false;
     }
-    for (size_t l = next; l < G.L1; ++l) {
-      if (!device_driven) stop_point();
-      launch_level_of(l, c, G, device_driven, proj_cap);
-    }
+    launch_levels(next, c, G, device_driven, proj_cap);
     after();
     if (device_driven) return CHUNK_OK;
     read_scal();

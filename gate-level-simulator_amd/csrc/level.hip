@@ -871,8 +871,8 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   unsigned long long wave_tiles = 0, wave_hbm = 0;
   if (A.scal[S_TRIP]) return;
   if (blockIdx.x == 0 && lane == 0) A.scal[S_CLOCK] = (uint64_t)wall_clock64();
-  const uint64_t ntiles = A.scal[S_TOT_A];  // uniform: one scalar load
-  uint32_t* const scratch = (uint32_t*)A.scal[S_SCRATCH];
+  const uint64_t ntiles = A.scal[S_NTILES + A.slot];  // uniform: one scalar load
+  uint32_t* const scratch = (uint32_t*)A.scal[S_SCRATCH + A.slot];
   unsigned int* const err = (unsigned int*)(A.scal + S_ERR);
   // Tiles are handed out in two parts.  The first half is split into
   // one run of consecutive tiles per workgroup (consecutive tiles of one gate
@@ -1048,28 +1048,34 @@ __device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* sh, uint64_
 __device__ __forceinline__ void put_part(uint64_t* p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool last_block(uint64_t* done) {
+__device__ __forceinline__ bool last_block(uint64_t* done, uint32_t nb) {
+  if (nb == 1) return true;
   __shared__ uint32_t s_last;
   if (threadIdx.x == 0) {  // the thread that stored the block's totals
     const unsigned long long n = __hip_atomic_fetch_add((unsigned long long*)done, 1ull,
                                                         __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = n + 1 == gridDim.x ? 1u : 0u;
+    s_last = n + 1 == nb ? 1u : 0u;
     if (s_last) *done = 0;  // for the next scan
   }
   __syncthreads();
   return s_last != 0;
 }
 // part[stride * b] for every block b: totals to exclusive prefixes; returns
-// the sum.
+// the sum (`own`: this block's total, all there is when it is the only one).
 template <int T>
-__device__ __forceinline__ uint64_t scan_parts(uint64_t* part, uint32_t stride, uint64_t* sh) {
+__device__ __forceinline__ uint64_t scan_parts(uint64_t* part, uint32_t stride, uint32_t nb,
+                                               uint64_t own, uint64_t* sh) {
+  if (nb == 1) {
+    if (threadIdx.x == 0) *part = 0;
+    return own;
+  }
   uint64_t carry = 0;
-  for (uint32_t b0 = 0; b0 < gridDim.x; b0 += T * 4) {
+  for (uint32_t b0 = 0; b0 < nb; b0 += T * 4) {
     uint64_t v[4], sum = 0;
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
       const uint32_t b = b0 + threadIdx.x * 4 + i;
-      v[i] = b < gridDim.x ? __hip_atomic_load(part + (uint64_t)stride * b, __ATOMIC_RELAXED,
+      v[i] = b < nb ? __hip_atomic_load(part + (uint64_t)stride * b, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT)
                            : 0;
       sum += v[i];
@@ -1078,7 +1084,7 @@ __device__ __forceinline__ uint64_t scan_parts(uint64_t* part, uint32_t stride, 
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
       const uint32_t b = b0 + threadIdx.x * 4 + i;
-      if (b < gridDim.x) part[(uint64_t)stride * b] = x;
+      if (b < nb) part[(uint64_t)stride * b] = x;
       x += v[i];
     }
     carry += tot;
@@ -1086,38 +1092,37 @@ __device__ __forceinline__ uint64_t scan_parts(uint64_t* part, uint32_t stride, 
   return carry;
 }
 
-// Plan of a level, four consecutive gates per thread: per gate its leader
-// (the input with the most words), words of the leader per tile, tiles and
-// output bound, and their prefixes over the level; then, in the block that
-// finishes last, whether the level has room, where its scratch lies, and the
-// walk's counters.  A tile of a gate of fan-in 1..4 holds 64 times the leader's
-// words of a lane share of about seg_target input words, spread evenly over the
-// gate's tiles; a wide gate's tiles hold wide_words input words (its tables
-// leave less LDS).
+// Plan of a level, one gate per thread: per gate its leader (the input with
+// the most words), words of the leader per tile, tiles and output bound, and
+// their prefixes over the level; then, in the block that finishes last, whether
+// the level has room, where its scratch lies, and the walk's counters.  A tile
+// of a gate of fan-in 1..4 holds 64 times the leader's words of a lane share of
+// about seg_target input words, spread evenly over the gate's tiles; a wide
+// gate's tiles hold wide_words input words (its tables leave less LDS).
 //
-// One launch: with the plan, two three-kernel scans, the capacity check and
-// the clears as launches of their own, a level of the 300-cell netlist spent
-// 9 of its 18 launches (25 of 48 us) before its first descriptor.
-__global__ __launch_bounds__(256) void k_plan(PlanArgs A) {
-  __shared__ uint64_t sh[4];
+// One launch at most: with the plan, two three-kernel scans, the capacity check
+// and the clears as launches of their own, a level of the 300-cell netlist spent
+// 9 of its 18 launches (25 of 48 us) before its first descriptor.  Every level
+// but a chunk's first is planned by blocks of the launch that copies the outputs
+// of the level before it (the lengths it reads are final by then).
+__device__ __forceinline__ void plan_block(const PlanArgs& A, uint32_t bi, uint32_t nb, uint64_t* sh) {
   if (A.scal[S_TRIP]) return;
-  const uint32_t g0 = blockIdx.x * kPlanGates + threadIdx.x * 4;
-  uint32_t nt4[4];
-  uint64_t bd4[4], nt_sum = 0, bd_sum = 0;
-#pragma unroll
-  for (uint32_t i = 0; i < 4; ++i) {
-    const uint32_t g = g0 + i;
-    nt4[i] = 0;
-    bd4[i] = 0;
-    if (g >= A.ng) continue;
+  const uint32_t g = bi * kPlanGates + threadIdx.x;
+  uint32_t nt = 0;
+  uint64_t bound = 0;
+  if (g < A.ng) {
     const GateRec& G = A.gates[g];
+    const uint32_t tail = A.tail_len[G.out_net];
+    uint32_t n6[6];
+#pragma unroll
+    for (uint32_t j = 0; j < kWideK; ++j) n6[j] = j < G.k ? A.wlen[G.in_net[j]] : 0u;
     uint64_t N = 0;
     uint32_t nl = 0, lead = 0;
-    for (int j = 0; j < G.k; ++j) {
-      const uint32_t n = A.wlen[G.in_net[j]];
-      N += n;
-      if (j == 0 || n > nl) {
-        nl = n;
+#pragma unroll
+    for (uint32_t j = 0; j < kWideK; ++j) {
+      N += n6[j];
+      if (n6[j] > nl) {
+        nl = n6[j];
         lead = j;
       }
     }
@@ -1128,44 +1133,47 @@ __global__ __launch_bounds__(256) void k_plan(PlanArgs A) {
       const uint32_t nt0 = (uint32_t)max<uint64_t>(1, (N + A.wide_words - 1) / A.wide_words);
       P.lt = max(1u, (nl + nt0 - 1) / nt0);
     } else {
-      uint64_t s = N > 0 ? (uint64_t)A.seg_target * nl / N : 1;
+      // (64-bit divisions only where 32 bits do not hold the product)
+      uint64_t s = 1;
+      if (N > 0)
+        s = N < (1ull << 31) && (uint64_t)A.seg_target * nl < (1ull << 32)
+                ? (uint64_t)(A.seg_target * nl / (uint32_t)N)
+                : (uint64_t)A.seg_target * nl / N;
       if (s < 1) s = 1;
       if (nl > 0) {
-        const uint64_t nt0 = ((nl + s - 1) / s + kLanes - 1) / kLanes;
-        s = (nl + nt0 * kLanes - 1) / (nt0 * kLanes);
+        if (s < (1u << 24) && nl < (1u << 31)) {
+          const uint32_t t = (uint32_t)s, nt0 = ((nl + t - 1) / t + kLanes - 1) / kLanes;
+          s = (nl + nt0 * kLanes - 1) / (nt0 * kLanes);
+        } else {
+          const uint64_t nt0 = ((nl + s - 1) / s + kLanes - 1) / kLanes;
+          s = (nl + nt0 * kLanes - 1) / (nt0 * kLanes);
+        }
       }
       P.lt = (uint32_t)min<uint64_t>(s * kLanes, 0xFFFFFFFFu);
     }
     P.lead = lead;
     A.plan[g] = P;
-    nt4[i] = max(1u, (uint32_t)(((uint64_t)nl + P.lt - 1) / P.lt));
-    A.ntile[g] = nt4[i];
+    nt = max(1u, nl / P.lt + (nl % P.lt ? 1u : 0u));
+    A.ntile[g] = nt;
     // scratch words of the gate's tile outputs: every tile keeps at most its
     // own input events + 1 entries; the gate's tail is added so that the
     // level's waveforms (tails + joined entries) never exceed the scratch
-    bd4[i] = N + nt4[i] + 1 + A.tail_len[G.out_net];
-    nt_sum += nt4[i];
-    bd_sum += bd4[i];
+    bound = N + nt + 1 + tail;
   }
   uint64_t nt_tot, bd_tot;
-  uint64_t t = block_scan<256>(nt_sum, sh, nt_tot);
-  uint64_t b = block_scan<256>(bd_sum, sh, bd_tot);
-#pragma unroll
-  for (uint32_t i = 0; i < 4; ++i) {
-    if (g0 + i < A.ng) {
-      A.tile_loc[g0 + i] = (uint32_t)t;
-      A.scr_loc[g0 + i] = b;
-    }
-    t += nt4[i];
-    b += bd4[i];
+  const uint64_t t = block_scan<256>(nt, sh, nt_tot);
+  const uint64_t b = block_scan<256>(bound, sh, bd_tot);
+  if (g < A.ng) {
+    A.tile_loc[g] = (uint32_t)t;
+    A.scr_loc[g] = b;
   }
   if (threadIdx.x == 0) {
-    put_part(A.part + 2 * blockIdx.x, nt_tot);
-    put_part(A.part + 2 * blockIdx.x + 1, bd_tot);
+    put_part(A.part + 2 * bi, nt_tot);
+    put_part(A.part + 2 * bi + 1, bd_tot);
   }
-  if (!last_block(A.scal + S_DONE)) return;
-  const uint64_t tiles = scan_parts<256>(A.part, 2, sh);
-  const uint64_t scr = scan_parts<256>(A.part + 1, 2, sh);
+  if (!last_block(A.scal + S_DONE, nb)) return;
+  const uint64_t tiles = scan_parts<256>(A.part, 2, nb, nt_tot, sh);
+  const uint64_t scr = scan_parts<256>(A.part + 1, 2, nb, bd_tot, sh);
   if (threadIdx.x < kTickets) A.ticket[threadIdx.x * kTicketStride] = 0;
   if (threadIdx.x != 0) return;
   const uint64_t used = A.scal[S_BUMP], stim = A.scal[S_STIM];
@@ -1175,30 +1183,41 @@ __global__ __launch_bounds__(256) void k_plan(PlanArgs A) {
     const double proj = (double)(used - stim) * A.all_gates / A.done_gates;
     if (((double)stim + proj) * 1.35 > A.proj_cap) why = TRIP_PROJECTED;
   }
-  // The level scratch lives in the unused top of the event pool when twice its
+  // The level scratch lies in the unused top of the event pool when twice its
   // size is free above the bump (the level's outputs, at most the scratch size,
-  // then land below it); otherwise in an allocation of its own.
+  // then land below it); otherwise in an allocation of its own.  (The scratch of
+  // the level before, still being copied, is not written before this level's
+  // walk.)
+  uint32_t* scratch = nullptr;
   if (!why) {
     if (tiles > A.tiles_cap) {
       why = TRIP_ROOM;
     } else if (used <= A.pool_words && 2 * scr <= A.pool_words - used) {
       A.scal[S_LIMIT] = A.pool_words - scr;
-      A.scal[S_SCRATCH] = (uint64_t)(A.pool + (A.pool_words - scr));
+      scratch = A.pool + (A.pool_words - scr);
     } else if (A.allow_apart && used + scr <= A.pool_words && scr <= A.apart_cap) {
       A.scal[S_LIMIT] = A.pool_words;
-      A.scal[S_SCRATCH] = (uint64_t)A.apart;
+      scratch = A.apart;
     } else {
       why = TRIP_ROOM;
     }
   }
   A.scal[S_TOT_A] = tiles;
   A.scal[S_TOT_B] = scr;
+  A.scal[S_NTILES + A.slot] = tiles;
+  A.scal[S_SCRATCH + A.slot] = (uint64_t)scratch;
   A.scal[S_EVL] = 0;
   A.scal[S_OVF_USED] = 0;
   if (why) {
-    A.scal[S_TRIP] = A.level;
     A.scal[S_WHY] = why;
+    // (the copy of the level before goes on: it is below S_TRIP)
+    __hip_atomic_store(A.scal + S_TRIP, (uint64_t)A.level, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+__global__ __launch_bounds__(256) void k_plan(PlanArgs A) {
+  __shared__ uint64_t sh[4];
+  plan_block(A, blockIdx.x, gridDim.x, sh);
 }
 
 // Per tile: its descriptor; thread j of the tile's four takes inputs j and
@@ -1208,12 +1227,12 @@ __global__ __launch_bounds__(256) void k_tile_desc(
     const uint32_t* __restrict__ tile_loc, const uint64_t* __restrict__ scr_loc,
     const uint64_t* __restrict__ part, const uint64_t* __restrict__ woff,
     const uint32_t* __restrict__ wlen, const uint32_t* __restrict__ pool,
-    TileDesc* __restrict__ tiles, const uint64_t* __restrict__ scal) {
+    TileDesc* __restrict__ tiles, const uint64_t* __restrict__ scal, uint32_t slot) {
   // a tile's first own word of each input is the previous tile's end: the
   // block's tiles pass them on through LDS (each boundary searched once)
   __shared__ uint32_t s_first[2][256];
   if (scal[S_TRIP]) return;
-  const uint64_t nt = scal[S_TOT_A];
+  const uint64_t nt = scal[S_NTILES + slot];
   const uint32_t nb = (ng + kPlanGates - 1) / kPlanGates;
   for (uint64_t t0 = (uint64_t)blockIdx.x * 64; t0 < nt; t0 += (uint64_t)gridDim.x * 64) {
     const uint64_t t = t0 + (threadIdx.x >> 2);
@@ -1475,6 +1494,7 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
   }
   __syncthreads();
   const unsigned int err = *(const unsigned int*)(A.scal + S_ERR);
+  uint64_t own = 0;        // the block's words, in the first wavefront
   if (threadIdx.x < 64) {  // the first wavefront: prefixes over the block's gates
     const uint32_t i = threadIdx.x;
     const uint64_t mine = i < kJoinGates ? s_cnt[i] : 0u;
@@ -1487,6 +1507,7 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
     const uint32_t gi = blockIdx.x * kJoinGates + i;
     if (i < kJoinGates && gi < A.ng) A.out_loc[gi] = x - mine;
     const uint64_t tot = __shfl(x, kJoinGates - 1, 64);
+    own = tot;
     if (i == 0) put_part(A.part + blockIdx.x, tot);
     // a level whose tiles ran out of overflow stacks runs again: counted then
     if (A.ev_job && !(err & ERR_OVERFLOW)) {
@@ -1502,8 +1523,8 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
       }
     }
   }
-  if (!last_block(A.scal + S_DONE)) return;
-  const uint64_t total = scan_parts<256>(A.part, 1, sh);
+  if (!last_block(A.scal + S_DONE, gridDim.x)) return;
+  const uint64_t total = scan_parts<256>(A.part, 1, gridDim.x, own, sh);
   if (threadIdx.x != 0) return;
   if (A.ovf_trip && (err & ERR_OVERFLOW)) {
     A.scal[S_TRIP] = A.level;
@@ -1525,23 +1546,32 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
 // Copy every tile's joined output from the scratch into the gate's dense
 // waveform in the pool (one wavefront per tile, coalesced); the gate's first
 // tile also copies the gate's tail (state and look-back entries, moved to
-// this chunk's time base) to the front.
-__global__ __launch_bounds__(256) void k_compact(
-    const TileDesc* __restrict__ tiles, const TileOut* __restrict__ tout,
-    const uint32_t* __restrict__ tile_off, const uint64_t* __restrict__ out_loc,
-    const uint64_t* __restrict__ part, uint32_t* __restrict__ pool, uint64_t* __restrict__ woff,
-    const uint64_t* __restrict__ scal, unsigned long long* __restrict__ saif,
-    const ChunkWin* __restrict__ cwin, uint32_t count_tc, TailArgs T) {
-  if (scal[S_TRIP]) return;
+// this chunk's time base) to the front.  The first nplan blocks plan the next
+// level.
+__global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, PlanArgs next,
+                                                 uint32_t nplan) {
+  __shared__ uint64_t sh[4];
+  if (blockIdx.x < nplan) {
+    plan_block(next, blockIdx.x, nplan, sh);
+    return;
+  }
+  // a trip of this level or one before it; the next one's plan may trip now
+  const uint64_t trip = __hip_atomic_load(A.scal + S_TRIP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (trip && trip <= A.level) return;
+  const TileDesc* __restrict__ tiles = A.tiles;
+  const TileOut* __restrict__ tout = A.tout;
+  const uint32_t* __restrict__ tile_off = A.tile_off;
+  uint32_t* __restrict__ pool = A.pool;
   const int lane = threadIdx.x & 63;
-  const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / 64);
-  const uint64_t nt = scal[S_TOT_A], base = scal[S_OUTBASE];
-  const uint32_t* scratch = (const uint32_t*)scal[S_SCRATCH];
-  for (uint64_t t = (uint64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; t < nt; t += waves) {
+  const uint32_t bi = blockIdx.x - nplan;
+  const uint64_t waves = (uint64_t)(gridDim.x - nplan) * (blockDim.x / 64);
+  const uint64_t nt = A.scal[S_NTILES + A.slot], base = A.scal[S_OUTBASE];
+  const uint32_t* __restrict__ scratch = (const uint32_t*)A.scal[S_SCRATCH + A.slot];
+  for (uint64_t t = (uint64_t)bi * (blockDim.x / 64) + threadIdx.x / 64; t < nt; t += waves) {
     const TileDesc& D = tiles[t];
-    const uint64_t gate = base + part[D.g / kJoinGates] + out_loc[D.g];
+    const uint64_t gate = base + A.part[D.g / kJoinGates] + A.out_loc[D.g];
     if (D.ti == 0) {
-      if (lane == 0) woff[D.out_net] = gate;
+      if (lane == 0) A.woff[D.out_net] = gate;
       const uint32_t tl = T.tail_len[D.out_net];
       const uint32_t* ts = T.tails + T.tail_off[D.out_net];
       uint32_t* td = pool + gate;
@@ -1567,11 +1597,11 @@ __global__ __launch_bounds__(256) void k_compact(
       dst[q + 192] = a3;
     }
     for (; q < n; q += 64) dst[q] = src[q];
-    if (count_tc) {
+    if (A.count_tc) {
       // SAIF TC inside the tile: 0<->1 changes between its consecutive
       // entries (the first entry against the previous tile is k_join's)
       const uint32_t* e = src - skip;
-      const ChunkWin W = cwin[D.job];
+      const ChunkWin W = A.cwin[D.job];
       uint32_t c = 0;
       for (uint32_t q = lane + 1; q < S.cnt; q += 64) {
         const uint32_t a = e[q - 1], b = e[q];
@@ -1579,7 +1609,8 @@ __global__ __launch_bounds__(256) void k_compact(
         c += (is_toggle(a & 3u, b & 3u) && tt > W.tc_lo && tt <= W.tc_hi) ? 1u : 0u;
       }
       c = wave_sum(c);
-      if (lane == 0 && c) atomicAdd(saif + (uint64_t)kSaifWords * D.out_net + 3, (unsigned long long)c);
+      if (lane == 0 && c)
+        atomicAdd(A.saif + (uint64_t)kSaifWords * D.out_net + 3, (unsigned long long)c);
     }
   }
 }
@@ -1625,12 +1656,12 @@ __global__ __launch_bounds__(256) void k_stim_plan(const uint64_t* __restrict__ 
   const uint64_t x = block_scan<256>(n, sh, tot);
   if (s < ns) loc[s] = x;
   if (threadIdx.x == 0) put_part(part + blockIdx.x, tot);
-  if (!last_block(scal + S_DONE)) return;
-  const uint64_t total = scan_parts<256>(part, 1, sh);
+  if (!last_block(scal + S_DONE, gridDim.x)) return;
+  const uint64_t total = scan_parts<256>(part, 1, gridDim.x, tot, sh);
   if (threadIdx.x != 0) return;
   scal[S_BUMP] = scal[S_STIM] = total;
   if (total + 1024 > pool_words) {
-    scal[S_TRIP] = ~0ull;
+    scal[S_TRIP] = 1;  // before every level
     scal[S_WHY] = TRIP_STIM;
   }
 }
@@ -1677,12 +1708,9 @@ __global__ __launch_bounds__(256) void k_tail_len(const GateRec* __restrict__ ga
   __shared__ uint64_t sh[4];
   if (scal[S_TRIP]) return;
   const uint32_t kw = key << 2;
-  uint64_t n4[4], sum = 0;
-#pragma unroll
-  for (uint32_t i = 0; i < 4; ++i) {
-    const uint32_t g = blockIdx.x * kPlanGates + threadIdx.x * 4 + i;
-    n4[i] = 0;
-    if (g >= ng) continue;
+  const uint32_t g = blockIdx.x * kPlanGates + threadIdx.x;
+  uint64_t mine = 0;
+  if (g < ng) {
     const uint32_t net = gates[g].out_net;
     const uint32_t* w = pool + woff[net];
     const uint32_t n = wlen[net];
@@ -1702,21 +1730,16 @@ __global__ __launch_bounds__(256) void k_tail_len(const GateRec* __restrict__ ga
       if (w[mid] < kw) lo = mid;
       else hi = mid;
     }
-    n4[i] = n - lo;
-    len[g] = n - lo;
+    mine = n - lo;
+    len[g] = mine;
     src[g] = woff[net] + lo;
-    sum += n - lo;
   }
-  uint64_t tot, x = block_scan<256>(sum, sh, tot);
-#pragma unroll
-  for (uint32_t i = 0; i < 4; ++i) {
-    const uint32_t g = blockIdx.x * kPlanGates + threadIdx.x * 4 + i;
-    if (g < ng) loc[g] = x;
-    x += n4[i];
-  }
+  uint64_t tot;
+  const uint64_t x = block_scan<256>(mine, sh, tot);
+  if (g < ng) loc[g] = x;
   if (threadIdx.x == 0) put_part(part + blockIdx.x, tot);
-  if (!last_block(scal + S_DONE)) return;
-  const uint64_t total = scan_parts<256>(part, 1, sh);
+  if (!last_block(scal + S_DONE, gridDim.x)) return;
+  const uint64_t total = scan_parts<256>(part, 1, gridDim.x, tot, sh);
   if (threadIdx.x == 0) scal[S_TAILS] = total;
 }
 
@@ -1802,10 +1825,11 @@ hipError_t launch_plan(const PlanArgs& a, hipStream_t st) {
 hipError_t launch_tile_desc(const GateRec* gates, uint32_t ng, const GatePlan* plan,
                             const uint32_t* tile_loc, const uint64_t* scr_loc, const uint64_t* part,
                             const uint64_t* woff, const uint32_t* wlen, const uint32_t* pool,
-                            TileDesc* tiles, const uint64_t* scal, uint64_t guess, hipStream_t st) {
+                            TileDesc* tiles, const uint64_t* scal, uint32_t slot, uint64_t guess,
+                            hipStream_t st) {
   const unsigned nb = (unsigned)std::min<uint64_t>(guess / 64 + 1, 8192);
   k_tile_desc<<<nb, 256, 0, st>>>(gates, ng, plan, tile_loc, scr_loc, part, woff, wlen, pool, tiles,
-                                  scal);
+                                  scal, slot);
   return hipGetLastError();
 }
 
@@ -1822,14 +1846,12 @@ hipError_t launch_join(const JoinArgs& a, const TailArgs& T, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_compact(const TileDesc* tiles, const TileOut* tout, const uint32_t* tile_off,
-                          const uint64_t* out_loc, const uint64_t* part, uint32_t* pool,
-                          uint64_t* woff, const uint64_t* scal, unsigned long long* saif,
-                          const ChunkWin* cwin, uint32_t count_tc, const TailArgs& T, uint64_t guess,
+// `next`: the plan of the level after it (null: none)
+hipError_t launch_compact(const CompactArgs& a, const TailArgs& T, const PlanArgs* next, uint64_t guess,
                           hipStream_t st) {
   const unsigned nb = (unsigned)std::min<uint64_t>(guess / 4 + 1, 8192);  // 4 wavefronts each
-  k_compact<<<nb, 256, 0, st>>>(tiles, tout, tile_off, out_loc, part, pool, woff, scal, saif, cwin,
-                                count_tc, T);
+  const unsigned np = next ? nblk(next->ng, kPlanGates) : 0;
+  k_compact<<<nb + np, 256, 0, st>>>(a, T, next ? *next : PlanArgs{}, np);
   return hipGetLastError();
 }
 
