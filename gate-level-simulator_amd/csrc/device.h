@@ -222,6 +222,9 @@ constexpr uint32_t kTickets = 4, kTicketStride = 32;
 // the stimulus cut.
 constexpr uint32_t kPlanGates = 256, kJoinGates = 32, kStimSignals = 256;
 
+// Tiles per block of the descriptors.
+constexpr uint32_t kDescTiles = 63;
+
 // Plan of one level.
 struct PlanArgs {
   const GateRec* gates;

@@ -1044,7 +1044,10 @@ __device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* sh, uint64_
 // Scans over blocks in one launch: every block leaves its totals in `part`
 // (agent-scope stores: the blocks run on XCDs with L2s of their own) and
 // counts itself done; the last one turns the totals into prefixes.  No block
-// waits for another.
+// waits for another.  The totals have left for memory before the block counts
+// itself (the wait for its stores), and they are all that the last block reads
+// of the others: a release fence here would write the XCD's whole L2 back, once
+// per block.
 __device__ __forceinline__ void put_part(uint64_t* p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1052,8 +1055,9 @@ __device__ __forceinline__ bool last_block(uint64_t* done, uint32_t nb) {
   if (nb == 1) return true;
   __shared__ uint32_t s_last;
   if (threadIdx.x == 0) {  // the thread that stored the block's totals
+    wait_vm();
     const unsigned long long n = __hip_atomic_fetch_add((unsigned long long*)done, 1ull,
-                                                        __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s_last = n + 1 == nb ? 1u : 0u;
     if (s_last) *done = 0;  // for the next scan
   }
@@ -1220,73 +1224,170 @@ __global__ __launch_bounds__(256) void k_plan(PlanArgs A) {
   plan_block(A, blockIdx.x, gridDim.x, sh);
 }
 
+// Words below `key` among the (at most) 8 of a sorted range [p, n) from p on.
+__device__ __forceinline__ uint32_t below8(const uint32_t* a, uint32_t p, uint32_t n, uint32_t key) {
+  uint32_t v[8], c = 0;
+  if (p + 8 <= n) {
+    __builtin_memcpy(v, a + p, 32);  // two 16-byte loads
+  } else {
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) v[i] = p + i < n ? a[p + i] : 0xFFFFFFFFu;
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < 8; ++i) c += v[i] < key ? 1u : 0u;
+  return c;
+}
+
+// First index of a sorted word range [0, n) at or after `key` (n if none),
+// looked for near `g` (< n): two probes corrected by the density `dens` (words per unit
+// of word value), a window of 16 words, then doubling strides away from it and
+// a search by halves inside the last one.
+//
+// The searches of a level's tile boundaries are bound by the cache lines that
+// they fetch from HBM and, on small levels, by the chain of dependent loads.
+// Event counts follow time closely, so the window is usually the end: about 4
+// lines in 3 rounds, against 11 lines in 15 rounds by halves over 20,000 words
+// (and 24 lines in 5 rounds with seven probes a round: 93 us a level against
+// 72 by halves on the busy 200,000-cell netlist).
+__device__ __forceinline__ uint32_t lb_near(const uint32_t* a, uint32_t n, uint32_t key, uint32_t g,
+                                            float dens) {
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const uint32_t v = a[g];
+    const float d = v < key ? (float)(key - v) : -(float)(v - key);
+    const float x = (float)g + d * dens;
+    g = (uint32_t)max(0.0f, min(x, (float)(n - 1)));
+    g = min(g, n - 1);
+  }
+  uint32_t s = g > 8 ? g - 8 : 0u;
+  const uint32_t c0 = below8(a, s, n, key), c1 = s + 8 < n ? below8(a, s + 8, n, key) : 0u;
+  const uint32_t c = c0 + c1;
+  if (c > 0 && c < 16) return s + c;
+  uint32_t lo, hi;  // every word before lo is below key, a[hi] is not (or hi = n)
+  if (c == 0) {
+    if (s == 0) return 0;
+    uint32_t d = 16;
+    hi = s;
+    for (;;) {
+      lo = 0;
+      if (d > hi) break;
+      if (a[hi - d] < key) {
+        lo = hi - d + 1;
+        break;
+      }
+      hi -= d;
+      d <<= 1;
+    }
+  } else {
+    uint32_t d = 16;
+    lo = s + 16;
+    for (;;) {
+      hi = n;
+      if (n - lo < d) break;
+      hi = lo + d - 1;
+      if (a[hi] >= key) break;
+      lo = hi + 1;
+      d <<= 1;
+    }
+  }
+  return lo + lb_words(a + lo, hi - lo, key);
+}
+
 // Per tile: its descriptor; thread j of the tile's four takes inputs j and
-// j + 4.
+// j + 4.  Bound by the latency of a chain of dependent loads (gate, lengths,
+// the boundary's time, the searches).  A block describes 63 tiles: the threads of the 64th only find where
+// its inputs start, which is where the 63rd ends.
 __global__ __launch_bounds__(256) void k_tile_desc(
     const GateRec* __restrict__ gates, uint32_t ng, const GatePlan* __restrict__ plan,
     const uint32_t* __restrict__ tile_loc, const uint64_t* __restrict__ scr_loc,
     const uint64_t* __restrict__ part, const uint64_t* __restrict__ woff,
     const uint32_t* __restrict__ wlen, const uint32_t* __restrict__ pool,
     TileDesc* __restrict__ tiles, const uint64_t* __restrict__ scal, uint32_t slot) {
+  constexpr uint32_t kRow = kDescTiles;  // row that only marks the end
   // a tile's first own word of each input is the previous tile's end: the
   // block's tiles pass them on through LDS (each boundary searched once)
   __shared__ uint32_t s_first[2][256];
+  __shared__ int32_t s_start[2 * kPlanGates];  // first tiles of the gates near, from t0
+  __shared__ uint32_t s_n[4];
   if (scal[S_TRIP]) return;
   const uint64_t nt = scal[S_NTILES + slot];
   const uint32_t nb = (ng + kPlanGates - 1) / kPlanGates;
-  for (uint64_t t0 = (uint64_t)blockIdx.x * 64; t0 < nt; t0 += (uint64_t)gridDim.x * 64) {
-    const uint64_t t = t0 + (threadIdx.x >> 2);
+  const uint32_t row = threadIdx.x >> 2, wid = threadIdx.x >> 6;
+  for (uint64_t t0 = (uint64_t)blockIdx.x * kDescTiles; t0 < nt; t0 += (uint64_t)gridDim.x * kDescTiles) {
+    const uint64_t t = t0 + row;
     const int j0 = (int)(threadIdx.x & 3);
     const bool valid = t < nt;
-    // gate of tile t: binary search over the plan's blocks, then in the block,
-    // by the tile's first thread, passed to the other three
-    uint32_t g = 0, ti = 0;
-    if (valid && j0 == 0) {
-      uint32_t lo = 0, hi = nb;
-      while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (part[2 * mid] <= t) lo = mid;
-        else hi = mid;
-      }
-      const uint32_t r = (uint32_t)(t - part[2 * lo]);
-      lo *= kPlanGates;
-      hi = min(lo + kPlanGates, ng);
-      while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (tile_loc[mid] <= r) lo = mid;
-        else hi = mid;
-      }
-      g = lo;
-      ti = r - tile_loc[lo];
+    // the plan's block with tile t0: the whole block probes
+    uint32_t b0 = 0, len = nb;
+    while (len > 1) {
+      const uint32_t st = (len + 255) / 256, at = threadIdx.x * st;
+      const uint64_t le = __ballot(at < len && part[2 * (b0 + (at < len ? at : 0u))] <= t0);
+      if ((threadIdx.x & 63) == 0) s_n[wid] = (uint32_t)__popcll(le);
+      __syncthreads();
+      const uint32_t c = max(s_n[0] + s_n[1] + s_n[2] + s_n[3], 1u) - 1;
+      __syncthreads();
+      b0 += c * st;
+      len = min(st, len - c * st);
     }
-    const int q0 = (int)((threadIdx.x & 63u) & ~3u);
-    g = __shfl(g, q0);
-    ti = __shfl(ti, q0);
+    // the tiles here are of its gates and of the next block's (every gate has
+    // at least one): the last gate that starts at or before the tile
+    __syncthreads();  // the block's tiles before these are done with s_first, s_start
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) {
+      const uint32_t g = (b0 + q) * kPlanGates + threadIdx.x;
+      int32_t s = 0x7FFFFFFF;
+      if (g < ng) {
+        const int64_t rel = (int64_t)(part[2 * (b0 + q)] + tile_loc[g]) - (int64_t)t0;
+        s = (int32_t)max((int64_t)-0x7FFFFFFF, min(rel, (int64_t)0x7FFFFFFF));
+      }
+      s_start[q * kPlanGates + threadIdx.x] = s;
+    }
+    __syncthreads();
+    uint32_t gl = 0;
+#pragma unroll
+    for (uint32_t st = kPlanGates; st; st >>= 1)
+      if (s_start[gl + st] <= (int32_t)row) gl += st;
+    const uint32_t g = valid ? b0 * kPlanGates + gl : 0u;
+    const uint32_t ti = (uint32_t)((int32_t)row - s_start[gl]);
     GateRec G;
     GatePlan P;
-    uint32_t nl = 0, L[2] = {0, 0};
+    uint32_t nl = 0, L[2] = {0, 0}, n2[2] = {0, 0}, tau_nx = 0;
+    uint64_t off2[2] = {0, 0};
     const uint32_t* lw = nullptr;
+    bool more = false;  // another tile of the gate follows
     if (valid) {
       G = gates[g];
       P = plan[g];
       lw = pool + woff[G.in_net[P.lead]];
       nl = wlen[G.in_net[P.lead]];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint32_t j = j0 + 4 * q;
+        if (j >= G.k) continue;
+        off2[q] = woff[G.in_net[j]];
+        n2[q] = wlen[G.in_net[j]];
+      }
+      more = (ti + 1) * (uint64_t)P.lt < nl;
+      const uint32_t tau_lo = ti > 0 ? lw[ti * P.lt] >> 2 : 0u;
+      tau_nx = more ? lw[(ti + 1) * P.lt] >> 2 : 0u;
       if (ti > 0) {
-        const uint32_t tau_lo = lw[ti * P.lt] >> 2;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
           const uint32_t j = j0 + 4 * q;
-          if (j < G.k)
-            L[q] = j == P.lead ? ti * P.lt
-                               : lb_words(pool + woff[G.in_net[j]], wlen[G.in_net[j]], tau_lo << 2);
+          if (j >= G.k) continue;
+          const uint32_t x = ti * P.lt, n = n2[q];
+          const float at = (float)x * ((float)n / (float)nl);
+          L[q] = j == P.lead ? x
+                 : n == 0    ? 0u
+                             : lb_near(pool + off2[q], n, tau_lo << 2, min((uint32_t)at, n - 1),
+                                       at / (float)(tau_lo << 2));
         }
       }
     }
-    __syncthreads();  // the block's tiles before these are done with s_first
     s_first[0][threadIdx.x] = L[0];
     s_first[1][threadIdx.x] = L[1];
     __syncthreads();
-    if (!valid) continue;
+    if (!valid || row == kRow) continue;
     TileDesc& D = tiles[t];
     // own input words of the tile (up to the next tile's first words), summed
     // over the tile's threads: its output region in the level scratch holds
@@ -1302,24 +1403,21 @@ __global__ __launch_bounds__(256) void k_tile_desc(
         }
         continue;
       }
-      const uint64_t off = woff[G.in_net[j]];
-      const uint32_t n = wlen[G.in_net[j]];
+      const uint64_t off = off2[q];
+      const uint32_t n = n2[q];
       const uint32_t* iw = pool + off;
       uint32_t E = n, Ln = n;
-      if ((ti + 1) * (uint64_t)P.lt < nl) {
+      if (more) {
         // the next tile is this gate's: its first words end this one
-        const uint32_t tau_nx = lw[(ti + 1) * P.lt] >> 2;
-        if (threadIdx.x + 4 < blockDim.x && t + 1 < nt)
-          Ln = s_first[q][threadIdx.x + 4];
-        else
-          Ln = j == P.lead ? (ti + 1) * P.lt : lb_words(iw, n, tau_nx << 2);
-        // halo end: the first word at or after tau_nx + dmax lies at or after
-        // Ln, usually at it; step forward with doubling strides, then search
-        // only inside the last stride (every word before a is below the key)
+        Ln = s_first[q][threadIdx.x + 4];
+        // halo end: the first word at or after tau_nx + dmax lies at or a few
+        // words after Ln; eight at once, then doubling strides and a search
+        // inside the last stride (every word before a is below the key)
         const uint32_t key = (tau_nx + G.dmax) << 2;
-        E = Ln;
-        if (E < n && iw[E] < key) {
-          uint32_t a = E, d = 1, b = a + 1;
+        const uint32_t c = below8(iw, Ln, n, key);
+        E = Ln + c;
+        if (c == 8) {
+          uint32_t a = E - 1, d = 8, b = a + d;
           while (b < n && iw[b] < key) {
             a = b;
             d <<= 1;
@@ -1827,7 +1925,7 @@ hipError_t launch_tile_desc(const GateRec* gates, uint32_t ng, const GatePlan* p
                             const uint64_t* woff, const uint32_t* wlen, const uint32_t* pool,
                             TileDesc* tiles, const uint64_t* scal, uint32_t slot, uint64_t guess,
                             hipStream_t st) {
-  const unsigned nb = (unsigned)std::min<uint64_t>(guess / 64 + 1, 8192);
+  const unsigned nb = (unsigned)std::min<uint64_t>(guess / kDescTiles + 1, 8192);
   k_tile_desc<<<nb, 256, 0, st>>>(gates, ng, plan, tile_loc, scr_loc, part, woff, wlen, pool, tiles,
                                   scal, slot);
   return hipGetLastError();
