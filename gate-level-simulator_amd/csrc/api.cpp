@@ -716,7 +716,7 @@ int gls_run_autotune(gls_run* r, gls_tune_report* rep) {
   gls_tune_report R;
   std::memset(&R, 0, sizeof R);
   auto trial = [&](uint32_t seg, uint32_t blocks, uint32_t pf) {
-    j.seg_target = seg;
+    j.seg_target = seg == Job::kDefaultSeg ? 0 : seg;  // the default adapts to small levels
     j.level_blocks_opt = blocks;
     j.prefetch = pf;
     j.run();
@@ -737,7 +737,7 @@ int gls_run_autotune(gls_run* r, gls_tune_report* rep) {
     double ms = trial(seg, 0, 1);
     if (ms < best) best = ms, best_seg = seg;
   }
-  j.seg_target = best_seg;
+  j.seg_target = best_seg == Job::kDefaultSeg ? 0 : best_seg;
   j.level_blocks_opt = 0;
   j.run();
   const uint32_t occ = (uint32_t)j.stats().level_blocks;
@@ -752,7 +752,7 @@ int gls_run_autotune(gls_run* r, gls_tune_report* rep) {
     double ms = trial(best_seg, best_blocks, 0);
     if (ms < best) best = ms, best_pf = 0;
   }
-  j.seg_target = best_seg;
+  j.seg_target = best_seg == Job::kDefaultSeg ? 0 : best_seg;
   j.level_blocks_opt = best_blocks;
   j.prefetch = best_pf;
   j.run();

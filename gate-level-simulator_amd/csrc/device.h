@@ -192,7 +192,6 @@ enum ScalSlot {
   S_TOT_B = 2,
   S_TOT_OUT = 3,  // output words of the level (two-pass path)
   S_EVC = 4,      // gate events of the run
-  S_EVL = 5,      // gate events of the level
   S_OVF_USED = 6, // overflow stack words the level asked for
   S_ERR = 7,      // error flags
   S_TILES = 8, S_TILES_HBM = 9,  // tiles walked, of them on the HBM path
@@ -222,6 +221,9 @@ constexpr uint32_t kTickets = 4, kTicketStride = 32;
 // the stimulus cut.
 constexpr uint32_t kPlanGates = 256, kJoinGates = 32, kStimSignals = 256;
 
+// Smallest lane share of a level too small for the chip (PlanArgs::spread).
+constexpr uint32_t kSpreadSeg = 16;
+
 // Tiles per block of the descriptors.
 constexpr uint32_t kDescTiles = 63;
 
@@ -232,6 +234,7 @@ struct PlanArgs {
   const uint32_t* wlen;
   const uint32_t* tail_len;
   uint32_t seg_target, wide_words;
+  float spread;         // 0, or: lane share of a small level per input word of the gate
   GatePlan* plan;
   uint32_t* ntile;      // tiles per gate
   uint32_t* tile_loc;   // tiles before the gate in its block
@@ -286,6 +289,7 @@ struct JoinArgs {
   uint64_t* scal;
   unsigned long long* ev_job;  // batches: gate events per instance (null: none)
   uint32_t level;       // level + 1, for S_TRIP
+  uint32_t slot;
   uint32_t ovf_trip;    // 1: a level that ran out of overflow stacks is run again
 };
 

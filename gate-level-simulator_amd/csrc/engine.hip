@@ -1299,6 +1299,15 @@ PlanArgs Job::plan_args(size_t l, const Group& G, uint32_t slot, bool device_dri
   p.tail_len = d_tail_len_;
   p.seg_target = seg_target ? seg_target : kDefaultSeg;
   p.wide_words = wide_words_;
+  // Levels too small for the chip: a tile is one wavefront's, and a level of
+  // fewer tiles than workgroups waits for one tile's walk (24 us of 2,048 words
+  // on the 2,000-cell netlist).  Lane shares from 16 words, twice the share that
+  // would give every workgroup a tile (the tiles' count is rounded up gate by
+  // gate; more than one a workgroup takes two rounds): 2,000 cells 1.09 -> 1.05
+  // ms a run, 6,000 cells of fan-in 5 and 6 1.54 -> 1.42, 5,000 and more no
+  // change; 8 words, or one tile a workgroup, lose up to 20%.  Not in a batch,
+  // whose instances count events by tile, nor with a size of the caller's.
+  p.spread = seg_target || net_base_.size() > 1 ? 0.0f : (float)p.ng / (32.0f * (float)std::max(1, level_blocks_));
   p.plan = d_plan_;
   p.ntile = d_ntile_;
   p.tile_loc = d_tileloc_;
@@ -1389,6 +1398,7 @@ void Job::launch_levels(size_t next, const Chunk& c, const Group& G, bool device
     j.scal = d_scal_;
     j.ev_job = d_evjob_chunk_;
     j.level = (uint32_t)l + 1;
+    j.slot = slot;
     j.ovf_trip = !device_driven && !static_ && (ovf_words_opt == 0 || pool_grow) ? 1u : 0u;
     HC(launch_join(j, T, stream_));
     CompactArgs k;

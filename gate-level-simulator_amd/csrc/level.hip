@@ -774,8 +774,7 @@ __device__ __forceinline__ void keep_entries(const LevelArgs& A, Lane<SP>& ln, b
 template <typename SP, typename F>
 __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const Lane<SP>& ln,
                                           uint32_t* dst, uint32_t out_cap, unsigned long long w_start,
-                                          unsigned long long w_end, unsigned long long& wave_ev,
-                                          F&& before_stores) {
+                                          unsigned long long w_end, F&& before_stores) {
   const int lane = threadIdx.x;
   const uint32_t n = (uint32_t)(ln.hi - ln.lo);
   const uint32_t e_first = n ? ln.lo[0] : 0u, e_last = n ? ln.hi[-1] : 0u;
@@ -851,7 +850,6 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
     o.tx = max(min(lt >> 2, e32), s32) - max(min(ft >> 2, e32), s32) - t0 - t1;
     o.ev = ev;
     A.tout[tk] = o;
-    wave_ev += ev;
   }
 }
 
@@ -867,8 +865,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   // dynamic LDS, A.lds_words: tables, inputs, ..., stacks (walk_lds_need)
   extern __shared__ uint32_t s_dyn[];
   const int lane = threadIdx.x;
-  unsigned long long wave_ev = 0;  // gate events of this wavefront (lane 0)
-  unsigned long long wave_tiles = 0, wave_hbm = 0;
+  unsigned long long wave_hbm = 0;  // of this wavefront's tiles
   if (A.scal[S_TRIP]) return;
   if (blockIdx.x == 0 && lane == 0) A.scal[S_CLOCK] = (uint64_t)wall_clock64();
   const uint64_t ntiles = A.scal[S_NTILES + A.slot];  // uniform: one scalar load
@@ -951,7 +948,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       const bool halo = D.xend != 0 && lane == kLanes - 1;
       keep_entries(A, ln, halo);
       if (halo) ln.nown = 0;
-      emit_tile(A, tk, ln, scratch + D.scr, D.out_cap, w_start, w_end, wave_ev, [&] {
+      emit_tile(A, tk, ln, scratch + D.scr, D.out_cap, w_start, w_end, [&] {
         if (staged) {
           wait_vm();
           put_sentinels(Dn);
@@ -1003,7 +1000,6 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       put_sentinels(Dn);
     }
     lds_fence();
-    ++wave_tiles;
     wave_hbm += fits ? 0u : 1u;
     if (!more_tiles) break;
     tk = tn;
@@ -1012,8 +1008,6 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   }
   if (lane == 0) {
     unsigned long long* n = (unsigned long long*)A.scal;
-    if (wave_ev) atomicAdd(n + S_EVL, wave_ev);
-    atomicAdd(n + S_TILES, wave_tiles);
     if (wave_hbm) atomicAdd(n + S_TILES_HBM, wave_hbm);
   }
 }
@@ -1051,18 +1045,27 @@ __device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* sh, uint64_
 __device__ __forceinline__ void put_part(uint64_t* p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool last_block(uint64_t* done, uint32_t nb) {
+// `v`: a total small enough (40 bits) to travel with the count (24 bits): in,
+// the block's; out, in the last block's first thread, the sum of all.
+__device__ __forceinline__ bool last_block(uint64_t* done, uint32_t nb, uint64_t& v) {
   if (nb == 1) return true;
   __shared__ uint32_t s_last;
   if (threadIdx.x == 0) {  // the thread that stored the block's totals
     wait_vm();
-    const unsigned long long n = __hip_atomic_fetch_add((unsigned long long*)done, 1ull,
+    const unsigned long long n = __hip_atomic_fetch_add((unsigned long long*)done, v << 24 | 1ull,
                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = n + 1 == nb ? 1u : 0u;
-    if (s_last) *done = 0;  // for the next scan
+    s_last = (n & 0xFFFFFFull) + 1 == nb ? 1u : 0u;
+    if (s_last) {
+      v += n >> 24;
+      *done = 0;  // for the next scan
+    }
   }
   __syncthreads();
   return s_last != 0;
+}
+__device__ __forceinline__ bool last_block(uint64_t* done, uint32_t nb) {
+  uint64_t none = 0;
+  return last_block(done, nb, none);
 }
 // part[stride * b] for every block b: totals to exclusive prefixes; returns
 // the sum (`own`: this block's total, all there is when it is the only one).
@@ -1133,16 +1136,19 @@ __device__ __forceinline__ void plan_block(const PlanArgs& A, uint32_t bi, uint3
     // a tile's offset inside its gate's waveform travels in 31 bits
     if (N + 1 >= (1ull << 30)) atomicOr((unsigned int*)(A.scal + S_ERR), ERR_RANGE);
     GatePlan P;
+    const uint32_t seg =
+        A.spread > 0 ? min(A.seg_target, max(kSpreadSeg, (uint32_t)((float)N * A.spread))) : A.seg_target;
     if (G.k > kTileK) {
-      const uint32_t nt0 = (uint32_t)max<uint64_t>(1, (N + A.wide_words - 1) / A.wide_words);
+      const uint32_t ww = (uint32_t)min<uint64_t>(A.wide_words, (uint64_t)seg * kLanes);
+      const uint32_t nt0 = (uint32_t)max<uint64_t>(1, (N + ww - 1) / ww);
       P.lt = max(1u, (nl + nt0 - 1) / nt0);
     } else {
       // (64-bit divisions only where 32 bits do not hold the product)
       uint64_t s = 1;
       if (N > 0)
-        s = N < (1ull << 31) && (uint64_t)A.seg_target * nl < (1ull << 32)
-                ? (uint64_t)(A.seg_target * nl / (uint32_t)N)
-                : (uint64_t)A.seg_target * nl / N;
+        s = N < (1ull << 31) && (uint64_t)seg * nl < (1ull << 32)
+                ? (uint64_t)(seg * nl / (uint32_t)N)
+                : (uint64_t)seg * nl / N;
       if (s < 1) s = 1;
       if (nl > 0) {
         if (s < (1u << 24) && nl < (1u << 31)) {
@@ -1210,7 +1216,6 @@ __device__ __forceinline__ void plan_block(const PlanArgs& A, uint32_t bi, uint3
   A.scal[S_TOT_B] = scr;
   A.scal[S_NTILES + A.slot] = tiles;
   A.scal[S_SCRATCH + A.slot] = (uint64_t)scratch;
-  A.scal[S_EVL] = 0;
   A.scal[S_OVF_USED] = 0;
   if (why) {
     A.scal[S_WHY] = why;
@@ -1489,20 +1494,23 @@ __global__ __launch_bounds__(256) void k_tile_desc(
 // The block that finishes last places the gates in the pool and closes the
 // level: bump pointer, gate events, or a trip when the level ran out of
 // overflow stacks.
-__global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
-  __shared__ uint64_t sh[4];
-  __shared__ uint32_t s_cnt[kJoinGates], s_job[kJoinGates];
+__global__ __launch_bounds__(8 * kJoinGates) void k_join(JoinArgs A, TailArgs T) {
+  constexpr int kThreads = 8 * kJoinGates;
+  __shared__ uint64_t sh[kThreads / 64], s_all[kThreads / 64];
+  __shared__ uint32_t s_job[kJoinGates];
   __shared__ unsigned long long s_ev[kJoinGates];
   if (A.scal[S_TRIP]) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     A.scal[S_EVAL] += (uint64_t)wall_clock64() - A.scal[S_CLOCK];
     A.scal[S_LEVELS] += 1;
+    A.scal[S_TILES] += A.scal[S_NTILES + A.slot];
   }
   const uint32_t grp = threadIdx.x >> 3, l8 = threadIdx.x & 7u;
   const int sh8 = (int)(threadIdx.x & 56u);  // the group's first lane in its wavefront
   const uint32_t g = blockIdx.x * kJoinGates + grp;
+  uint32_t words = 0;  // the gate's, in its first lane
+  uint64_t ev = 0;     // events of the lane's tiles
   if (l8 == 0) {
-    s_cnt[grp] = 0;
     s_ev[grp] = 0;
     s_job[grp] = 0xFFFFFFFFu;
   }
@@ -1552,6 +1560,7 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
       // an instance counts the events of its tiles with entries; the tiles of a
       // wide gate count as one
       gev += ne || G.k > kTileK ? S.ev : 0u;
+      ev += S.ev;
       any |= mask;
       // inclusive scan of the joined counts over the step
       uint32_t incl = mine;
@@ -1579,7 +1588,7 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
       gev += __shfl_xor(gev, d, 8);
     }
     if (l8 == 0) {
-      s_cnt[grp] = cnt;
+      words = cnt;
       s_job[grp] = G.job;
       s_ev[grp] = any ? gev : 0ull;
       A.wlen[G.out_net] = cnt;
@@ -1590,39 +1599,35 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
       sa[3] = tc;
     }
   }
-  __syncthreads();
   const unsigned int err = *(const unsigned int*)(A.scal + S_ERR);
-  uint64_t own = 0;        // the block's words, in the first wavefront
-  if (threadIdx.x < 64) {  // the first wavefront: prefixes over the block's gates
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) ev += __shfl_xor(ev, d);
+  if ((threadIdx.x & 63) == 0) s_all[threadIdx.x >> 6] = ev;
+  uint64_t own;  // the block's words
+  const uint64_t x = block_scan<kThreads>(words, sh, own);  // (its barriers: s_all, s_ev, s_job)
+  if (l8 == 0 && g < A.ng) A.out_loc[g] = x;
+  uint64_t events = 0;
+  if (threadIdx.x == 0) {
+    put_part(A.part + blockIdx.x, own);
+#pragma unroll
+    for (int i = 0; i < kThreads / 64; ++i) events += s_all[i];
+  }
+  // a level whose tiles ran out of overflow stacks runs again: counted then
+  if (A.ev_job && !(err & ERR_OVERFLOW) && threadIdx.x < 64) {
     const uint32_t i = threadIdx.x;
-    const uint64_t mine = i < kJoinGates ? s_cnt[i] : 0u;
-    uint64_t x = mine;
+    const uint32_t job = i < kJoinGates ? s_job[i] : 0xFFFFFFFFu;
+    unsigned long long e = i < kJoinGates ? s_ev[i] : 0ull;
+    const uint32_t job0 = __shfl(job, 0, 64);
+    if (__ballot(job != job0 && job != 0xFFFFFFFFu)) {
+      if (job != 0xFFFFFFFFu && e) atomicAdd(A.ev_job + job, e);
+    } else {
 #pragma unroll
-    for (int d = 1; d < (int)kJoinGates; d <<= 1) {
-      const uint64_t y = __shfl_up(x, d, 64);
-      if ((int)i >= d) x += y;
-    }
-    const uint32_t gi = blockIdx.x * kJoinGates + i;
-    if (i < kJoinGates && gi < A.ng) A.out_loc[gi] = x - mine;
-    const uint64_t tot = __shfl(x, kJoinGates - 1, 64);
-    own = tot;
-    if (i == 0) put_part(A.part + blockIdx.x, tot);
-    // a level whose tiles ran out of overflow stacks runs again: counted then
-    if (A.ev_job && !(err & ERR_OVERFLOW)) {
-      const uint32_t job = i < kJoinGates ? s_job[i] : 0xFFFFFFFFu;
-      unsigned long long ev = i < kJoinGates ? s_ev[i] : 0ull;
-      const uint32_t job0 = __shfl(job, 0, 64);
-      if (__ballot(job != job0 && job != 0xFFFFFFFFu)) {
-        if (job != 0xFFFFFFFFu && ev) atomicAdd(A.ev_job + job, ev);
-      } else {
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) ev += __shfl_xor(ev, d);
-        if (i == 0 && ev) atomicAdd(A.ev_job + job0, ev);
-      }
+      for (int d = 1; d < 64; d <<= 1) e += __shfl_xor(e, d);
+      if (i == 0 && e) atomicAdd(A.ev_job + job0, e);
     }
   }
-  if (!last_block(A.scal + S_DONE, gridDim.x)) return;
-  const uint64_t total = scan_parts<256>(A.part, 1, gridDim.x, own, sh);
+  if (!last_block(A.scal + S_DONE, gridDim.x, events)) return;
+  const uint64_t total = scan_parts<kThreads>(A.part, 1, gridDim.x, own, sh);
   if (threadIdx.x != 0) return;
   if (A.ovf_trip && (err & ERR_OVERFLOW)) {
     A.scal[S_TRIP] = A.level;
@@ -1638,7 +1643,7 @@ __global__ __launch_bounds__(256) void k_join(JoinArgs A, TailArgs T) {
   }
   A.scal[S_OUTBASE] = base;
   A.scal[S_BUMP] = base + total;
-  A.scal[S_EVC] += A.scal[S_EVL];
+  A.scal[S_EVC] += events;
 }
 
 // Copy every tile's joined output from the scratch into the gate's dense
@@ -1940,7 +1945,7 @@ hipError_t launch_fill_u64(unsigned long long* p, uint64_t n, unsigned long long
 
 hipError_t launch_join(const JoinArgs& a, const TailArgs& T, hipStream_t st) {
   if (a.ng == 0) return hipSuccess;
-  k_join<<<nblk(a.ng, kJoinGates), 256, 0, st>>>(a, T);
+  k_join<<<nblk(a.ng, kJoinGates), 8 * kJoinGates, 0, st>>>(a, T);
   return hipGetLastError();
 }
 

@@ -67,3 +67,32 @@ def test_tile_boundaries_of_uneven_inputs(ctx, seed, cells, levels, t_end, gap, 
         assert r.waves_hash() == want["waves_hash"], seg
         assert r.saif_text() == want["saif"], seg
         r.close()
+
+
+@pytest.mark.parametrize("cells,t_end,gap", [(12, 40000, 20.0), (300, 30000, 40.0)])
+def test_lane_shares_of_small_levels(ctx, cells, t_end, gap, tmp_path):
+    """The default lane share depends on how many workgroups a level has to
+    fill (16 to 32 words); any share gives the same waveforms, and in a batch
+    it stays fixed."""
+    print("shares", cells, flush=True)
+    sys.stdout.flush()
+    d = gls.Design.generate(3, 700 + cells, cells, 4, 8)
+    paths = [str(tmp_path / n) for n in ("lib.vlib", "n.gv", "n.sdf", "s.vcd")]
+    d.write(*paths[:3])
+    s = gls.Stimulus.generate(d, 71, t_end, gap, 0.05)
+    s.write_vcd(paths[3])
+    want = oracle_bind.run(*paths, 0, t_end, str(tmp_path))
+    tiles = []
+    for blocks in (1, 8, 64, 0):
+        r = ctx.simulate(d, s, 0, t_end, keep_waves=True, level_blocks=blocks)
+        assert r.stats()["n_events"] == want["n_events"], blocks
+        assert r.waves_hash() == want["waves_hash"], blocks
+        assert r.saif_text() == want["saif"], blocks
+        tiles.append(r.stats()["tiles"])
+        r.close()
+    assert tiles[0] <= tiles[1] <= tiles[2] <= tiles[3] and tiles[0] < tiles[3]
+    run = ctx.prepare_batch([d, d], [s, s], [0, 0], [t_end, t_end])
+    run.execute()
+    assert run.stats()["tiles"] == 2 * tiles[0]
+    assert run.instance_saif_text(1) == want["saif"]
+    run.close()
