@@ -95,17 +95,6 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
   return __builtin_amdgcn_readlane(wave_scan(x), 63);
 }
 
-// Inclusive prefix maximum over the wavefront.
-__device__ __forceinline__ uint32_t wave_max_scan(uint32_t x) {
-  x = max(x, dpp<0x111>(x));
-  x = max(x, dpp<0x112>(x));
-  x = max(x, dpp<0x114>(x));
-  x = max(x, dpp<0x118>(x));
-  x = max(x, dpp<0x142, 0xA>(x));
-  x = max(x, dpp<0x143, 0xC>(x));
-  return x;
-}
-
 // Minimum over the lanes after this one (all ones for lane 63): within rows
 // by row shifts, the later rows' minima from their first lanes.
 __device__ __forceinline__ uint32_t wave_min_after(uint32_t x) {
@@ -327,9 +316,12 @@ struct Lane {
 //   fan-in 2: binary search on the merge path's diagonal (exact: 11 steps of
 //     two LDS reads for 2,000 words).
 //   fan-in 3+: a start is an event of the leader input: its index at the
-//     leader's share of the rank, the other inputs' positions by binary
-//     search, then one correction by the rank error and a second search (the
-//     merged rank of 3..6 ranges has no direct search).
+//     leader's share of the rank, the other inputs' positions and with them the
+//     exact rank by binary search, then interpolation between the two lanes
+//     around the wanted rank and a short second search (the merged rank of
+//     3..6 ranges has no direct search).  Of 32.5 words a lane on average the
+//     longest lane has 41; corrected by its own rank error alone it had 48, and
+//     a tile's walk lasts as long as its longest lane's.
 template <int K>
 __device__ __forceinline__ void lane_bounds(const uint32_t (&in)[K], const Tile& D, uint32_t k,
                                             uint32_t (&a)[K], uint32_t& t0, uint32_t& t1) {
@@ -394,25 +386,31 @@ __device__ __forceinline__ void lane_bounds(const uint32_t (&in)[K], const Tile&
     uint32_t rank = 0;
 #pragma unroll
     for (int j = 0; j < K; ++j) rank += (uint32_t)j < k ? (p[j] - in[j]) / 4 : 0u;
-    const int dx = __float2int_rn((float)((int)d - (int)rank) * r);
-    x = halo ? x : min(max(x + dx, 1), top);
-    x = (int)wave_max_scan((uint32_t)x);  // starts stay in order
+    // the lanes' guesses are 64 knots of the exact rank over the leader: take
+    // the knots around the wanted rank (i the last at or below it) and
+    // interpolate; the positions follow knot i's
+    const uint32_t knot = rank << 16 | (uint32_t)x, past = D.own << 16 | last;
+    uint32_t i = 0;
+#pragma unroll
+    for (uint32_t s = 32; s; s >>= 1) i += (uint32_t)__shfl((int)knot, (int)(i + s)) >> 16 <= d ? s : 0u;
+    const uint32_t ka = (uint32_t)__shfl((int)knot, (int)i), kn = (uint32_t)__shfl((int)knot, (int)(i + 1));
+    const uint32_t kb = i < 63 ? kn : past;
+    const int xa = (int)(ka & 0xFFFFu), xb = (int)(kb & 0xFFFFu);
+    const float per = (float)(xb - xa) * __builtin_amdgcn_rcpf((float)max((kb >> 16) - (ka >> 16), 1u));
+    const int dx = (int)((float)(d - (ka >> 16)) * per + 0.5f);
+    const int xi = max(min(min(xa + dx, xb), top), 1);
+#pragma unroll
+    for (int j = 0; j < K; ++j) p[j] = (uint32_t)__shfl((int)p[j], (int)i);
+    x = halo ? x : xi;
     t0 = lane == 0 ? 4u : lds32(il + 4 * x) & ~3u;
-    // the correction is small: search 32 words around the first positions,
-    // and everywhere only when a lane's lies outside
+    // 31 words from knot i's positions, and everywhere when a lane's lies beyond
     uint32_t p0[K];
     bool miss = false;
 #pragma unroll
-    for (int j = 0; j < K; ++j) p[j] = p0[j] = max(p[j], in[j] + 4 * 16) - 4 * 16;
+    for (int j = 0; j < K; ++j) p0[j] = p[j];
     descend(16);
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-      if ((uint32_t)j >= k) continue;
-      // the word before p0 must be before t0 (or p0 be the range's start), and
-      // the search must not have run to its end
-      miss |= p0[j] > in[j] && lds32(p0[j]) >= t0;
-      miss |= p[j] == p0[j] + 4 * 31;
-    }
+    for (int j = 0; j < K; ++j) miss |= (uint32_t)j < k && p[j] == p0[j] + 4 * 31;
     if (__ballot(miss)) {
 #pragma unroll
       for (int j = 0; j < K; ++j) p[j] = in[j];
