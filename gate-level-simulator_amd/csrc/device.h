@@ -103,6 +103,14 @@ __host__ __device__ inline constexpr uint32_t walk_lds_need(uint32_t id, uint32_
   return walk_dt_words(id, k) + walk_tt_words(id, k) + (words + 8 * k) + (words + kStackSlack);
 }
 
+// LDS words of one input range's slot: n words from pool word lo.  The slots
+// follow the tables; the range starts lo mod 4 words into its slot, so that it
+// is copied with 16-byte loads from the aligned word before it, and the word
+// behind it is its sentinel's.  At most n + 7 words.
+__host__ __device__ inline constexpr uint32_t range_words(uint32_t lo, uint32_t n) {
+  return ((lo & 3u) + n + 4) & ~3u;
+}
+
 // Per-gate tiling of one level: tile i covers the leader input's words
 // [i * lt, (i + 1) * lt).
 struct GatePlan {
@@ -127,7 +135,9 @@ struct alignas(16) TileDesc {
   uint32_t out_cap;        // words of the tile's output region in the level scratch
   uint32_t g, ti;          // gate (index in the level), tile of the gate
   uint32_t out_net;
-  uint32_t pad[5];
+  uint32_t at2[3];         // where the ranges are staged: LDS words, two inputs a word (range_words)
+  uint32_t words;          // sum of n
+  uint32_t tab;            // words of the gate's delay table | truth bytes << 16
 };
 static_assert(sizeof(TileDesc) == 128, "TileDesc layout");
 

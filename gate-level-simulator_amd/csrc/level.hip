@@ -140,6 +140,12 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
+// Global memory behind an address that travelled as a number: without the
+// address space its accesses would be flat ones, which also count as LDS
+// accesses and hold up the waits for them.
+typedef __attribute__((address_space(1))) uint32_t glb_u32;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef __attribute__((address_space(1))) u32x4 glb_u32x4;
 
 // LDS by byte address (32-bit local pointers: the reads are ds_read with the
 // constant part of the address in the instruction).
@@ -173,7 +179,7 @@ __device__ __forceinline__ void wait_vm() {
 struct Tile {
   uint32_t in_lo[6], n[6], in_hi[2];
   uint64_t scr;
-  uint32_t own, xend, meta, dt_off, tt_off, dmax, job, out_cap, g;
+  uint32_t own, xend, meta, dt_off, tt_off, dmax, job, out_cap, g, at2[3], words, tab;
 
   __device__ __forceinline__ uint32_t id() const { return meta & 15u; }
   __device__ __forceinline__ uint32_t k() const { return (meta >> 4) & 15u; }
@@ -183,25 +189,27 @@ struct Tile {
   __device__ __forceinline__ uint64_t src(int j) const {
     return ((uint64_t)((in_hi[j >> 2] >> (8 * (j & 3))) & 0xFFu) << 32) | in_lo[j];
   }
-  __device__ __forceinline__ uint32_t words() const {
-    uint32_t t = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kWideK; ++j) t += n[j];  // 0 beyond the fan-in
-    return t;
-  }
+  __device__ __forceinline__ uint32_t dt_words() const { return tab & 0xFFFFu; }
+  __device__ __forceinline__ uint32_t tt_words() const { return tab >> 16; }
+  // LDS word of input j's range (range_at)
+  __device__ __forceinline__ uint32_t at(int j) const { return (at2[j >> 1] >> (16 * (j & 1))) & 0xFFFFu; }
 };
 
 // A tile descriptor is read with one coalesced load (lane i < 32 holds
 // dword i), a tile ahead, and broadcast with readlane: its fields are scalars
-// and no load of theirs waits behind the staging loads in flight.
+// and no load of theirs waits behind the staging loads in flight.  The loaded
+// word is what a loop carries, not the scalars: uniform for a reader, they are
+// divergent for the compiler wherever a branch of single lanes meets the loop's,
+// and it then keeps them in vector registers and walks every branch on them with
+// the execution mask (a quarter of the instructions of a tile's fixed part).
 __device__ __forceinline__ uint32_t desc_word(const TileDesc* p) {
   return threadIdx.x < 32 ? ((const uint32_t*)p)[threadIdx.x] : 0u;
 }
 
 __device__ __forceinline__ Tile tile_of(uint32_t dw) {
-  uint32_t w[25];
+  uint32_t w[32];
 #pragma unroll
-  for (int i = 0; i < 25; ++i) w[i] = __builtin_amdgcn_readlane(dw, i);
+  for (int i = 0; i < 32; ++i) w[i] = __builtin_amdgcn_readlane(dw, i);
   Tile D;
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
@@ -220,46 +228,43 @@ __device__ __forceinline__ Tile tile_of(uint32_t dw) {
   D.job = w[22];
   D.out_cap = w[23];
   D.g = w[24];
+  D.at2[0] = w[27];
+  D.at2[1] = w[28];
+  D.at2[2] = w[29];
+  D.words = w[30];
+  D.tab = w[31];
   return D;
 }
 
-// LDS layout of a tile's input ranges (byte address of each range's index 0):
-// range j (n_j words from pool word G_j) starts at word P_j = R_j + G_j mod 4
-// with R_j a multiple of 4 words, so it is copied with 16-byte loads from the
-// aligned word G_j - G_j mod 4; R_{j+1} = the multiple of 4 at or above
-// P_j + n_j + 1 keeps the sentinel word after each range.  The layout needs at
-// most sum(n_j) + 7 K words.
-__device__ __forceinline__ void range_layout(const Tile& D, uint32_t base, uint32_t P[6]) {
-  uint32_t R = base;
-#pragma unroll
-  for (uint32_t j = 0; j < kWideK; ++j) {
-    P[j] = R + 4 * (D.in_lo[j] & 3u);
-    if (j < D.k()) R = (P[j] + 4 * D.n[j] + 16) & ~15u;
-  }
+// A value that is the same in every lane, for the compiler too.
+__device__ __forceinline__ uint32_t uni(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ uint64_t uni(uint64_t x) {
+  return ((uint64_t)uni((uint32_t)(x >> 32)) << 32) | uni((uint32_t)x);
 }
 
-// First byte of the tile's input ranges: after its gate's tables.
-__device__ __forceinline__ uint32_t in_base(const Tile& D) {
-  return 4 * (walk_dt_words(D.id(), D.k()) + walk_tt_words(D.id(), D.k()));
-}
 __device__ __forceinline__ bool tile_fits(const LevelArgs& A, const Tile& D) {
-  return D.id() < W_COUNT && walk_lds_need(D.id(), D.k(), D.words()) <= A.lds_words;
+  return D.id() < W_COUNT &&
+         D.dt_words() + D.tt_words() + 2 * D.words + 8 * D.k() + kStackSlack <= A.lds_words;
 }
-// First byte of the tile's stacks: they end with the workgroup's LDS, so the
+// First word behind the tile's input ranges.
+__device__ __forceinline__ uint32_t in_end(const Tile& D) {
+  return D.dt_words() + D.tt_words() + D.words + 8 * D.k();
+}
+// First word of the tile's stacks: they end with the workgroup's LDS, so the
 // next tile's inputs can be staged at the front while they are read.
-__device__ __forceinline__ uint32_t stack_base(const LevelArgs& A, const Tile& D) {
-  return 4 * (A.lds_words - D.words() - kStackSlack);
+__device__ __forceinline__ uint32_t stack_at(const LevelArgs& A, const Tile& D) {
+  return A.lds_words - D.words - kStackSlack;
 }
 
 // Issue the loads of a tile into LDS: its gate's tables (unless the tile
-// before was of the same gate) and its input ranges (laid out by
-// range_layout; the 16-byte copies may also bring up to 3 words before and
-// after a range, inside its slot).  Completion: wait_vm().
+// before was of the same gate) and its input ranges (the 16-byte copies may also
+// bring up to 3 words before and after a range, inside its slot).  Completion:
+// wait_vm().
 __device__ __forceinline__ void stage_tile(const LevelArgs& A, const Tile& D, bool tables,
                                            uint32_t* lds) {
   const uint32_t lane = threadIdx.x;
   if (tables) {
-    const uint32_t dw = walk_dt_words(D.id(), D.k()), tw = walk_tt_words(D.id(), D.k());
+    const uint32_t dw = D.dt_words(), tw = D.tt_words();
     const uint32_t* dsrc = A.dtab + D.dt_off;
     const uint32_t* tsrc = A.ttab + D.tt_off;
 #pragma unroll 1
@@ -269,29 +274,27 @@ __device__ __forceinline__ void stage_tile(const LevelArgs& A, const Tile& D, bo
     for (uint32_t i = 0; i < tw; i += 4 * kLanes)
       if (i + 4 * lane < tw) dma_x4(tsrc + i + 4 * lane, lds + dw + i);
   }
-  uint32_t P[6];
-  range_layout(D, in_base(D), P);
 #pragma unroll
   for (uint32_t j = 0; j < kWideK; ++j) {
     if (j >= D.k()) break;
     const uint32_t a = D.in_lo[j] & 3u;
     const uint32_t m = (a + D.n[j] + 3) & ~3u;  // words copied, a multiple of 4
     const uint32_t* src = A.pool + (D.src(j) - a);
-    uint32_t* l = lds + (P[j] / 4 - a);
+    uint32_t* l = lds + (D.at(j) - a);
 #pragma unroll 1
     for (uint32_t i = 0; i < m; i += 4 * kLanes)
       if (i + 4 * lane < m) dma_x4(src + i + 4 * lane, l + i);
   }
 }
 
-// INF after every input range of a staged tile (its loads have arrived).
+// INF after every input range of a staged tile (its loads have arrived).  Every
+// lane writes the same word: a branch for one lane is dearer.
 __device__ __forceinline__ void put_sentinels(const Tile& D) {
-  if (threadIdx.x != 0) return;
-  uint32_t P[6];
-  range_layout(D, in_base(D), P);
 #pragma unroll
-  for (uint32_t j = 0; j < kWideK; ++j)
-    if (j < D.k()) *(lds_u32*)(P[j] + 4 * D.n[j]) = kWordInf;
+  for (uint32_t j = 0; j < kWideK; ++j) {
+    if (j >= D.k()) break;
+    *(lds_u32*)(4 * (D.at(j) + D.n[j])) = kWordInf;
+  }
 }
 
 // What one lane's walk leaves: candidates (or, later, kept entries) at
@@ -440,15 +443,14 @@ __device__ __forceinline__ Lane<lds_u32*> lane_walk(const LevelArgs& A, const Ti
   const uint32_t k = GEN ? D.k() : (uint32_t)K;
   const uint32_t lane = threadIdx.x;
   const uint32_t ttb = 4 * walk_dt_words(ID, K);  // truth bytes; the delay table is at 0
-  uint32_t P[6], in[K], a[K];
-  range_layout(D, in_base(D), P);
+  uint32_t in[K], a[K];
 #pragma unroll
-  for (int j = 0; j < K; ++j) in[j] = P[j];
+  for (int j = 0; j < K; ++j) in[j] = 4 * D.at(j);
   if (GEN) {
     // unused inputs stand at input 0's sentinel
 #pragma unroll
     for (int j = 0; j < K; ++j)
-      if ((uint32_t)j >= k) in[j] = P[0] + 4 * D.n[0];
+      if ((uint32_t)j >= k) in[j] = in[0] + 4 * D.n[0];
   }
   uint32_t t0, t1;
   lane_bounds<K>(in, D, k, a, t0, t1);
@@ -461,7 +463,7 @@ __device__ __forceinline__ Lane<lds_u32*> lane_walk(const LevelArgs& A, const Ti
     x = __builtin_amdgcn_alignbit(pw[j], x, 2);
   }
   Lane<lds_u32*> ln;
-  uint32_t sp = stack_base(A, D) + 4 * soff;
+  uint32_t sp = 4 * (stack_at(A, D) + soff);
   ln.lo = (lds_u32*)sp;
   // the gate's value before the first event: X at t = 0 (src/simulate.cpp:933),
   // else the function of the values
@@ -771,7 +773,7 @@ __device__ __forceinline__ void keep_entries(const LevelArgs& A, Lane<SP>& ln, b
 // `before_stores` runs just before the first store.
 template <typename SP, typename F>
 __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const Lane<SP>& ln,
-                                          uint32_t* dst, uint32_t out_cap, unsigned long long w_start,
+                                          glb_u32* dst, uint32_t out_cap, unsigned long long w_start,
                                           unsigned long long w_end, F&& before_stores) {
   const int lane = threadIdx.x;
   const uint32_t n = (uint32_t)(ln.hi - ln.lo);
@@ -806,7 +808,9 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
     // the interval before the lane's first entry, which is not stored again
     // when it repeats the value before it
     add(e_first);
-    uint32_t* dp = dst + w;
+    // (the tile's region is uniform: lanes add 32-bit offsets to it)
+    auto to = [&](uint32_t q) { return (glb_u32*)((__attribute__((address_space(1))) char*)dst + q); };
+    uint32_t dp = 4 * w;
     uint32_t left = min(mine, out_cap - w);  // entries that the region takes
     SP p = ln.lo + dup;
     // whole groups of four: four reads in flight, one store
@@ -816,8 +820,8 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
       for (int q = 0; q < 4; ++q) e4[q] = p[q];
 #pragma unroll
       for (int q = 0; q < 4; ++q) add(e4[q]);
-      __builtin_memcpy(dp, e4, 16);
-      dp += 4;
+      *(glb_u32x4*)to(dp) = u32x4{e4[0], e4[1], e4[2], e4[3]};
+      dp += 16;
       p += 4;
       left -= 4;
     }
@@ -829,7 +833,7 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         add(e4[q]);
-        if ((uint32_t)q < left) dp[q] = e4[q];
+        if ((uint32_t)q < left) *to(dp + 4 * q) = e4[q];
       }
     }
   }
@@ -867,7 +871,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   if (A.scal[S_TRIP]) return;
   if (blockIdx.x == 0 && lane == 0) A.scal[S_CLOCK] = (uint64_t)wall_clock64();
   const uint64_t ntiles = A.scal[S_NTILES + A.slot];  // uniform: one scalar load
-  uint32_t* const scratch = (uint32_t*)A.scal[S_SCRATCH + A.slot];
+  glb_u32* const scratch = (glb_u32*)A.scal[S_SCRATCH + A.slot];
   unsigned int* const err = (unsigned int*)(A.scal + S_ERR);
   // Tiles are handed out in two parts.  The first half is split into
   // one run of consecutive tiles per workgroup (consecutive tiles of one gate
@@ -891,8 +895,9 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   };
   auto drawn_batch = [&]() -> uint64_t {  // first tile of the drawn batch (ntiles: none left)
     while (t_drawn < ntiles && used_up < kTickets) {
-      const uint64_t i = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(drawn >> 32)) << 32) |
-                         (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)drawn);
+      counter = uni(counter);
+      used_up = uni(used_up);
+      const uint64_t i = uni((uint64_t)drawn);
       const uint64_t t = t_drawn + (counter + kTickets * i) * B;
       if (t < ntiles) return t;
       if (++used_up == kTickets) break;
@@ -902,16 +907,22 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
     return ntiles;
   };
   if (tk + 1 >= bend) draw();
-  Tile D = tile_of(desc_word(A.tiles + tk));
-  bool fits = tile_fits(A, D);
+  uint32_t dw = desc_word(A.tiles + tk);
   uint32_t tab_g = 0xFFFFFFFFu;  // gate whose tables are in LDS
-  if (fits) {
-    stage_tile(A, D, true, s_dyn);
-    tab_g = D.g;
-    wait_vm();
-    put_sentinels(D);
+  {
+    const Tile D = tile_of(dw);
+    if (tile_fits(A, D)) {
+      stage_tile(A, D, true, s_dyn);
+      tab_g = D.g;
+      wait_vm();
+      put_sentinels(D);
+    }
   }
   for (;;) {
+    tk = uni(tk);
+    tab_g = uni(tab_g);
+    const Tile D = tile_of(dw);
+    const bool fits = tile_fits(A, D);
     // the tile after this one: the next of its run, or the first of the batch
     // drawn a tile ago
     uint64_t tn = tk + 1;
@@ -919,30 +930,21 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       tn = drawn_batch();
       bend = min(tn + B, ntiles);
     }
+    tn = uni(tn);
+    bend = uni(bend);
     const bool more_tiles = tn < ntiles;
     const uint32_t dwn = more_tiles ? desc_word(A.tiles + tn) : 0u;
     if (more_tiles && tn + 1 >= bend) draw();
     const ChunkWin* W = A.cwin + D.job;
     const unsigned long long w_start = W->lo, w_end = W->hi;
     lds_fence();
-    Tile Dn = D;
-    bool fits_n = false, staged = false;
-    auto stage_next = [&] {
-      if (!fits_n || staged) return;
-      stage_tile(A, Dn, Dn.g != tab_g, s_dyn);
-      tab_g = Dn.g;
-      staged = true;
-    };
+    bool staged = false;  // the next tile's loads are on their way
     auto finish = [&](auto& ln) {
       // inputs and tables are no longer read
       lds_fence();
-      if (more_tiles) {
-        Dn = tile_of(dwn);
-        fits_n = tile_fits(A, Dn);
-        if (A.prefetch &&
-            !(fits && in_base(Dn) + 4 * (Dn.words() + 8 * Dn.k()) > stack_base(A, D)))
-          stage_next();
-      }
+      const Tile Dn = tile_of(dwn);
+      staged = more_tiles && A.prefetch && tile_fits(A, Dn) && !(fits && in_end(Dn) > stack_at(A, D));
+      if (staged) stage_tile(A, Dn, Dn.g != tab_g, s_dyn);
       const bool halo = D.xend != 0 && lane == kLanes - 1;
       keep_entries(A, ln, halo);
       if (halo) ln.nown = 0;
@@ -974,11 +976,10 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       ln.lo = ln.hi = A.ovf;
       ln.nown = 0;
       if (D.id() < W_COUNT) {
-        const unsigned long long need = (unsigned long long)D.words() + kStackSlack;
+        const unsigned long long need = (unsigned long long)D.words + kStackSlack;
         unsigned long long base = 0;
         if (lane == 0) base = atomicAdd((unsigned long long*)(A.scal + S_OVF_USED), need);
-        base = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
-               (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)base);  // lane 0's value
+        base = uni((uint64_t)base);  // lane 0's value
         uint32_t bad = 0;
         if (base + need > A.ovf_cap) {
           // no room: the tile's output is left empty (so the level's waveforms
@@ -991,18 +992,21 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       }
       finish(ln);
     }
-    if (more_tiles && fits_n && !staged) {
-      lds_fence();
-      stage_next();
-      wait_vm();
-      put_sentinels(Dn);
-    }
     lds_fence();
     wave_hbm += fits ? 0u : 1u;
     if (!more_tiles) break;
+    const Tile Dn = tile_of(dwn);
+    if (tile_fits(A, Dn)) {
+      if (!staged) {
+        stage_tile(A, Dn, Dn.g != tab_g, s_dyn);
+        wait_vm();
+        put_sentinels(Dn);
+      }
+      tab_g = Dn.g;
+    }
+    lds_fence();
     tk = tn;
-    fits = fits_n;
-    D = Dn;
+    dw = dwn;
   }
   if (lane == 0) {
     unsigned long long* n = (unsigned long long*)A.scal;
@@ -1392,6 +1396,8 @@ __global__ __launch_bounds__(256) void k_tile_desc(
     __syncthreads();
     if (!valid || row == kRow) continue;
     TileDesc& D = tiles[t];
+    const uint32_t dtw = walk_dt_words(G.walk, G.k), ttw = walk_tt_words(G.walk, G.k);
+    uint32_t slot8[2] = {0, 0}, nq[2] = {0, 0}, in_lo8[2] = {0, 0};
     // own input words of the tile (up to the next tile's first words), summed
     // over the tile's threads: its output region in the level scratch holds
     // that many entries plus one
@@ -1432,8 +1438,9 @@ __global__ __launch_bounds__(256) void k_tile_desc(
         if (j == P.lead) xend = (ti + 1) * P.lt - (L[q] > 0 ? L[q] - 1 : 0u);
       }
       const uint32_t B = L[q] > 0 ? L[q] - 1 : 0u;
-      D.in_lo[j] = (uint32_t)(off + B);
-      D.n[j] = E - B;
+      D.in_lo[j] = in_lo8[q] = (uint32_t)(off + B);
+      D.n[j] = nq[q] = E - B;
+      slot8[q] = range_words(in_lo8[q], E - B);
       hi8[q] = (uint32_t)((off + B) >> 32) << (8 * j0);
       span += Ln - L[q];
       own += Ln - max(L[q], 1u);
@@ -1450,7 +1457,25 @@ __global__ __launch_bounds__(256) void k_tile_desc(
       hi8[0] |= __shfl_xor(hi8[0], d);
       hi8[1] |= __shfl_xor(hi8[1], d);
     }
+    // where the ranges start in LDS: the slots before, and the words that the
+    // first one's 16-byte copies bring before it
+    uint32_t words = nq[0] + nq[1], at[2];
+    words += __shfl_xor(words, 1);
+    words += __shfl_xor(words, 2);
+    const uint32_t b1 = __shfl_up(slot8[0], 1, 4), b2 = __shfl_up(slot8[0], 2, 4), b3 = __shfl_up(slot8[0], 3, 4);
+    uint32_t all4 = slot8[0] + __shfl_xor(slot8[0], 1);
+    all4 += __shfl_xor(all4, 2);
+    at[0] = dtw + ttw + (j0 > 0 ? b1 : 0u) + (j0 > 1 ? b2 : 0u) + (j0 > 2 ? b3 : 0u) + (in_lo8[0] & 3u);
+    const uint32_t c0 = __shfl(slot8[1], 0, 4);
+    at[1] = dtw + ttw + all4 + (j0 > 0 ? c0 : 0u) + (in_lo8[1] & 3u);
+    uint32_t pair[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) pair[q] = (at[q] & 0xFFFFu) | __shfl_down(at[q], 1, 4) << 16;
+    if (j0 == 0 || j0 == 2) D.at2[j0 / 2] = pair[0];
     if (j0 == 0) {
+      D.at2[2] = pair[1];
+      D.words = words;
+      D.tab = dtw | ttw << 16;
       D.in_hi[0] = hi8[0];
       D.in_hi[1] = hi8[1];
       // a gate's region, then the tile's first own event in the gate's merged
@@ -1667,7 +1692,7 @@ __global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, Plan
   const uint32_t bi = blockIdx.x - nplan;
   const uint64_t waves = (uint64_t)(gridDim.x - nplan) * (blockDim.x / 64);
   const uint64_t nt = A.scal[S_NTILES + A.slot], base = A.scal[S_OUTBASE];
-  const uint32_t* __restrict__ scratch = (const uint32_t*)A.scal[S_SCRATCH + A.slot];
+  const glb_u32* scratch = (const glb_u32*)A.scal[S_SCRATCH + A.slot];
   for (uint64_t t = (uint64_t)bi * (blockDim.x / 64) + threadIdx.x / 64; t < nt; t += waves) {
     const TileDesc& D = tiles[t];
     const uint64_t gate = base + A.part[D.g / kJoinGates] + A.out_loc[D.g];
@@ -1685,7 +1710,7 @@ __global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, Plan
     if (!((S.flags >> 4) & 1u)) continue;
     const uint32_t off = tile_off[t] & 0x7FFFFFFFu, skip = tile_off[t] >> 31;
     const uint32_t n = S.cnt - skip;
-    const uint32_t* src = scratch + (((uint64_t)D.scr_hi << 32) | D.scr_lo) + skip;
+    const glb_u32* src = scratch + (((uint64_t)D.scr_hi << 32) | D.scr_lo) + skip;
     uint32_t* dst = pool + gate + off;
     // four loads in flight per lane before their stores: the copy of a tile
     // waits for memory about n / 256 times instead of n / 64
@@ -1701,7 +1726,7 @@ __global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, Plan
     if (A.count_tc) {
       // SAIF TC inside the tile: 0<->1 changes between its consecutive
       // entries (the first entry against the previous tile is k_join's)
-      const uint32_t* e = src - skip;
+      const glb_u32* e = src - skip;
       const ChunkWin W = A.cwin[D.job];
       uint32_t c = 0;
       for (uint32_t q = lane + 1; q < S.cnt; q += 64) {
