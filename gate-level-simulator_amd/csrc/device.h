@@ -141,17 +141,15 @@ struct alignas(16) TileDesc {
 };
 static_assert(sizeof(TileDesc) == 128, "TileDesc layout");
 
-// What the walk kernel leaves for one tile, 32 bytes: its output entries
-// (deduplicated inside the tile) sit in the level scratch; the per-gate
-// carry pass joins consecutive tiles.
+// What the walk kernel leaves for one tile, 16 bytes: its output entries
+// (deduplicated inside the tile) sit in the level scratch; the join places
+// them behind the tiles before.
 struct alignas(16) TileOut {
-  uint32_t cnt;         // entries after dedup inside the tile
-  uint32_t ft, lt;      // times of the first and last entries
-  uint32_t flags;       // first value | last value << 2 | has entries << 4
-  uint32_t t0, t1, tx;  // SAIF durations between the tile's own entries (clipped)
-  uint32_t ev;          // gate events of the tile (input-event times from the chunk start on)
+  uint32_t cnt;          // entries after dedup inside the tile
+  uint32_t first, last;  // the first and the last of them
+  uint32_t ev;           // gate events of the tile (input-event times from the chunk start on)
 };
-static_assert(sizeof(TileOut) == 32, "TileOut layout");
+static_assert(sizeof(TileOut) == 16, "TileOut layout");
 
 // SAIF counters per net: T0, T1, TX durations and TC, the number of direct
 // 0<->1 transitions at times in (dumpon, dumpoff].

@@ -131,11 +131,6 @@ __device__ __forceinline__ uint32_t lb_words(P a, uint32_t n, uint32_t key) {
   return lo;
 }
 
-// Bit fields of TileOut::flags.
-__device__ __forceinline__ uint32_t out_flags(uint32_t fv, uint32_t lv, uint32_t has) {
-  return fv | (lv << 2) | (has << 4);
-}
-
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
@@ -304,6 +299,7 @@ template <typename SP>
 struct Lane {
   SP lo, hi;
   uint32_t nown;
+  bool look;  // (uniform) some lane's events lie before the chunk
 };
 
 // The lanes' segments.  The tile's own words, in the merged time order of
@@ -494,6 +490,7 @@ __device__ __forceinline__ Lane<lds_u32*> lane_walk(const LevelArgs& A, const Ti
   const uint32_t lo_w = A.lo_rel << 2;
   uint32_t bound = t1;
   bool look = __ballot(w < lo_w && w < t1) != 0;
+  ln.look = look;
   if (look) bound = min(lo_w, t1);
   uint32_t nown = 0;
   // The two lookups of a step and its push are spread over the steps after it,
@@ -713,6 +710,7 @@ __device__ __forceinline__ void hbm_walk(const LevelArgs& A, const Tile& D, uint
   ln.lo = st;
   ln.hi = st + nc;
   ln.nown = nown;
+  ln.look = true;
 }
 
 // The preemption rule of src/simulate.cpp:990-1009 in its closed form: a
@@ -722,38 +720,75 @@ __device__ __forceinline__ void hbm_walk(const LevelArgs& A, const Tile& D, uint
 // an entry that repeats its predecessor's value dropped; then the later
 // lanes' minimum (one suffix minimum over the wavefront) and the chunk's end
 // (candidates at or above hi_rel belong to the next chunk) cut the list from
-// the end.  Look-back candidates below lo_rel only pre-empt.
+// the end.  Look-back candidates below lo_rel only pre-empt: a lane has some
+// only where the tile has events before the chunk.
+//
+// Without them the step has no branch: the last kept entry `last` holds both
+// the running minimum and the value to compare with, and a candidate that is
+// not kept writes `last` once more where it stands.  Seven VALU instructions a
+// candidate; with the two conditions as branches a tile's pass took 6,080 cycles
+// of its 29,600 (200,000 cells at gap 500 ps).
 template <typename SP>
 __device__ __forceinline__ void keep_entries(const LevelArgs& A, Lane<SP>& ln, bool halo_lane) {
   SP q = ln.hi, jp = ln.hi;
-  uint32_t rm = 0xFFFFFFFFu, lastv = 4u, left = (uint32_t)(ln.hi - ln.lo);
-  const uint32_t lo_w = A.lo_rel << 2;
-  auto take = [&](uint32_t e) {
-    if (e < rm) {
-      rm = e & ~3u;
-      if (e >= lo_w) {
-        const uint32_t v = e & 3u;
-        jp -= v != lastv ? 1 : 0;
-        *jp = e;
-        lastv = v;
-      }
+  uint32_t rm = 0xFFFFFFFFu, left = (uint32_t)(ln.hi - ln.lo);
+  // four reads in flight; `ahead`: the next four before this four's steps
+  // (their words lie below those that the steps write)
+  auto pass = [&](auto& take, auto ahead) {
+    uint32_t e4[4];
+    auto read4 = [&](uint32_t n) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e4[i] = (uint32_t)i < n ? q[-1 - i] : kWordInf;
+    };
+    if (decltype(ahead)::value) read4(4);
+    while (left >= 4) {
+      if (!decltype(ahead)::value) read4(4);
+      uint32_t t4[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) t4[i] = e4[i];
+      q -= 4;
+      left -= 4;
+      if (decltype(ahead)::value) read4(4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) take(t4[i]);
+    }
+    if (left) {
+      if (!decltype(ahead)::value) read4(left);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) take((uint32_t)i < left ? e4[i] : kWordInf);
     }
   };
-  while (left >= 4) {
-    uint32_t e4[4];  // four reads in flight
-#pragma unroll
-    for (int i = 0; i < 4; ++i) e4[i] = q[-1 - i];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) take(e4[i]);
-    q -= 4;
-    left -= 4;
-  }
-  if (left) {
-    uint32_t e4[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) e4[i] = (uint32_t)i < left ? q[-1 - i] : kWordInf;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) take(e4[i]);
+  // (reading ahead may read words below the lane's: inputs, in LDS)
+  constexpr bool kLds = std::is_same<SP, lds_u32*>::value;
+  if (!kLds || ln.look) {
+    uint32_t lastv = 4u;
+    const uint32_t lo_w = A.lo_rel << 2;
+    auto take = [&](uint32_t e) {
+      if (e < rm) {
+        rm = e & ~3u;
+        if (e >= lo_w) {
+          const uint32_t v = e & 3u;
+          jp -= v != lastv ? 1 : 0;
+          *jp = e;
+          lastv = v;
+        }
+      }
+    };
+    pass(take, std::false_type{});
+  } else {
+    // (the first candidate is below 0xFFFFFFFC, and its value is not that of the
+    // initial `last`; a lane without candidates writes nothing)
+    const bool some = left != 0;
+    uint32_t last = ~q[-1] | 0xFFFFFFFCu;
+    auto take = [&](uint32_t e) {
+      const bool kept = e < (last & ~3u);
+      const bool other = ((e ^ last) & 3u) != 0u;
+      jp -= kept && other ? 1 : 0;
+      last = kept ? e : last;
+      *jp = last;
+    };
+    pass(take, std::true_type{});
+    rm = some ? last & ~3u : 0xFFFFFFFFu;
   }
   const uint32_t hi_w = A.hi_rel == 0xFFFFFFFFu ? 0xFFFFFFFFu : A.hi_rel << 2;
   const uint32_t cut = min(wave_min_after(rm), hi_w);
@@ -765,16 +800,15 @@ __device__ __forceinline__ void keep_entries(const LevelArgs& A, Lane<SP>& ln, b
 }
 
 // Join the lanes' lists (a list that starts with the value before it drops
-// that entry), store the tile's entries at dst, sum the SAIF durations
-// between them (32 bits per lane: times < 2^30; the lanes' intervals are
-// disjoint pieces of the tile's span, so the sums fit too) and write the tile
-// summary.  out_cap: words of the tile's output region (never reached for
-// time-ordered inputs; entries beyond it are dropped, with ERR_ORDER).
-// `before_stores` runs just before the first store.
+// that entry), store the tile's entries at dst and write the tile summary.
+// (The SAIF durations between them are summed where the entries are copied,
+// one wavefront instruction for 64 of them: here it was one for as many as the
+// lanes have at the same place of their lists.)  out_cap: words of the tile's
+// output region (never reached for time-ordered inputs; entries beyond it are
+// dropped, with ERR_ORDER).  `before_stores` runs just before the first store.
 template <typename SP, typename F>
 __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const Lane<SP>& ln,
-                                          glb_u32* dst, uint32_t out_cap, unsigned long long w_start,
-                                          unsigned long long w_end, F&& before_stores) {
+                                          glb_u32* dst, uint32_t out_cap, F&& before_stores) {
   const int lane = threadIdx.x;
   const uint32_t n = (uint32_t)(ln.hi - ln.lo);
   const uint32_t e_first = n ? ln.lo[0] : 0u, e_last = n ? ln.hi[-1] : 0u;
@@ -785,29 +819,16 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
   const uint32_t mine = n - dup;
   const uint32_t incl = wave_scan(mine);
   const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
-  uint32_t ft = 0, lt = 0;  // the tile's first and last entries
-  if (mask) {
-    ft = __builtin_amdgcn_readlane(e_first, __ffsll((long long)mask) - 1);
-    lt = __builtin_amdgcn_readlane(e_last, 63 - __clzll((long long)mask));
+  uint32_t first = 0, last = 0;  // the tile's first and last entries
+  const uint64_t with = __ballot(mine > 0);
+  if (with) {
+    first = __builtin_amdgcn_readlane(e_first, __ffsll((long long)with) - 1);
+    last = __builtin_amdgcn_readlane(e_last, 63 - __clzll((long long)with));
   }
-  const uint32_t s32 = (uint32_t)min(w_start, 0x7FFFFFFFull);
-  const uint32_t e32 = (uint32_t)min(w_end, 0x7FFFFFFFull);
+  const uint32_t ev = wave_sum(ln.nown);
   const uint32_t w = min(incl - mine, out_cap);
-  uint32_t a0 = 0, a3 = 0;
-  uint32_t pv = below ? prev & 3u : 4u;
-  uint32_t pt = max(min((below ? prev : e_first) >> 2, e32), s32);
-  auto add = [&](uint32_t e) {
-    const uint32_t t = max(min(e >> 2, e32), s32), len = t - pt;
-    a0 += pv == 0u ? len : 0u;
-    a3 += pv == 3u ? len : 0u;
-    pv = e & 3u;
-    pt = t;
-  };
   before_stores();
-  if (n) {
-    // the interval before the lane's first entry, which is not stored again
-    // when it repeats the value before it
-    add(e_first);
+  if (mine) {
     // (the tile's region is uniform: lanes add 32-bit offsets to it)
     auto to = [&](uint32_t q) { return (glb_u32*)((__attribute__((address_space(1))) char*)dst + q); };
     uint32_t dp = 4 * w;
@@ -815,41 +836,24 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
     SP p = ln.lo + dup;
     // whole groups of four: four reads in flight, one store
     while (left >= 4) {
-      uint32_t e4[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) e4[q] = p[q];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) add(e4[q]);
-      *(glb_u32x4*)to(dp) = u32x4{e4[0], e4[1], e4[2], e4[3]};
+      *(glb_u32x4*)to(dp) = u32x4{p[0], p[1], p[2], p[3]};
       dp += 16;
       p += 4;
       left -= 4;
     }
-    // the rest; repeating the last entry adds nothing
-    if (left) {
-      uint32_t e4[3];
+    uint32_t e4[3];
 #pragma unroll
-      for (int q = 0; q < 3; ++q) e4[q] = (uint32_t)q < left ? p[q] : e_last;
+    for (int q = 0; q < 3; ++q) e4[q] = (uint32_t)q < left ? p[q] : 0u;
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        add(e4[q]);
-        if ((uint32_t)q < left) *to(dp + 4 * q) = e4[q];
-      }
-    }
+    for (int q = 0; q < 3; ++q)
+      if ((uint32_t)q < left) *to(dp + 4 * q) = e4[q];
   }
-  const uint32_t t0 = wave_sum(a0), t1 = wave_sum(a3);
-  const uint32_t ev = wave_sum(ln.nown);
   if (lane == 0) {
     TileOut o;
     o.cnt = min(total, out_cap);
     if (total > out_cap) atomicOr((unsigned int*)(A.scal + S_ERR), ERR_ORDER);
-    o.ft = ft >> 2;
-    o.lt = lt >> 2;
-    o.flags = out_flags(ft & 3u, lt & 3u, mask ? 1u : 0u);
-    o.t0 = t0;
-    o.t1 = t1;
-    // the intervals between the tile's entries add up to its span
-    o.tx = max(min(lt >> 2, e32), s32) - max(min(ft >> 2, e32), s32) - t0 - t1;
+    o.first = first;
+    o.last = last;
     o.ev = ev;
     A.tout[tk] = o;
   }
@@ -935,8 +939,6 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
     const bool more_tiles = tn < ntiles;
     const uint32_t dwn = more_tiles ? desc_word(A.tiles + tn) : 0u;
     if (more_tiles && tn + 1 >= bend) draw();
-    const ChunkWin* W = A.cwin + D.job;
-    const unsigned long long w_start = W->lo, w_end = W->hi;
     lds_fence();
     bool staged = false;  // the next tile's loads are on their way
     auto finish = [&](auto& ln) {
@@ -948,7 +950,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       const bool halo = D.xend != 0 && lane == kLanes - 1;
       keep_entries(A, ln, halo);
       if (halo) ln.nown = 0;
-      emit_tile(A, tk, ln, scratch + D.scr, D.out_cap, w_start, w_end, [&] {
+      emit_tile(A, tk, ln, scratch + D.scr, D.out_cap, [&] {
         if (staged) {
           wait_vm();
           put_sentinels(Dn);
@@ -975,6 +977,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       Lane<uint32_t*> ln;
       ln.lo = ln.hi = A.ovf;
       ln.nown = 0;
+      ln.look = true;
       if (D.id() < W_COUNT) {
         const unsigned long long need = (unsigned long long)D.words + kStackSlack;
         unsigned long long base = 0;
@@ -1503,8 +1506,8 @@ __global__ __launch_bounds__(256) void k_tile_desc(
 // Per gate, in tile order: join the tiles' outputs (a tile whose first
 // entry repeats the last value before it drops that entry), place each
 // tile's output (offset inside the gate, bit 31: first entry dropped), and
-// add up the SAIF durations: inside tiles, between tiles, and from the last
-// entry to the window end.  Eight lanes per gate, 8 tiles per step: each
+// add up the SAIF durations between tiles and from the last entry to the window
+// end (the copy adds those inside tiles).  Eight lanes per gate, 8 tiles per step: each
 // lane takes the last value and time of the nearest non-empty tile before
 // it (a ballot of the non-empty lanes, then a shuffle; the step's first
 // non-empty tile takes them from the previous step), the offsets are an
@@ -1560,9 +1563,9 @@ __global__ __launch_bounds__(8 * kJoinGates) void k_join(JoinArgs A, TailArgs T)
       const uint64_t t = t0 + c + l8;
       TileOut S = {};
       if (in) S = A.tout[t];
-      const bool ne = in && ((S.flags >> 4) & 1u);
+      const bool ne = S.cnt != 0;
       const uint32_t mask = (uint32_t)(__ballot(ne) >> sh8) & 0xFFu;
-      const uint32_t my_lv = (S.flags >> 2) & 3u, my_lt = S.lt, my_fv = S.flags & 3u;
+      const uint32_t my_lv = S.last & 3u, my_lt = S.last >> 2, my_fv = S.first & 3u, my_ft = S.first >> 2;
       // nearest non-empty tile below this lane in the step, if any
       const uint32_t below = mask & ((1u << l8) - 1u);
       const int pl = below ? 31 - __clz((int)below) : 0;
@@ -1573,12 +1576,9 @@ __global__ __launch_bounds__(8 * kJoinGates) void k_join(JoinArgs A, TailArgs T)
       if (ne) {
         skip = (p_has && p_lv == my_fv) ? 1u : 0u;
         mine = S.cnt - skip;
-        if (p_has) saif_acc(acc, p_lv, p_lt, S.ft, start, end);
-        acc[0] += S.t0;
-        acc[1] += S.t1;
-        acc[2] += S.tx;
+        if (p_has) saif_acc(acc, p_lv, p_lt, my_ft, start, end);
         // the tile's first entry against the previous tile's last value
-        tc += (p_has && is_toggle(p_lv, my_fv) && S.ft > W.tc_lo && S.ft <= W.tc_hi) ? 1u : 0u;
+        tc += (p_has && is_toggle(p_lv, my_fv) && my_ft > W.tc_lo && my_ft <= W.tc_hi) ? 1u : 0u;
       }
       // an instance counts the events of its tiles with entries; the tiles of a
       // wide gate count as one
@@ -1672,8 +1672,10 @@ __global__ __launch_bounds__(8 * kJoinGates) void k_join(JoinArgs A, TailArgs T)
 // Copy every tile's joined output from the scratch into the gate's dense
 // waveform in the pool (one wavefront per tile, coalesced); the gate's first
 // tile also copies the gate's tail (state and look-back entries, moved to
-// this chunk's time base) to the front.  The first nplan blocks plan the next
-// level.
+// this chunk's time base) to the front.  On its way every entry adds its SAIF
+// durations (and toggles when asked) to its net's record: the copy waits for
+// memory, and the walk that left the entries waits for its VALU.  The first nplan
+// blocks plan the next level.
 __global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, PlanArgs next,
                                                  uint32_t nplan) {
   __shared__ uint64_t sh[4];
@@ -1707,37 +1709,63 @@ __global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, Plan
       }
     }
     const TileOut S = tout[t];
-    if (!((S.flags >> 4) & 1u)) continue;
+    if (!S.cnt) continue;
     const uint32_t off = tile_off[t] & 0x7FFFFFFFu, skip = tile_off[t] >> 31;
     const uint32_t n = S.cnt - skip;
     const glb_u32* src = scratch + (((uint64_t)D.scr_hi << 32) | D.scr_lo) + skip;
     uint32_t* dst = pool + gate + off;
+    const ChunkWin W = A.cwin[D.job];
+    // SAIF durations between the tile's entries, in 32 bits (times < 2^30; a
+    // lane's intervals are disjoint pieces of the tile's span): an entry ends the
+    // interval of the one before it, which is the lane's below, and lane 0's is
+    // the last of the 64 entries before
+    const uint32_t s32 = (uint32_t)min(W.lo, 0x7FFFFFFFull);
+    const uint32_t e32 = (uint32_t)min(W.hi, 0x7FFFFFFFull);
+    uint32_t carry = S.first, a0 = 0, a3 = 0, tc = 0;
+    auto add = [&](uint32_t e) {
+      const uint32_t p = dpp<0x138>(e, carry);
+      carry = __builtin_amdgcn_readlane(e, 63);
+      const uint32_t len = max(min(e >> 2, e32), s32) - max(min(p >> 2, e32), s32), pv = p & 3u;
+      a0 += pv == 0u ? len : 0u;
+      a3 += pv == 3u ? len : 0u;
+      // SAIF TC: 0<->1 changes (the first entry against the tile before is the join's)
+      if (A.count_tc) {
+        const unsigned long long tt = e >> 2;
+        tc += (is_toggle(pv, e & 3u) && tt > W.tc_lo && tt <= W.tc_hi) ? 1u : 0u;
+      }
+    };
     // four loads in flight per lane before their stores: the copy of a tile
     // waits for memory about n / 256 times instead of n / 64
-    uint32_t q = lane;
-    for (; q + 192 < n; q += 256) {
-      const uint32_t a0 = src[q], a1 = src[q + 64], a2 = src[q + 128], a3 = src[q + 192];
-      dst[q] = a0;
-      dst[q + 64] = a1;
-      dst[q + 128] = a2;
-      dst[q + 192] = a3;
-    }
-    for (; q < n; q += 64) dst[q] = src[q];
-    if (A.count_tc) {
-      // SAIF TC inside the tile: 0<->1 changes between its consecutive
-      // entries (the first entry against the previous tile is k_join's)
-      const glb_u32* e = src - skip;
-      const ChunkWin W = A.cwin[D.job];
-      uint32_t c = 0;
-      for (uint32_t q = lane + 1; q < S.cnt; q += 64) {
-        const uint32_t a = e[q - 1], b = e[q];
-        const unsigned long long tt = b >> 2;
-        c += (is_toggle(a & 3u, b & 3u) && tt > W.tc_lo && tt <= W.tc_hi) ? 1u : 0u;
+    uint32_t q = 0;
+    for (; q + 256 <= n; q += 256) {
+      uint32_t a[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = src[q + 64 * i + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dst[q + 64 * i + lane] = a[i];
+        add(a[i]);
       }
-      c = wave_sum(c);
-      if (lane == 0 && c)
-        atomicAdd(A.saif + (uint64_t)kSaifWords * D.out_net + 3, (unsigned long long)c);
     }
+    if (q < n) {  // the rest; lanes behind the end repeat the last entry, which adds nothing
+      uint32_t a[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a[i] = q + 64 * i + lane < n ? src[q + 64 * i + lane] : S.last;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (q + 64 * i >= n) break;
+        if (q + 64 * i + lane < n) dst[q + 64 * i + lane] = a[i];
+        add(a[i]);
+      }
+    }
+    const uint32_t t0 = wave_sum(a0), t1 = wave_sum(a3);
+    // the intervals between the tile's entries add up to its span
+    const uint32_t span = max(min(S.last >> 2, e32), s32) - max(min(S.first >> 2, e32), s32);
+    if (A.count_tc) tc = wave_sum(tc);
+    const uint32_t v = lane == 0 ? t0 : (lane == 1 ? t1 : (lane == 2 ? span - t0 - t1 : tc));
+    if (lane < (int)kSaifWords && v)
+      atomicAdd(A.saif + (uint64_t)kSaifWords * D.out_net + lane, (unsigned long long)v);
   }
 }
 
