@@ -1722,9 +1722,7 @@ __global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, Plan
     const uint32_t s32 = (uint32_t)min(W.lo, 0x7FFFFFFFull);
     const uint32_t e32 = (uint32_t)min(W.hi, 0x7FFFFFFFull);
     uint32_t carry = S.first, a0 = 0, a3 = 0, tc = 0;
-    auto add = [&](uint32_t e) {
-      const uint32_t p = dpp<0x138>(e, carry);
-      carry = __builtin_amdgcn_readlane(e, 63);
+    auto add = [&](uint32_t p, uint32_t e) {
       const uint32_t len = max(min(e >> 2, e32), s32) - max(min(p >> 2, e32), s32), pv = p & 3u;
       a0 += pv == 0u ? len : 0u;
       a3 += pv == 3u ? len : 0u;
@@ -1734,30 +1732,35 @@ __global__ __launch_bounds__(256) void k_compact(CompactArgs A, TailArgs T, Plan
         tc += (is_toggle(pv, e & 3u) && tt > W.tc_lo && tt <= W.tc_hi) ? 1u : 0u;
       }
     };
-    // four loads in flight per lane before their stores: the copy of a tile
-    // waits for memory about n / 256 times instead of n / 64
-    uint32_t q = 0;
-    for (; q + 256 <= n; q += 256) {
-      uint32_t a[4];
+    // four entries a lane in one access, four accesses in flight: a tile of
+    // 1,000 entries waits for memory once.  (The copy is bound by those waits: a
+    // wavefront's chain is descriptor, place, entries.)
+    const uint32_t n4 = n / 4;
+    for (uint32_t b = 0; b < n4; b += 256) {
+      const uint32_t left = n4 - b;
+      u32x4 w[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = src[q + 64 * i + lane];
+      for (uint32_t i = 0; i < 4; ++i)
+        if (64 * i + lane < left) w[i] = ((const glb_u32x4*)src)[b + 64 * i + lane];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        dst[q + 64 * i + lane] = a[i];
-        add(a[i]);
+      for (uint32_t i = 0; i < 4; ++i) {
+        if (64 * i >= left) break;
+        const bool in = 64 * i + lane < left;
+        if (in) *(u32x4*)(dst + 4 * (b + 64 * i + lane)) = w[i];
+        // (lanes behind the end repeat the entry before, which adds nothing)
+        const uint32_t p = dpp<0x138>(w[i].w, carry);
+        carry = __builtin_amdgcn_readlane(w[i].w, min(left - 64 * i, 64u) - 1);
+        const uint32_t e0 = in ? w[i].x : p, e1 = in ? w[i].y : p, e2 = in ? w[i].z : p;
+        add(p, e0);
+        add(e0, e1);
+        add(e1, e2);
+        add(e2, in ? w[i].w : p);
       }
     }
-    if (q < n) {  // the rest; lanes behind the end repeat the last entry, which adds nothing
-      uint32_t a[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        a[i] = q + 64 * i + lane < n ? src[q + 64 * i + lane] : S.last;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (q + 64 * i >= n) break;
-        if (q + 64 * i + lane < n) dst[q + 64 * i + lane] = a[i];
-        add(a[i]);
-      }
+    if (n & 3u) {
+      const uint32_t e = 4 * n4 + lane < n ? src[4 * n4 + lane] : S.last;
+      if (4 * n4 + lane < n) dst[4 * n4 + lane] = e;
+      add(dpp<0x138>(e, carry), e);
     }
     const uint32_t t0 = wave_sum(a0), t1 = wave_sum(a3);
     // the intervals between the tile's entries add up to its span
