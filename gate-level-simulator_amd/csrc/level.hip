@@ -882,9 +882,11 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   // keep its tables in LDS).  The rest is drawn by ticket in batches of B, so
   // that workgroups with slow tiles take fewer and the level's tail stays
   // short.  One counter serves about 70 M tickets a second, which held levels of
-  // short waveforms (one or two tiles a gate) to 70 M tiles a second: four
-  // counters hand out every fourth batch each, and a workgroup whose counter
-  // has run out goes on to the next.
+  // short waveforms (one or two tiles a gate) to 70 M tiles a second: up to four
+  // counters hand out every fourth batch each, to a quarter of the workgroups
+  // each.  (A workgroup whose counter had run out went on to the other three,
+  // one wait after the other and 6,000 tickets a level that found nothing: of
+  // 200,000 quiet cells' 26,200 cycles a tile, 2,300.)
   const uint64_t n_run = max(1ull, (unsigned long long)(ntiles / 2 / gridDim.x));
   const uint64_t t_drawn = n_run * gridDim.x;  // first tile handed out by ticket
   const uint32_t B = (uint32_t)max(
@@ -892,23 +894,18 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   uint64_t tk = (uint64_t)blockIdx.x * n_run;
   if (tk >= ntiles) return;
   uint64_t bend = min(tk + n_run, ntiles);  // end of the current run or batch
-  uint32_t counter = (blockIdx.x >> 3) & (kTickets - 1), used_up = 0;
-  unsigned long long drawn = 0;  // lane 0: the drawn ticket
+  const uint32_t counters = min(kTickets, (gridDim.x + 7) / 8);  // every one has workgroups
+  const uint32_t counter = (blockIdx.x >> 3) % counters;
+  // lane 0: the ticket on its way; and the last one that has arrived.  It is
+  // taken from `drawn` where the tile's loads are waited for: taken where it is
+  // used, after the tile's stores, it would wait for those too.
+  unsigned long long drawn = 0;
+  uint64_t ticket = 0;
   auto draw = [&] {
     if (lane == 0 && t_drawn < ntiles) drawn = atomicAdd(A.ticket + counter * kTicketStride, 1ull);
   };
-  auto drawn_batch = [&]() -> uint64_t {  // first tile of the drawn batch (ntiles: none left)
-    while (t_drawn < ntiles && used_up < kTickets) {
-      counter = uni(counter);
-      used_up = uni(used_up);
-      const uint64_t i = uni((uint64_t)drawn);
-      const uint64_t t = t_drawn + (counter + kTickets * i) * B;
-      if (t < ntiles) return t;
-      if (++used_up == kTickets) break;
-      counter = (counter + 1) & (kTickets - 1);
-      draw();
-    }
-    return ntiles;
+  auto drawn_batch = [&]() -> uint64_t {  // first tile of the drawn batch (at least ntiles: none left)
+    return t_drawn + (counter + counters * ticket) * B;
   };
   if (tk + 1 >= bend) draw();
   uint32_t dw = desc_word(A.tiles + tk);
@@ -922,6 +919,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       put_sentinels(D);
     }
   }
+  ticket = uni((uint64_t)drawn);
   for (;;) {
     tk = uni(tk);
     tab_g = uni(tab_g);
@@ -932,7 +930,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
     uint64_t tn = tk + 1;
     if (tn >= bend) {
       tn = drawn_batch();
-      bend = min(tn + B, ntiles);
+      bend = tn + B < ntiles ? tn + B : ntiles;
     }
     tn = uni(tn);
     bend = uni(bend);
@@ -951,10 +949,9 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
       keep_entries(A, ln, halo);
       if (halo) ln.nown = 0;
       emit_tile(A, tk, ln, scratch + D.scr, D.out_cap, [&] {
-        if (staged) {
-          wait_vm();
-          put_sentinels(Dn);
-        }
+        wait_vm();
+        ticket = uni((uint64_t)drawn);
+        if (staged) put_sentinels(Dn);
       });
     };
     if (fits) {
@@ -994,6 +991,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
         if (bad) atomicOr(err, ERR_ORDER);
       }
       finish(ln);
+      wait_vm();
     }
     lds_fence();
     wave_hbm += fits ? 0u : 1u;
