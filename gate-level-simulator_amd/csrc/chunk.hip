@@ -55,8 +55,7 @@ __global__ void k_saif_accum(const GateRec* __restrict__ gates, uint32_t ng,
 }
 
 // SAIF of the resident stimulus signals over the whole window (once per
-// run; they are never re-computed per chunk): one wavefront per signal, the
-// net is X before its first entry, an entry holds until the next one (the
+// run; they are never re-computed per chunk): one block per signal, the net is X before its first entry, an entry holds until the next one (the
 // last until the window end), src/simulate.cpp:102-163.
 __device__ __forceinline__ void saif_add64(unsigned long long* acc, uint32_t v, uint64_t a,
                                            uint64_t b, uint64_t start, uint64_t end) {
@@ -68,38 +67,53 @@ __device__ __forceinline__ void saif_add64(unsigned long long* acc, uint32_t v, 
   else acc[2] += len;
 }
 
-__global__ void k_saif_stim(const uint64_t* __restrict__ store, const uint64_t* __restrict__ soff,
-                            const uint32_t* __restrict__ slen, const uint32_t* __restrict__ snet,
-                            const uint32_t* __restrict__ sjob, uint32_t ns,
-                            unsigned long long* __restrict__ saif,
-                            const unsigned long long* __restrict__ win,
-                            unsigned long long* __restrict__ wtot) {
-  const uint32_t s = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-  const int lane = threadIdx.x & 63;
-  if (s >= ns) return;
+// (One wavefront per signal waited for its loads 31 times over 2,000 events: 25
+// us, three of a hundred of a run of 2,000 cells.)
+__global__ __launch_bounds__(256) void k_saif_stim(
+    const uint64_t* __restrict__ store, const uint64_t* __restrict__ soff,
+    const uint32_t* __restrict__ slen, const uint32_t* __restrict__ snet,
+    const uint32_t* __restrict__ sjob, unsigned long long* __restrict__ saif,
+    const unsigned long long* __restrict__ win, unsigned long long* __restrict__ wtot) {
+  __shared__ unsigned long long s_acc[4][4];
+  const uint32_t s = blockIdx.x;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const uint64_t start = win[2 * sjob[s]], end = win[2 * sjob[s] + 1];
   const uint64_t* w = store + soff[s];
   const uint32_t n = slen[s];
   unsigned long long acc[4] = {0, 0, 0, 0};
-  if (lane == 0) saif_add64(acc, 1u, 0, n ? (w[0] >> 2) : end, start, end);
-  for (uint32_t q = lane; q < n; q += 64) {
-    const uint64_t e = w[q], t = e >> 2;
-    const uint64_t tn = q + 1 < n ? (w[q + 1] >> 2) : (end > t ? end : t);
-    saif_add64(acc, (uint32_t)(e & 3u), t, tn, start, end);
-    // stimulus waveforms may repeat a value (scalars are not de-duplicated)
-    if (q > 0 && is_toggle((uint32_t)(w[q - 1] & 3u), (uint32_t)(e & 3u)) && t > start && t <= end)
-      ++acc[3];
+  if (threadIdx.x == 0) saif_add64(acc, 1u, 0, n ? (w[0] >> 2) : end, start, end);
+  constexpr uint32_t kAhead = 4;  // rounds whose loads are in flight together
+  for (uint64_t q0 = threadIdx.x; q0 < n; q0 += 256 * kAhead) {
+    uint64_t p[kAhead], e[kAhead], x[kAhead];
+#pragma unroll
+    for (uint32_t i = 0; i < kAhead; ++i) {
+      const uint64_t q = q0 + 256 * i;
+      e[i] = q < n ? w[q] : 0;
+      p[i] = q < n && q > 0 ? w[q - 1] : 0;
+      x[i] = q + 1 < n ? w[q + 1] : 0;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kAhead; ++i) {
+      const uint64_t q = q0 + 256 * i;
+      if (q >= n) break;
+      const uint64_t t = e[i] >> 2;
+      const uint64_t tn = q + 1 < n ? (x[i] >> 2) : (end > t ? end : t);
+      saif_add64(acc, (uint32_t)(e[i] & 3u), t, tn, start, end);
+      // stimulus waveforms may repeat a value (scalars are not de-duplicated)
+      if (q > 0 && is_toggle((uint32_t)(p[i] & 3u), (uint32_t)(e[i] & 3u)) && t > start && t <= end)
+        ++acc[3];
+    }
   }
-  for (int k = 0; k < 4; ++k)
+  for (int k = 0; k < 4; ++k) {
     for (int o = 32; o > 0; o >>= 1) acc[k] += __shfl_down(acc[k], o, 64);
-  if (lane == 0) {
-    unsigned long long* d = saif + (uint64_t)kSaifWords * snet[s];
-    d[0] = acc[0];
-    d[1] = acc[1];
-    d[2] = acc[2];
-    d[3] = acc[3];
-    wtot[snet[s]] = n;
+    if (lane == 0) s_acc[wid][k] = acc[k];
   }
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    const uint32_t k = threadIdx.x;
+    saif[(uint64_t)kSaifWords * snet[s] + k] = s_acc[0][k] + s_acc[1][k] + s_acc[2][k] + s_acc[3][k];
+  }
+  if (threadIdx.x == 0) wtot[snet[s]] = n;
 }
 
 static inline unsigned nblk(uint64_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
@@ -140,7 +154,7 @@ hipError_t launch_saif_stim(const uint64_t* store, const uint64_t* soff, const u
                             unsigned long long* saif, const unsigned long long* win,
                             unsigned long long* wtot, hipStream_t st) {
   if (ns == 0) return hipSuccess;
-  k_saif_stim<<<nblk(ns, 4), 256, 0, st>>>(store, soff, slen, snet, sjob, ns, saif, win, wtot);
+  k_saif_stim<<<ns, 256, 0, st>>>(store, soff, slen, snet, sjob, saif, win, wtot);
   return hipGetLastError();
 }
 

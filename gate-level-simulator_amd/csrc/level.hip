@@ -1821,28 +1821,27 @@ __global__ __launch_bounds__(256) void k_stim_plan(const uint64_t* __restrict__ 
   }
 }
 
-// One wavefront per stimulus signal: state entry at relative time 0, then
-// the range in relative time (abs - lb + 1 >= 1); sets the net's waveform.
+// One block per stimulus signal: state entry at relative time 0, then the range
+// in relative time (abs - lb + 1 >= 1); sets the net's waveform.
 __global__ __launch_bounds__(256) void k_stim_copy(
     const uint64_t* __restrict__ store, const uint64_t* __restrict__ soff,
-    const uint32_t* __restrict__ snet, uint32_t ns, uint64_t lb, const uint64_t* __restrict__ cnt,
+    const uint32_t* __restrict__ snet, uint64_t lb, const uint64_t* __restrict__ cnt,
     const uint32_t* __restrict__ first, const uint64_t* __restrict__ loc,
     const uint64_t* __restrict__ part, uint32_t* __restrict__ pool, uint64_t* __restrict__ woff,
     uint32_t* __restrict__ wlen, const uint64_t* __restrict__ scal) {
   if (scal[S_TRIP]) return;
-  const uint32_t s = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-  const int lane = threadIdx.x & 63;
-  if (s >= ns) return;
+  const uint32_t s = blockIdx.x;
   const uint64_t base = part[s / kStimSignals] + loc[s];
   const uint64_t* w = store + soff[s] + first[s];
   const uint32_t n = (uint32_t)(cnt[s] - 1);
   uint32_t* d = pool + base;
-  if (lane == 0) {
+  if (threadIdx.x == 0) {
     d[0] = first[s] > 0 ? (uint32_t)(w[-1] & 3u) : 1u;  // X before the first entry
     woff[snet[s]] = base;
     wlen[snet[s]] = n + 1;
   }
-  for (uint32_t q = lane; q < n; q += 64) {
+#pragma unroll 4
+  for (uint64_t q = threadIdx.x; q < n; q += 256) {
     const uint64_t e = w[q];
     d[1 + q] = (uint32_t)((((e >> 2) - lb + 1) << 2) | (e & 3u));
   }
@@ -2039,8 +2038,7 @@ hipError_t launch_stim_copy(const uint64_t* store, const uint64_t* soff, const u
                             const uint64_t* loc, const uint64_t* part, uint32_t* pool, uint64_t* woff,
                             uint32_t* wlen, const uint64_t* scal, hipStream_t st) {
   if (ns == 0) return hipSuccess;
-  k_stim_copy<<<nblk(ns, 4), 256, 0, st>>>(store, soff, snet, ns, lb, cnt, first, loc, part, pool, woff,
-                                           wlen, scal);
+  k_stim_copy<<<ns, 256, 0, st>>>(store, soff, snet, lb, cnt, first, loc, part, pool, woff, wlen, scal);
   return hipGetLastError();
 }
 
