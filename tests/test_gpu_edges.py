@@ -1,0 +1,87 @@
+"""Counts at which the kernels' rounds end, against the oracle: signals of as
+many events as a block takes in one round (256 threads, four rounds in flight)
+and one less or more, tiles of 64, 256 and 1,024 words (the copy of a tile's
+entries takes 64 accesses of four, four of them in flight), and tiles handed
+out to so few workgroups that only some of the ticket counters are used."""
+import re
+import sys
+
+import pytest
+
+import gls
+import oracle_bind
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = (1, 3, 255, 256, 257, 1023, 1024, 1025, 4097)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = gls.Context(0)
+    yield c
+    c.close()
+
+
+def cut_vcd(src, dst):
+    """Keeps the first LENGTHS[k] changes of the k-th signal."""
+    head, body = open(src).read().split("$enddefinitions $end\n")
+    left, out = {}, []
+    for tok in body.split():
+        if tok[0] in "01xzXZ":
+            sig = tok[1:]
+            if sig not in left:
+                left[sig] = LENGTHS[len(left) % len(LENGTHS)]
+            left[sig] -= 1
+            if left[sig] < 0:
+                continue
+        out.append(tok)
+    with open(dst, "w") as f:
+        f.write(head + "$enddefinitions $end\n" + "\n".join(out) + "\n")
+
+
+@pytest.fixture(scope="module")
+def case(tmp_path_factory):
+    t = str(tmp_path_factory.mktemp("edges"))
+    d = gls.Design.generate(3, 811, 60, 3, len(LENGTHS))
+    paths = [t + "/" + n for n in ("lib.vlib", "n.gv", "n.sdf", "s.vcd")]
+    d.write(*paths[:3])
+    gls.Stimulus.generate(d, 812, 60000, 10.0, 0.05).write_vcd(t + "/all.vcd")
+    cut_vcd(t + "/all.vcd", paths[3])
+    window = (7001, 59000)
+    return d, gls.Stimulus.from_vcd(paths[3]), window, oracle_bind.run(*paths, *window, t)
+
+
+def toggles(wave, on, off):
+    return sum(1 for (_, p), (t, v) in zip(wave, wave[1:]) if {p, v} == {0, 3} and on < t <= off)
+
+
+def check(r, want, what):
+    assert r.stats()["n_events"] == want["n_events"], what
+    assert r.waves_hash() == want["waves_hash"], what
+    assert re.sub(r" \(TC \d+\)", "", r.saif_text()) == want["saif"], what
+
+
+@pytest.mark.parametrize("seg,chunk", [(0, 0), (1, 0), (4, 0), (16, 0), (16, 17011)])
+def test_round_ends(ctx, case, seg, chunk):
+    print("round ends", seg, chunk, flush=True)
+    sys.stdout.flush()
+    d, s, (on, off), want = case
+    r = ctx.simulate(d, s, on, off, keep_waves=True, saif_tc=True, seg_events=seg, chunk_ps=chunk)
+    check(r, want, (seg, chunk))
+    names = re.findall(r"^      \((\S+)\n         \(T0", r.saif_text(), re.M)
+    assert len(names) > 20
+    for net in names:
+        assert r.net_toggles(net) == toggles(r.waveform(net), on, off), net
+    r.close()
+
+
+@pytest.mark.parametrize("blocks", [1, 7, 8, 9, 17, 25, 40])
+def test_few_workgroups(ctx, case, blocks):
+    print("workgroups", blocks, flush=True)
+    sys.stdout.flush()
+    d, s, (on, off), want = case
+    r = ctx.simulate(d, s, on, off, keep_waves=True, seg_events=1, level_blocks=blocks)
+    assert r.stats()["tiles"] > 8 * blocks
+    check(r, want, blocks)
+    r.close()
