@@ -19,27 +19,35 @@
 //      (keep_entries);
 //   4. the lanes' lists are joined (a list that starts with the value before
 //      it drops that entry) and stored into the level scratch, and lane 0
-//      writes the tile summary (count, first/last value and time, SAIF
-//      durations) (emit_tile).
+//      writes the tile summary (count, first and last entry, gate events)
+//      (emit_tile).
 //   The next tile's loads are issued when the walk no longer reads its inputs.
 //
-// What bounds the walk: VALU issue, at 67% of the SIMDs' cycles with two
-// wavefronts per SIMD (LDS-limited).  1.39 VALU wave-instructions per gate
-// event on the 200k-cell configuration (gap 500 ps): about 22 (fan-in 2) to 34
-// (fan-in 4) a step and 43 steps a tile where 31 would do if the lanes' shares
-// were exact; 1,200 a tile besides.  With delays looked up by an edge class and
-// per-input event and edge bits computed each step, a halo walked by every lane,
-// the candidate lists joined by a wavefront scan of 3-word aggregates, 16 bytes a
-// store fewer and all tiles handed out by one ticket counter it was 2.04, and
-// that configuration took 154 ms over 10 Mps where it now takes 99 ms (the 2M-cell
-// configuration over 2 Mps: 615 -> 405 ms; 5- and 6-input cells, walked by one
-// thread a gate before, 6,007 cells over 150 kps: 122 -> 0.7 ms).
-// k_gate_carry: per gate, joins its tiles in order (a tile whose first entry
-//   repeats the value before it drops that entry), places them, and finishes
-//   the gate's SAIF record.
-// k_compact: copies each tile's joined entries into the gate's dense
-//   waveform in the pool (coalesced), so the pool holds exactly the outputs,
-//   and counts SAIF toggles inside tiles when asked.
+// What bounds the walk: VALU issue (61% of the SIMDs' cycles) and, with two
+// wavefronts per SIMD (LDS-limited), the latency of LDS reads (bank conflicts take
+// 38% of the LDS's cycles: lanes read their inputs at unrelated places).  On the
+// 200k-cell configuration (gap 500 ps) it issues 0.97 VALU and 0.29 scalar
+// wave-instructions per gate event, and a tile of 1,940 events takes 24,000 cycles
+// of a wavefront: 4,700 to the lanes' bounds, 10,800 in the steps (41 of 22 to 34
+// VALU instructions, where 31 would do if the lanes' shares were exact), 3,800
+// for preemption, 2,000 to issue the next tile's loads, 900 waiting for them, 1,800
+// to store.  Per run over 10 Mps (2M cells over 2 Mps):
+//   154 ms (615)  delays by edge class and event bits each step, a halo walked by
+//                 every lane, a wavefront scan of 3-word aggregates
+//    99 ms (405)  table lookups, equal lane shares, one lane's halo
+//    96 ms (395)  lane starts from exact ranks, lighter level ends
+//    87 ms        descriptor fields as scalars
+//    79 ms (323)  preemption without branches, SAIF durations left to the copy
+//    76 ms (310)  no wait for a tile's stores, a ticket counter of its own
+// Tried and slower: tiles of 16, 24 or 28 words a lane at the more workgroups a CU
+// that they allow, less LDS around a tile's words (tiles in HBM cost 40 us each),
+// searches that start in a window around the even split.
+// k_join: per gate, joins its tiles in order (a tile whose first entry repeats
+//   the value before it drops that entry), places them, and adds the SAIF
+//   durations between them.
+// k_compact: copies each tile's joined entries into the gate's dense waveform
+//   in the pool (coalesced), so the pool holds exactly the outputs, and sums the
+//   SAIF durations (and toggles when asked) inside tiles.
 //
 // Event rules: src/simulate.cpp:919-1201 (Calculate, AddDelay, CheckDelay),
 // src/simulate.cpp:1365-1506 (Process, GetValueAt).
@@ -860,13 +868,16 @@ __device__ __forceinline__ void emit_tile(const LevelArgs& A, uint64_t tk, const
 }
 
 // Persistent, software-pipelined walk kernel.  Tiles are independent (no
-// tile waits for another): workgroup b starts with tile b and then draws
-// tickets for the next one.  The next tile's descriptor and ticket are on the
+// tile waits for another): a workgroup walks a run of consecutive tiles and then
+// draws batches by ticket.  The next tile's descriptor and ticket are on the
 // way during the walk; its inputs are staged into LDS from the end of the
 // walk on, behind the current tile's stacks, and waited for before the current
 // tile's first store (a later wait would include the stores).  A static
 // round-robin schedule left the workgroups that drew many tiles too long for
-// LDS as a long tail (14% slower on the 200k-cell workload).
+// LDS as a long tail (14% slower on the 200k-cell workload).  Whatever a tile
+// leaves in flight on either path is waited for on that path: what may be in
+// flight anywhere, the compiler waits for at the next tile's start, together with
+// this one's stores.
 __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   // dynamic LDS, A.lds_words: tables, inputs, ..., stacks (walk_lds_need)
   extern __shared__ uint32_t s_dyn[];
