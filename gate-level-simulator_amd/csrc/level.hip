@@ -249,6 +249,10 @@ __device__ __forceinline__ bool tile_fits(const LevelArgs& A, const Tile& D) {
   return D.id() < W_COUNT &&
          D.dt_words() + D.tt_words() + 2 * D.words + 8 * D.k() + kStackSlack <= A.lds_words;
 }
+// A tile whose inputs fit, but not its stacks beside them.
+__device__ __forceinline__ bool inputs_fit(const LevelArgs& A, const Tile& D) {
+  return D.id() < W_COUNT && D.dt_words() + D.tt_words() + D.words + 8 * D.k() <= A.lds_words;
+}
 // First word behind the tile's input ranges.
 __device__ __forceinline__ uint32_t in_end(const Tile& D) {
   return D.dt_words() + D.tt_words() + D.words + 8 * D.k();
@@ -602,13 +606,14 @@ __device__ __forceinline__ Lane<lds_u32*> lane_walk(const LevelArgs& A, const Ti
   return ln;
 }
 
-// The same walk for a tile too long for LDS: inputs read from HBM, the
-// gate's tables too, stacks in the overflow buffer, lanes at equal shares of
-// the leader's words.  Rare (a tile's words are kept to its LDS share), so it
+// The same walk for a tile too long for LDS: stacks in the overflow buffer,
+// tables read from HBM, inputs too unless they fit LDS by themselves (`lds`: where
+// they are staged), lanes at equal shares of the leader's words.  Rare (a tile's words are kept to its LDS share), so it
 // is one form for every gate.  Writes that would leave the lane's buffer
 // (inputs out of order) land on its last word and set bad.
-__device__ __forceinline__ void hbm_walk(const LevelArgs& A, const Tile& D, uint32_t* stk,
-                                      uint32_t stk_words, Lane<uint32_t*>& ln, uint32_t& bad) {
+__device__ __forceinline__ void hbm_walk(const LevelArgs& A, const Tile& D, const uint32_t* lds,
+                                         uint32_t* stk, uint32_t stk_words, Lane<uint32_t*>& ln,
+                                         uint32_t& bad) {
   const uint32_t lane = threadIdx.x;
   const uint32_t k = D.k(), id = D.id();
   const bool more = D.xend != 0;
@@ -618,7 +623,7 @@ __device__ __forceinline__ void hbm_walk(const LevelArgs& A, const Tile& D, uint
   uint32_t nl = 0;
 #pragma unroll
   for (uint32_t j = 0; j < kWideK; ++j) {
-    in[j] = A.pool + D.src(j);
+    in[j] = lds ? lds + D.at(j) : A.pool + D.src(j);
     if (j == D.lead()) {
       lead = in[j];
       nl = D.n[j];
@@ -923,7 +928,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
   uint32_t tab_g = 0xFFFFFFFFu;  // gate whose tables are in LDS
   {
     const Tile D = tile_of(dw);
-    if (tile_fits(A, D)) {
+    if (inputs_fit(A, D)) {
       stage_tile(A, D, true, s_dyn);
       tab_g = D.g;
       wait_vm();
@@ -997,7 +1002,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
           // stay in time order) and the run reports the error
           if (lane == 0) atomicOr(err, ERR_OVERFLOW);
         } else {
-          hbm_walk(A, D, A.ovf + base, (uint32_t)need, ln, bad);
+          hbm_walk(A, D, inputs_fit(A, D) ? s_dyn : nullptr, A.ovf + base, (uint32_t)need, ln, bad);
         }
         if (bad) atomicOr(err, ERR_ORDER);
       }
@@ -1008,7 +1013,7 @@ __global__ __launch_bounds__(kLanes) void k_level(LevelArgs A) {
     wave_hbm += fits ? 0u : 1u;
     if (!more_tiles) break;
     const Tile Dn = tile_of(dwn);
-    if (tile_fits(A, Dn)) {
+    if (inputs_fit(A, Dn)) {
       if (!staged) {
         stage_tile(A, Dn, Dn.g != tab_g, s_dyn);
         wait_vm();

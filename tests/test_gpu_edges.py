@@ -85,3 +85,33 @@ def test_few_workgroups(ctx, case, blocks):
     assert r.stats()["tiles"] > 8 * blocks
     check(r, want, blocks)
     r.close()
+
+
+@pytest.mark.parametrize("burst", [900, 1400, 1700, 2900, 3400, 5000])
+def test_tiles_too_long_for_lds(ctx, burst, tmp_path):
+    """Half of the signals change all along, the others `burst` times in a short
+    stretch: at one word a lane its tiles hold more than LDS does, with their
+    stacks (about 1,500 words) or without them (about 3,000)."""
+    print("too long", burst, flush=True)
+    sys.stdout.flush()
+    t = str(tmp_path)
+    d = gls.Design.generate(3, 813, 40, 2, 8)
+    paths = [t + "/" + n for n in ("lib.vlib", "n.gv", "n.sdf", "s.vcd")]
+    d.write(*paths[:3])
+    gls.Stimulus.generate(d, 814, 1000, 10.0, 0.05).write_vcd(t + "/all.vcd")
+    head, body = open(t + "/all.vcd").read().split("$enddefinitions $end\n")
+    events = []
+    for k, sig in enumerate(sorted({tok[1:] for tok in body.split() if tok[0] in "01xzXZ"})):
+        n, at, gap = (1100, 10 + k, 50) if k % 2 == 0 else (burst, 20000 + k, 3)
+        events += [(at + gap * i, sig, "01"[(i + k) & 1]) for i in range(n)]
+    events.sort()
+    with open(paths[3], "w") as f:
+        f.write(head + "$enddefinitions $end\n")
+        for at, sig, v in events:
+            f.write("#%d\n%s%s\n" % (at, v, sig))
+    s = gls.Stimulus.from_vcd(paths[3])
+    want = oracle_bind.run(*paths, 100, 60000, t)
+    r = ctx.simulate(d, s, 100, 60000, keep_waves=True, seg_events=1)
+    assert r.stats()["tiles_hbm"] > 0 or burst < 1500
+    check(r, want, burst)
+    r.close()
