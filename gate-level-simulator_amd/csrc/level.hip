@@ -8,8 +8,8 @@
 //   1. the tile's input ranges (one event before the tile for the starting
 //      values, a D_max look-ahead halo after it) and the gate's two tables
 //      are copied into LDS with direct-to-LDS loads, each range followed by an
-//      INF sentinel (tiles too long for LDS read HBM instead and keep their
-//      stacks in the overflow buffer);
+//      INF sentinel (tiles too long for LDS keep their stacks in the overflow
+//      buffer and, where even their inputs do not fit, read HBM instead);
 //   2. the tile's words are cut into equal shares, one per lane (lane_bounds);
 //      every lane merges its share in time order and looks every event up:
 //      a truth byte by the input values, then a delay word by the gate's old
@@ -608,9 +608,13 @@ __device__ __forceinline__ Lane<lds_u32*> lane_walk(const LevelArgs& A, const Ti
 
 // The same walk for a tile too long for LDS: stacks in the overflow buffer,
 // tables read from HBM, inputs too unless they fit LDS by themselves (`lds`: where
-// they are staged), lanes at equal shares of the leader's words.  Rare (a tile's words are kept to its LDS share), so it
-// is one form for every gate.  Writes that would leave the lane's buffer
-// (inputs out of order) land on its last word and set bad.
+// they are staged), lanes at equal shares of the leader's words.  Rare (a tile's
+// words are kept to its LDS share), so it is one form for every gate, and what it
+// reads may be either kind of memory.  A step that waited for HBM made such a tile
+// last about 40 us, a quarter of a level of 200,000 quiet cells, of which one in
+// three has one (its walks 6.39 -> 6.15 ms a run with the inputs in LDS).  Writes
+// that would leave the lane's buffer (inputs out of order) land on its last word
+// and set bad.
 __device__ __forceinline__ void hbm_walk(const LevelArgs& A, const Tile& D, const uint32_t* lds,
                                          uint32_t* stk, uint32_t stk_words, Lane<uint32_t*>& ln,
                                          uint32_t& bad) {
