@@ -94,11 +94,13 @@ int level_max_blocks(uint32_t lds_words);
 // words twice (inputs and stacks) and 4 KiB for the gate's tables, the halo and
 // the spread of a tile's words around their mean; at least what the largest
 // tables (fan-in 6) need and at most what a CU gives one workgroup.  A tile that
-// does not fit reads HBM (0.07% of the tiles of the 200k-cell configuration; a
-// `seg` beyond every LDS size sends all of them there).  At the default of 32
-// it is 20 KiB, eight workgroups a CU: with 24 (nine) the 200k-cell
-// configuration's walk took 108 ms instead of 101, the fixed work of a tile
-// outweighing the ninth.
+// does not fit keeps its stacks in memory (50 of 14.2 M tiles of the 200k-cell
+// configuration; a `seg` beyond every LDS size sends all of them there).  At the
+// default of 32 it is 20 KiB, eight workgroups a CU: with 22 (ten) the 200k-cell
+// configuration's walk takes 75.2 ms instead of 75.7, and what is done per tile
+// beside it 38 ms instead of 32; with 24 (nine) and 28 (eight) the walk is slower
+// too.  3 KiB around the tiles' words instead of 4 made a hundred times as many
+// tiles too long (81 ms).
 static uint32_t walk_lds_words(uint32_t seg) {
   return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(128ull * seg + 1024, 3328), 33792);
 }

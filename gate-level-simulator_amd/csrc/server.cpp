@@ -119,10 +119,13 @@ void Server::worker(int slot) {
   hip_check(hipSetDevice(device_), "hipSetDevice");
   hipStream_t stream = nullptr;
   hip_check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
+  bool ran = false, more = false;
   for (;;) {
     std::vector<Rec*> group;
     {
       std::unique_lock<std::mutex> lk(mu_);
+      if (ran) --busy_;
+      ran = false;
       for (;;) {
         if (stop_ && queue_.empty()) break;
         // queued jobs cancelled or past their deadline leave the queue first
@@ -149,7 +152,8 @@ void Server::worker(int slot) {
         // a job may pass the head of the queue only while the head does not
         // fit.  A job that can never fit fails and the scan goes on past it.
         // With batching, later queued jobs without a deadline that also fit
-        // join the first one's run.
+        // join the first one's run when no other worker is free for them (so
+        // which jobs share a run does not hang on which thread wakes first).
         uint64_t taken = 0;
         for (auto it = queue_.begin(); it != queue_.end();) {
           Rec* c = jobs_[*it].get();
@@ -174,7 +178,7 @@ void Server::worker(int slot) {
             group.push_back(c);
             taken += need;
             it = queue_.erase(it);
-            if (group.size() >= std::max<uint32_t>(1, opt_.max_batch)) break;
+            if (group.size() >= std::max<uint32_t>(1, opt_.max_batch) || busy_ + 1 < opt_.max_running) break;
             continue;
           }
           if (group.empty()) {
@@ -198,7 +202,11 @@ void Server::worker(int slot) {
       peak_bytes_ = std::max(peak_bytes_, in_use_);
       peak_running_ = std::max(peak_running_, running_);
       for (Rec* r : group) r->info.overlap = running_ - 1;
+      ++busy_;
+      ran = true;
+      more = !queue_.empty();
     }
+    if (more) cv_work_.notify_all();
     if (group.size() > 1 && run_group(group, stream)) {
       cv_done_.notify_all();
       cv_work_.notify_all();

@@ -144,6 +144,7 @@ class Server {
   std::map<uint64_t, std::unique_ptr<Rec>> jobs_;
   uint64_t next_id_ = 1, in_use_ = 0, peak_bytes_ = 0;
   uint32_t running_ = 0, peak_running_ = 0;
+  uint32_t busy_ = 0;  // workers that run something
   bool stop_ = false;
   std::vector<std::thread> workers_;
   std::chrono::steady_clock::time_point t0_;
