@@ -107,6 +107,9 @@ uint64_t Server::submit(RunInst inst, std::shared_ptr<const Stimulus> keep, doub
     }
     id = next_id_++;
     r->id = id;
+    uint32_t taken = busy_;  // workers that run something or have a job waiting for them
+    for (uint64_t q : queue_) taken += jobs_[q]->alone ? 1u : 0u;
+    r->alone = taken < opt_.max_running;
     jobs_[id] = std::move(r);
     queue_.push_back(id);
   }
@@ -119,13 +122,11 @@ void Server::worker(int slot) {
   hip_check(hipSetDevice(device_), "hipSetDevice");
   hipStream_t stream = nullptr;
   hip_check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
-  bool ran = false, more = false;
+  bool more = false;
   for (;;) {
     std::vector<Rec*> group;
     {
       std::unique_lock<std::mutex> lk(mu_);
-      if (ran) --busy_;
-      ran = false;
       for (;;) {
         if (stop_ && queue_.empty()) break;
         // queued jobs cancelled or past their deadline leave the queue first
@@ -152,8 +153,9 @@ void Server::worker(int slot) {
         // a job may pass the head of the queue only while the head does not
         // fit.  A job that can never fit fails and the scan goes on past it.
         // With batching, later queued jobs without a deadline that also fit
-        // join the first one's run when no other worker is free for them (so
-        // which jobs share a run does not hang on which thread wakes first).
+        // join the first one's run, unless a worker was free for one of them
+        // when it came (which jobs share a run does not hang on which thread
+        // wakes first).
         uint64_t taken = 0;
         for (auto it = queue_.begin(); it != queue_.end();) {
           Rec* c = jobs_[*it].get();
@@ -173,12 +175,12 @@ void Server::worker(int slot) {
             cv_done_.notify_all();
             continue;
           }
-          const bool joinable = group.empty() || (!c->has_deadline && !group[0]->has_deadline);
+          const bool joinable = group.empty() || (!c->has_deadline && !group[0]->has_deadline && !c->alone);
           if (joinable && in_use_ + taken + need <= opt_.device_budget) {
             group.push_back(c);
             taken += need;
             it = queue_.erase(it);
-            if (group.size() >= std::max<uint32_t>(1, opt_.max_batch) || busy_ + 1 < opt_.max_running) break;
+            if (group.size() >= std::max<uint32_t>(1, opt_.max_batch) || group[0]->alone) break;
             continue;
           }
           if (group.empty()) {
@@ -203,7 +205,7 @@ void Server::worker(int slot) {
       peak_running_ = std::max(peak_running_, running_);
       for (Rec* r : group) r->info.overlap = running_ - 1;
       ++busy_;
-      ran = true;
+      group.back()->last = true;
       more = !queue_.empty();
     }
     if (more) cv_work_.notify_all();
@@ -342,6 +344,7 @@ void Server::finish(Rec* r, int status, uint64_t events, uint64_t bytes, uint32_
   r->saif = std::move(saif);
   in_use_ -= r->reserve;
   --running_;
+  if (r->last) --busy_;
 }
 
 void Server::fail_queued(Rec* r) {

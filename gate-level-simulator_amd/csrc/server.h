@@ -115,6 +115,8 @@ class Server {
     uint64_t pool_words = 0, reserve = 0;
     std::vector<uint64_t> saif;
     std::chrono::steady_clock::time_point t_submit, t_start, t_end, deadline;
+    bool alone = false;  // a worker was free for it when it came
+    bool last = false;   // of the jobs that its worker took with it
     bool has_deadline = false;
     std::atomic<bool> stop{false};  // cancel asked for a running job
   };

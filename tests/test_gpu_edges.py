@@ -115,3 +115,28 @@ def test_tiles_too_long_for_lds(ctx, burst, tmp_path):
     assert r.stats()["tiles_hbm"] > 0 or burst < 1500
     check(r, want, burst)
     r.close()
+
+
+@pytest.mark.parametrize("workers,max_batch", [(1, 4), (3, 4), (4, 1)])
+def test_jobs_that_find_a_free_worker_run_alone(ctx, workers, max_batch):
+    """Every job's results are its own run's; the first jobs, one a worker, run
+    by themselves however fast they are submitted, so that their counts too are
+    those of a run of their own."""
+    print("workers", workers, max_batch, flush=True)
+    sys.stdout.flush()
+    d = gls.Design.generate(1, 815, 900, 12, 20)
+    ss = [gls.Stimulus.generate(d, 820 + i, 40000, 150.0, 0.02) for i in range(7)]
+    alone = []
+    for s in ss:
+        r = ctx.simulate(d, s, 0, 40001)
+        alone.append((r.saif_text(), r.stats()["n_events"]))
+        r.close()
+    srv = gls.Server(ctx, max_running=workers, max_batch=max_batch)
+    for _ in range(3):
+        jobs = [srv.submit(d, s, 0, 40001) for s in ss]
+        for i, j in enumerate(jobs):
+            assert srv.wait(j) == 0
+            assert srv.saif_text(j) == alone[i][0], i
+            if i < workers:
+                assert srv.info(j)["n_events"] == alone[i][1], i
+    srv.close()
